@@ -78,7 +78,7 @@ def listed():
 # a stable timestep per planet and row length (dt scales with the spacing)
 _DT = {
     ea.HELD_SUAREZ: {16: 900, 32: 600, 64: 400, 128: 200},
-    ea.VENUS_LIKE: {16: 300, 32: 300, 64: 200, 128: 100, 256: 60, 512: 30},
+    ea.VENUS_LIKE: {16: 300, 32: 300, 64: 200, 128: 100, 256: 30, 512: 15},
     ea.JUPITER_LIKE: {16: 60, 32: 60, 64: 60, 128: 60, 256: 40, 512: 30, 1024: 15},
     ea.SATURN_LIKE: {16: 60, 32: 60, 64: 60, 128: 60, 256: 40, 512: 25},
     ea.HOT_JUPITER: {64: 30, 128: 30, 256: 30, 512: 30, 1024: 30},
@@ -108,7 +108,7 @@ def draw(rng):
         case["adv_nonmass"] = 1
     if rng.random() < 0.15:
         case["pv_scheme"] = 1
-    if rng.random() < 0.1:
+    if planet in (ea.JUPITER_LIKE, ea.SATURN_LIKE) and rng.random() < 0.2:
         case["pgrad_traditional"] = 1
     if rng.random() < 0.2:
         case["nudiv"] = 0.1
