@@ -22,6 +22,25 @@ namespace epic {
 
 constexpr int KMAX = 66;  // nk <= 64
 
+// A pointer to device memory held in a descriptor.  A generic pointer that a
+// kernel loads from memory makes every access through it a flat instruction,
+// which counts as a vector-memory and an LDS access at once and is waited
+// for by waiting for everything in flight.  Held as a pointer to global
+// memory (device code only; the host sees a plain pointer of the same size)
+// the accesses are global instructions, and a kernel waits only for the load
+// it needs next.
+template <class T>
+struct gptr {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __attribute__((address_space(1))) T *raw;
+#else
+  T *raw;
+#endif
+  __host__ __device__ __forceinline__ T *get() const { return (T *)raw; }
+  __host__ __device__ __forceinline__ operator T *() const { return get(); }
+  __host__ __device__ __forceinline__ T *operator->() const { return get(); }
+};
+
 struct MemberDyn {
   int it0, itm1, itm2;  // IT_ZERO, IT_MINUS1, IT_MINUS2
   int itime;            // value of grid.itime during the next step
@@ -57,35 +76,35 @@ struct MemberDesc {
   int adv_akima[3];
   // PV averaging of uv_core and gz_from_u: 1 Arakawa-Lamb (1981), 0 Sadourny
   int pv_al81;
-  const double *snd_x, *snd_y, *snd_d, *cool_x, *cool_y, *cool_d;
+  gptr<const double> snd_x, snd_y, snd_d, cool_x, cool_y, cool_d;
   // host-libm tables: cos(lat), cos(lat)^4 per h-row J, cos(lon) per column I
-  const double *coslat_h, *coslat4_h, *coslon_h;
+  gptr<const double> coslat_h, coslat4_h, coslon_h;
   // reciprocals formed once on the host (the same IEEE quotients the
   // kernels would form per cell): 1/m on v-rows J = 0..nj+1 (0 at the
   // poles, as the meridional advection takes it) and 1/n on h-rows 0..nj
-  const double *minv_v, *ninv_h;
+  gptr<const double> minv_v, ninv_h;
   // per layer K >= k_sigma: THETA2's interval in the sigmatheta table and its width
-  const int *t2_kay;
-  const double *t2_h;
+  gptr<const int> t2_kay;
+  gptr<const double> t2_h;
   // 1-D metrics and tables
-  const double *lat, *lon, *m, *n, *mn, *f, *g, *rln, *rlt, *sgth, *dsgth, *dsgth_inv, *h_min, *t_sponge;
-  const double *mn_inv, *hl_h, *hl_pv, *hcx, *hcy, *hcz, *vcx, *vcy, *vcz;
-  const double *tw_f, *tw_i, *tr_f, *tr_i;  // four1 / realft twiddles, forward and inverse
-  const float *tw_f32, *tw_i32, *tr_f32, *tr_i32;
-  const int *rows_h, *rows_v;
-  const int *rflag_h, *rflag_v;  // 1 where row J is in the filter band
+  gptr<const double> lat, lon, m, n, mn, f, g, rln, rlt, sgth, dsgth, dsgth_inv, h_min, t_sponge;
+  gptr<const double> mn_inv, hl_h, hl_pv, hcx, hcy, hcz, vcx, vcy, vcz;
+  gptr<const double> tw_f, tw_i, tr_f, tr_i;  // four1 / realft twiddles, forward and inverse
+  gptr<const float> tw_f32, tw_i32, tr_f32, tr_i32;
+  gptr<const int> rows_h, rows_v;
+  gptr<const int> rflag_h, rflag_v;  // 1 where row J is in the filter band
   // state and diagnostics
-  double *U, *V, *DUDT, *DVDT, *HDRY, *THETA, *P3, *P2, *THETA2, *H3, *T2, *T3, *RHO2, *RHO3;
-  double *EXNER3, *GZ3, *MONT3, *HEAT3, *PV3, *DIV, *W3, *DZDT3, *USPIN, *GZS;
-  double *RI2;  // formed on demand (epic_engine_read, the drop-in's write-back)
+  gptr<double> U, V, DUDT, DVDT, HDRY, THETA, P3, P2, THETA2, H3, T2, T3, RHO2, RHO3;
+  gptr<double> EXNER3, GZ3, MONT3, HEAT3, PV3, DIV, W3, DZDT3, USPIN, GZS;
+  gptr<double> RI2;  // formed on demand (epic_engine_read, the drop-in's write-back)
   // mixed mode: DUDT, DVDT are one FP64 plane (the current step's sum) and
   // DUDTf, DVDTf the three FP32 Adams-Bashforth history planes
-  float *DUDTf, *DVDTf;
+  gptr<float> DUDTf, DVDTf;
   // sA..sD: scratch, three 3-D copies each (the batched advection gives each
   // advected field its own copy; every other user takes the first)
-  double *gz, *sA, *sB, *sC, *sD, *unity, *old, *spl;
-  double *rowbuf;  // 8*(nj+3) doubles: zonal means and meridional profiles
-  MemberDyn *dyn;
+  gptr<double> gz, sA, sB, sC, sD, unity, old, spl;
+  gptr<double> rowbuf;  // 8*(nj+3) doubles: zonal means and meridional profiles
+  gptr<MemberDyn> dyn;
 };
 
 __device__ __forceinline__ size_t ix3(const MemberDesc &d, int K, int J, int I) {
@@ -483,10 +502,10 @@ template <> __device__ __forceinline__ float *fld_ptr_t<float>(const MemberDesc 
   switch (f) {
     case F_DUDT_T: return d.DUDTf + (size_t)d.dyn->it0 * d.N3;
     case F_DVDT_T: return d.DVDTf + (size_t)d.dyn->it0 * d.N3;
-    case F_SA: return reinterpret_cast<float *>(d.sA);
-    case F_SB: return reinterpret_cast<float *>(d.sB);
-    case F_SC: return reinterpret_cast<float *>(d.sC);
-    case F_SD: return reinterpret_cast<float *>(d.sD);
+    case F_SA: return reinterpret_cast<float *>(d.sA.get());
+    case F_SB: return reinterpret_cast<float *>(d.sB.get());
+    case F_SC: return reinterpret_cast<float *>(d.sC.get());
+    case F_SD: return reinterpret_cast<float *>(d.sD.get());
   }
   return nullptr;
 }

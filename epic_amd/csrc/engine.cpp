@@ -546,7 +546,7 @@ void member_plan(const epic_case *c, bool mixed, const epic_tables &T, MemberDes
   add(&d.P3, sizeof(double) * N3, c->p3, EPIC_F_P3);
   add(&d.USPIN, sizeof(double) * N3, c->u_spinup);
   add(&d.GZS, sizeof(double) * N2, c->gz_surface, EPIC_F_GZ_SURFACE);
-  struct { double **p; int f; } fields[] = {
+  struct { gptr<double> *p; int f; } fields[] = {
       {&d.HDRY, EPIC_F_HDRY},     {&d.P2, EPIC_F_P2},       {&d.THETA2, EPIC_F_THETA2}, {&d.H3, EPIC_F_H3},
       {&d.T2, EPIC_F_T2},         {&d.T3, EPIC_F_T3},       {&d.RHO2, EPIC_F_RHO2},     {&d.RHO3, EPIC_F_RHO3},
       {&d.EXNER3, EPIC_F_EXNER3}, {&d.GZ3, EPIC_F_GZ3},     {&d.MONT3, EPIC_F_MONT3},   {&d.HEAT3, EPIC_F_HEAT3},

@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   // update on the tile's rows: the FP64 field plus the flux divergence; sB
   // (the copy the zonal pass filters) in the flux type
   double *sA = d.sA + so + o;
-  T *sB = reinterpret_cast<T *>(d.sB) + so + o;
+  T *sB = reinterpret_cast<T *>(d.sB.get()) + so + o;
   for (int r = r0; r < MER_TJ; r += RS) {
     const int J = J0 + r;
     if (J > nj) break;
@@ -322,7 +322,7 @@ __global__ void __launch_bounds__(256) k_hsu_zonal(const MemberDesc *D, int mb, 
   // it (twice per cell, by the same expression)
   T *A = sh + (size_t)m.g * 3 * W;
   T *UV = A + W, *AP = A + 2 * W, *FF = UV;
-  const T *af = reinterpret_cast<const T *>(d.sB) + so + (size_t)K * d.N2;
+  const T *af = reinterpret_cast<const T *>(d.sB.get()) + so + (size_t)K * d.N2;
   const double ninv = d.ninv_h[J];
   const T mn = T(d.mn[2 * J + 1]), DT = T(d.dt);
   const T amin = (which == AV_HDRY) ? T(d.h_min[K]) : T(0.);
@@ -527,7 +527,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   }
   __syncthreads();
   double *sA = d.sA + so + o;
-  T *sB = reinterpret_cast<T *>(d.sB) + so + o;
+  T *sB = reinterpret_cast<T *>(d.sB.get()) + so + o;
   for (int r = r0; r < MER_TJ; r += RS) {
     const int J = J0 + r;
     if (J > nj) break;
@@ -554,7 +554,7 @@ __global__ void __launch_bounds__(256) k_ak_zonal(const MemberDesc *D, int mb, i
   T *sh = reinterpret_cast<T *>(sh_raw);
   const int ni = d.ni, W = ni + 2;
   T *A = sh + (size_t)m.g * 3 * W, *DL = A + W, *FF = A + 2 * W;
-  const T *af = reinterpret_cast<const T *>(d.sB) + so + (size_t)K * d.N2;
+  const T *af = reinterpret_cast<const T *>(d.sB.get()) + so + (size_t)K * d.N2;
   const double ninv = d.ninv_h[J];
   const T mn = T(d.mn[2 * J + 1]), DT = T(d.dt);
   auto wr = [ni](int I) { return I < 1 ? I + ni : (I > ni ? I - ni : I); };

@@ -644,7 +644,7 @@ __global__ void __launch_bounds__(256) k_d2dy2_cols(const MemberDesc *D, int mb,
   if (J0 > jmax) return;  // uniform per block (the grid covers the v rows)
   const int I = 1 + chunk * (int)blockDim.x + (int)threadIdx.x;
   const double *hh = fld_ptr(d, f) + (size_t)K * d.N2;
-  T *out = reinterpret_cast<T *>(d.sB) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
+  T *out = reinterpret_cast<T *>(d.sB.get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
   const double *cx = vg ? d.vcx : d.hcx, *cy = vg ? d.vcy : d.hcy, *cz = vg ? d.vcz : d.hcz;
   const T c2 = T(d.coef2), c4 = T(d.coef4);
   T w[TJ + 4];  // rows J0-2 .. J0+TJ+1
@@ -705,7 +705,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   const int J = live ? Jr : 0, ni = d.ni, vg = (kind == 1);
   T *x = lds + (size_t)m.g * 2 * ni, *work = x + ni;
   double *a = fld_ptr(d, f) + (size_t)K * d.N2;
-  T *dd = reinterpret_cast<T *>(src ? d.sC : d.sB) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
+  T *dd = reinterpret_cast<T *>((src ? d.sC : d.sB).get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
   const bool upd = live && J >= r.jbot && J <= d.nj;
   if (upd)
     for (int I = 1 + m.lane; I <= ni; I += m.stride) x[I - 1] = dd[ix2(d, J, I)];
@@ -742,8 +742,8 @@ __global__ void __launch_bounds__(256) k_d2dy2_pass(const MemberDesc *D, int mb,
   if (t >= (jmax + 1) * d.ni) return;
   const int J = t / d.ni, I = 1 + t - J * d.ni;
   const size_t o = (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
-  const T *hh = reinterpret_cast<const T *>(src ? d.sC : d.sB) + o;
-  T *out = reinterpret_cast<T *>(src ? d.sB : d.sC) + o;
+  const T *hh = reinterpret_cast<const T *>((src ? d.sC : d.sB).get()) + o;
+  T *out = reinterpret_cast<T *>((src ? d.sB : d.sC).get()) + o;
   const double *cx = vg ? d.vcx : d.hcx, *cy = vg ? d.vcy : d.hcy, *cz = vg ? d.vcz : d.hcz;
   int j0, j1, j2;
   if (J == 0) { j0 = 0; j1 = 1; j2 = 2; }
@@ -990,7 +990,7 @@ __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, i
   const bool live = Jr <= d.nj + 1;
   const int J = live ? Jr : 0, vg = (kind == 1);
   double *a = fld_ptr(d, f) + (size_t)K * d.N2;
-  const T *dd = reinterpret_cast<const T *>(d.sB) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
+  const T *dd = reinterpret_cast<const T *>(d.sB.get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
   const bool upd = live && J >= r.jbot && J <= d.nj;
   // the row of A and the row of D, both loads in flight together
   double v[4];

@@ -47,9 +47,9 @@ static inline dim3 grid2(int nJ, int nI, int nK, int nm) {
 // the current step's tendency plane (FP64) and the FP32 history ring
 __device__ __forceinline__ double *curU(const MemberDesc &d) { return d.DUDT; }
 __device__ __forceinline__ double *curV(const MemberDesc &d) { return d.DVDT; }
-__device__ __forceinline__ float *sAf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sA); }
-__device__ __forceinline__ float *sBf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sB); }
-__device__ __forceinline__ float *sCf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sC); }
+__device__ __forceinline__ float *sAf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sA.get()); }
+__device__ __forceinline__ float *sBf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sB.get()); }
+__device__ __forceinline__ float *sCf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sC.get()); }
 
 // ------------------------------------------------------------ tendencies
 // UH, VH, KIN (FP32 views of sA, sB, sC) on planes 1..nk-1 with zonal pads
