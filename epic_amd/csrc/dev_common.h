@@ -440,21 +440,44 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // s + a[0] + a[1] + ... + a[n-1] (or s - a[0] - a[1] - ...), accumulated left
-// to right as the reference's loops do; the loads are issued eight at a time
-// ahead of the additions so the chain waits on additions only.
+// to right as the reference's loops do.  The chain of additions bounds it,
+// and only if no load stands in the chain: eight values are added while the
+// next eight are on their way from LDS (the scheduling barriers keep the
+// loads in front of the additions they pass behind; left to itself the
+// compiler sinks them and the chain waits for every group).
 template <bool SUB = false, class T = double>
 __device__ __forceinline__ T seq_acc(const T *a, int n, T s = T(0)) {
   int i = 0;
+  if (n >= 8) {
+    T x[8], y[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = a[u];
+    for (; i + 24 <= n; i += 16) {
+#pragma unroll
+      for (int u = 0; u < 8; u++) y[u] = a[i + 8 + u];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 8; u++) s = SUB ? s - x[u] : s + x[u];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 8; u++) x[u] = a[i + 16 + u];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 8; u++) s = SUB ? s - y[u] : s + y[u];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) s = SUB ? s - x[u] : s + x[u];
+    i += 8;
+  }
   for (; i + 8 <= n; i += 8) {
-    const T v0 = a[i], v1 = a[i + 1], v2 = a[i + 2], v3 = a[i + 3];
-    const T v4 = a[i + 4], v5 = a[i + 5], v6 = a[i + 6], v7 = a[i + 7];
-    if (SUB) { s -= v0; s -= v1; s -= v2; s -= v3; s -= v4; s -= v5; s -= v6; s -= v7; }
-    else { s += v0; s += v1; s += v2; s += v3; s += v4; s += v5; s += v6; s += v7; }
+    T x[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = a[i + u];
+#pragma unroll
+    for (int u = 0; u < 8; u++) s = SUB ? s - x[u] : s + x[u];
   }
-  for (; i < n; i++) {
-    if (SUB) s -= a[i];
-    else s += a[i];
-  }
+  for (; i < n; i++) s = SUB ? s - a[i] : s + a[i];
   return s;
 }
 

@@ -800,13 +800,19 @@ void L_merid_hv(hipStream_t s, const Bucket &b, const FieldSet &fs) {
 
 // zonal hyperviscosity: a block holds RB = 4*RW consecutive (K,J) rows in
 // LDS, wavefront w owning rows w + 4u (u < RW), each lane the points
-// I = 1 + lane + 64q (q < NQ) of them, whose second differences it keeps in
-// registers; the row array is rewritten with them for the zonal means, which
-// are sequential sums, as the reference sums them, lane r of the first
-// wavefront summing row r (one chain of additions serves RB rows).  One row
-// array per row (not two) lets a CU hold twice the rows, i.e. run twice the
-// serial chains side by side.  Rows are strided by an odd number of doubles
-// so the lanes of the serial phase fall in distinct LDS banks.
+// I = 1 + lane + 64q (q < NQ) of them, which stay in registers (the field is
+// read and written once); the row array is rewritten with their second
+// differences for the zonal means, which are sequential sums, as the reference sums them, lane r of the
+// first wavefront summing row r (one chain of additions serves RB rows).
+// One row array per row (not two) lets a CU hold twice the rows, i.e. run
+// twice the serial chains side by side.  Rows are strided by an odd number
+// of doubles so the lanes of the serial phase fall in distinct LDS banks.
+// A row is its wavefront's own except to the lane that sums it: block
+// barriers stand on both sides of the sums only.
+// NQ > 1 means rows of exactly 64 NQ points: no point is tested against ni,
+// so all of a lane's loads are in flight together (with the test each load,
+// of LDS and of memory, was waited for in its own branch: 1346 -> 841 us a
+// step at 1024x512x64 with the pipelined sums of seq_acc).
 template <class T, int RW, int NQ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_zonal_hv(const MemberDesc *D, int mb, int nm, FieldSet fs) {
   SET_MEMBER;
@@ -822,10 +828,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   T *meanv = X + (size_t)RB * WS;
   double *a = fld_ptr(d, f) + (size_t)K * d.N2;
   const int J0 = blockIdx.x * RB, jlast = d.nj + 1;
+  const bool on = NQ > 1 || lane < ni;  // lane holds points of the row
+  double v[RW][NQ];
+  // rows past the last one take its values and are not stored
+#pragma unroll
   for (int u = 0; u < RW; u++) {
-    const int t = wv + 4 * u, J = J0 + t;
-    T *x = X + t * WS;
-    for (int I = lane; I < W; I += 64) x[I] = (J <= jlast) ? T(a[ix2(d, J, I)]) : T(0.);
+    const double *row = a + ix2(d, min(J0 + wv + 4 * u, jlast), 0);
+    T *x = X + (wv + 4 * u) * WS;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) v[u][q] = on ? row[1 + lane + 64 * q] : 0.;
+    if (lane < 2) x[lane ? ni + 1 : 0] = T(row[lane ? ni + 1 : 0]);
   }
   // m (or m0 poleward of LAT0) of each row; pass p's coefficient of the
   // row is (coef[2(p+1)] mm) mm, as the reference forms it
@@ -836,74 +848,64 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     const bool taper = fabs(d.lat[2 * Jc + r.jh]) > 45.;
     mm[u] = taper ? d.m0z : d.m[2 * Jc + r.jh];
   }
-  __syncthreads();
-  T y[RW][NQ];
+#pragma unroll
+  for (int u = 0; u < RW; u++)
+    if (on)
+#pragma unroll
+      for (int q = 0; q < NQ; q++) X[(wv + 4 * u) * WS + 1 + lane + 64 * q] = T(v[u][q]);
+  wave_sync();
   for (int pass = 0; pass < np; pass++) {
     const double cp = hv_coef(d, pass);
+    if (on)
 #pragma unroll
-    for (int u = 0; u < RW; u++) {
-      const T *x = X + (wv + 4 * u) * WS;
-      const T dcu = T(cp * mm[u] * mm[u]);
+      for (int u = 0; u < RW; u++) {
+        T *x = X + (wv + 4 * u) * WS + 1 + lane, y[NQ];
+        const T dcu = T(cp * mm[u] * mm[u]);
 #pragma unroll
-      for (int q = 0; q < NQ; q++) {
-        const int I = 1 + lane + 64 * q;
-        if (I <= ni) y[u][q] = dcu * (x[I - 1] - T(2.) * x[I] + x[I + 1]);
+        for (int q = 0; q < NQ; q++) y[q] = dcu * (x[64 * q - 1] - T(2.) * x[64 * q] + x[64 * q + 1]);
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < NQ; q++) x[64 * q] = y[q];
       }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < RW; u++) {
-      T *x = X + (wv + 4 * u) * WS;
-#pragma unroll
-      for (int q = 0; q < NQ; q++) {
-        const int I = 1 + lane + 64 * q;
-        if (I <= ni) x[I] = y[u][q];
-      }
-    }
     __syncthreads();
     if (wv == 0 && lane < RB) meanv[lane] = seq_acc(X + lane * WS + 1, ni) / T(ni);
     __syncthreads();
     // every point (and the zonal pads, copies of points ni and 1) less the
-    // mean; the last pass's result stays in registers
-#pragma unroll
-    for (int u = 0; u < RW; u++) {
-      const int t = wv + 4 * u;
-      T *x = X + t * WS;
-      const T fm = meanv[t];
-#pragma unroll
-      for (int q = 0; q < NQ; q++) {
-        const int I = 1 + lane + 64 * q;
-        if (I <= ni) {
-          y[u][q] -= fm;
-          if (pass < np - 1) {
-            x[I] = y[u][q];
-            if (I == ni) x[0] = y[u][q];
-            if (I == 1) x[ni + 1] = y[u][q];
-          }
-        }
-      }
-    }
-    __syncthreads();
-    if (hv_nu(d, pass) == 0.) continue;
-    // an order with nu > 0: A += DT*sign*D on the rows of the range (sign
-    // -1 for del^4 and del^8, +1 for del^6), then pads
+    // mean; an order with nu > 0: A += DT*sign*D on the rows of the range
+    // (sign -1 for del^4 and del^8, +1 for del^6)
+    const bool more = pass < np - 1;
     const double sign = (pass & 1) ? -1. : 1.;
 #pragma unroll
     for (int u = 0; u < RW; u++) {
       const int J = J0 + wv + 4 * u;
-      if (J > jlast) break;
-      const bool upd = J >= r.jbot && J <= d.nj;
+      const T fm = meanv[wv + 4 * u];
+      T *x = X + (wv + 4 * u) * WS + 1 + lane, y[NQ];
 #pragma unroll
-      for (int q = 0; q < NQ; q++) {
-        const int I = 1 + lane + 64 * q;
-        if (I > ni) break;
-        double v = a[ix2(d, J, I)];
-        if (upd) v += d.dt * sign * (double)y[u][q];
-        a[ix2(d, J, I)] = v;
-        if (I == ni) a[ix2(d, J, 0)] = v;
-        if (I == 1) a[ix2(d, J, ni + 1)] = v;
+      for (int q = 0; q < NQ; q++) y[q] = on ? x[64 * q] - fm : T(0.);
+      if (more && on) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) x[64 * q] = y[q];
+        if (1 + lane + 64 * (NQ - 1) == ni) X[(wv + 4 * u) * WS] = y[NQ - 1];
+        if (lane == 0) X[(wv + 4 * u) * WS + ni + 1] = y[0];
+      }
+      if (hv_nu(d, pass) != 0. && J >= r.jbot && J <= d.nj) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) v[u][q] += d.dt * sign * (double)y[q];
       }
     }
+    wave_sync();
+  }
+  // the rows and their pads (the last pass has nu > 0: hv_passes)
+#pragma unroll
+  for (int u = 0; u < RW; u++) {
+    const int J = J0 + wv + 4 * u;
+    if (J > jlast) break;
+    double *row = a + ix2(d, J, 0);
+    if (on)
+#pragma unroll
+      for (int q = 0; q < NQ; q++) row[1 + lane + 64 * q] = v[u][q];
+    if (1 + lane + 64 * (NQ - 1) == ni) row[0] = v[u][NQ - 1];
+    if (lane == 0) row[ni + 1] = v[u][0];
   }
 }
 
