@@ -2,8 +2,8 @@
 // filter rows: the NR real FFT of src/shared/epic_funcs_util.c:4023-4135
 // (four1 stages and the realft split step, with the twiddles of the
 // reference's recurrences tabulated on the host), one butterfly per lane,
-// and filter_row_lds(), which filters one latitude row held in LDS inside
-// a consumer kernel (src/shared/epic_adjust.c:102-242, TWODIM).
+// and filter_row_regs(), which filters one latitude row held by its lanes
+// inside a consumer kernel (src/shared/epic_adjust.c:102-242, TWODIM).
 #pragma once
 #include "dev_common.h"
 
@@ -160,34 +160,43 @@ __device__ __forceinline__ RowMap row_map(int ni) {
 }
 static inline int rows_per_block(int ni) { return 1024 / ni; }
 
-// Filter one latitude row held in LDS, in place: x[0..ni) holds I = 1..ni
-// in natural order; work is ni values of scratch LDS; lane is the caller's
-// index within its row (RowMap::lane), the row's ni/4 lanes being the
-// transform team.  When ni <= 256 the team lies in one wavefront and the
-// stages are separated by wavefront barriers; when ni > 256 by block
-// barriers, so every lane of the block must call.  The caller places a
-// block barrier after the call before other lanes read x.  filt = whether row J is in
-// the filter band; the row is untouched otherwise.  The arithmetic is that
-// of k_fft_filter, operation for operation.
+// Whether some row of this lane's synchronisation group (its wavefront when
+// a row's ni/4 lanes lie in one, else its block) is to be filtered: the same
+// answer in every lane of the group, which may then skip the transform's
+// barriers and stages together.  Half of the rows lie outside the band.
+__device__ __forceinline__ bool filter_any(int ni, bool active) {
+  return (ni >> 2) <= 64 ? __any(active) : __syncthreads_or(active);
+}
+
+// Filter one latitude row held in registers, in place: v[q] is point
+// I = 1 + lane + q ni/4 of the row, lane the caller's index within its row
+// (RowMap::lane), the row's ni/4 lanes being the transform team; work is ni
+// values of scratch LDS of the row's own.  When ni <= 256 the team lies in
+// one wavefront and the stages are separated by wavefront barriers; when
+// ni > 256 by block barriers, so every lane of the block must call.  active =
+// the row is in the filter band; it is untouched otherwise.  work is free
+// for other use when the call returns.  The arithmetic is that of
+// k_fft_filter, operation for operation.
 template <class T>
-__device__ __forceinline__ void filter_row_lds(const MemberDesc &d, T *x, T *work, int J, int vgrid, bool filt,
-                                               int lane) {
-  const int n = d.ni, nq = n >> 2;
-  if (nq <= 64 && lane >= nq) return;
-  const bool active = filt && lane < nq;
-  const int bits = d.nlogn - 1;
+__device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], T *work, int J, int vgrid, bool active,
+                                                int lane) {
+  const int n = d.ni, nq = n >> 2, bits = d.nlogn - 1;
   LaneTw<T> tf, ti;
   load_tw(tf, tw_fwd<T>(d), tr_fwd<T>(d), n, lane);
   load_tw(ti, tw_inv<T>(d), tr_inv<T>(d), n, lane);
   const double *hl = (vgrid ? d.hl_pv : d.hl_h) + (size_t)J * (n / 2 + 2);
   T gain[4];
-  if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) {
-      int gi = (e == 0) ? 1 : (e == 1 ? n / 2 + 1 : (e >> 1) + 1);
+  int rev[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int e = lane + q * nq;
+    rev[q] = (brev(e >> 1, bits) << 1) | (e & 1);
+    if (active) {
+      const int gi = (e == 0) ? 1 : (e == 1 ? n / 2 + 1 : (e >> 1) + 1);
       gain[q] = T(hl[gi]);
-      int k = e >> 1, c = e & 1;
-      work[(brev(k, bits) << 1) | c] = x[e];
+      work[rev[q]] = v[q];
     }
+  }
   row_sync(nq);
   four1_stages(work, n, lane, tf, active);
   split_step(work, n, lane, tf, T(-0.5), active);
@@ -198,7 +207,8 @@ __device__ __forceinline__ void filter_row_lds(const MemberDesc &d, T *x, T *wor
   }
   row_sync(nq);
   if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) work[e] *= gain[q];
+#pragma unroll
+    for (int q = 0; q < 4; q++) work[lane + q * nq] *= gain[q];
   row_sync(nq);
   split_step(work, n, lane, ti, T(0.5), active);
   if (active && lane == 0) {
@@ -207,19 +217,18 @@ __device__ __forceinline__ void filter_row_lds(const MemberDesc &d, T *x, T *wor
     work[1] = T(0.5) * (h1r - work[1]);
   }
   row_sync(nq);
-  T v[4];
   if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) v[q] = work[e];
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq];
   row_sync(nq);
   if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) {
-      int k = e >> 1, c = e & 1;
-      work[(brev(k, bits) << 1) | c] = v[q];
-    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) work[rev[q]] = v[q];
   row_sync(nq);
   four1_stages(work, n, lane, ti, active);
   if (active)
-    for (int e = lane; e < n; e += nq) x[e] = work[e] * T(2. / (n));
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq] * T(2. / (n));
   row_sync(nq);
 }
 

@@ -946,8 +946,10 @@ void L_calc_w(hipStream_t s, const Bucket &b, int with_source) {
 
 // ------------------------------------------------ vorticity / divergence
 // PV3 planes k0..k1 from U (uu) and the zonally filtered V (vv), with H3.
-// One block per (K,J) pv-row group: row J of vv is filtered in LDS (rows of
-// the v-grid filter band), then one lane per I.  bx is the row group.
+// One block per (K,J) pv-row group: row J of vv is filtered by its lanes
+// (rows of the v-grid filter band), which hand each other their neighbours
+// through the row's ni values of LDS.  A lane's four points are written out,
+// so their loads are in flight together.  bx is the row group.
 __device__ __forceinline__ void vort_interior_rows(const MemberDesc &d, double *lds, int bx, int K, int uf, int vf) {
   const RowMap m = row_map(d.ni);
   const int Jr = 1 + bx * m.rpb + m.g, ni = d.ni;
@@ -956,27 +958,37 @@ __device__ __forceinline__ void vort_interior_rows(const MemberDesc &d, double *
   const double *uu = fld_ptr(d, uf) + (size_t)K * d.N2, *vv = fld_ptr(d, vf) + (size_t)K * d.N2;
   const double *hh = d.H3 + (size_t)K * d.N2;
   double *pv = d.PV3 + (size_t)K * d.N2;
-  double *xv = lds + (size_t)m.g * 2 * ni, *work = xv + ni;  // xv[I-1] = filtered vv(J,I)
-  if (live)
-    for (int I = 1 + m.lane; I <= ni; I += m.stride) xv[I - 1] = vv[ix2(d, J, I)];
-  __syncthreads();
-  filter_row_lds(d, xv, work, J, 1, live && d.rflag_v[J] != 0, m.lane);
-  __syncthreads();
+  double *xv = lds + (size_t)m.g * ni;  // xv[I-1] = filtered vv(J,I)
+  double v[4], u0[4], u1[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    v[q] = vv[ix2(d, J, I)];
+    u0[q] = uu[ix2(d, J - 1, I)];
+    u1[q] = uu[ix2(d, J, I)];
+  }
+  const bool filt = live && d.rflag_v[J] != 0;
+  if (filter_any(ni, filt)) filter_row_regs(d, v, xv, J, 1, filt, m.lane);
+#pragma unroll
+  for (int q = 0; q < 4; q++) xv[m.lane + m.stride * q] = v[q];
+  row_sync(m.stride);
   if (!live) return;
   double f2j = d.f[2 * J], m2j = d.m[2 * J], n2j = d.n[2 * J];
   double mm1i = 1. / d.m[2 * J - 1], mp1i = 1. / d.m[2 * J + 1];
   double mnm1i = 1. / d.mn[2 * J - 1], mnp1i = 1. / d.mn[2 * J + 1];
   double mn_pv = .5 / (mnm1i + mnp1i);
-  for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-    const double vc = xv[I - 1], vw = xv[I == 1 ? ni - 1 : I - 2];
-    double ze = m2j * ((vc - vw) + n2j * (uu[ix2(d, J - 1, I)] * mm1i - uu[ix2(d, J, I)] * mp1i));
-    double v = (ze + f2j);
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    const double vc = v[q], vw = xv[I == 1 ? ni - 1 : I - 2];
+    double ze = m2j * ((vc - vw) + n2j * (u0[q] * mm1i - u1[q] * mp1i));
+    double w = (ze + f2j);
     double h_pv = ((hh[ix2(d, J, I)] + hh[ix2(d, J, I - 1)]) * mnp1i +
                    (hh[ix2(d, J - 1, I)] + hh[ix2(d, J - 1, I - 1)]) * mnm1i) * mn_pv;
-    v /= h_pv;
-    pv[ix2(d, J, I)] = v;
-    if (I == ni) pv[ix2(d, J, 0)] = v;
-    if (I == 1) pv[ix2(d, J, ni + 1)] = v;
+    w /= h_pv;
+    pv[ix2(d, J, I)] = w;
+    if (I == ni) pv[ix2(d, J, 0)] = w;
+    if (I == 1) pv[ix2(d, J, ni + 1)] = w;
   }
 }
 // pole PV from the circulation of the adjacent u-row (north = 1: J = nj+1
@@ -1015,7 +1027,7 @@ __device__ __forceinline__ void vort_pole(const MemberDesc &d, double *row, int 
   for (int I = threadIdx.x; I <= ni + 1; I += blockDim.x) pv[ix2(d, Jd, I)] = val;
 }
 // DIV of (uu zonally filtered, vv) on plane K: one block per (K,J) h-row
-// group, row J of uu filtered in LDS (rows of the h-grid filter band)
+// group, row J of uu filtered by its lanes (rows of the h-grid filter band)
 __device__ __forceinline__ void divergence_rows(const MemberDesc &d, double *lds, int bx, int K, int uf, int vf, int df) {
   const RowMap m = row_map(d.ni);
   const int Jr = bx * m.rpb + m.g, ni = d.ni;
@@ -1023,27 +1035,37 @@ __device__ __forceinline__ void divergence_rows(const MemberDesc &d, double *lds
   const int J = live ? Jr : 0;
   const double *uu = fld_ptr(d, uf) + (size_t)K * d.N2, *vv = fld_ptr(d, vf) + (size_t)K * d.N2;
   double *di = fld_ptr(d, df) + (size_t)K * d.N2;
-  double *xu = lds + (size_t)m.g * 2 * ni, *work = xu + ni;  // xu[I-1] = filtered uu(J,I)
-  if (live)
-    for (int I = 1 + m.lane; I <= ni; I += m.stride) xu[I - 1] = uu[ix2(d, J, I)];
-  __syncthreads();
-  filter_row_lds(d, xu, work, J, 0, live && d.rflag_h[J] != 0, m.lane);
-  __syncthreads();
+  double *xu = lds + (size_t)m.g * ni;  // xu[I-1] = filtered uu(J,I)
+  double u[4], v0[4], v1[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    u[q] = uu[ix2(d, J, I)];
+    v0[q] = vv[ix2(d, J, I)];
+    v1[q] = vv[ix2(d, J + 1, I)];
+  }
+  const bool filt = live && d.rflag_h[J] != 0;
+  if (filter_any(ni, filt)) filter_row_regs(d, u, xu, J, 0, filt, m.lane);
+#pragma unroll
+  for (int q = 0; q < 4; q++) xu[m.lane + m.stride * q] = u[q];
+  row_sync(m.stride);
   if (!live) return;
   int jj = 2 * J + 1;
   double n_inv = 1. / d.n[jj], mn = d.mn[jj];
   double m2j_inv = (J == 0) ? 0. : 1. / d.m[jj - 1];
   double m2jp2_inv = (J == d.nj) ? 0. : 1. / d.m[jj + 1];
-  for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-    const double ue = xu[I == ni ? 0 : I], uc = xu[I - 1];
-    double v = mn * ((ue * n_inv - uc * n_inv) + (vv[ix2(d, J + 1, I)] * m2jp2_inv - vv[ix2(d, J, I)] * m2j_inv));
-    di[ix2(d, J, I)] = v;
-    if (I == ni) di[ix2(d, J, 0)] = v;
-    if (I == 1) di[ix2(d, J, ni + 1)] = v;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    const double ue = xu[I == ni ? 0 : I], uc = u[q];
+    double w = mn * ((ue * n_inv - uc * n_inv) + (v1[q] * m2jp2_inv - v0[q] * m2j_inv));
+    di[ix2(d, J, I)] = w;
+    if (I == ni) di[ix2(d, J, 0)] = w;
+    if (I == 1) di[ix2(d, J, ni + 1)] = w;
   }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_vort_interior(const MemberDesc *D, int mb, int uf, int vf, int k0) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_vort_interior(const MemberDesc *D, int mb, int uf, int vf, int k0) {
   MEMBER;
   extern __shared__ double lds[];
   vort_interior_rows(d, lds, blockIdx.x, k0 + blockIdx.y, uf, vf);
@@ -1056,12 +1078,12 @@ __global__ void __launch_bounds__(256) k_vort_poles(const MemberDesc *D, int mb,
 void L_vorticity(hipStream_t s, const Bucket &b, int uu, int vv, int k0, int k1) {
   int nK = k1 - k0 + 1;
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_vort_interior, dim3((b.nj + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * 2 * b.ni, s, b.D,
+  LAUNCH(k_vort_interior, dim3((b.nj + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s, b.D,
          b.mb, uu, vv, k0);
   LAUNCH(k_vort_poles, dim3(2 * nK, 1, b.nm), dim3(64), sizeof(double) * (2 * b.ni + 2), s, b.D, b.mb, uu, k0);
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_divergence(const MemberDesc *D, int mb, int uf, int vf, int df, int k0) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_divergence(const MemberDesc *D, int mb, int uf, int vf, int df, int k0) {
   MEMBER;
   extern __shared__ double lds[];
   divergence_rows(d, lds, blockIdx.x, k0 + blockIdx.y, uf, vf, df);
@@ -1074,7 +1096,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
 // time planes (IT_ZERO <- IT_MINUS2 <- IT_MINUS1 <- IT_ZERO) and advances
 // itime: the step's last use of them was its Adams-Bashforth update, and no
 // block of this launch reads them.
-__global__ void __launch_bounds__(256) k_store_diag(const MemberDesc *D, int mb, int nv, int nd, int rotate) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_store_diag(const MemberDesc *D, int mb, int nv, int nd, int rotate) {
   MEMBER;
   extern __shared__ double lds[];
   const int bx = blockIdx.x, K = blockIdx.y;
@@ -1093,13 +1115,13 @@ __global__ void __launch_bounds__(256) k_store_diag(const MemberDesc *D, int mb,
 void L_store_diag(hipStream_t s, const Bucket &b, int rotate) {
   const int rpb = rows_per_block(b.ni);
   const int nv = (b.nj + rpb - 1) / rpb, nd = (b.nj + 1 + rpb - 1) / rpb;
-  const size_t shm = sizeof(double) * std::max(rpb * 2 * b.ni, 2 * b.ni + 2);
+  const size_t shm = sizeof(double) * std::max(rpb * b.ni, 2 * b.ni + 2);
   LAUNCH(k_store_diag, dim3(nv + nd + 2, b.nk + 1, b.nm), dim3(256), shm, s, b.D, b.mb, nv, nd, rotate);
 }
 void L_divergence(hipStream_t s, const Bucket &b, int uu, int vv, int dst, int k0, int k1) {
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_divergence, dim3((b.nj + 1 + rpb - 1) / rpb, k1 - k0 + 1, b.nm), dim3(256), sizeof(double) * rpb * 2 * b.ni,
-         s, b.D, b.mb, uu, vv, dst, k0);
+  LAUNCH(k_divergence, dim3((b.nj + 1 + rpb - 1) / rpb, k1 - k0 + 1, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
+         b.D, b.mb, uu, vv, dst, k0);
 }
 
 }  // namespace epic

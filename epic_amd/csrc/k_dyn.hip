@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(256) k_dvdt_core(const MemberDesc *D, int mb) 
 // DUDT = (DUDT + PV*VH terms + dKIN/dx with filtered KIN) - vertical
 // advection.  One block per (K,J) u-row: the KIN row is zonally filtered in
 // LDS (rows of the filter band) and its pad refreshed, then one lane per I.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_dudt_core(const MemberDesc *D, int mb) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_dudt_core(const MemberDesc *D, int mb) {
   MEMBER;
   extern __shared__ double lds[];
   const RowMap m = row_map(d.ni);
@@ -131,12 +131,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   const int J = live ? Jr : 0;
   const size_t o = (size_t)K * d.N2;
   const double *uh = d.sA + o, *vh = d.sB + o, *kin = d.sC + o, *pv = d.PV3 + o;
-  double *kr = lds + (size_t)m.g * 2 * ni, *work = kr + ni;  // kr[I-1] = KIN(J,I)
-  if (live)
-    for (int I = 1 + m.lane; I <= ni; I += m.stride) kr[I - 1] = kin[ix2(d, J, I)];
-  __syncthreads();
-  filter_row_lds(d, kr, work, J, 0, live && d.rflag_h[J] != 0, m.lane);
-  __syncthreads();
+  double *kr = lds + (size_t)m.g * ni;  // kr[I-1] = filtered KIN(J,I)
+  double kv[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) kv[q] = kin[ix2(d, J, 1 + m.lane + m.stride * q)];
+  const bool filt = live && d.rflag_h[J] != 0;
+  if (filter_any(ni, filt)) filter_row_regs(d, kv, kr, J, 0, filt, m.lane);
+#pragma unroll
+  for (int q = 0; q < 4; q++) kr[m.lane + m.stride * q] = kv[q];
+  row_sync(m.stride);
   if (!live) return;
   double *du = cur_tend(d, d.DUDT) + o;
   for (int I = 1 + m.lane; I <= ni; I += m.stride) {
@@ -163,7 +166,7 @@ void L_uv_core(hipStream_t s, const Bucket &b) {
   LAUNCH(k_uvh_kin, grid2(b.nj + 2, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   LAUNCH(k_dvdt_core, grid2(b.nj, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_dudt_core, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * 2 * b.ni, s,
+  LAUNCH(k_dudt_core, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
          b.D, b.mb);
 }
 
@@ -577,30 +580,31 @@ __global__ void __launch_bounds__(256) k_gz_filtercopy(const MemberDesc *D, int 
   MEMBER;
   extern __shared__ double lds[];
   const RowMap m = row_map(d.ni);
-  const int Jr = (int)(blockIdx.x * m.rpb + m.g) - 1, K = blockIdx.y, ni = d.ni, W = ni + 2;
+  const int Jr = (int)(blockIdx.x * m.rpb + m.g) - 1, K = blockIdx.y, ni = d.ni;
   const bool live = Jr <= d.nj + 1;
   const int J = live ? Jr : 0;
-  double *x = lds + (size_t)m.g * (W + ni), *work = x + W;
   const double *src = d.GZ3 + (size_t)K * d.N2;
   double *dst = d.gz + (size_t)K * d.N2;
-  if (live)
-    for (int I = m.lane; I < W; I += m.stride) x[I] = src[ix2(d, J, I)];
-  __syncthreads();
+  double v[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) v[q] = src[ix2(d, J, 1 + m.lane + m.stride * q)];
+  // the lanes that hold points 1 and ni also move the pads
+  const bool first = m.lane == 0, last = m.lane == m.stride - 1;
+  double pe = 0., pw = 0.;
+  if (first) pe = src[ix2(d, J, ni + 1)];
+  if (last) pw = src[ix2(d, J, 0)];
   const bool filt = live && K <= d.nk - 1 && J >= 0 && J <= d.nj && d.rflag_h[J] != 0;
-  filter_row_lds(d, x + 1, work, J < 0 ? 0 : J, 0, filt, m.lane);
-  __syncthreads();
+  if (filter_any(ni, filt)) filter_row_regs(d, v, lds + (size_t)m.g * ni, J < 0 ? 0 : J, 0, filt, m.lane);
   if (!live) return;
-  for (int I = m.lane; I < W; I += m.stride) {
-    double v = x[I];
-    if (filt && I == 0) v = x[ni];
-    if (filt && I == ni + 1) v = x[1];
-    dst[ix2(d, J, I)] = v;
-  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) dst[ix2(d, J, 1 + m.lane + m.stride * q)] = v[q];
+  if (first) dst[ix2(d, J, ni + 1)] = filt ? v[0] : pe;
+  if (last) dst[ix2(d, J, 0)] = filt ? v[3] : pw;
 }
 void L_gz_filtercopy(hipStream_t s, const Bucket &b) {
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_gz_filtercopy, dim3((b.nj + 3 + rpb - 1) / rpb, b.nk + 2, b.nm), dim3(256),
-         sizeof(double) * rpb * (2 * b.ni + 2), s, b.D, b.mb);
+  LAUNCH(k_gz_filtercopy, dim3((b.nj + 3 + rpb - 1) / rpb, b.nk + 2, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
+         b.D, b.mb);
 }
 
 void L_gz_mono(hipStream_t s, const Bucket &b) {
@@ -693,7 +697,7 @@ __global__ void __launch_bounds__(256) k_d2dy2_cols(const MemberDesc *D, int mb,
 // place, src/shared/epic_subgrid.c:960-975).  Members that do not apply
 // the order leave D and A as they are.
 template <class T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_hv_apply(const MemberDesc *D, int mb, int nm, FieldSet fs, int pass, int src) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_hv_apply(const MemberDesc *D, int mb, int nm, FieldSet fs, int pass, int src) {
   SET_MEMBER;
   extern __shared__ double lds_raw[];
   T *lds = reinterpret_cast<T *>(lds_raw);
@@ -703,27 +707,33 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   if (K > r.k1 || hv_nu(d, pass) == 0. || hv_passes(d) <= pass) return;  // uniform per block
   const bool live = Jr <= d.nj + 1;
   const int J = live ? Jr : 0, ni = d.ni, vg = (kind == 1);
-  T *x = lds + (size_t)m.g * 2 * ni, *work = x + ni;
   double *a = fld_ptr(d, f) + (size_t)K * d.N2;
   T *dd = reinterpret_cast<T *>((src ? d.sC : d.sB).get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
   const bool upd = live && J >= r.jbot && J <= d.nj;
-  if (upd)
-    for (int I = 1 + m.lane; I <= ni; I += m.stride) x[I - 1] = dd[ix2(d, J, I)];
-  __syncthreads();
-  filter_row_lds(d, x, work, J, vg, upd && (vg ? d.rflag_v[J] : d.rflag_h[J]) != 0, m.lane);
-  __syncthreads();
+  // the row of A and the row of D, all loads in flight together
+  double v[4];
+  T x[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const size_t i = ix2(d, J, 1 + m.lane + m.stride * q);
+    v[q] = a[i];
+    x[q] = dd[i];
+  }
+  const bool filt = upd && (vg ? d.rflag_v[J] : d.rflag_h[J]) != 0;
+  if (filter_any(ni, filt)) filter_row_regs(d, x, lds + (size_t)m.g * ni, J, vg, filt, m.lane);
   if (!live) return;
   const bool back = upd && hv_passes(d) > pass + 1;
   const double sign = (pass & 1) ? -1. : 1.;
-  for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-    double v = a[ix2(d, J, I)];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
     if (upd) {
-      v += d.dt * sign * (double)x[I - 1];
-      a[ix2(d, J, I)] = v;
+      v[q] += d.dt * sign * (double)x[q];
+      a[ix2(d, J, I)] = v[q];
     }
-    if (back) dd[ix2(d, J, I)] = x[I - 1];
-    if (I == d.ni) a[ix2(d, J, 0)] = v;
-    if (I == 1) a[ix2(d, J, d.ni + 1)] = v;
+    if (back) dd[ix2(d, J, I)] = x[q];
+    if (I == ni) a[ix2(d, J, 0)] = v[q];
+    if (I == 1) a[ix2(d, J, ni + 1)] = v[q];
   }
 }
 
@@ -784,13 +794,13 @@ static void merid_hv_t(hipStream_t s, const Bucket &b, const FieldSet &fs) {
   d2dy2_del4<T>(s, b, fs);
   const int rpb = rows_per_block(b.ni);
   const dim3 ga((b.nj + 2 + rpb - 1) / rpb, b.nk, fs.n * b.nm);
-  LAUNCH(k_hv_apply<T>, ga, dim3(256), sizeof(T) * rpb * 2 * b.ni, s, b.D, b.mb, b.nm, fs, 1, 0);
+  LAUNCH(k_hv_apply<T>, ga, dim3(256), sizeof(T) * rpb * b.ni, s, b.D, b.mb, b.nm, fs, 1, 0);
   // del^6 (pass 2, into sC) and del^8 (pass 3, back into sB)
   const dim3 gp((jrows * b.ni + TPB - 1) / TPB, b.nk, fs.n * b.nm);
   for (int pass = 2; pass < b.hv_passes; pass++) {
     const int src = (pass == 2) ? 0 : 1;
     LAUNCH(k_d2dy2_pass<T>, gp, dim3(TPB), 0, s, b.D, b.mb, b.nm, fs, pass, src);
-    LAUNCH(k_hv_apply<T>, ga, dim3(256), sizeof(T) * rpb * 2 * b.ni, s, b.D, b.mb, b.nm, fs, pass, 1 - src);
+    LAUNCH(k_hv_apply<T>, ga, dim3(256), sizeof(T) * rpb * b.ni, s, b.D, b.mb, b.nm, fs, pass, 1 - src);
   }
 }
 void L_merid_hv(hipStream_t s, const Bucket &b, const FieldSet &fs) {
@@ -1003,22 +1013,10 @@ __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, i
     v[q] = live ? a[ix2(d, J, I)] : 0.;
     dq[q] = upd ? dd[ix2(d, J, I)] : T(0.);
   }
-  // the meridional part: D filtered in place (x = z0[1..ni], work = z1) in
-  // blocks that hold a row of the filter band (a block-uniform test)
-  const int *rflag = vg ? d.rflag_v : d.rflag_h;
-  bool anyf = false;
-  for (int g = 0, J1 = blockIdx.x * m.rpb; g < m.rpb; g++, J1++)
-    anyf |= (J1 >= r.jbot && J1 <= d.nj && rflag[J1] != 0);
-  T *x = z0 + 1;
-  if (anyf) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) x[m.lane + m.stride * q] = dq[q];
-    row_bar();
-    filter_row_lds(d, x, z1, J, vg, upd && rflag[J] != 0, m.lane);
-    row_bar();
-#pragma unroll
-    for (int q = 0; q < 4; q++) dq[q] = x[m.lane + m.stride * q];
-  }
+  // the meridional part: D filtered (work = z1) where the row's wavefront or
+  // block holds a row of the filter band
+  const bool filt = upd && (vg ? d.rflag_v : d.rflag_h)[J] != 0;
+  if (filter_any(ni, filt)) filter_row_regs(d, dq, z1, J, vg, filt, m.lane);
   const double sign = -1.;  // del^4
 #pragma unroll
   for (int q = 0; q < 4; q++)

@@ -130,12 +130,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   const int J = live ? Jr : 0;
   const size_t o = (size_t)K * d.N2;
   const float *uh = sAf(d) + o, *vh = sBf(d) + o, *kin = sCf(d) + o;
-  float *kr = lds + (size_t)m.g * 2 * ni, *work = kr + ni;  // kr[I-1] = KIN(J,I)
-  if (live)
-    for (int I = 1 + m.lane; I <= ni; I += m.stride) kr[I - 1] = kin[ix2(d, J, I)];
-  __syncthreads();
-  filter_row_lds(d, kr, work, J, 0, live && d.rflag_h[J] != 0, m.lane);
-  __syncthreads();
+  float *kr = lds + (size_t)m.g * ni;  // kr[I-1] = filtered KIN(J,I)
+  float kv[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) kv[q] = kin[ix2(d, J, 1 + m.lane + m.stride * q)];
+  const bool filt = live && d.rflag_h[J] != 0;
+  if (filter_any(ni, filt)) filter_row_regs(d, kv, kr, J, 0, filt, m.lane);
+#pragma unroll
+  for (int q = 0; q < 4; q++) kr[m.lane + m.stride * q] = kv[q];
+  row_sync(m.stride);
   if (!live) return;
   const double *pv = d.PV3 + o;
   double *du = curU(d) + o;
@@ -310,7 +313,7 @@ void LM_uv_core(hipStream_t s, const Bucket &b) {
   LAUNCH(km_uvh_kin, grid2(b.nj + 2, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   LAUNCH(km_dvdt_core, grid2(b.nj, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(km_dudt_core, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(float) * rpb * 2 * b.ni, s,
+  LAUNCH(km_dudt_core, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(float) * rpb * b.ni, s,
          b.D, b.mb);
 }
 void LM_uv_drag(hipStream_t s, const Bucket &b) {
