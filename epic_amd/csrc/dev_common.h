@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 // FP64 exp, log and pow of every kernel: correctly rounded, from the same
 // source the oracle's attribution build uses (crmath.h)
 #include "crmath.h"
@@ -100,19 +102,30 @@ struct MemberDesc {
   // mixed mode: DUDT, DVDT are one FP64 plane (the current step's sum) and
   // DUDTf, DVDTf the three FP32 Adams-Bashforth history planes
   gptr<float> DUDTf, DVDTf;
-  // sA..sD: scratch, three 3-D copies each (the batched advection gives each
-  // advected field its own copy; every other user takes the first)
-  gptr<double> gz, sA, sB, sC, sD, unity, old, spl;
+  // sA..sD: scratch, three 3-D copies each; vunity, vtheta: unity and theta
+  // after the advection's column pass
+  gptr<double> gz, sA, sB, sC, sD, vunity, vtheta, spl;
   gptr<double> rowbuf;  // 8*(nj+3) doubles: zonal means and meridional profiles
   gptr<MemberDyn> dyn;
 };
 
+// ix2 indexes a plane: a plane of a member is well below 2^32 bytes, so the
+// byte offset within it fits 32 bits and an access is one instruction on a
+// scalar base and a 32-bit offset (Plane).  ix3 indexes a field in 64 bits:
+// neighbours in I then share one address (an immediate offset), which the
+// point stencils over several planes need more than short arithmetic.
 __device__ __forceinline__ size_t ix3(const MemberDesc &d, int K, int J, int I) {
   return (size_t)I + (size_t)(J + 1) * d.Ia + (size_t)K * d.N2;
 }
-__device__ __forceinline__ size_t ix2(const MemberDesc &d, int J, int I) {
-  return (size_t)I + (size_t)(J + 1) * d.Ia;
-}
+__device__ __forceinline__ uint32_t ix2(const MemberDesc &d, int J, int I) { return (uint32_t)(I + (J + 1) * d.Ia); }
+template <class T>
+struct Plane {
+  T *p;
+  __device__ __forceinline__ T &operator[](uint32_t i) const {
+    using C = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+    return *(T *)((C *)p + (uint32_t)(i * (uint32_t)sizeof(T)));
+  }
+};
 
 __device__ __forceinline__ double dmax(double x, double y) { return x > y ? x : y; }
 
@@ -484,7 +497,7 @@ __device__ __forceinline__ T seq_acc(const T *a, int n, T s = T(0)) {
 // field selector: which 3-D array of the descriptor
 enum Fld : int {
   F_U, F_V, F_HDRY, F_THETA, F_P3, F_P2, F_THETA2, F_H3, F_GZ3, F_HEAT3, F_PV3, F_DIV, F_W3, F_DZDT3,
-  F_GZ, F_SA, F_SB, F_SC, F_SD, F_UNITY, F_OLD, F_DUDT_T, F_DVDT_T
+  F_GZ, F_SA, F_SB, F_SC, F_SD, F_DUDT_T, F_DVDT_T
 };
 
 __device__ __forceinline__ double *fld_ptr(const MemberDesc &d, int f) {
@@ -508,8 +521,6 @@ __device__ __forceinline__ double *fld_ptr(const MemberDesc &d, int f) {
     case F_SB: return d.sB;
     case F_SC: return d.sC;
     case F_SD: return d.sD;
-    case F_UNITY: return d.unity;
-    case F_OLD: return d.old;
     // the mixed mode keeps one FP64 plane for the current step's tendency
     case F_DUDT_T: return d.mixed ? d.DUDT : d.DUDT + (size_t)d.dyn->it0 * d.N3;
     case F_DVDT_T: return d.mixed ? d.DVDT : d.DVDT + (size_t)d.dyn->it0 * d.N3;

@@ -551,7 +551,7 @@ void member_plan(const epic_case *c, bool mixed, const epic_tables &T, MemberDes
       {&d.T2, EPIC_F_T2},         {&d.T3, EPIC_F_T3},       {&d.RHO2, EPIC_F_RHO2},     {&d.RHO3, EPIC_F_RHO3},
       {&d.EXNER3, EPIC_F_EXNER3}, {&d.GZ3, EPIC_F_GZ3},     {&d.MONT3, EPIC_F_MONT3},   {&d.HEAT3, EPIC_F_HEAT3},
       {&d.PV3, EPIC_F_PV3},       {&d.DIV, EPIC_F_DIV_UV3}, {&d.W3, EPIC_F_W3},         {&d.DZDT3, EPIC_F_DZDT3},
-      {&d.RI2, EPIC_F_RI2},       {&d.gz, -1},              {&d.unity, -1},             {&d.old, -1}};
+      {&d.RI2, EPIC_F_RI2},       {&d.gz, -1},              {&d.vunity, -1},            {&d.vtheta, -1}};
   for (auto &p : fields) add(p.p, sizeof(double) * N3, nul, p.f);
   // scratch: three copies each, one per field of the batched advection
   for (auto p : {&d.sA, &d.sB, &d.sC, &d.sD}) add(p, sizeof(double) * 3 * N3, nul);

@@ -13,10 +13,14 @@ __device__ __forceinline__ int brev(int k, int bits) { return bits ? (int)(__bre
 
 // Barrier between the transform stages of one row.  A row's ni/4 lanes lie
 // in one wavefront when ni <= 256, and rows never exchange data, so a
-// wavefront-level barrier suffices there; larger rows span waves.
-__device__ __forceinline__ void row_sync(int nq) {
-  if (nq <= 64) wave_sync();
-  else __syncthreads();
+// wavefront-level barrier suffices there; larger rows (WIDE, ni > 256) span
+// waves.  WIDE is a template argument of every row kernel: tested at each
+// barrier, it had the compiler duplicate the code behind it (the zonal
+// advection pass took 134 VGPRs instead of 78).
+template <bool WIDE>
+__device__ __forceinline__ void row_sync() {
+  if constexpr (WIDE) __syncthreads();
+  else wave_sync();
 }
 
 // The stage twiddles stay in their table (global, cache-resident: the
@@ -72,7 +76,7 @@ template <> __device__ __forceinline__ const float *tr_inv<float>(const MemberDe
 // with one stage per pass, with half the LDS round trips and barriers.  n/8
 // lanes take part in a pair of stages; an odd last stage runs one butterfly
 // per lane on n/4 lanes.
-template <class T>
+template <bool WIDE, class T>
 __device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const LaneTw<T> &t, bool active) {
   const T *tw = t.tw;
   int S = 0;
@@ -101,7 +105,7 @@ __device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const Lane
       buf[i3] = x3r;
       buf[i3 + 1] = x3i;
     }
-    row_sync(n >> 2);
+    row_sync<WIDE>();
   }
   if (s < S) {
     const int mmax = 2 << s, half = 1 << s;
@@ -115,12 +119,12 @@ __device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const Lane
       buf[j0] = yr;
       buf[j0 + 1] = yi;
     }
-    row_sync(n >> 2);
+    row_sync<WIDE>();
   }
 }
 
 // split step of the real transform; c2 = -0.5 forward, +0.5 inverse
-template <class T>
+template <bool WIDE, class T>
 __device__ __forceinline__ void split_step(T *buf, int n, int lane, const LaneTw<T> &t, T c2, bool active) {
   const T c1 = T(0.5);
   if (active && lane < n / 4 - 1) {
@@ -137,7 +141,7 @@ __device__ __forceinline__ void split_step(T *buf, int n, int lane, const LaneTw
     buf[i3] = h1r - wr * h2r + wi * h2i;
     buf[i4] = -h1i + wr * h2i + wi * h2r;
   }
-  row_sync(n >> 2);
+  row_sync<WIDE>();
 }
 
 // Rows per block of the row kernels: a row takes ni/4 lanes (the transform
@@ -159,13 +163,21 @@ __device__ __forceinline__ RowMap row_map(int ni) {
   return m;
 }
 static inline int rows_per_block(int ni) { return 1024 / ni; }
+// launch of a row kernel: its WIDE form for rows of more than 256 points
+#define ROWS_LAUNCH(b, name, kw, kn, g, blk, shm, s, ...)            \
+  do {                                                              \
+    if ((b).ni > 256) LAUNCH_AS(name, kw, g, blk, shm, s, __VA_ARGS__); \
+    else LAUNCH_AS(name, kn, g, blk, shm, s, __VA_ARGS__);          \
+  } while (0)
 
 // Whether some row of this lane's synchronisation group (its wavefront when
 // a row's ni/4 lanes lie in one, else its block) is to be filtered: the same
 // answer in every lane of the group, which may then skip the transform's
 // barriers and stages together.  Half of the rows lie outside the band.
-__device__ __forceinline__ bool filter_any(int ni, bool active) {
-  return (ni >> 2) <= 64 ? __any(active) : __syncthreads_or(active);
+template <bool WIDE>
+__device__ __forceinline__ bool filter_any(bool active) {
+  if constexpr (WIDE) return __syncthreads_or(active);
+  else return __any(active);
 }
 
 // Filter one latitude row held in registers, in place: v[q] is point
@@ -175,9 +187,9 @@ __device__ __forceinline__ bool filter_any(int ni, bool active) {
 // one wavefront and the stages are separated by wavefront barriers; when
 // ni > 256 by block barriers, so every lane of the block must call.  active =
 // the row is in the filter band; it is untouched otherwise.  work is free
-// for other use when the call returns.  The arithmetic is that of
-// k_fft_filter, operation for operation.
-template <class T>
+// for other use when the call returns.  The operations are those
+// of the reference's realft, in its order.
+template <bool WIDE, class T>
 __device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], T *work, int J, int vgrid, bool active,
                                                 int lane) {
   const int n = d.ni, nq = n >> 2, bits = d.nlogn - 1;
@@ -197,39 +209,39 @@ __device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], 
       work[rev[q]] = v[q];
     }
   }
-  row_sync(nq);
-  four1_stages(work, n, lane, tf, active);
-  split_step(work, n, lane, tf, T(-0.5), active);
+  row_sync<WIDE>();
+  four1_stages<WIDE>(work, n, lane, tf, active);
+  split_step<WIDE>(work, n, lane, tf, T(-0.5), active);
   if (active && lane == 0) {
     T h1r;
     work[0] = (h1r = work[0]) + work[1];
     work[1] = h1r - work[1];
   }
-  row_sync(nq);
+  row_sync<WIDE>();
   if (active)
 #pragma unroll
     for (int q = 0; q < 4; q++) work[lane + q * nq] *= gain[q];
-  row_sync(nq);
-  split_step(work, n, lane, ti, T(0.5), active);
+  row_sync<WIDE>();
+  split_step<WIDE>(work, n, lane, ti, T(0.5), active);
   if (active && lane == 0) {
     T h1r;
     work[0] = T(0.5) * ((h1r = work[0]) + work[1]);
     work[1] = T(0.5) * (h1r - work[1]);
   }
-  row_sync(nq);
+  row_sync<WIDE>();
   if (active)
 #pragma unroll
     for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq];
-  row_sync(nq);
+  row_sync<WIDE>();
   if (active)
 #pragma unroll
     for (int q = 0; q < 4; q++) work[rev[q]] = v[q];
-  row_sync(nq);
-  four1_stages(work, n, lane, ti, active);
+  row_sync<WIDE>();
+  four1_stages<WIDE>(work, n, lane, ti, active);
   if (active)
 #pragma unroll
     for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq] * T(2. / (n));
-  row_sync(nq);
+  row_sync<WIDE>();
 }
 
 }  // namespace epic

@@ -14,8 +14,19 @@
 //
 // The three advected fields (unity on the pressure grid, theta, hdry) are
 // independent of one another until the theta correction that follows them,
-// so every launch carries all three: blockIdx.z = field * members + member,
-// each field with its own scratch copies (sA..sD + field * N3).
+// so every launch of the column and meridional passes carries all three:
+// blockIdx.z = field * members + member, each field with its own scratch
+// copy (sA + field * N3).
+//
+// The passes run out of place, field -> adv_out -> sA -> field, so that no
+// copy of a field is made: the column pass reads the field (unity is the
+// constant 1 and is not read at all; hdry is read with the restore_mass that
+// precedes the advection) and leaves its result in adv_out; the meridional
+// pass leaves its in sA; the zonal pass filters its row in place of a copy
+// of the field and writes the field, theta with its correction (the theta of
+// before the passes is still in place then, and the same block has advected
+// unity) and hdry with the restore_mass that follows.  Of unity only the
+// levels whose correction is used, K >= k_sigma-1, are advected.
 //
 // The reference keeps its column work arrays in statics across calls: the
 // theta call starts at K = k_sigma-1 and reads wm[k_sigma-2] and
@@ -37,12 +48,23 @@ constexpr int ADV_FIELDS = 3;
 
 enum { AV_P3 = 0, AV_THETA = 1, AV_HDRY = 2 };
 
+// the field as the advection reads and writes it (theta and hdry)
 __device__ __forceinline__ double *adv_field(const MemberDesc &d, int which) {
-  return which == AV_P3 ? d.unity : (which == AV_THETA ? d.THETA : d.HDRY);
+  return which == AV_THETA ? d.THETA : d.HDRY;
 }
+// where the column pass leaves its result
+__device__ __forceinline__ double *adv_out(const MemberDesc &d, int which) {
+  return which == AV_P3 ? d.vunity : (which == AV_THETA ? d.vtheta : d.sC);
+}
+// a field's value on level K at offset q as the column pass takes it
+__device__ __forceinline__ double adv_value(const MemberDesc &d, int which, int K, size_t q) {
+  return which == AV_P3 ? 1. : which == AV_THETA ? d.THETA[q] : dmax(d.h_min[K], d.HDRY[q]);
+}
+// first level of a field that is advected
+__device__ __forceinline__ int adv_kfirst(const MemberDesc &d, int which) { return which == AV_HDRY ? 1 : d.ks - 1; }
 
 // ------------------------------------------------------------ vertical
-// Column tiles of C columns (J = 0..nj, I = 0..ni+1) with every level in LDS.
+// Column tiles of C columns (J = 0..nj, I = 1..ni) with every level in LDS.
 // The pass is a chain of K-stencils (first-guess flux, predictor, centred
 // flux, limiter correction, update) with no recurrence, so each stage runs
 // on all lanes over (column, level) pairs, separated by barriers.
@@ -75,6 +97,10 @@ __device__ __forceinline__ T tt_iface(const T *wa, int K, int nk, T ep) {
 // computes in FP64 (the same bits), else a re-read of the FP64 field
 __device__ __forceinline__ double old_value(double staged, const double *) { return staged; }
 __device__ __forceinline__ double old_value(float, const double *p) { return *p; }
+__device__ __forceinline__ double col_value(double staged, const MemberDesc &, int, int, size_t) { return staged; }
+__device__ __forceinline__ double col_value(float, const MemberDesc &d, int which, int K, size_t q) {
+  return adv_value(d, which, K, q);
+}
 
 template <class T>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_hsu_vert(const MemberDesc *D, int mb, int nm, int C) {
@@ -83,15 +109,15 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
   extern __shared__ double lds_raw[];
   T *lds = reinterpret_cast<T *>(lds_raw);
   const int c = threadIdx.x % C, kk = threadIdx.x / C, KS = blockDim.x / C;
-  const int nI = d.ni + 2, col = blockIdx.x * C + c;
-  const bool live = col < (d.nj + 1) * nI;
-  const int J = live ? col / nI : 0, I = live ? col % nI : 0;
+  const int col = blockIdx.x * C + c;
+  const bool live = col < (d.nj + 1) * d.ni;
+  const int J = live ? col >> d.nlogn : 0, I = live ? 1 + (col & (d.ni - 1)) : 1;
   const int nk = d.nk, L = nk + 2;
   const int layer = (which == AV_HDRY);
   const int kf = (which == AV_THETA) ? d.ks - 1 : 1;
   const T ep = T(1.e-10), DT = T(d.dt);
   const double *dsi = d.dsgth_inv;
-  double *b = adv_field(d, which);
+  double *out = adv_out(d, which);
   T *wa = lds + c * L, *wv = lds + (C + c) * L, *pr = lds + (2 * C + c) * L, *ff = lds + (3 * C + c) * L;
   // stage 1: field and vertical velocity (wv holds w on the points the
   // field lives on: W3 itself for layers, the interface average otherwise)
@@ -99,10 +125,10 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
     for (int K = kk; K <= nk + 1; K += KS) {
       double x = 0., w = 0.;
       if (layer) {
-        if (K >= kf && K <= nk) x = b[ix3(d, K, J, I)];
+        if (K >= kf && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
         if (K >= kf - 1 && K <= nk) w = d.W3[ix3(d, K, J, I)];
       } else {
-        if (K >= kf - 1 && K <= nk) x = b[ix3(d, K, J, I)];
+        if (K >= kf - 1 && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
         if (K >= kf && K <= nk) w = (K == 1 || K == nk) ? 0. : .5 * (d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K - 1, J, I)]);
         // statics left by the unity pass (wm[kf-1], wa[kf-2] of its last column)
         if (which == AV_THETA && K == kf - 1 && K >= 1) {
@@ -153,22 +179,26 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
     __syncthreads();
     if (live)
       for (int K = kf + kk; K <= nk; K += KS)
-        b[ix3(d, K, J, I)] = old_value(wa[K], b + ix3(d, K, J, I)) + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
+        out[ix3(d, K, J, I)] =
+            col_value(wa[K], d, which, K, ix3(d, K, J, I)) + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
   } else {
+    // unity's levels above k_sigma-1 serve their neighbours only: flux and
+    // predictor from k_sigma-2, the corrected flux from k_sigma-1
+    const int k1 = max(kf, d.ks - 2), k2 = max(kf, d.ks - 1);
     // first-guess flux on layers kf..nk (zero below the bottom)
     if (live)
-      for (int K = kf + kk; K <= nk + 1; K += KS) ff[K] = (K == nk + 1) ? T(0.) : WP(K) * wa[K] + WM(K) * wa[K - 1];
+      for (int K = k1 + kk; K <= nk + 1; K += KS) ff[K] = (K == nk + 1) ? T(0.) : WP(K) * wa[K] + WM(K) * wa[K - 1];
     __syncthreads();
     if (live)
-      for (int K = kf - 1 + kk; K <= nk; K += KS)
+      for (int K = max(kf - 1, d.ks - 2) + kk; K <= nk; K += KS)
         pr[K] = (K == kf - 1) ? wa[K] : wa[K] + (ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT;
     __syncthreads();
     if (live)
-      for (int K = kf + kk; K <= nk; K += KS)
+      for (int K = k2 + kk; K <= nk; K += KS)
         ff[K] = T(.5) * (WP(K) * (pr[K - 1] + wa[K]) + WM(K) * (pr[K] + wa[K - 1]));
     __syncthreads();
     if (live)
-      for (int K = kf + kk; K <= nk; K += KS) {
+      for (int K = k2 + kk; K <= nk; K += KS) {
         const T d1K = pr[K - 1] - wa[K];
         const T d2K = pr[K] - wa[K - 1];
         const T d2M = (K == kf) ? T(0.) : pr[K - 1] - wa[K - 2];
@@ -193,8 +223,9 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
       }
     __syncthreads();
     if (live)
-      for (int K = kf + kk; K <= nk; K += KS)
-        b[ix3(d, K, J, I)] = old_value(wa[K], b + ix3(d, K, J, I)) + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
+      for (int K = k2 + kk; K <= nk; K += KS)
+        out[ix3(d, K, J, I)] =
+            col_value(wa[K], d, which, K, ix3(d, K, J, I)) + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
   }
 #undef WM
 #undef WP
@@ -207,13 +238,12 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
 // J0-1..J0+TJ+1, the smoothness terms aq and the predictor ap on rows
 // J0-1..J0+TJ and the corrected flux on v-rows J0..J0+TJ, each formed once per
 // cell by the reference's expression (the halo rows are formed again by the
-// neighbouring tile: the same values).  The update goes to sA and to its copy
-// sB (which the zonal pass filters), with sB's zonal pads.
+// neighbouring tile: the same values).  The update goes to sA.
 template <class T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_hsu_mer(const MemberDesc *D, int mb, int nm, int CW, int MER_TJ) {
   ADV_MEMBER;
   const int K = 1 + blockIdx.y;
-  if (d.adv_akima[which] || (which == AV_THETA && K <= d.ks - 2)) return;  // uniform per block
+  if (d.adv_akima[which] || K < adv_kfirst(d, which)) return;  // uniform per block
   extern __shared__ double sh_raw[];
   T *sh = reinterpret_cast<T *>(sh_raw);
   const int nj = d.nj, nchunk = d.ni / CW;
@@ -224,7 +254,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   T *ta = sh, *tvp = ta + RA * CW, *tvm = tvp + RV * CW, *taq = tvm + RV * CW, *tap = taq + RP * CW;
   T *tff = tap + RP * CW;
   const size_t o = (size_t)K * d.N2;
-  const double *A = adv_field(d, which) + o;
+  const Plane<const double> A{adv_out(d, which) + o};
   const T amin = (which == AV_HDRY) ? T(d.h_min[K]) : T(0.), DT = T(d.dt), ep = T(1.e-10);
   // row index helpers: field rows from J0-2, v-rows and predictor rows from J0-1
   auto a = [&](int J) { return ta[(J - J0 + 2) * CW + c]; };
@@ -284,106 +314,167 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
     tff[r * CW + c] = fc + -al * (VP * bp * d1J - vhp * bhp * d1m + VM * bm * d2m - vhm * bhm * d2J);
   }
   __syncthreads();
-  // update on the tile's rows: the FP64 field plus the flux divergence; sB
-  // (the copy the zonal pass filters) in the flux type
-  double *sA = d.sA + so + o;
-  T *sB = reinterpret_cast<T *>(d.sB.get()) + so + o;
+  // update on the tile's rows: the FP64 field plus the flux divergence
+  const Plane<double> sA{d.sA + so + o};
   for (int r = r0; r < MER_TJ; r += RS) {
     const int J = J0 + r;
     if (J > nj) break;
     const T f0 = (J >= 1) ? tff[r * CW + c] : T(0.), f1 = (J + 1 <= nj) ? tff[(r + 1) * CW + c] : T(0.);
-    const double v = old_value(a(J), A + ix2(d, J, I)) + (double)((f0 - f1) * T(d.mn[2 * J + 1]) * DT);
-    sA[ix2(d, J, I)] = v;
-    sB[ix2(d, J, I)] = T(v);
-    if (I == d.ni) sB[ix2(d, J, 0)] = T(v);
-    if (I == 1) sB[ix2(d, J, d.ni + 1)] = T(v);
+    sA[ix2(d, J, I)] = old_value(a(J), &A[ix2(d, J, I)]) + (double)((f0 - f1) * T(d.mn[2 * J + 1]) * DT);
   }
 }
 
 // --------------------------------------------------------------- zonal
-// Rows of the zonally filtered copy sB (1024/ni rows per block), staged in
-// LDS with their pads: velocities, first-guess fluxes, predictor, corrected
-// fluxes and the update sA + d(flux) each run on all lanes of the row,
-// periodic in I.
-template <class T>
-__global__ void __launch_bounds__(256) k_hsu_zonal(const MemberDesc *D, int mb, int nm) {
-  ADV_MEMBER;
-  const RowMap m = row_map(d.ni);
-  const int K = 1 + blockIdx.y, Jr = blockIdx.x * m.rpb + m.g;
-  if (d.adv_akima[which] || (which == AV_THETA && K <= d.ks - 2)) return;  // uniform per block
-  const bool live = Jr <= d.nj;
-  const int J = live ? Jr : 0;
-  extern __shared__ double sh_raw[];
-  T *sh = reinterpret_cast<T *>(sh_raw);
+// The zonal pass of row J by its ni/4 lanes, a lane holding the four points
+// I = 1 + lane + q ni/4: a is the plane as the meridional pass left it (sA),
+// y receives the row's result.  The row is rounded to the flux type, zonally
+// filtered where it lies in the filter band, and staged in LDS with its pads
+// beside the velocity u/n; first-guess flux, predictor and corrected flux
+// follow on all lanes, periodic in I.  The filter runs here, on the row in registers, rather than
+// in a launch of its own over a copy: the copy was a write and two reads of
+// every field, and a wavefront without a row in the band skips the transform.
+// Three row arrays: field, velocity (split by sign where it is used; the
+// corrected flux overwrites it once every lane has read it) and predictor
+// (before that, the filter's scratch); the first-guess flux is formed where
+// the predictor needs it (twice per cell, by the same expression).
+// the velocity on u-row J: U of the interface for unity and theta, the mean
+// of the interfaces above and below for hdry (whose pads are the points they
+// copy)
+__device__ __forceinline__ double adv_u(const MemberDesc &d, bool layer, int K, int J, int I) {
+  const Plane<const double> u{d.U + (size_t)K * d.N2};
+  if (!layer) return u[ix2(d, J, I)];
+  const Plane<const double> up{d.U + (size_t)(K - 1) * d.N2};
+  const uint32_t i = ix2(d, J, I < 1 ? I + d.ni : (I > d.ni ? I - d.ni : I));
+  return .5 * (u[i] + up[i]);
+}
+template <bool WIDE, class T>
+__device__ __forceinline__ void hsu_zonal_row(const MemberDesc &d, const RowMap &m, bool layer, int K, int J, bool filt, T amin,
+                                              const Plane<const double> &a, double (&y)[4], T *A) {
   const int ni = d.ni, W = ni + 2;
-  // three row arrays: the field, the velocity u/n (split by sign where it is
-  // used; the corrected flux overwrites it once every lane has read it) and
-  // the predictor; the first-guess flux is formed where the predictor needs
-  // it (twice per cell, by the same expression)
-  T *A = sh + (size_t)m.g * 3 * W;
-  T *UV = A + W, *AP = A + 2 * W, *FF = UV;
-  const T *af = reinterpret_cast<const T *>(d.sB.get()) + so + (size_t)K * d.N2;
   const double ninv = d.ninv_h[J];
+  T *UV = A + W, *AP = A + 2 * W, *FF = UV;
   const T mn = T(d.mn[2 * J + 1]), DT = T(d.dt);
-  const T amin = (which == AV_HDRY) ? T(d.h_min[K]) : T(0.);
   auto wr = [ni](int I) { return I < 1 ? I + ni : (I > ni ? I - ni : I); };
-  if (live)
-    for (int I = m.lane; I < W; I += m.stride) {
-      A[I] = af[ix2(d, J, I)];
-      double u2;
-      if (which == AV_HDRY) {
-        int Ii = wr(I);
-        u2 = .5 * (d.U[ix3(d, K, J, Ii)] + d.U[ix3(d, K - 1, J, Ii)]);
-      } else {
-        u2 = d.U[ix3(d, K, J, I)];
-      }
-      UV[I] = T(u2 * ninv);
-    }
-  __syncthreads();
+  T x[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) x[q] = T(a[ix2(d, J, 1 + m.lane + m.stride * q)]);
+  // (the velocity and the FP64 row are read behind the transform, which
+  // needs the registers they would hold)
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, x, AP, J, 0, filt, m.lane);
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    A[I] = x[q];
+    UV[I] = T(adv_u(d, layer, K, J, I) * ninv);
+  }
+  if (m.lane == 0) {
+    A[ni + 1] = x[0];
+    UV[ni + 1] = T(adv_u(d, layer, K, J, ni + 1) * ninv);
+  }
+  if (m.lane == m.stride - 1) {
+    A[0] = x[3];
+    UV[0] = T(adv_u(d, layer, K, J, 0) * ninv);
+  }
+  row_sync<WIDE>();
   // T(min(0, x)) = min(0, T(x)): rounding is monotone and keeps zero
   auto UP = [UV](int I) { return tmax(T(0.), UV[I]); };
   auto UM = [UV](int I) { return tmin(T(0.), UV[I]); };
   auto FP = [&](int c) { return UP(c) * A[c - 1] + UM(c) * A[c]; };
-  if (live)
-    for (int c = 1 + m.lane; c <= ni; c += m.stride) AP[c] = A[c] + (FP(c) - FP(wr(c + 1))) * mn * DT;
-  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int c = 1 + m.lane + m.stride * q;
+    AP[c] = A[c] + (FP(c) - FP(wr(c + 1))) * mn * DT;
+  }
+  row_sync<WIDE>();
   // a lane's four corrected fluxes (c = 1 + lane + q*stride) in registers
   T ffr[4];
-  if (live)
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int c = 1 + m.lane + q * m.stride;
-      const int cm = wr(c - 1);
-      T UPc = UP(c), UMc = UM(c), APc = AP[c], APm = AP[cm], Am = A[c - 1], Ac = A[c];
-      T fc = T(.5) * (UPc * (APc + Am) + UMc * (APm + Ac));
-      T d1c = APc - Am, d2c = APc - A[c + 1];
-      T d1m = APm - A[cm - 1], d2m = APm - A[cm + 1];
-      T uhp = sqrt(UPc * UP(c - 1)), uhm = -sqrt(UMc * UM(c + 1));
-      T mu = (UPc - UMc) * mn * DT, al = (T(1.) + mu) / T(6.);
-      T t0 = fabs(A[cm - 1] - T(2.) * A[cm] + A[cm + 1]) + T(1.e-10), q0 = t0 * t0;
-      T t1 = fabs(A[c - 1] - T(2.) * A[c] + A[c + 1]) + T(1.e-10), q1 = t1 * t1;
-      T gp = q0 / (q0 + (Am - amin) * (Ac - amin));
-      gp = gp * gp;
-      T gm = q1 / (q1 + (Am - amin) * (Ac - amin));
-      gm = gm * gm;
-      T bp = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gp, bm = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gm;
-      T bhp = T(1.) - gp, bhm = T(1.) - gm;
-      ffr[q] = fc + -al * (UPc * bp * d1c - uhp * bhp * d1m + UMc * bm * d2m - uhm * bhm * d2c);
-    }
-  __syncthreads();
-  if (live)
-#pragma unroll
-    for (int q = 0; q < 4; q++) FF[1 + m.lane + q * m.stride] = ffr[q];
-  __syncthreads();
-  if (!live) return;
-  double *out = adv_field(d, which);
-  for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-    const size_t q = ix3(d, K, J, I);
-    const double y = d.sA[so + q] + (double)((FF[I] - FF[wr(I + 1)]) * mn * DT);
-    out[q] = y;
-    if (I == ni) out[ix3(d, K, J, 0)] = y;
-    if (I == 1) out[ix3(d, K, J, ni + 1)] = y;
+  for (int q = 0; q < 4; q++) {
+    const int c = 1 + m.lane + q * m.stride;
+    const int cm = wr(c - 1);
+    T UPc = UP(c), UMc = UM(c), APc = AP[c], APm = AP[cm], Am = A[c - 1], Ac = A[c];
+    T fc = T(.5) * (UPc * (APc + Am) + UMc * (APm + Ac));
+    T d1c = APc - Am, d2c = APc - A[c + 1];
+    T d1m = APm - A[cm - 1], d2m = APm - A[cm + 1];
+    T uhp = sqrt(UPc * UP(c - 1)), uhm = -sqrt(UMc * UM(c + 1));
+    T mu = (UPc - UMc) * mn * DT, al = (T(1.) + mu) / T(6.);
+    T t0 = fabs(A[cm - 1] - T(2.) * A[cm] + A[cm + 1]) + T(1.e-10), q0 = t0 * t0;
+    T t1 = fabs(A[c - 1] - T(2.) * A[c] + A[c + 1]) + T(1.e-10), q1 = t1 * t1;
+    T gp = q0 / (q0 + (Am - amin) * (Ac - amin));
+    gp = gp * gp;
+    T gm = q1 / (q1 + (Am - amin) * (Ac - amin));
+    gm = gm * gm;
+    T bp = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gp, bm = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gm;
+    T bhp = T(1.) - gp, bhm = T(1.) - gm;
+    ffr[q] = fc + -al * (UPc * bp * d1c - uhp * bhp * d1m + UMc * bm * d2m - uhm * bhm * d2c);
+    // one point at a time: interleaved, the four need 192 VGPRs
+    __builtin_amdgcn_sched_barrier(0);
   }
+  row_sync<WIDE>();
+#pragma unroll
+  for (int q = 0; q < 4; q++) FF[1 + m.lane + q * m.stride] = ffr[q];
+  row_sync<WIDE>();
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + q * m.stride;
+    y[q] = a[ix2(d, J, I)] + (double)((ffr[q] - FF[wr(I + 1)]) * mn * DT);
+  }
+}
+// the Akima scheme's zonal pass of one row, in the same form
+template <bool WIDE, class T>
+__device__ __forceinline__ void ak_zonal_row(const MemberDesc &d, const RowMap &m, bool layer, int K, int J, bool filt,
+                                             const Plane<const double> &a, double (&y)[4], T *A);
+
+// Zonal pass of a row group (1024/ni rows of plane K per block).  layer: hdry,
+// stored with the restore_mass that follows the advection.  Otherwise theta
+// and, before it by the same lanes, unity, whose result corrects theta
+// (theta - old (unity - 1), old the theta of before the advection, still in
+// place) and is written nowhere.  The two go through one copy of the code (a
+// loop): written out twice the transform's operands are kept from one to the
+// other and cost a wave of occupancy.
+template <bool WIDE, class T, bool AKIMA>
+__device__ __forceinline__ void adv_zonal_rows(const MemberDesc &d, bool layer, T *sh) {
+  const RowMap m = row_map(d.ni);
+  const int K = 1 + blockIdx.y, Jr = blockIdx.x * m.rpb + m.g, ni = d.ni;
+  const bool live = Jr <= d.nj;
+  const int J = live ? Jr : 0;
+  T *A = sh + (size_t)m.g * 3 * (ni + 2);
+  const bool filt = live && d.rflag_h[J] != 0;
+  const size_t o = (size_t)K * d.N2;
+  double y[4], cor[4];  // the field's row; unity's advected row less 1
+#pragma unroll 1
+  for (int which = layer ? AV_HDRY : AV_P3;; which = AV_THETA) {
+    const Plane<const double> a{d.sA + (size_t)which * d.N3 + o};
+    if constexpr (AKIMA) ak_zonal_row<WIDE, T>(d, m, layer, K, J, filt, a, y, A);
+    else hsu_zonal_row<WIDE, T>(d, m, layer, K, J, filt, layer ? T(d.h_min[K]) : T(0.), a, y, A);
+    if (which != AV_P3) break;
+#pragma unroll
+    for (int q = 0; q < 4; q++) cor[q] = y[q] - 1.;
+    row_sync<WIDE>();
+  }
+  if (!live) return;
+  const Plane<double> out{(layer ? d.HDRY : d.THETA) + o};
+  const double hmin = d.h_min[K];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    double v = y[q];
+    if (layer) v = dmax(hmin, v);
+    else v -= out[ix2(d, J, I)] * cor[q];
+    out[ix2(d, J, I)] = v;
+    if (I == ni) out[ix2(d, J, 0)] = v;
+    if (I == 1) out[ix2(d, J, ni + 1)] = v;
+  }
+}
+// blockIdx.z = member for unity with theta, members + member for hdry
+template <bool WIDE, class T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_hsu_zonal(const MemberDesc *D, int mb, int nm) {
+  extern __shared__ double sh_raw[];
+  const bool layer = (int)blockIdx.z >= nm;
+  const MemberDesc &d = D[mb + (int)blockIdx.z - (layer ? nm : 0)];
+  const int which = layer ? AV_HDRY : AV_THETA;
+  if (d.adv_akima[which] || 1 + (int)blockIdx.y < adv_kfirst(d, which)) return;  // uniform per block
+  adv_zonal_rows<WIDE, T, false>(d, layer, reinterpret_cast<T *>(sh_raw));
 }
 
 // ------------------------------------------------------------- Akima
@@ -394,7 +485,7 @@ __global__ void __launch_bounds__(256) k_hsu_zonal(const MemberDesc *D, int mb, 
 // sign (0 otherwise), and the flux: the velocity times the edge value
 // .5 (a- + a+) - (dela+ - dela-) / 6, each by the reference's expression.
 // A block whose field takes the other scheme returns at once (uniform per
-// block); the two schemes share the filtered copy sB and its filter launch.
+// block).
 // The reference also runs the column pass on the pad rows J = -1 and nj+1,
 // where W3 is zero and the pass changes nothing.
 template <class T>
@@ -403,7 +494,7 @@ __device__ __forceinline__ T ak_dela(T d0, T d1) {
   return (tmp > T(0.)) ? T(2.) * tmp / (d0 + d1) : T(0.);
 }
 
-// column pass: columns J = 0..nj, I = 0..ni+1 in LDS tiles; the stages
+// column pass: columns J = 0..nj, I = 1..ni in LDS tiles; the stages
 // (differences, slopes, fluxes, update) run on all lanes over (column,
 // level) pairs, separated by barriers (no recurrence in K)
 template <class T>
@@ -413,25 +504,25 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
   extern __shared__ double lds_raw[];
   T *lds = reinterpret_cast<T *>(lds_raw);
   const int c = threadIdx.x % C, kk = threadIdx.x / C, KS = blockDim.x / C;
-  const int nI = d.ni + 2, col = blockIdx.x * C + c;
-  const bool live = col < (d.nj + 1) * nI;
-  const int J = live ? col / nI : 0, I = live ? col % nI : 0;
+  const int col = blockIdx.x * C + c;
+  const bool live = col < (d.nj + 1) * d.ni;
+  const int J = live ? col >> d.nlogn : 0, I = live ? 1 + (col & (d.ni - 1)) : 1;
   const int nk = d.nk, L = nk + 2;
   const int layer = (which == AV_HDRY);
   const int kf = (which == AV_THETA) ? d.ks - 1 : 1;
   const T DT = T(d.dt);
   const double *dsi = d.dsgth_inv;
-  double *b = adv_field(d, which);
+  double *out = adv_out(d, which);
   // the flux reuses the difference column once the slopes are formed
   T *wa = lds + c * L, *wv = lds + (C + c) * L, *da = lds + (2 * C + c) * L, *dl = lds + (3 * C + c) * L, *ff = da;
   if (live)
     for (int K = kk; K <= nk + 1; K += KS) {
       double x = 0., w = 0.;
       if (layer) {
-        if (K >= kf && K <= nk) x = b[ix3(d, K, J, I)];
+        if (K >= kf && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
         if (K >= kf - 1 && K <= nk) w = d.W3[ix3(d, K, J, I)];
       } else {
-        if (K >= kf - 1 && K <= nk) x = b[ix3(d, K, J, I)];
+        if (K >= kf - 1 && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
         if (K >= kf && K <= nk) w = (K == 1 || K == nk) ? 0. : .5 * (d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K - 1, J, I)]);
       }
       wa[K] = T(x);
@@ -467,22 +558,23 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
     }
   __syncthreads();
   if (live)
-    for (int K = kf + kk; K <= nk; K += KS) {
+    for (int K = max(kf, adv_kfirst(d, which)) + kk; K <= nk; K += KS) {
       const size_t q = ix3(d, K, J, I);
-      if (layer) b[q] = old_value(wa[K], b + q) + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
-      else b[q] = old_value(wa[K], b + q) + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
+      const double x = col_value(wa[K], d, which, K, q);
+      if (layer) out[q] = x + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
+      else out[q] = x + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
     }
 }
 
 // meridional pass: a tile of TJ rows x CW columns of one plane, with the
 // field on rows J0-2..J0+TJ+1, the slopes on J0-1..J0+TJ, the velocity and
-// the fluxes on v-rows J0..J0+TJ; the update goes to sA and its copy sB
-// (with sB's zonal pads), as the predictor-corrector's does
+// the fluxes on v-rows J0..J0+TJ; the update goes to sA, as the
+// predictor-corrector's does
 template <class T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_ak_mer(const MemberDesc *D, int mb, int nm, int CW, int MER_TJ) {
   ADV_MEMBER;
   const int K = 1 + blockIdx.y;
-  if (!d.adv_akima[which] || (which == AV_THETA && K <= d.ks - 2)) return;  // uniform per block
+  if (!d.adv_akima[which] || K < adv_kfirst(d, which)) return;  // uniform per block
   extern __shared__ double sh_raw[];
   T *sh = reinterpret_cast<T *>(sh_raw);
   const int nj = d.nj, nchunk = d.ni / CW;
@@ -492,7 +584,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   const int RA = MER_TJ + 4, RV = MER_TJ + 1, RD = MER_TJ + 2;
   T *ta = sh, *tv = ta + RA * CW, *tdl = tv + RV * CW, *tff = tdl + RD * CW;
   const size_t o = (size_t)K * d.N2;
-  const double *A = adv_field(d, which) + o;
+  const Plane<const double> A{adv_out(d, which) + o};
   const T DT = T(d.dt);
   auto a = [&](int J) { return ta[(J - J0 + 2) * CW + c]; };
   auto dl = [&](int J) { return tdl[(J - J0 + 1) * CW + c]; };
@@ -526,70 +618,74 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
     tff[r * CW + c] = f;
   }
   __syncthreads();
-  double *sA = d.sA + so + o;
-  T *sB = reinterpret_cast<T *>(d.sB.get()) + so + o;
+  const Plane<double> sA{d.sA + so + o};
   for (int r = r0; r < MER_TJ; r += RS) {
     const int J = J0 + r;
     if (J > nj) break;
-    const double v =
-        old_value(a(J), A + ix2(d, J, I)) + (double)((tff[r * CW + c] - tff[(r + 1) * CW + c]) * T(d.mn[2 * J + 1]) * DT);
-    sA[ix2(d, J, I)] = v;
-    sB[ix2(d, J, I)] = T(v);
-    if (I == d.ni) sB[ix2(d, J, 0)] = T(v);
-    if (I == 1) sB[ix2(d, J, d.ni + 1)] = T(v);
+    sA[ix2(d, J, I)] =
+        old_value(a(J), &A[ix2(d, J, I)]) + (double)((tff[r * CW + c] - tff[(r + 1) * CW + c]) * T(d.mn[2 * J + 1]) * DT);
   }
 }
 
-// zonal pass: rows of the filtered copy sB with its pads in LDS; slopes,
-// fluxes and the update sA + d(flux) on all lanes of the row, periodic in I
-template <class T>
-__global__ void __launch_bounds__(256) k_ak_zonal(const MemberDesc *D, int mb, int nm) {
-  ADV_MEMBER;
-  const RowMap m = row_map(d.ni);
-  const int K = 1 + blockIdx.y, Jr = blockIdx.x * m.rpb + m.g;
-  if (!d.adv_akima[which] || (which == AV_THETA && K <= d.ks - 2)) return;  // uniform per block
-  const bool live = Jr <= d.nj;
-  const int J = live ? Jr : 0;
-  extern __shared__ double sh_raw[];
-  T *sh = reinterpret_cast<T *>(sh_raw);
+// zonal pass of one row: the filtered row with its pads in LDS; slopes,
+// fluxes and the update on all lanes of the row, periodic in I
+template <bool WIDE, class T>
+__device__ __forceinline__ void ak_zonal_row(const MemberDesc &d, const RowMap &m, bool layer, int K, int J, bool filt,
+                                             const Plane<const double> &a, double (&y)[4], T *A) {
   const int ni = d.ni, W = ni + 2;
-  T *A = sh + (size_t)m.g * 3 * W, *DL = A + W, *FF = A + 2 * W;
-  const T *af = reinterpret_cast<const T *>(d.sB.get()) + so + (size_t)K * d.N2;
-  const double ninv = d.ninv_h[J];
+  T *DL = A + W, *FF = A + 2 * W;
   const T mn = T(d.mn[2 * J + 1]), DT = T(d.dt);
+  const double ninv = d.ninv_h[J];
   auto wr = [ni](int I) { return I < 1 ? I + ni : (I > ni ? I - ni : I); };
-  if (live)
-    for (int I = m.lane; I < W; I += m.stride) A[I] = af[ix2(d, J, I)];
-  __syncthreads();
+  T x[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) x[q] = T(a[ix2(d, J, 1 + m.lane + m.stride * q)]);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, x, FF, J, 0, filt, m.lane);
+#pragma unroll
+  for (int q = 0; q < 4; q++) A[1 + m.lane + m.stride * q] = x[q];
+  if (m.lane == 0) A[ni + 1] = x[0];
+  if (m.lane == m.stride - 1) A[0] = x[3];
+  row_sync<WIDE>();
   // differences A(I) - A(I-1) on I = 1..ni, the pad of I = ni+1 that of I = 1
   auto dA = [&](int I) { return A[I] - A[I - 1]; };
-  if (live)
-    for (int I = 1 + m.lane; I <= ni; I += m.stride) DL[I] = ak_dela(dA(I), dA(wr(I + 1)));
-  __syncthreads();
-  if (live)
-    for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-      const double u2 =
-          (which == AV_HDRY) ? .5 * (d.U[ix3(d, K, J, I)] + d.U[ix3(d, K - 1, J, I)]) : d.U[ix3(d, K, J, I)];
-      FF[I] = T(u2) * (T(.5) * (A[I] + A[I - 1]) - (DL[I] - DL[wr(I - 1)]) / T(6.)) * T(ninv);
-    }
-  __syncthreads();
-  if (!live) return;
-  double *out = adv_field(d, which);
-  for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-    const size_t q = ix3(d, K, J, I);
-    const double y = d.sA[so + q] + (double)((FF[I] - FF[wr(I + 1)]) * mn * DT);
-    out[q] = y;
-    if (I == ni) out[ix3(d, K, J, 0)] = y;
-    if (I == 1) out[ix3(d, K, J, ni + 1)] = y;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    DL[I] = ak_dela(dA(I), dA(wr(I + 1)));
+  }
+  row_sync<WIDE>();
+  T f[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    f[q] = T(adv_u(d, layer, K, J, I)) * (T(.5) * (A[I] + A[I - 1]) - (DL[I] - DL[wr(I - 1)]) / T(6.)) * T(ninv);
+    FF[I] = f[q];
+  }
+  row_sync<WIDE>();
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = 1 + m.lane + m.stride * q;
+    y[q] = a[ix2(d, J, I)] + (double)((f[q] - FF[wr(I + 1)]) * mn * DT);
   }
 }
+template <bool WIDE, class T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_ak_zonal(const MemberDesc *D, int mb, int nm) {
+  extern __shared__ double sh_raw[];
+  const bool layer = (int)blockIdx.z >= nm;
+  const MemberDesc &d = D[mb + (int)blockIdx.z - (layer ? nm : 0)];
+  const int which = layer ? AV_HDRY : AV_THETA;
+  if (!d.adv_akima[which] || 1 + (int)blockIdx.y < adv_kfirst(d, which)) return;  // uniform per block
+  adv_zonal_rows<WIDE, T, true>(d, layer, reinterpret_cast<T *>(sh_raw));
+}
 
-// one advection pass over all three fields of every member; the mixed mode
-// forms the fluxes in FP32 (sB, the filtered copy, FP32 too).  Each scheme's
-// launches run where some field of the bucket takes it.
+// restore_mass, one advection pass over all three fields of every member,
+// restore_mass (src/shared/epic_timestep.c, src/shared/epic_flux.c); the mixed
+// mode forms the fluxes in FP32.  Each scheme's launches run where some field
+// of the bucket takes it.  set_p2etc(DONT_UPDATE_THETA) follows, with
+// store_pgrad_vars.
 template <class T>
-static void hsu3_t(hipStream_t s, const Bucket &b) {
-  const int ncol = (b.nj + 1) * (b.ni + 2), nz = ADV_FIELDS * b.nm;
+static void advection_t(hipStream_t s, const Bucket &b) {
+  const int ncol = (b.nj + 1) * b.ni, nz = ADV_FIELDS * b.nm;
   // columns per block: as many as keep the four LDS columns within 40 KB
   int C = 64;
   while (C > 16 && (size_t)4 * C * (b.nk + 2) * sizeof(double) > 40 * 1024) C /= 2;
@@ -609,55 +705,14 @@ static void hsu3_t(hipStream_t s, const Bucket &b) {
   if (akima)
     LAUNCH(k_ak_mer<T>, gm, dim3(256), sizeof(T) * CW * ((TJ + 4) + 2 * (TJ + 1) + (TJ + 2)), s, b.D, b.mb, b.nm, CW,
            TJ);
-  // the zonal pass reads a zonally filtered copy (the reference filters it
-  // per level before the zonal sweep); a separate launch packs the rows of
-  // the filter band, which is faster here than filtering inside the pass
-  if (sizeof(T) == sizeof(double)) L_filter(s, b, F_SB, 1, b.nk, 0, 0, ADV_FIELDS);
-  else L_filter_f32(s, b, F_SB, 1, b.nk, 0, 0, ADV_FIELDS);
   const int rpb = rows_per_block(b.ni);
-  const dim3 gz((b.nj + 1 + rpb - 1) / rpb, b.nk, nz);
-  if (hsu) LAUNCH(k_hsu_zonal<T>, gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm);
-  if (akima) LAUNCH(k_ak_zonal<T>, gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm);
+  const dim3 gz((b.nj + 1 + rpb - 1) / rpb, b.nk, 2 * b.nm);
+  if (hsu) ROWS_LAUNCH(b, "k_hsu_zonal<T>", (k_hsu_zonal<true, T>), (k_hsu_zonal<false, T>), gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm);
+  if (akima) ROWS_LAUNCH(b, "k_ak_zonal<T>", (k_ak_zonal<true, T>), (k_ak_zonal<false, T>), gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm);
 }
-static void hsu3(hipStream_t s, const Bucket &b) {
-  if (b.mixed) hsu3_t<float>(s, b);
-  else hsu3_t<double>(s, b);
-}
-
-// op 0: unity = 1 on K = 0..nk+1, J = 0..nj, I = 0..ni+1, and OLD = THETA
-// on K = k_sigma-1..nk+1 over the same rows; op 1: the theta correction
-// there.  Both also apply restore_mass (HDRY = max(h_min, HDRY) on K = 1..nk
-// over the same rows), which the reference runs right before advection
-// (src/shared/epic_timestep.c) and right after it (src/shared/epic_flux.c)
-// and which touches HDRY only.
-__global__ void __launch_bounds__(256) k_adv_elem(const MemberDesc *D, int mb, int op) {
-  MEMBER;
-  int t = blockIdx.x * TPB + threadIdx.x;
-  const int nI = d.ni + 2;
-  if (t >= (d.nj + 1) * nI) return;
-  const int J = t / nI, I = t % nI, K = blockIdx.y;
-  if (K > d.nk + 1) return;
-  size_t q = ix3(d, K, J, I);
-  if (op == 0) {
-    d.unity[q] = 1.;
-    if (K >= d.ks - 1) d.old[q] = d.THETA[q];
-  } else if (K >= d.ks - 1) {
-    d.THETA[q] -= d.old[q] * (d.unity[q] - 1.);
-  }
-  if (K >= 1 && K <= d.nk) d.HDRY[q] = dmax(d.h_min[K], d.HDRY[q]);
-}
-
-// restore_mass, advection, restore_mass (the two restore_mass calls run
-// inside the element-wise launches around the advection passes)
 void L_advection(hipStream_t s, const Bucket &b) {
-  int ncol = (b.nj + 1) * (b.ni + 2);
-  dim3 ge((ncol + TPB - 1) / TPB, b.nk + 2, b.nm);
-  // unity, theta and hdry advected together; the theta correction after
-  // them (hdry's advection reads neither theta nor unity)
-  LAUNCH(k_adv_elem, ge, dim3(TPB), 0, s, b.D, b.mb, 0);
-  hsu3(s, b);
-  LAUNCH(k_adv_elem, ge, dim3(TPB), 0, s, b.D, b.mb, 1);
-  // set_p2etc(DONT_UPDATE_THETA) follows, with store_pgrad_vars
+  if (b.mixed) advection_t<float>(s, b);
+  else advection_t<double>(s, b);
 }
 
 }  // namespace epic

@@ -57,39 +57,6 @@ void L_fill(hipStream_t s, const Bucket &b, int f, double v) {
   LAUNCH(k_fill, dim3(256, 1, b.nm), dim3(TPB), 0, s, b.D, b.mb, f, v);
 }
 
-// zonal periodicity of a whole 3-D array (bc_lateral THREEDIM,
-// src/single/s_epic_functions.c:72-88): K = 0..nk+1, J = 0..nj+1
-__global__ void __launch_bounds__(256) k_bc3(const MemberDesc *D, int mb, int f) {
-  MEMBER;
-  double *a = fld_ptr(d, f);
-  int t = blockIdx.x * TPB + threadIdx.x;
-  int nrow = (d.nj + 2) * (d.nk + 2);
-  if (t >= nrow) return;
-  int K = t / (d.nj + 2), J = t % (d.nj + 2);
-  a[ix3(d, K, J, 0)] = a[ix3(d, K, J, d.ni)];
-  a[ix3(d, K, J, d.ni + 1)] = a[ix3(d, K, J, 1)];
-}
-void L_bc3(hipStream_t s, const Bucket &b, int f) {
-  int nrow = (b.nj + 2) * (b.nk + 2);
-  LAUNCH(k_bc3, dim3((nrow + TPB - 1) / TPB, 1, b.nm), dim3(TPB), 0, s, b.D, b.mb, f);
-}
-
-// copy planes k0..k1 (whole planes) src -> dst
-__global__ void __launch_bounds__(256) k_copy_planes(const MemberDesc *D, int mb, int src, int dst, int k0) {
-  MEMBER;
-  const double *a = fld_ptr(d, src);
-  double *o = fld_ptr(d, dst);
-  int t = blockIdx.x * TPB + threadIdx.x;
-  if (t >= d.N2) return;
-  size_t off = (size_t)(k0 + blockIdx.y) * d.N2 + t;
-  o[off] = a[off];
-}
-void L_copy_planes(hipStream_t s, const Bucket &b, int src, int dst, int k0, int k1) {
-  int N2 = (b.ni + 2) * (b.nj + 3);
-  LAUNCH(k_copy_planes, dim3((N2 + TPB - 1) / TPB, k1 - k0 + 1, b.nm), dim3(TPB), 0, s, b.D, b.mb,
-                     src, dst, k0);
-}
-
 // ------------------------------------------------------------ column tiles
 // A block holds C consecutive (J,I) columns (J = 0..nj, I = 0..ni+1) and
 // all their levels.  The per-level work (transcendentals, Leslie-Purser
@@ -950,14 +917,15 @@ void L_calc_w(hipStream_t s, const Bucket &b, int with_source) {
 // (rows of the v-grid filter band), which hand each other their neighbours
 // through the row's ni values of LDS.  A lane's four points are written out,
 // so their loads are in flight together.  bx is the row group.
+template <bool WIDE>
 __device__ __forceinline__ void vort_interior_rows(const MemberDesc &d, double *lds, int bx, int K, int uf, int vf) {
   const RowMap m = row_map(d.ni);
   const int Jr = 1 + bx * m.rpb + m.g, ni = d.ni;
   const bool live = Jr <= d.nj;
   const int J = live ? Jr : 1;
-  const double *uu = fld_ptr(d, uf) + (size_t)K * d.N2, *vv = fld_ptr(d, vf) + (size_t)K * d.N2;
-  const double *hh = d.H3 + (size_t)K * d.N2;
-  double *pv = d.PV3 + (size_t)K * d.N2;
+  const Plane<const double> uu{fld_ptr(d, uf) + (size_t)K * d.N2}, vv{fld_ptr(d, vf) + (size_t)K * d.N2};
+  const Plane<const double> hh{d.H3 + (size_t)K * d.N2};
+  const Plane<double> pv{d.PV3 + (size_t)K * d.N2};
   double *xv = lds + (size_t)m.g * ni;  // xv[I-1] = filtered vv(J,I)
   double v[4], u0[4], u1[4];
 #pragma unroll
@@ -968,10 +936,10 @@ __device__ __forceinline__ void vort_interior_rows(const MemberDesc &d, double *
     u1[q] = uu[ix2(d, J, I)];
   }
   const bool filt = live && d.rflag_v[J] != 0;
-  if (filter_any(ni, filt)) filter_row_regs(d, v, xv, J, 1, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, v, xv, J, 1, filt, m.lane);
 #pragma unroll
   for (int q = 0; q < 4; q++) xv[m.lane + m.stride * q] = v[q];
-  row_sync(m.stride);
+  row_sync<WIDE>();
   if (!live) return;
   double f2j = d.f[2 * J], m2j = d.m[2 * J], n2j = d.n[2 * J];
   double mm1i = 1. / d.m[2 * J - 1], mp1i = 1. / d.m[2 * J + 1];
@@ -996,9 +964,9 @@ __device__ __forceinline__ void vort_interior_rows(const MemberDesc &d, double *
 // 0/1 form the two zonal sums in the reference's sequential order.  Every
 // lane of the block reaches both barriers.
 __device__ __forceinline__ void vort_pole(const MemberDesc &d, double *row, int K, int north, int uf) {
-  const double *uu = fld_ptr(d, uf) + (size_t)K * d.N2;
-  const double *hh = d.H3 + (size_t)K * d.N2;
-  double *pv = d.PV3 + (size_t)K * d.N2;
+  const Plane<const double> uu{fld_ptr(d, uf) + (size_t)K * d.N2};
+  const Plane<const double> hh{d.H3 + (size_t)K * d.N2};
+  const Plane<double> pv{d.PV3 + (size_t)K * d.N2};
   const int ni = d.ni, nj = d.nj, Jr = north ? nj : 0;
   for (int i = threadIdx.x; i < ni; i += blockDim.x) {
     row[i] = uu[ix2(d, Jr, i + 1)];
@@ -1028,13 +996,14 @@ __device__ __forceinline__ void vort_pole(const MemberDesc &d, double *row, int 
 }
 // DIV of (uu zonally filtered, vv) on plane K: one block per (K,J) h-row
 // group, row J of uu filtered by its lanes (rows of the h-grid filter band)
+template <bool WIDE>
 __device__ __forceinline__ void divergence_rows(const MemberDesc &d, double *lds, int bx, int K, int uf, int vf, int df) {
   const RowMap m = row_map(d.ni);
   const int Jr = bx * m.rpb + m.g, ni = d.ni;
   const bool live = Jr <= d.nj;
   const int J = live ? Jr : 0;
-  const double *uu = fld_ptr(d, uf) + (size_t)K * d.N2, *vv = fld_ptr(d, vf) + (size_t)K * d.N2;
-  double *di = fld_ptr(d, df) + (size_t)K * d.N2;
+  const Plane<const double> uu{fld_ptr(d, uf) + (size_t)K * d.N2}, vv{fld_ptr(d, vf) + (size_t)K * d.N2};
+  const Plane<double> di{fld_ptr(d, df) + (size_t)K * d.N2};
   double *xu = lds + (size_t)m.g * ni;  // xu[I-1] = filtered uu(J,I)
   double u[4], v0[4], v1[4];
 #pragma unroll
@@ -1045,10 +1014,10 @@ __device__ __forceinline__ void divergence_rows(const MemberDesc &d, double *lds
     v1[q] = vv[ix2(d, J + 1, I)];
   }
   const bool filt = live && d.rflag_h[J] != 0;
-  if (filter_any(ni, filt)) filter_row_regs(d, u, xu, J, 0, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, u, xu, J, 0, filt, m.lane);
 #pragma unroll
   for (int q = 0; q < 4; q++) xu[m.lane + m.stride * q] = u[q];
-  row_sync(m.stride);
+  row_sync<WIDE>();
   if (!live) return;
   int jj = 2 * J + 1;
   double n_inv = 1. / d.n[jj], mn = d.mn[jj];
@@ -1065,28 +1034,11 @@ __device__ __forceinline__ void divergence_rows(const MemberDesc &d, double *lds
   }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_vort_interior(const MemberDesc *D, int mb, int uf, int vf, int k0) {
-  MEMBER;
-  extern __shared__ double lds[];
-  vort_interior_rows(d, lds, blockIdx.x, k0 + blockIdx.y, uf, vf);
-}
-__global__ void __launch_bounds__(256) k_vort_poles(const MemberDesc *D, int mb, int uf, int k0) {
-  MEMBER;
-  extern __shared__ double row[];
-  vort_pole(d, row, k0 + (blockIdx.x >> 1), blockIdx.x & 1, uf);
-}
-void L_vorticity(hipStream_t s, const Bucket &b, int uu, int vv, int k0, int k1) {
-  int nK = k1 - k0 + 1;
-  const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_vort_interior, dim3((b.nj + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s, b.D,
-         b.mb, uu, vv, k0);
-  LAUNCH(k_vort_poles, dim3(2 * nK, 1, b.nm), dim3(64), sizeof(double) * (2 * b.ni + 2), s, b.D, b.mb, uu, k0);
-}
-
+template <bool WIDE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_divergence(const MemberDesc *D, int mb, int uf, int vf, int df, int k0) {
   MEMBER;
   extern __shared__ double lds[];
-  divergence_rows(d, lds, blockIdx.x, k0 + blockIdx.y, uf, vf, df);
+  divergence_rows<WIDE>(d, lds, blockIdx.x, k0 + blockIdx.y, uf, vf, df);
 }
 
 // store_diag in one launch: on planes K = 0..nk, blocks [0, nv) form the PV
@@ -1096,12 +1048,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
 // time planes (IT_ZERO <- IT_MINUS2 <- IT_MINUS1 <- IT_ZERO) and advances
 // itime: the step's last use of them was its Adams-Bashforth update, and no
 // block of this launch reads them.
+template <bool WIDE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_store_diag(const MemberDesc *D, int mb, int nv, int nd, int rotate) {
   MEMBER;
   extern __shared__ double lds[];
   const int bx = blockIdx.x, K = blockIdx.y;
-  if (bx < nv) vort_interior_rows(d, lds, bx, K, F_U, F_V);
-  else if (bx < nv + nd) divergence_rows(d, lds, bx - nv, K, F_U, F_V, F_DIV);
+  if (bx < nv) vort_interior_rows<WIDE>(d, lds, bx, K, F_U, F_V);
+  else if (bx < nv + nd) divergence_rows<WIDE>(d, lds, bx - nv, K, F_U, F_V, F_DIV);
   else vort_pole(d, lds, K, bx - nv - nd, F_U);
   if (rotate && bx == 0 && K == 0 && threadIdx.x == 0) {
     MemberDyn *y = d.dyn;
@@ -1116,11 +1069,11 @@ void L_store_diag(hipStream_t s, const Bucket &b, int rotate) {
   const int rpb = rows_per_block(b.ni);
   const int nv = (b.nj + rpb - 1) / rpb, nd = (b.nj + 1 + rpb - 1) / rpb;
   const size_t shm = sizeof(double) * std::max(rpb * b.ni, 2 * b.ni + 2);
-  LAUNCH(k_store_diag, dim3(nv + nd + 2, b.nk + 1, b.nm), dim3(256), shm, s, b.D, b.mb, nv, nd, rotate);
+  ROWS_LAUNCH(b, "k_store_diag", k_store_diag<true>, k_store_diag<false>, dim3(nv + nd + 2, b.nk + 1, b.nm), dim3(256), shm, s, b.D, b.mb, nv, nd, rotate);
 }
 void L_divergence(hipStream_t s, const Bucket &b, int uu, int vv, int dst, int k0, int k1) {
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_divergence, dim3((b.nj + 1 + rpb - 1) / rpb, k1 - k0 + 1, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
+  ROWS_LAUNCH(b, "k_divergence", k_divergence<true>, k_divergence<false>, dim3((b.nj + 1 + rpb - 1) / rpb, k1 - k0 + 1, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
          b.D, b.mb, uu, vv, dst, k0);
 }
 

@@ -58,8 +58,8 @@ __global__ void __launch_bounds__(256) k_uvh_kin(const MemberDesc *D, int mb) {
   MEMBER_X;
   FLAT2_X(0, d.nj + 2, 1, d.ni);
   const int K = 1 + bx_.y;
-  const double *u = d.U + (size_t)K * d.N2, *v = d.V + (size_t)K * d.N2, *h3 = d.H3 + (size_t)K * d.N2;
-  double *uh = d.sA + (size_t)K * d.N2, *vh = d.sB + (size_t)K * d.N2, *kin = d.sC + (size_t)K * d.N2;
+  const Plane<const double> u{d.U + (size_t)K * d.N2}, v{d.V + (size_t)K * d.N2}, h3{d.H3 + (size_t)K * d.N2};
+  const Plane<double> uh{d.sA + (size_t)K * d.N2}, vh{d.sB + (size_t)K * d.N2}, kin{d.sC + (size_t)K * d.N2};
   const int ni = d.ni, nj = d.nj;
   if (J <= nj) {
     double havg = .5 * (h3[ix2(d, J, I)] + h3[ix2(d, J, I - 1)]);
@@ -102,8 +102,8 @@ __global__ void __launch_bounds__(256) k_dvdt_core(const MemberDesc *D, int mb) 
   FLAT2_X(1, d.nj, 1, d.ni);
   const int K = 1 + bx_.y;
   const size_t o = (size_t)K * d.N2;
-  const double *uh = d.sA + o, *vh = d.sB + o, *kin = d.sC + o, *pv = d.PV3 + o;
-  double *dv = cur_tend(d, d.DVDT) + o;
+  const Plane<const double> uh{d.sA + o}, vh{d.sB + o}, kin{d.sC + o}, pv{d.PV3 + o};
+  const Plane<double> dv{cur_tend(d, d.DVDT) + o};
   auto PV = [&](int j, int i) { return pv[ix2(d, j, i)]; };
   const PvW<double> w = pv_weights_v<double>(d.pv_al81, PV, J, I);
   double x = dv[ix2(d, J, I)];
@@ -122,6 +122,7 @@ __global__ void __launch_bounds__(256) k_dvdt_core(const MemberDesc *D, int mb) 
 // DUDT = (DUDT + PV*VH terms + dKIN/dx with filtered KIN) - vertical
 // advection.  One block per (K,J) u-row: the KIN row is zonally filtered in
 // LDS (rows of the filter band) and its pad refreshed, then one lane per I.
+template <bool WIDE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_dudt_core(const MemberDesc *D, int mb) {
   MEMBER;
   extern __shared__ double lds[];
@@ -130,18 +131,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
   const bool live = Jr <= d.nj;
   const int J = live ? Jr : 0;
   const size_t o = (size_t)K * d.N2;
-  const double *uh = d.sA + o, *vh = d.sB + o, *kin = d.sC + o, *pv = d.PV3 + o;
+  const Plane<const double> uh{d.sA + o}, vh{d.sB + o}, kin{d.sC + o}, pv{d.PV3 + o};
   double *kr = lds + (size_t)m.g * ni;  // kr[I-1] = filtered KIN(J,I)
   double kv[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) kv[q] = kin[ix2(d, J, 1 + m.lane + m.stride * q)];
   const bool filt = live && d.rflag_h[J] != 0;
-  if (filter_any(ni, filt)) filter_row_regs(d, kv, kr, J, 0, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, kv, kr, J, 0, filt, m.lane);
 #pragma unroll
   for (int q = 0; q < 4; q++) kr[m.lane + m.stride * q] = kv[q];
-  row_sync(m.stride);
+  row_sync<WIDE>();
   if (!live) return;
-  double *du = cur_tend(d, d.DUDT) + o;
+  const Plane<double> du{cur_tend(d, d.DUDT) + o};
   for (int I = 1 + m.lane; I <= ni; I += m.stride) {
     auto PV = [&](int j, int i) { return pv[ix2(d, j, i)]; };
     const PvW<double> w = pv_weights_u<double>(d.pv_al81, PV, J, I);
@@ -166,7 +167,7 @@ void L_uv_core(hipStream_t s, const Bucket &b) {
   LAUNCH(k_uvh_kin, grid2(b.nj + 2, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   LAUNCH(k_dvdt_core, grid2(b.nj, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_dudt_core, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
+  ROWS_LAUNCH(b, "k_dudt_core", k_dudt_core<true>, k_dudt_core<false>, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
          b.D, b.mb);
 }
 
@@ -492,7 +493,7 @@ __global__ void __launch_bounds__(256) k_divdamp(const MemberDesc *D, int mb) {
   FLAT2_X(0, d.nj + 1, 1, d.ni);
   const int K = 1 + bx_.y;
   if (d.nudiv == 0.) return;
-  const double *div = d.sB + (size_t)K * d.N2;
+  const Plane<const double> div{d.sB + (size_t)K * d.N2};
   double *du = cur_tend(d, d.DUDT), *dv = cur_tend(d, d.DVDT);
   double coef = (d.lat[2 * J + 1] > 45.) ? d.nudiv * d.m0z : d.nudiv * d.m[2 * J + 1];
   du[ix3(d, K, J, I)] += coef * (div[ix2(d, J, I)] - div[ix2(d, J, I - 1)]);
@@ -576,6 +577,7 @@ __global__ void __launch_bounds__(256) k_gz_mono(const MemberDesc *D, int mb) {
 }
 // gz = GZ3 with planes 0..nk-1 zonally filtered (rows of the h-grid band),
 // one block per (K,J) row of the whole plane (J = -1..nj+1), pads included
+template <bool WIDE>
 __global__ void __launch_bounds__(256) k_gz_filtercopy(const MemberDesc *D, int mb) {
   MEMBER;
   extern __shared__ double lds[];
@@ -583,8 +585,8 @@ __global__ void __launch_bounds__(256) k_gz_filtercopy(const MemberDesc *D, int 
   const int Jr = (int)(blockIdx.x * m.rpb + m.g) - 1, K = blockIdx.y, ni = d.ni;
   const bool live = Jr <= d.nj + 1;
   const int J = live ? Jr : 0;
-  const double *src = d.GZ3 + (size_t)K * d.N2;
-  double *dst = d.gz + (size_t)K * d.N2;
+  const Plane<const double> src{d.GZ3 + (size_t)K * d.N2};
+  const Plane<double> dst{d.gz + (size_t)K * d.N2};
   double v[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) v[q] = src[ix2(d, J, 1 + m.lane + m.stride * q)];
@@ -594,7 +596,7 @@ __global__ void __launch_bounds__(256) k_gz_filtercopy(const MemberDesc *D, int 
   if (first) pe = src[ix2(d, J, ni + 1)];
   if (last) pw = src[ix2(d, J, 0)];
   const bool filt = live && K <= d.nk - 1 && J >= 0 && J <= d.nj && d.rflag_h[J] != 0;
-  if (filter_any(ni, filt)) filter_row_regs(d, v, lds + (size_t)m.g * ni, J < 0 ? 0 : J, 0, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, v, lds + (size_t)m.g * ni, J < 0 ? 0 : J, 0, filt, m.lane);
   if (!live) return;
 #pragma unroll
   for (int q = 0; q < 4; q++) dst[ix2(d, J, 1 + m.lane + m.stride * q)] = v[q];
@@ -603,7 +605,7 @@ __global__ void __launch_bounds__(256) k_gz_filtercopy(const MemberDesc *D, int 
 }
 void L_gz_filtercopy(hipStream_t s, const Bucket &b) {
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(k_gz_filtercopy, dim3((b.nj + 3 + rpb - 1) / rpb, b.nk + 2, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
+  ROWS_LAUNCH(b, "k_gz_filtercopy", k_gz_filtercopy<true>, k_gz_filtercopy<false>, dim3((b.nj + 3 + rpb - 1) / rpb, b.nk + 2, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
          b.D, b.mb);
 }
 
@@ -647,8 +649,8 @@ __global__ void __launch_bounds__(256) k_d2dy2_cols(const MemberDesc *D, int mb,
   const int J0 = tile * TJ;
   if (J0 > jmax) return;  // uniform per block (the grid covers the v rows)
   const int I = 1 + chunk * (int)blockDim.x + (int)threadIdx.x;
-  const double *hh = fld_ptr(d, f) + (size_t)K * d.N2;
-  T *out = reinterpret_cast<T *>(d.sB.get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
+  const Plane<const double> hh{fld_ptr(d, f) + (size_t)K * d.N2};
+  const Plane<T> out{reinterpret_cast<T *>(d.sB.get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2};
   const double *cx = vg ? d.vcx : d.hcx, *cy = vg ? d.vcy : d.hcy, *cz = vg ? d.vcz : d.hcz;
   const T c2 = T(d.coef2), c4 = T(d.coef4);
   T w[TJ + 4];  // rows J0-2 .. J0+TJ+1
@@ -696,7 +698,7 @@ __global__ void __launch_bounds__(256) k_d2dy2_cols(const MemberDesc *D, int mb,
 // order's meridional second difference reads (the reference filters it in
 // place, src/shared/epic_subgrid.c:960-975).  Members that do not apply
 // the order leave D and A as they are.
-template <class T>
+template <bool WIDE, class T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_hv_apply(const MemberDesc *D, int mb, int nm, FieldSet fs, int pass, int src) {
   SET_MEMBER;
   extern __shared__ double lds_raw[];
@@ -707,8 +709,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
   if (K > r.k1 || hv_nu(d, pass) == 0. || hv_passes(d) <= pass) return;  // uniform per block
   const bool live = Jr <= d.nj + 1;
   const int J = live ? Jr : 0, ni = d.ni, vg = (kind == 1);
-  double *a = fld_ptr(d, f) + (size_t)K * d.N2;
-  T *dd = reinterpret_cast<T *>((src ? d.sC : d.sB).get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
+  const Plane<double> a{fld_ptr(d, f) + (size_t)K * d.N2};
+  const Plane<T> dd{reinterpret_cast<T *>((src ? d.sC : d.sB).get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2};
   const bool upd = live && J >= r.jbot && J <= d.nj;
   // the row of A and the row of D, all loads in flight together
   double v[4];
@@ -720,7 +722,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
     x[q] = dd[i];
   }
   const bool filt = upd && (vg ? d.rflag_v[J] : d.rflag_h[J]) != 0;
-  if (filter_any(ni, filt)) filter_row_regs(d, x, lds + (size_t)m.g * ni, J, vg, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, x, lds + (size_t)m.g * ni, J, vg, filt, m.lane);
   if (!live) return;
   const bool back = upd && hv_passes(d) > pass + 1;
   const double sign = (pass & 1) ? -1. : 1.;
@@ -752,8 +754,8 @@ __global__ void __launch_bounds__(256) k_d2dy2_pass(const MemberDesc *D, int mb,
   if (t >= (jmax + 1) * d.ni) return;
   const int J = t / d.ni, I = 1 + t - J * d.ni;
   const size_t o = (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
-  const T *hh = reinterpret_cast<const T *>((src ? d.sC : d.sB).get()) + o;
-  T *out = reinterpret_cast<T *>((src ? d.sB : d.sC).get()) + o;
+  const Plane<const T> hh{reinterpret_cast<const T *>((src ? d.sC : d.sB).get()) + o};
+  const Plane<T> out{reinterpret_cast<T *>((src ? d.sB : d.sC).get()) + o};
   const double *cx = vg ? d.vcx : d.hcx, *cy = vg ? d.vcy : d.hcy, *cz = vg ? d.vcz : d.hcz;
   int j0, j1, j2;
   if (J == 0) { j0 = 0; j1 = 1; j2 = 2; }
@@ -794,13 +796,13 @@ static void merid_hv_t(hipStream_t s, const Bucket &b, const FieldSet &fs) {
   d2dy2_del4<T>(s, b, fs);
   const int rpb = rows_per_block(b.ni);
   const dim3 ga((b.nj + 2 + rpb - 1) / rpb, b.nk, fs.n * b.nm);
-  LAUNCH(k_hv_apply<T>, ga, dim3(256), sizeof(T) * rpb * b.ni, s, b.D, b.mb, b.nm, fs, 1, 0);
+  ROWS_LAUNCH(b, "k_hv_apply<T>", (k_hv_apply<true, T>), (k_hv_apply<false, T>), ga, dim3(256), sizeof(T) * rpb * b.ni, s, b.D, b.mb, b.nm, fs, 1, 0);
   // del^6 (pass 2, into sC) and del^8 (pass 3, back into sB)
   const dim3 gp((jrows * b.ni + TPB - 1) / TPB, b.nk, fs.n * b.nm);
   for (int pass = 2; pass < b.hv_passes; pass++) {
     const int src = (pass == 2) ? 0 : 1;
     LAUNCH(k_d2dy2_pass<T>, gp, dim3(TPB), 0, s, b.D, b.mb, b.nm, fs, pass, src);
-    LAUNCH(k_hv_apply<T>, ga, dim3(256), sizeof(T) * rpb * b.ni, s, b.D, b.mb, b.nm, fs, pass, 1 - src);
+    ROWS_LAUNCH(b, "k_hv_apply<T>", (k_hv_apply<true, T>), (k_hv_apply<false, T>), ga, dim3(256), sizeof(T) * rpb * b.ni, s, b.D, b.mb, b.nm, fs, pass, 1 - src);
   }
 }
 void L_merid_hv(hipStream_t s, const Bucket &b, const FieldSet &fs) {
@@ -983,17 +985,11 @@ __device__ __forceinline__ float mean_butterfly(float p, int ni) {
 // otherwise sums left to right, as the reference and k_zonal_hv form them,
 // each lane of a row forming the same sum itself (which spares a barrier
 // to hand it round).
-template <class T, bool BFLY>
+template <bool WIDE, class T, bool BFLY>
 __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, int nm, FieldSet fs) {
   SET_MEMBER;
   extern __shared__ double lds_raw[];
   const RowMap m = row_map(d.ni);
-  // a row's lanes exchange data only among themselves: within one
-  // wavefront when ni <= 256, so a wavefront barrier suffices there
-  auto row_bar = [&]() {
-    if (m.stride <= 64) wave_sync();
-    else __syncthreads();
-  };
   const int ni = d.ni, WS = ni + 2;
   T *z0 = reinterpret_cast<T *>(lds_raw) + (size_t)m.g * 3 * WS, *z1 = z0 + WS, *z2 = z1 + WS;
   HvRange r = hv_range(d, kind);
@@ -1001,8 +997,8 @@ __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, i
   if (K > r.k1 || hv_passes(d) != 2) return;  // uniform per block
   const bool live = Jr <= d.nj + 1;
   const int J = live ? Jr : 0, vg = (kind == 1);
-  double *a = fld_ptr(d, f) + (size_t)K * d.N2;
-  const T *dd = reinterpret_cast<const T *>(d.sB.get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2;
+  const Plane<double> a{fld_ptr(d, f) + (size_t)K * d.N2};
+  const Plane<const T> dd{reinterpret_cast<const T *>(d.sB.get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2};
   const bool upd = live && J >= r.jbot && J <= d.nj;
   // the row of A and the row of D, both loads in flight together
   double v[4];
@@ -1016,7 +1012,7 @@ __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, i
   // the meridional part: D filtered (work = z1) where the row's wavefront or
   // block holds a row of the filter band
   const bool filt = upd && (vg ? d.rflag_v : d.rflag_h)[J] != 0;
-  if (filter_any(ni, filt)) filter_row_regs(d, dq, z1, J, vg, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, dq, z1, J, vg, filt, m.lane);
   const double sign = -1.;  // del^4
 #pragma unroll
   for (int q = 0; q < 4; q++)
@@ -1034,7 +1030,7 @@ __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, i
   const int Jc = min(J, d.nj);
   const double mm = fabs(d.lat[2 * Jc + r.jh]) > 45. ? d.m0z : d.m[2 * Jc + r.jh];
   T y[4];
-  row_bar();
+  row_sync<WIDE>();
   for (int pass = 0; pass < 2; pass++) {
     // pass 0 reads z0 and leaves its raw result in z1; pass 1 reads z2 (pass
     // 0 less its mean) and leaves its raw result in z0
@@ -1047,7 +1043,7 @@ __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, i
       y[q] = dcu * (xin[I - 1] - T(2.) * xin[I] + xin[I + 1]);
       raw[I] = y[q];
     }
-    row_bar();
+    row_sync<WIDE>();
     T fm;
     if constexpr (BFLY) {
       // each wavefront of the row's lanes forms the 64 partials itself
@@ -1068,7 +1064,7 @@ __global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, i
         if (I == ni) z2[0] = y[q];
         if (I == 1) z2[ni + 1] = y[q];
       }
-      row_bar();
+      row_sync<WIDE>();
     }
   }
   if (!live) return;
@@ -1097,8 +1093,9 @@ static void hv4_mixed(hipStream_t s, const Bucket &b, const FieldSet &fs) {
   const int rpb = rows_per_block(b.ni);
   const dim3 ga((b.nj + 2 + rpb - 1) / rpb, b.nk, fs.n * b.nm);
   const size_t shm = sizeof(T) * rpb * 3 * (b.ni + 2);
-  if (b.ni >= 256) LAUNCH_AS("k_hv4_rows", (k_hv4_rows<T, true>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
-  else LAUNCH_AS("k_hv4_rows", (k_hv4_rows<T, false>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
+  if (b.ni > 256) LAUNCH_AS("k_hv4_rows", (k_hv4_rows<true, T, true>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
+  else if (b.ni == 256) LAUNCH_AS("k_hv4_rows", (k_hv4_rows<false, T, true>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
+  else LAUNCH_AS("k_hv4_rows", (k_hv4_rows<false, T, false>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
 }
 void L_hv(hipStream_t s, const Bucket &b, const FieldSet &fs) {
   if (b.mixed && b.hv_passes == 2 && b.ni >= 16 && b.ni <= 1024) {

@@ -21,93 +21,6 @@ namespace epic {
 
 #define MEMBER const MemberDesc &d = D[mb + blockIdx.z]
 
-template <class T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_fft_filter(const MemberDesc *D, int mb, int f, int k0, int kn, int vgrid,
-                                                    int pads) {
-  MEMBER;
-  extern __shared__ double lds_raw[];
-  T *lds = reinterpret_cast<T *>(lds_raw);
-  const int n = d.ni, nq = n >> 2, RB = TPB / nq;
-  const int rs = threadIdx.x / nq, lane = threadIdx.x - rs * nq;
-  const int nrows = vgrid ? d.nrow_v : d.nrow_h;
-  const int r = blockIdx.x * RB + rs;
-  const bool active = r < nrows;
-  const int J = active ? (vgrid ? d.rows_v[r] : d.rows_h[r]) : 0;
-  // planes k0..k0+kn-1 of each of gridDim.y/kn contiguous copies of the array
-  const int copy = blockIdx.y / kn, K = k0 + blockIdx.y - copy * kn;
-  T *a = fld_ptr_t<T>(d, f) + (size_t)copy * d.N3 + (size_t)K * d.N2;
-  T *buf = lds + (size_t)rs * n;
-  const int bits = d.nlogn - 1;
-  const double *hl = (vgrid ? d.hl_pv : d.hl_h) + (size_t)J * (n / 2 + 2);
-  LaneTw<T> tf, ti;
-  load_tw(tf, tw_fwd<T>(d), tr_fwd<T>(d), n, lane);
-  load_tw(ti, tw_inv<T>(d), tr_inv<T>(d), n, lane);
-  T gain[4];
-  if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) {
-      int gi = (e == 0) ? 1 : (e == 1 ? n / 2 + 1 : (e >> 1) + 1);
-      gain[q] = T(hl[gi]);
-      int k = e >> 1, c = e & 1;
-      buf[(brev(k, bits) << 1) | c] = a[ix2(d, J, e + 1)];
-    }
-  row_sync(nq);
-  four1_stages(buf, n, lane, tf, active);
-  split_step(buf, n, lane, tf, T(-0.5), active);
-  if (active && lane == 0) {
-    T h1r;
-    buf[0] = (h1r = buf[0]) + buf[1];
-    buf[1] = h1r - buf[1];
-  }
-  row_sync(nq);
-  if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) buf[e] *= gain[q];
-  row_sync(nq);
-  split_step(buf, n, lane, ti, T(0.5), active);
-  if (active && lane == 0) {
-    T h1r;
-    buf[0] = T(0.5) * ((h1r = buf[0]) + buf[1]);
-    buf[1] = T(0.5) * (h1r - buf[1]);
-  }
-  row_sync(nq);
-  T v[4];
-  if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) v[q] = buf[e];
-  row_sync(nq);
-  if (active)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) {
-      int k = e >> 1, c = e & 1;
-      buf[(brev(k, bits) << 1) | c] = v[q];
-    }
-  row_sync(nq);
-  four1_stages(buf, n, lane, ti, active);
-  if (active)
-    for (int e = lane; e < n; e += nq) {
-      const T y = buf[e] * T(2. / (n));
-      a[ix2(d, J, e + 1)] = y;
-      if (pads && e == n - 1) a[ix2(d, J, 0)] = y;
-      if (pads && e == 0) a[ix2(d, J, n + 1)] = y;
-    }
-}
-
-template <class T>
-static void launch_fft(hipStream_t s, const Bucket &b, int f, int k0, int k1, int vgrid, int pads, int copies) {
-  const int n = b.ni, nq = n / 4, RB = TPB / nq;
-  const int rows = b.nj + 1;  // upper bound on the listed rows
-  dim3 g((rows + RB - 1) / RB, (k1 - k0 + 1) * copies, b.nm);
-  size_t shm = sizeof(T) * (size_t)RB * n;
-  LAUNCH(k_fft_filter<T>, g, dim3(TPB), shm, s, b.D, b.mb, f, k0, k1 - k0 + 1, vgrid, pads);
-}
-
-// mode 0: also refresh the zonal pads of the filtered rows (the producers of
-// every filtered copy write the pads of the rows they fill); mode 1: no pads
-void L_filter(hipStream_t s, const Bucket &b, int f, int k0, int k1, int vgrid, int mode, int copies) {
-  launch_fft<double>(s, b, f, k0, k1, vgrid, mode == 0, copies);
-}
-// the same on an FP32 array (mixed precision)
-void L_filter_f32(hipStream_t s, const Bucket &b, int f, int k0, int k1, int vgrid, int mode, int copies) {
-  launch_fft<float>(s, b, f, k0, k1, vgrid, mode == 0, copies);
-}
-
 // ------------------------------------------------------------- 3-D form
 __device__ __forceinline__ double geez(const MemberDesc &d, int kind, int K, int J, int I) {
   const double *gz = d.gz;
@@ -255,7 +168,7 @@ __global__ void __launch_bounds__(256) k_spline_prep(const MemberDesc *D, int mb
 // band come out as (a - v) + v, as in the reference, which subtracts and adds
 // the profile on every row.  HDRY is stored with the restore_mass that
 // follows the filters in the step.  RB rows per block, ni/4 lanes per row.
-template <class T, bool F>
+template <bool WIDE, class T, bool F>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k_filter3(const MemberDesc *D, int mb, int nm, FieldSet fs) {
   SET_MEMBER;
   extern __shared__ double lds_raw[];
@@ -274,8 +187,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
   T *buf = reinterpret_cast<T *>(tabs + (size_t)RB * 5 * KT) + (size_t)rs * n;
   if (live)
     for (int e = lane; e < 3 * KT; e += nq) tab[e] = d.spl[(size_t)(fi * (d.nj + 2) + J) * 3 * KT + e];
-  row_sync(nq);
-  T *a = fld_ptr_t<T>(d, f) + (size_t)K * d.N2;
+  row_sync<WIDE>();
+  const Plane<T> a{fld_ptr_t<T>(d, f) + (size_t)K * d.N2};
   const double *tx = tab, *ty = tab + KT, *tz = tab + 2 * KT;
   // the cubic of each interval k depends on the table alone (splint_pchip,
   // src/shared/epic_funcs_util.c:926-999): its coefficients are formed once
@@ -290,7 +203,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
       tc3[k] = (e1 + e2) / h;
       tc2[k] = -(e1 + e1 + e2);
     }
-  row_sync(nq);
+  row_sync<WIDE>();
   double v[4];
   T x[4];
   if (live)
@@ -318,36 +231,36 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
       int kq = e >> 1, c = e & 1;
       buf[(brev(kq, bits) << 1) | c] = x[q];
     }
-  row_sync(nq);
-  four1_stages(buf, n, lane, tf, filt);
-  split_step(buf, n, lane, tf, T(-0.5), filt);
+  row_sync<WIDE>();
+  four1_stages<WIDE>(buf, n, lane, tf, filt);
+  split_step<WIDE>(buf, n, lane, tf, T(-0.5), filt);
   if (filt && lane == 0) {
     T h1r;
     buf[0] = (h1r = buf[0]) + buf[1];
     buf[1] = h1r - buf[1];
   }
-  row_sync(nq);
+  row_sync<WIDE>();
   if (filt)
     for (int q = 0, e = lane; q < 4; q++, e += nq) buf[e] *= gain[q];
-  row_sync(nq);
-  split_step(buf, n, lane, ti, T(0.5), filt);
+  row_sync<WIDE>();
+  split_step<WIDE>(buf, n, lane, ti, T(0.5), filt);
   if (filt && lane == 0) {
     T h1r;
     buf[0] = T(0.5) * ((h1r = buf[0]) + buf[1]);
     buf[1] = T(0.5) * (h1r - buf[1]);
   }
-  row_sync(nq);
+  row_sync<WIDE>();
   T w[4];
   if (filt)
     for (int q = 0, e = lane; q < 4; q++, e += nq) w[q] = buf[e];
-  row_sync(nq);
+  row_sync<WIDE>();
   if (filt)
     for (int q = 0, e = lane; q < 4; q++, e += nq) {
       int kq = e >> 1, c = e & 1;
       buf[(brev(kq, bits) << 1) | c] = w[q];
     }
-  row_sync(nq);
-  four1_stages(buf, n, lane, ti, filt);
+  row_sync<WIDE>();
+  four1_stages<WIDE>(buf, n, lane, ti, filt);
   if (filt)
     for (int q = 0, e = lane; q < 4; q++, e += nq) x[q] = buf[e] * T(2. / (n));
   // hdry leaves with restore_mass applied (max(h_min, h), every cell of
@@ -372,8 +285,8 @@ void L_filter3(hipStream_t s, const Bucket &b, const FieldSet &fs) {
   const int nq = b.ni / 4, RB = (256 / nq) < 16 ? (256 / nq) : 16;
   dim3 g((nrow + RB - 1) / RB, b.nk, nz);
   size_t shm = sizeof(double) * (size_t)RB * 5 * (b.nk + 2) + sizeof(double) * (size_t)RB * b.ni;
-  if (b.mixed) LAUNCH_AS("k_filter3<double>", (k_filter3<double, true>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
-  else LAUNCH_AS("k_filter3<double>", (k_filter3<double, false>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
+  if (b.mixed) ROWS_LAUNCH(b, "k_filter3<double>", (k_filter3<true, double, true>), (k_filter3<false, double, true>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
+  else ROWS_LAUNCH(b, "k_filter3<double>", (k_filter3<true, double, false>), (k_filter3<false, double, false>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
 }
 
 }  // namespace epic

@@ -58,8 +58,8 @@ __global__ void __launch_bounds__(256) km_uvh_kin(const MemberDesc *D, int mb) {
   FLAT2_X(0, d.nj + 2, 1, d.ni);
   const int K = 1 + bx_.y;
   const size_t o = (size_t)K * d.N2;
-  const double *u = d.U + o, *v = d.V + o, *h3 = d.H3 + o;
-  float *uh = sAf(d) + o, *vh = sBf(d) + o, *kin = sCf(d) + o;
+  const Plane<const double> u{d.U + o}, v{d.V + o}, h3{d.H3 + o};
+  const Plane<float> uh{sAf(d) + o}, vh{sBf(d) + o}, kin{sCf(d) + o};
   const int ni = d.ni, nj = d.nj;
   if (J <= nj) {
     float havg = .5f * ((float)h3[ix2(d, J, I)] + (float)h3[ix2(d, J, I - 1)]);
@@ -101,9 +101,9 @@ __global__ void __launch_bounds__(256) km_dvdt_core(const MemberDesc *D, int mb)
   FLAT2_X(1, d.nj, 1, d.ni);
   const int K = 1 + bx_.y;
   const size_t o = (size_t)K * d.N2;
-  const float *uh = sAf(d) + o, *vh = sBf(d) + o, *kin = sCf(d) + o;
-  const double *pv = d.PV3 + o;
-  double *dv = curV(d) + o;
+  const Plane<const float> uh{sAf(d) + o}, vh{sBf(d) + o}, kin{sCf(d) + o};
+  const Plane<const double> pv{d.PV3 + o};
+  const Plane<double> dv{curV(d) + o};
   auto PV = [&](int j, int i) { return (float)pv[ix2(d, j, i)]; };
   const PvW<float> w = pv_weights_v<float>(d.pv_al81, PV, J, I);
   float t = -w.ga * uh[ix2(d, J, I + 1)] - w.de * uh[ix2(d, J, I)] - w.al * uh[ix2(d, J - 1, I)] -
@@ -120,6 +120,7 @@ __global__ void __launch_bounds__(256) km_dvdt_core(const MemberDesc *D, int mb)
 // One block per (K,J) u-row group: the row of KIN is zonally filtered in
 // LDS (rows of the filter band, the FP32 filter of the 2-D zonal filter),
 // then one lane per I forms the u tendency, as k_dudt_core does in FP64.
+template <bool WIDE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) km_dudt_core(const MemberDesc *D, int mb) {
   MEMBER;
   extern __shared__ double lds_raw[];
@@ -129,19 +130,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
   const bool live = Jr <= d.nj;
   const int J = live ? Jr : 0;
   const size_t o = (size_t)K * d.N2;
-  const float *uh = sAf(d) + o, *vh = sBf(d) + o, *kin = sCf(d) + o;
+  const Plane<const float> uh{sAf(d) + o}, vh{sBf(d) + o}, kin{sCf(d) + o};
   float *kr = lds + (size_t)m.g * ni;  // kr[I-1] = filtered KIN(J,I)
   float kv[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) kv[q] = kin[ix2(d, J, 1 + m.lane + m.stride * q)];
   const bool filt = live && d.rflag_h[J] != 0;
-  if (filter_any(ni, filt)) filter_row_regs(d, kv, kr, J, 0, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, kv, kr, J, 0, filt, m.lane);
 #pragma unroll
   for (int q = 0; q < 4; q++) kr[m.lane + m.stride * q] = kv[q];
-  row_sync(m.stride);
+  row_sync<WIDE>();
   if (!live) return;
-  const double *pv = d.PV3 + o;
-  double *du = curU(d) + o;
+  const Plane<const double> pv{d.PV3 + o};
+  const Plane<double> du{curU(d) + o};
   const int kk = 2 * K + 1;
   const float ds_inv = (float)(1. / (d.sgth[kk - 2] - d.sgth[kk + 2])), mj = (float)d.m[2 * J + 1];
   for (int I = 1 + m.lane; I <= ni; I += m.stride) {
@@ -259,7 +260,7 @@ __global__ void __launch_bounds__(256) km_divdamp(const MemberDesc *D, int mb) {
   FLAT2(0, d.nj + 1, 1, d.ni);
   const int K = 1 + blockIdx.y;
   if (d.nudiv == 0.) return;
-  const double *div = d.sB + (size_t)K * d.N2;
+  const Plane<const double> div{d.sB + (size_t)K * d.N2};
   double *du = curU(d), *dv = curV(d);
   float coef = (float)((d.lat[2 * J + 1] > 45.) ? d.nudiv * d.m0z : d.nudiv * d.m[2 * J + 1]);
   du[ix3(d, K, J, I)] += (double)(coef * (float)(div[ix2(d, J, I)] - div[ix2(d, J, I - 1)]));
@@ -313,7 +314,7 @@ void LM_uv_core(hipStream_t s, const Bucket &b) {
   LAUNCH(km_uvh_kin, grid2(b.nj + 2, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   LAUNCH(km_dvdt_core, grid2(b.nj, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   const int rpb = rows_per_block(b.ni);
-  LAUNCH(km_dudt_core, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(float) * rpb * b.ni, s,
+  ROWS_LAUNCH(b, "km_dudt_core", km_dudt_core<true>, km_dudt_core<false>, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(float) * rpb * b.ni, s,
          b.D, b.mb);
 }
 void LM_uv_drag(hipStream_t s, const Bucket &b) {

@@ -81,11 +81,8 @@ void L_richardson(hipStream_t s, const Bucket &b);
 void L_gz_from_u(hipStream_t s, const Bucket &b);
 void L_gz3(hipStream_t s, const Bucket &b);
 void L_dzdt3(hipStream_t s, const Bucket &b);
-void L_bc3(hipStream_t s, const Bucket &b, int fld);
 void L_heating(hipStream_t s, const Bucket &b, int adjust, bool in_thermo);
 void L_calc_w(hipStream_t s, const Bucket &b, int with_source);
-void L_copy_planes(hipStream_t s, const Bucket &b, int src, int dst, int k0, int k1);
-void L_vorticity(hipStream_t s, const Bucket &b, int uu, int vv, int k0, int k1);
 void L_divergence(hipStream_t s, const Bucket &b, int uu, int vv, int dst, int k0, int k1);
 // store_diag (PV3 and DIV_UV3 of U, V on K = 0..nk) in one launch; rotate:
 // also rotate the time planes and advance itime (the step's last action)
@@ -94,11 +91,6 @@ void L_store_diag(hipStream_t s, const Bucket &b, int rotate);
 void L_thermo(hipStream_t s, const Bucket &b);
 
 // ---- zonal filter (k_filter.hip)
-// 2-D filter of planes k0..k1 of fld; vgrid selects the v/pv rows; mode 0
-// also refreshes the zonal pads of every row, mode 1 leaves pads alone;
-// copies > 1 filters the same planes of that many consecutive 3-D copies.
-void L_filter(hipStream_t s, const Bucket &b, int fld, int k0, int k1, int vgrid, int mode, int copies = 1);
-void L_filter_f32(hipStream_t s, const Bucket &b, int fld, int k0, int k1, int vgrid, int mode, int copies = 1);
 // the 3-D filter with the PCHIP profile removal, on every field of the set
 void L_filter3(hipStream_t s, const Bucket &b, const FieldSet &fs);
 
