@@ -1,7 +1,8 @@
 // filter_row.h -- the polar-filter transform shared by the kernels that
 // filter rows: the NR real FFT of src/shared/epic_funcs_util.c:4023-4135
 // (four1 stages and the realft split step, with the twiddles of the
-// reference's recurrences tabulated on the host), one butterfly per lane,
+// reference's recurrences tabulated on the host; the stage-s twiddle m is
+// complex entry 2^s - 1 + m), one butterfly per lane,
 // and filter_row_regs(), which filters one latitude row held by its lanes
 // inside a consumer kernel (src/shared/epic_adjust.c:102-242, TWODIM).
 #pragma once
@@ -21,25 +22,6 @@ template <bool WIDE>
 __device__ __forceinline__ void row_sync() {
   if constexpr (WIDE) __syncthreads();
   else wave_sync();
-}
-
-// The stage twiddles stay in their table (global, cache-resident: the
-// stage-s twiddle m is complex entry 2^s - 1 + m); the lane's split-step
-// twiddle is held in registers.
-constexpr int MAX_STAGES = 9;  // n <= 1024: stages with 2 << s < n
-
-template <class T>
-struct LaneTw {
-  const T *tw;  // stage twiddles
-  T sr, si;     // split-step twiddle of this lane
-};
-
-template <class T>
-__device__ __forceinline__ void load_tw(LaneTw<T> &t, const T *tw, const T *tr, int n, int lane) {
-  t.tw = tw;
-  const bool on = lane < n / 4 - 1;
-  t.sr = on ? tr[2 * lane] : T(0);
-  t.si = on ? tr[2 * lane + 1] : T(0);
 }
 
 // one radix-2 butterfly of the reference's four1 on (xr, xi) and (yr, yi)
@@ -77,8 +59,7 @@ template <> __device__ __forceinline__ const float *tr_inv<float>(const MemberDe
 // lanes take part in a pair of stages; an odd last stage runs one butterfly
 // per lane on n/4 lanes.
 template <bool WIDE, class T>
-__device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const LaneTw<T> &t, bool active) {
-  const T *tw = t.tw;
+__device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const T *tw, bool active) {
   int S = 0;
   while ((2 << S) < n) S++;  // stages s with 2 << s < n
   int s = 0;
@@ -123,25 +104,50 @@ __device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const Lane
   }
 }
 
-// split step of the real transform; c2 = -0.5 forward, +0.5 inverse
-template <bool WIDE, class T>
-__device__ __forceinline__ void split_step(T *buf, int n, int lane, const LaneTw<T> &t, T c2, bool active) {
+// One lane's four values between the forward and the inverse transform: the
+// split step of the forward real transform, the filter's gains and the split
+// step of the inverse.  Unit l < n/4-1 holds the complex elements k = l+1
+// (ar, ai) and n/2-k (br, bi), which the split steps mix with each other and
+// with nothing else; unit n/4-1 holds what they leave alone, the pair of DC
+// and Nyquist (ar, ai) and the middle element n/4 (br, bi).  One pass over the
+// row instead of five (split, DC, gains, split, DC), every value by the same
+// operations in the same order.
+__device__ __forceinline__ int unit_k(int n, int l) { return (l == n / 4 - 1) ? 0 : l + 1; }
+__device__ __forceinline__ int unit_kb(int n, int l) { return (l == n / 4 - 1) ? n / 4 : n / 2 - (l + 1); }
+template <class T>
+__device__ __forceinline__ void split_mix(T &ar, T &ai, T &br, T &bi, T wr, T wi, T c2) {
   const T c1 = T(0.5);
-  if (active && lane < n / 4 - 1) {
-    int i = lane + 2;
-    int i1 = i + i - 1, i2 = 1 + i1, i3 = n + 3 - i2, i4 = 1 + i3;
-    i1--; i2--; i3--; i4--;
-    T wr = t.sr, wi = t.si;
-    T h1r = c1 * (buf[i1] + buf[i3]);
-    T h1i = c1 * (buf[i2] - buf[i4]);
-    T h2r = -c2 * (buf[i2] + buf[i4]);
-    T h2i = c2 * (buf[i1] - buf[i3]);
-    buf[i1] = h1r + wr * h2r - wi * h2i;
-    buf[i2] = h1i + wr * h2i + wi * h2r;
-    buf[i3] = h1r - wr * h2r + wi * h2i;
-    buf[i4] = -h1i + wr * h2i + wi * h2r;
+  const T h1r = c1 * (ar + br), h1i = c1 * (ai - bi), h2r = -c2 * (ai + bi), h2i = c2 * (ar - br);
+  ar = h1r + wr * h2r - wi * h2i;
+  ai = h1i + wr * h2i + wi * h2r;
+  br = h1r - wr * h2r + wi * h2i;
+  bi = -h1i + wr * h2i + wi * h2r;
+}
+template <class T>
+__device__ __forceinline__ void split_gain(T &ar, T &ai, T &br, T &bi, int n, int l, const T *trf, const T *tri,
+                                           const double *hl) {
+  if (l < n / 4 - 1) {
+    const T g1 = T(hl[l + 2]), g2 = T(hl[n / 2 - l]);
+    const T wr = trf[2 * l], wi = trf[2 * l + 1], vr = tri[2 * l], vi = tri[2 * l + 1];
+    split_mix(ar, ai, br, bi, wr, wi, T(-0.5));
+    ar *= g1;
+    ai *= g1;
+    br *= g2;
+    bi *= g2;
+    split_mix(ar, ai, br, bi, vr, vi, T(0.5));
+  } else {
+    const T g0 = T(hl[1]), gn = T(hl[n / 2 + 1]), gm = T(hl[n / 4 + 1]);
+    T h1r = ar;
+    ar = h1r + ai;
+    ai = h1r - ai;
+    ar *= g0;
+    ai *= gn;
+    h1r = ar;
+    ar = T(0.5) * (h1r + ai);
+    ai = T(0.5) * (h1r - ai);
+    br *= gm;
+    bi *= gm;
   }
-  row_sync<WIDE>();
 }
 
 // Rows per block of the row kernels: a row takes ni/4 lanes (the transform
@@ -193,51 +199,34 @@ template <bool WIDE, class T>
 __device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], T *work, int J, int vgrid, bool active,
                                                 int lane) {
   const int n = d.ni, nq = n >> 2, bits = d.nlogn - 1;
-  LaneTw<T> tf, ti;
-  load_tw(tf, tw_fwd<T>(d), tr_fwd<T>(d), n, lane);
-  load_tw(ti, tw_inv<T>(d), tr_inv<T>(d), n, lane);
   const double *hl = (vgrid ? d.hl_pv : d.hl_h) + (size_t)J * (n / 2 + 2);
-  T gain[4];
-  int rev[4];
+  if (active)
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int e = lane + q * nq;
-    rev[q] = (brev(e >> 1, bits) << 1) | (e & 1);
-    if (active) {
-      const int gi = (e == 0) ? 1 : (e == 1 ? n / 2 + 1 : (e >> 1) + 1);
-      gain[q] = T(hl[gi]);
-      work[rev[q]] = v[q];
+    for (int q = 0; q < 4; q++) {
+      const int e = lane + q * nq;
+      work[(brev(e >> 1, bits) << 1) | (e & 1)] = v[q];
     }
+  row_sync<WIDE>();
+  four1_stages<WIDE>(work, n, lane, tw_fwd<T>(d), active);
+  const int ka = unit_k(n, lane), kb = unit_kb(n, lane);
+  T ar, ai, br, bi;
+  if (active) {
+    ar = work[2 * ka];
+    ai = work[2 * ka + 1];
+    br = work[2 * kb];
+    bi = work[2 * kb + 1];
+    split_gain(ar, ai, br, bi, n, lane, tr_fwd<T>(d), tr_inv<T>(d), hl);
   }
   row_sync<WIDE>();
-  four1_stages<WIDE>(work, n, lane, tf, active);
-  split_step<WIDE>(work, n, lane, tf, T(-0.5), active);
-  if (active && lane == 0) {
-    T h1r;
-    work[0] = (h1r = work[0]) + work[1];
-    work[1] = h1r - work[1];
+  if (active) {
+    const int pa = brev(ka, bits) << 1, pb = brev(kb, bits) << 1;
+    work[pa] = ar;
+    work[pa + 1] = ai;
+    work[pb] = br;
+    work[pb + 1] = bi;
   }
   row_sync<WIDE>();
-  if (active)
-#pragma unroll
-    for (int q = 0; q < 4; q++) work[lane + q * nq] *= gain[q];
-  row_sync<WIDE>();
-  split_step<WIDE>(work, n, lane, ti, T(0.5), active);
-  if (active && lane == 0) {
-    T h1r;
-    work[0] = T(0.5) * ((h1r = work[0]) + work[1]);
-    work[1] = T(0.5) * (h1r - work[1]);
-  }
-  row_sync<WIDE>();
-  if (active)
-#pragma unroll
-    for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq];
-  row_sync<WIDE>();
-  if (active)
-#pragma unroll
-    for (int q = 0; q < 4; q++) work[rev[q]] = v[q];
-  row_sync<WIDE>();
-  four1_stages<WIDE>(work, n, lane, ti, active);
+  four1_stages<WIDE>(work, n, lane, tw_inv<T>(d), active);
   if (active)
 #pragma unroll
     for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq] * T(2. / (n));

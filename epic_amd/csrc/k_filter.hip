@@ -178,17 +178,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
   if (K > r.kend) return;  // uniform per block
   const int n = d.ni, nq = n >> 2, RB = blockDim.x / nq;
   const int rs = threadIdx.x / nq, lane = threadIdx.x - rs * nq;
-  const int J = r.jstart + blockIdx.x * RB + rs;
-  const bool live = J <= d.nj;
+  const int Jr = r.jstart + blockIdx.x * RB + rs;
+  const bool live = Jr <= d.nj;
+  const int J = live ? Jr : d.nj;
   const int vg = (kind == 1);
   const bool filt = live && (vg ? d.rflag_v[J] : d.rflag_h[J]);
   const int KT = d.nk + 2, nt = r.kend - r.kstart + 1;
   double *tab = tabs + (size_t)rs * 5 * KT;
   T *buf = reinterpret_cast<T *>(tabs + (size_t)RB * 5 * KT) + (size_t)rs * n;
-  if (live)
-    for (int e = lane; e < 3 * KT; e += nq) tab[e] = d.spl[(size_t)(fi * (d.nj + 2) + J) * 3 * KT + e];
-  row_sync<WIDE>();
+  // the lane's four points and their filtered geopotential, on their way
+  // while the row's table is set up
   const Plane<T> a{fld_ptr_t<T>(d, f) + (size_t)K * d.N2};
+  double xx[4];
+  T x[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int I = lane + q * nq + 1;
+    xx[q] = geez(d, kind, K, J, I);
+    x[q] = a[ix2(d, J, I)];
+  }
+  for (int e = lane; e < 3 * KT; e += nq) tab[e] = d.spl[(size_t)(fi * (d.nj + 2) + J) * 3 * KT + e];
+  row_sync<WIDE>();
   const double *tx = tab, *ty = tab + KT, *tz = tab + 2 * KT;
   // the cubic of each interval k depends on the table alone (splint_pchip,
   // src/shared/epic_funcs_util.c:926-999): its coefficients are formed once
@@ -205,69 +215,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
     }
   row_sync<WIDE>();
   double v[4];
-  T x[4];
   if (live)
+#pragma unroll
     for (int q = 0; q < 4; q++) {
-      const int I = lane + q * nq + 1;
-      double xx = geez(d, kind, K, J, I), h;
+      double h;
       // entry e of the table is level kend - e of the column at Imin
-      int k = near ? table_place_near(nt, tx, xx, r.kend - K, &h) : table_place(nt, tx, xx, &h);
-      double xr = xx - tx[k];
+      int k = near ? table_place_near(nt, tx, xx[q], r.kend - K, &h) : table_place(nt, tx, xx[q], &h);
+      double xr = xx[q] - tx[k];
       double val = ty[k] + xr * (tz[k] + xr * (tc2[k] + xr * tc3[k]));
       if (kind == 2) val = m_exp<F>(val);
       v[q] = val;
-      x[q] = T((double)a[ix2(d, J, I)] - val);
+      x[q] = T((double)x[q] - val);
     }
-  LaneTw<T> tf, ti;
-  load_tw(tf, tw_fwd<T>(d), tr_fwd<T>(d), n, lane);
-  load_tw(ti, tw_inv<T>(d), tr_inv<T>(d), n, lane);
-  const int bits = d.nlogn - 1;
-  const double *hl = (vg ? d.hl_pv : d.hl_h) + (size_t)(live ? J : 0) * (n / 2 + 2);
-  T gain[4];
-  if (filt)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) {
-      int gi = (e == 0) ? 1 : (e == 1 ? n / 2 + 1 : (e >> 1) + 1);
-      gain[q] = T(hl[gi]);
-      int kq = e >> 1, c = e & 1;
-      buf[(brev(kq, bits) << 1) | c] = x[q];
-    }
-  row_sync<WIDE>();
-  four1_stages<WIDE>(buf, n, lane, tf, filt);
-  split_step<WIDE>(buf, n, lane, tf, T(-0.5), filt);
-  if (filt && lane == 0) {
-    T h1r;
-    buf[0] = (h1r = buf[0]) + buf[1];
-    buf[1] = h1r - buf[1];
-  }
-  row_sync<WIDE>();
-  if (filt)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) buf[e] *= gain[q];
-  row_sync<WIDE>();
-  split_step<WIDE>(buf, n, lane, ti, T(0.5), filt);
-  if (filt && lane == 0) {
-    T h1r;
-    buf[0] = T(0.5) * ((h1r = buf[0]) + buf[1]);
-    buf[1] = T(0.5) * (h1r - buf[1]);
-  }
-  row_sync<WIDE>();
-  T w[4];
-  if (filt)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) w[q] = buf[e];
-  row_sync<WIDE>();
-  if (filt)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) {
-      int kq = e >> 1, c = e & 1;
-      buf[(brev(kq, bits) << 1) | c] = w[q];
-    }
-  row_sync<WIDE>();
-  four1_stages<WIDE>(buf, n, lane, ti, filt);
-  if (filt)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) x[q] = buf[e] * T(2. / (n));
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, x, buf, J, vg, filt, lane);
   // hdry leaves with restore_mass applied (max(h_min, h), every cell of
   // K = 1..nk, J = 0..nj, I = 0..ni+1 is written here)
   const double hmin = (kind == 2) ? d.h_min[K] : 0.;
   if (live)
-    for (int q = 0, e = lane; q < 4; q++, e += nq) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int e = lane + q * nq;
       T out = T((double)x[q] + v[q]);
       if (kind == 2) out = T(dmax(hmin, (double)out));
       a[ix2(d, J, e + 1)] = out;
