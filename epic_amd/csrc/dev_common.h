@@ -465,6 +465,7 @@ __device__ __forceinline__ T seq_acc(const T *a, int n, T s = T(0)) {
     T x[8], y[8];
 #pragma unroll
     for (int u = 0; u < 8; u++) x[u] = a[u];
+#pragma unroll 1
     for (; i + 24 <= n; i += 16) {
 #pragma unroll
       for (int u = 0; u < 8; u++) y[u] = a[i + 8 + u];
@@ -483,6 +484,7 @@ __device__ __forceinline__ T seq_acc(const T *a, int n, T s = T(0)) {
     for (int u = 0; u < 8; u++) s = SUB ? s - x[u] : s + x[u];
     i += 8;
   }
+#pragma unroll 1
   for (; i + 8 <= n; i += 8) {
     T x[8];
 #pragma unroll
@@ -490,6 +492,7 @@ __device__ __forceinline__ T seq_acc(const T *a, int n, T s = T(0)) {
 #pragma unroll
     for (int u = 0; u < 8; u++) s = SUB ? s - x[u] : s + x[u];
   }
+#pragma unroll 1
   for (; i < n; i++) s = SUB ? s - a[i] : s + a[i];
   return s;
 }

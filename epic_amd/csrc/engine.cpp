@@ -280,7 +280,6 @@ static void rec_step(hipStream_t s, const Bucket &b, bool hv, bool divd, bool ad
   L_calc_w(s, b, 1);  // source_sink + calc_w, and the step's tendency planes cleared
   // hdry and theta take their hyperviscosity together (neither reads the
   // other, and restore_mass touches hdry only)
-  const FieldSet hth = {2, {F_HDRY, F_THETA}, {2, 3}, 1};
   // forked only for buckets of 2^18 grid points or more: at 256x128x20 the
   // branch saves 3% of the FP64 step, at 64x32x10 the cross-queue join
   // costs more than the branch (+9%)
@@ -290,7 +289,7 @@ static void rec_step(hipStream_t s, const Bucket &b, bool hv, bool divd, bool ad
   if (fork) {
     (void)hipEventRecord(side->fork, s);
     (void)hipStreamWaitEvent(side->s2, side->fork, 0);
-    L_hv(side->s2, b, hth);
+    L_hv_hth(side->s2, b);
     (void)hipEventRecord(side->join, side->s2);
   }
   L_uv_core(s, b);
@@ -298,7 +297,7 @@ static void rec_step(hipStream_t s, const Bucket &b, bool hv, bool divd, bool ad
   if (fork) {
     (void)hipStreamWaitEvent(s, side->join, 0);
   } else if (hv) {
-    L_hv(s, b, hth);
+    L_hv_hth(s, b);
   }
   L_advection(s, b);  // restore_mass first, inside
   rec_p2etc_pgrad_vars(s, b, 0, side);
@@ -314,10 +313,7 @@ static void rec_step(hipStream_t s, const Bucket &b, bool hv, bool divd, bool ad
   L_pgrad(s, b);
   if (divd) L_divdamp(s, b);
   L_ab(s, b);
-  if (hv) {
-    const FieldSet uv = {2, {F_U, F_V}, {0, 1}};
-    L_hv(s, b, uv);
-  }
+  if (hv) L_hv_uv(s, b);
   // store_diag, then the time planes rotated (in the same launch: nothing
   // after the Adams-Bashforth update reads them)
   rec_store_diag(s, b, 1);

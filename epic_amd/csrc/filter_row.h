@@ -50,6 +50,45 @@ template <> __device__ __forceinline__ const float *tw_inv<float>(const MemberDe
 template <> __device__ __forceinline__ const float *tr_fwd<float>(const MemberDesc &d) { return d.tr_f32; }
 template <> __device__ __forceinline__ const float *tr_inv<float>(const MemberDesc &d) { return d.tr_i32; }
 
+// unit `lane` (of n/8) of the stages s and s+1, h = 2^s, on a row in LDS: the
+// four points p, p+h, p+2h, p+3h go through stage s as (p, p+h) and
+// (p+2h, p+3h) and through stage s+1 as (p, p+2h) and (p+h, p+3h), in
+// registers
+template <class T>
+__device__ __forceinline__ void four1_pair(T *buf, int s, int lane, const T *tw) {
+  const int half = 1 << s, mm = lane & (half - 1), g = lane >> s;
+  const int i0 = 2 * (mm + g * 4 * half), i1 = i0 + 2 * half, i2 = i1 + 2 * half, i3 = i2 + 2 * half;
+  T x0r = buf[i0], x0i = buf[i0 + 1], x1r = buf[i1], x1i = buf[i1 + 1];
+  T x2r = buf[i2], x2i = buf[i2 + 1], x3r = buf[i3], x3i = buf[i3 + 1];
+  const int ka = half - 1 + mm, kb = 2 * half - 1 + mm;
+  const T ar = tw[2 * ka], ai = tw[2 * ka + 1];
+  const T br = tw[2 * kb], bi = tw[2 * kb + 1], cr = tw[2 * (kb + half)], ci = tw[2 * (kb + half) + 1];
+  bfly(x0r, x0i, x1r, x1i, ar, ai);
+  bfly(x2r, x2i, x3r, x3i, ar, ai);
+  bfly(x0r, x0i, x2r, x2i, br, bi);
+  bfly(x1r, x1i, x3r, x3i, cr, ci);
+  buf[i0] = x0r;
+  buf[i0 + 1] = x0i;
+  buf[i1] = x1r;
+  buf[i1 + 1] = x1i;
+  buf[i2] = x2r;
+  buf[i2 + 1] = x2i;
+  buf[i3] = x3r;
+  buf[i3 + 1] = x3i;
+}
+// unit `lane` (of n/4) of one stage s: the odd last one
+template <class T>
+__device__ __forceinline__ void four1_last(T *buf, int s, int lane, const T *tw) {
+  const int mmax = 2 << s, half = 1 << s, g = lane >> s, mm = lane & (half - 1);
+  const int i0 = 2 * mm + g * 2 * mmax, j0 = i0 + mmax, k = half - 1 + mm;
+  T xr = buf[i0], xi = buf[i0 + 1], yr = buf[j0], yi = buf[j0 + 1];
+  bfly(xr, xi, yr, yi, tw[2 * k], tw[2 * k + 1]);
+  buf[i0] = xr;
+  buf[i0 + 1] = xi;
+  buf[j0] = yr;
+  buf[j0 + 1] = yi;
+}
+
 // complex radix-2 stages on buf[0..n) (n doubles = n/2 complex), in the
 // reference's stage order.  Stages go two at a time: a lane loads the four
 // points p, p+h, p+2h, p+3h (h = 2^s) into registers, applies stage s to
@@ -64,42 +103,11 @@ __device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const T *t
   while ((2 << S) < n) S++;  // stages s with 2 << s < n
   int s = 0;
   for (; s + 1 < S; s += 2) {
-    const int half = 1 << s;
-    if (active && lane < (n >> 3)) {
-      const int mm = lane & (half - 1), g = lane >> s;
-      const int i0 = 2 * (mm + g * 4 * half), i1 = i0 + 2 * half, i2 = i1 + 2 * half, i3 = i2 + 2 * half;
-      T x0r = buf[i0], x0i = buf[i0 + 1], x1r = buf[i1], x1i = buf[i1 + 1];
-      T x2r = buf[i2], x2i = buf[i2 + 1], x3r = buf[i3], x3i = buf[i3 + 1];
-      const int ka = half - 1 + mm, kb = 2 * half - 1 + mm;
-      const T ar = tw[2 * ka], ai = tw[2 * ka + 1];
-      const T br = tw[2 * kb], bi = tw[2 * kb + 1], cr = tw[2 * (kb + half)], ci = tw[2 * (kb + half) + 1];
-      bfly(x0r, x0i, x1r, x1i, ar, ai);
-      bfly(x2r, x2i, x3r, x3i, ar, ai);
-      bfly(x0r, x0i, x2r, x2i, br, bi);
-      bfly(x1r, x1i, x3r, x3i, cr, ci);
-      buf[i0] = x0r;
-      buf[i0 + 1] = x0i;
-      buf[i1] = x1r;
-      buf[i1 + 1] = x1i;
-      buf[i2] = x2r;
-      buf[i2 + 1] = x2i;
-      buf[i3] = x3r;
-      buf[i3 + 1] = x3i;
-    }
+    if (active && lane < (n >> 3)) four1_pair(buf, s, lane, tw);
     row_sync<WIDE>();
   }
   if (s < S) {
-    const int mmax = 2 << s, half = 1 << s;
-    if (active) {
-      const int g = lane >> s, mm = lane & (half - 1);
-      const int i0 = 2 * mm + g * 2 * mmax, j0 = i0 + mmax, k = half - 1 + mm;
-      T xr = buf[i0], xi = buf[i0 + 1], yr = buf[j0], yi = buf[j0 + 1];
-      bfly(xr, xi, yr, yi, tw[2 * k], tw[2 * k + 1]);
-      buf[i0] = xr;
-      buf[i0 + 1] = xi;
-      buf[j0] = yr;
-      buf[j0 + 1] = yi;
-    }
+    if (active) four1_last(buf, s, lane, tw);
     row_sync<WIDE>();
   }
 }
@@ -231,6 +239,71 @@ __device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], 
 #pragma unroll
     for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq] * T(2. / (n));
   row_sync<WIDE>();
+}
+
+// The same filter by one wavefront on `rows` rows that lie in LDS at X + r*WS
+// (rows 1/64 of the NV values a lane holds of them: NV = rows*ni/64, at least
+// 1); on[r] tells whether row r, row J of the grid at r = 0, is in the filter
+// band (rows that are not stay as they are).  The lanes share the units of
+// all rows, so that short rows fill the wavefront too, and only wavefront
+// barriers separate the stages.  On entry (behind a barrier) a row that is on
+// holds its points in bit-reversed order (rev_pos); on exit (behind one) the
+// unscaled result in natural order, to be multiplied by 2/ni.
+__device__ __forceinline__ int rev_pos(int e, int bits) { return (brev(e >> 1, bits) << 1) | (e & 1); }
+template <class T, int NV>
+__device__ __forceinline__ void filter_wave(const MemberDesc &d, T *X, int WS, int rows, const int *on, int J,
+                                            int vgrid, int lane) {
+  const int n = d.ni, lg = d.nlogn, bits = lg - 1, S = lg - 1;
+  auto stages = [&](const T *tw) {
+    int s = 0;
+    for (; s + 1 < S; s += 2) {
+#pragma unroll
+      for (int i = 0; i < (NV + 7) / 8; i++) {
+        const int u = lane + 64 * i, r = u >> (lg - 3);
+        if (r < rows && on[r]) four1_pair(X + r * WS, s, u & ((n >> 3) - 1), tw);
+      }
+      wave_sync();
+    }
+    if (s < S) {
+#pragma unroll
+      for (int i = 0; i < (NV + 3) / 4; i++) {
+        const int u = lane + 64 * i, r = u >> (lg - 2);
+        if (r < rows && on[r]) four1_last(X + r * WS, s, u & ((n >> 2) - 1), tw);
+      }
+      wave_sync();
+    }
+  };
+  stages(tw_fwd<T>(d));
+  T ar[(NV + 3) / 4], ai[(NV + 3) / 4], br[(NV + 3) / 4], bi[(NV + 3) / 4];
+#pragma unroll
+  for (int i = 0; i < (NV + 3) / 4; i++) {
+    const int u = lane + 64 * i, r = u >> (lg - 2), l = u & ((n >> 2) - 1);
+    if (r < rows && on[r]) {
+      const T *x = X + r * WS;
+      const int ka = unit_k(n, l), kb = unit_kb(n, l);
+      ar[i] = x[2 * ka];
+      ai[i] = x[2 * ka + 1];
+      br[i] = x[2 * kb];
+      bi[i] = x[2 * kb + 1];
+      const double *hl = (vgrid ? d.hl_pv : d.hl_h) + (size_t)(J + r) * (n / 2 + 2);
+      split_gain(ar[i], ai[i], br[i], bi[i], n, l, tr_fwd<T>(d), tr_inv<T>(d), hl);
+    }
+  }
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < (NV + 3) / 4; i++) {
+    const int u = lane + 64 * i, r = u >> (lg - 2), l = u & ((n >> 2) - 1);
+    if (r < rows && on[r]) {
+      T *x = X + r * WS;
+      const int pa = brev(unit_k(n, l), bits) << 1, pb = brev(unit_kb(n, l), bits) << 1;
+      x[pa] = ar[i];
+      x[pa + 1] = ai[i];
+      x[pb] = br[i];
+      x[pb + 1] = bi[i];
+    }
+  }
+  wave_sync();
+  stages(tw_inv<T>(d));
 }
 
 }  // namespace epic

@@ -48,17 +48,22 @@ constexpr int ADV_FIELDS = 3;
 
 enum { AV_P3 = 0, AV_THETA = 1, AV_HDRY = 2 };
 
-// the field as the advection reads and writes it (theta and hdry)
-__device__ __forceinline__ double *adv_field(const MemberDesc &d, int which) {
-  return which == AV_THETA ? d.THETA : d.HDRY;
-}
 // where the column pass leaves its result
 __device__ __forceinline__ double *adv_out(const MemberDesc &d, int which) {
   return which == AV_P3 ? d.vunity : (which == AV_THETA ? d.vtheta : d.sC);
 }
-// a field's value on level K at offset q as the column pass takes it
-__device__ __forceinline__ double adv_value(const MemberDesc &d, int which, int K, size_t q) {
-  return which == AV_P3 ? 1. : which == AV_THETA ? d.THETA[q] : dmax(d.h_min[K], d.HDRY[q]);
+// the field as it enters the advection: hv set, the hyperviscosity left theta
+// and hdry in sD's copies 2 and 1 (k_hv4)
+__device__ __forceinline__ const double *adv_in(const MemberDesc &d, int which, int hv) {
+  if (hv) return d.sD + (size_t)(which == AV_THETA ? 2 : 1) * d.N3;
+  return which == AV_THETA ? d.THETA : d.HDRY;
+}
+// its value on level K at offset q as the column pass takes it (theta above
+// its first advected level, which the pass reads too, is the field's)
+__device__ __forceinline__ double adv_value(const MemberDesc &d, int which, int K, size_t q, int hv) {
+  if (which == AV_P3) return 1.;
+  if (which == AV_THETA) return adv_in(d, which, hv && K >= d.ks - 1)[q];
+  return dmax(d.h_min[K], adv_in(d, which, hv)[q]);
 }
 // first level of a field that is advected
 __device__ __forceinline__ int adv_kfirst(const MemberDesc &d, int which) { return which == AV_HDRY ? 1 : d.ks - 1; }
@@ -97,13 +102,13 @@ __device__ __forceinline__ T tt_iface(const T *wa, int K, int nk, T ep) {
 // computes in FP64 (the same bits), else a re-read of the FP64 field
 __device__ __forceinline__ double old_value(double staged, const double *) { return staged; }
 __device__ __forceinline__ double old_value(float, const double *p) { return *p; }
-__device__ __forceinline__ double col_value(double staged, const MemberDesc &, int, int, size_t) { return staged; }
-__device__ __forceinline__ double col_value(float, const MemberDesc &d, int which, int K, size_t q) {
-  return adv_value(d, which, K, q);
+__device__ __forceinline__ double col_value(double staged, const MemberDesc &, int, int, size_t, int) { return staged; }
+__device__ __forceinline__ double col_value(float, const MemberDesc &d, int which, int K, size_t q, int hv) {
+  return adv_value(d, which, K, q, hv);
 }
 
 template <class T>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_hsu_vert(const MemberDesc *D, int mb, int nm, int C) {
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_hsu_vert(const MemberDesc *D, int mb, int nm, int C, int hv) {
   ADV_MEMBER;
   if (d.adv_akima[which]) return;  // the field takes the Akima scheme (uniform per block)
   extern __shared__ double lds_raw[];
@@ -125,10 +130,10 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
     for (int K = kk; K <= nk + 1; K += KS) {
       double x = 0., w = 0.;
       if (layer) {
-        if (K >= kf && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
+        if (K >= kf && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I), hv);
         if (K >= kf - 1 && K <= nk) w = d.W3[ix3(d, K, J, I)];
       } else {
-        if (K >= kf - 1 && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
+        if (K >= kf - 1 && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I), hv);
         if (K >= kf && K <= nk) w = (K == 1 || K == nk) ? 0. : .5 * (d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K - 1, J, I)]);
         // statics left by the unity pass (wm[kf-1], wa[kf-2] of its last column)
         if (which == AV_THETA && K == kf - 1 && K >= 1) {
@@ -180,7 +185,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
     if (live)
       for (int K = kf + kk; K <= nk; K += KS)
         out[ix3(d, K, J, I)] =
-            col_value(wa[K], d, which, K, ix3(d, K, J, I)) + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
+            col_value(wa[K], d, which, K, ix3(d, K, J, I), hv) + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
   } else {
     // unity's levels above k_sigma-1 serve their neighbours only: flux and
     // predictor from k_sigma-2, the corrected flux from k_sigma-1
@@ -225,7 +230,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
     if (live)
       for (int K = k2 + kk; K <= nk; K += KS)
         out[ix3(d, K, J, I)] =
-            col_value(wa[K], d, which, K, ix3(d, K, J, I)) + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
+            col_value(wa[K], d, which, K, ix3(d, K, J, I), hv) + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
   }
 #undef WM
 #undef WP
@@ -428,12 +433,12 @@ __device__ __forceinline__ void ak_zonal_row(const MemberDesc &d, const RowMap &
 // Zonal pass of a row group (1024/ni rows of plane K per block).  layer: hdry,
 // stored with the restore_mass that follows the advection.  Otherwise theta
 // and, before it by the same lanes, unity, whose result corrects theta
-// (theta - old (unity - 1), old the theta of before the advection, still in
-// place) and is written nowhere.  The two go through one copy of the code (a
+// (theta - old (unity - 1), old the theta of before the advection, still where
+// the column pass read it) and is written nowhere.  The two go through one copy of the code (a
 // loop): written out twice the transform's operands are kept from one to the
 // other and cost a wave of occupancy.
 template <bool WIDE, class T, bool AKIMA>
-__device__ __forceinline__ void adv_zonal_rows(const MemberDesc &d, bool layer, T *sh) {
+__device__ __forceinline__ void adv_zonal_rows(const MemberDesc &d, bool layer, int hv, T *sh) {
   const RowMap m = row_map(d.ni);
   const int K = 1 + blockIdx.y, Jr = blockIdx.x * m.rpb + m.g, ni = d.ni;
   const bool live = Jr <= d.nj;
@@ -454,13 +459,14 @@ __device__ __forceinline__ void adv_zonal_rows(const MemberDesc &d, bool layer, 
   }
   if (!live) return;
   const Plane<double> out{(layer ? d.HDRY : d.THETA) + o};
+  const Plane<const double> old{adv_in(d, AV_THETA, hv) + o};
   const double hmin = d.h_min[K];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     const int I = 1 + m.lane + m.stride * q;
     double v = y[q];
     if (layer) v = dmax(hmin, v);
-    else v -= out[ix2(d, J, I)] * cor[q];
+    else v -= old[ix2(d, J, I)] * cor[q];
     out[ix2(d, J, I)] = v;
     if (I == ni) out[ix2(d, J, 0)] = v;
     if (I == 1) out[ix2(d, J, ni + 1)] = v;
@@ -468,13 +474,13 @@ __device__ __forceinline__ void adv_zonal_rows(const MemberDesc &d, bool layer, 
 }
 // blockIdx.z = member for unity with theta, members + member for hdry
 template <bool WIDE, class T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_hsu_zonal(const MemberDesc *D, int mb, int nm) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_hsu_zonal(const MemberDesc *D, int mb, int nm, int hv) {
   extern __shared__ double sh_raw[];
   const bool layer = (int)blockIdx.z >= nm;
   const MemberDesc &d = D[mb + (int)blockIdx.z - (layer ? nm : 0)];
   const int which = layer ? AV_HDRY : AV_THETA;
   if (d.adv_akima[which] || 1 + (int)blockIdx.y < adv_kfirst(d, which)) return;  // uniform per block
-  adv_zonal_rows<WIDE, T, false>(d, layer, reinterpret_cast<T *>(sh_raw));
+  adv_zonal_rows<WIDE, T, false>(d, layer, hv, reinterpret_cast<T *>(sh_raw));
 }
 
 // ------------------------------------------------------------- Akima
@@ -498,7 +504,7 @@ __device__ __forceinline__ T ak_dela(T d0, T d1) {
 // (differences, slopes, fluxes, update) run on all lanes over (column,
 // level) pairs, separated by barriers (no recurrence in K)
 template <class T>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_ak_vert(const MemberDesc *D, int mb, int nm, int C) {
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_ak_vert(const MemberDesc *D, int mb, int nm, int C, int hv) {
   ADV_MEMBER;
   if (!d.adv_akima[which]) return;  // uniform per block
   extern __shared__ double lds_raw[];
@@ -519,10 +525,10 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
     for (int K = kk; K <= nk + 1; K += KS) {
       double x = 0., w = 0.;
       if (layer) {
-        if (K >= kf && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
+        if (K >= kf && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I), hv);
         if (K >= kf - 1 && K <= nk) w = d.W3[ix3(d, K, J, I)];
       } else {
-        if (K >= kf - 1 && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I));
+        if (K >= kf - 1 && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I), hv);
         if (K >= kf && K <= nk) w = (K == 1 || K == nk) ? 0. : .5 * (d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K - 1, J, I)]);
       }
       wa[K] = T(x);
@@ -560,7 +566,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
   if (live)
     for (int K = max(kf, adv_kfirst(d, which)) + kk; K <= nk; K += KS) {
       const size_t q = ix3(d, K, J, I);
-      const double x = col_value(wa[K], d, which, K, q);
+      const double x = col_value(wa[K], d, which, K, q, hv);
       if (layer) out[q] = x + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
       else out[q] = x + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
     }
@@ -669,13 +675,13 @@ __device__ __forceinline__ void ak_zonal_row(const MemberDesc &d, const RowMap &
   }
 }
 template <bool WIDE, class T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_ak_zonal(const MemberDesc *D, int mb, int nm) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_ak_zonal(const MemberDesc *D, int mb, int nm, int hv) {
   extern __shared__ double sh_raw[];
   const bool layer = (int)blockIdx.z >= nm;
   const MemberDesc &d = D[mb + (int)blockIdx.z - (layer ? nm : 0)];
   const int which = layer ? AV_HDRY : AV_THETA;
   if (!d.adv_akima[which] || 1 + (int)blockIdx.y < adv_kfirst(d, which)) return;  // uniform per block
-  adv_zonal_rows<WIDE, T, true>(d, layer, reinterpret_cast<T *>(sh_raw));
+  adv_zonal_rows<WIDE, T, true>(d, layer, hv, reinterpret_cast<T *>(sh_raw));
 }
 
 // restore_mass, one advection pass over all three fields of every member,
@@ -685,6 +691,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 // store_pgrad_vars.
 template <class T>
 static void advection_t(hipStream_t s, const Bucket &b) {
+  const int hv = hv_fused(b) ? 1 : 0;
   const int ncol = (b.nj + 1) * b.ni, nz = ADV_FIELDS * b.nm;
   // columns per block: as many as keep the four LDS columns within 40 KB
   int C = 64;
@@ -694,8 +701,8 @@ static void advection_t(hipStream_t s, const Bucket &b) {
   const bool hsu = b.adv_schemes & 1, akima = b.adv_schemes & 2;
   const dim3 gv((ncol + C - 1) / C, 1, nz);
   if (hsu)
-    LAUNCH(k_hsu_vert<T>, gv, dim3(knob_threads(v, b.nk + 2)), sizeof(T) * 4 * C * (b.nk + 2), s, b.D, b.mb, b.nm, C);
-  if (akima) LAUNCH(k_ak_vert<T>, gv, dim3(knob_threads(v, b.nk + 2)), sizeof(T) * 4 * C * (b.nk + 2), s, b.D, b.mb, b.nm, C);
+    LAUNCH(k_hsu_vert<T>, gv, dim3(knob_threads(v, b.nk + 2)), sizeof(T) * 4 * C * (b.nk + 2), s, b.D, b.mb, b.nm, C, hv);
+  if (akima) LAUNCH(k_ak_vert<T>, gv, dim3(knob_threads(v, b.nk + 2)), sizeof(T) * 4 * C * (b.nk + 2), s, b.D, b.mb, b.nm, C, hv);
   const int TJ = b.knob[KN_ROWS_MER] ? b.knob[KN_ROWS_MER] : 4;
   const int CW = b.ni < 64 ? b.ni : 64, tiles = (b.nj + 1 + TJ - 1) / TJ;
   const dim3 gm(tiles * (b.ni / CW), b.nk, nz);
@@ -707,8 +714,8 @@ static void advection_t(hipStream_t s, const Bucket &b) {
            TJ);
   const int rpb = rows_per_block(b.ni);
   const dim3 gz((b.nj + 1 + rpb - 1) / rpb, b.nk, 2 * b.nm);
-  if (hsu) ROWS_LAUNCH(b, "k_hsu_zonal<T>", (k_hsu_zonal<true, T>), (k_hsu_zonal<false, T>), gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm);
-  if (akima) ROWS_LAUNCH(b, "k_ak_zonal<T>", (k_ak_zonal<true, T>), (k_ak_zonal<false, T>), gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm);
+  if (hsu) ROWS_LAUNCH(b, "k_hsu_zonal<T>", (k_hsu_zonal<true, T>), (k_hsu_zonal<false, T>), gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm, hv);
+  if (akima) ROWS_LAUNCH(b, "k_ak_zonal<T>", (k_ak_zonal<true, T>), (k_ak_zonal<false, T>), gz, dim3(256), sizeof(T) * rpb * 3 * (b.ni + 2), s, b.D, b.mb, b.nm, hv);
 }
 void L_advection(hipStream_t s, const Bucket &b) {
   if (b.mixed) advection_t<float>(s, b);

@@ -515,7 +515,9 @@ void L_divdamp(hipStream_t s, const Bucket &b) {
 // ------------------------------------------------------ Adams-Bashforth
 // Coefficients from the FLAT_MAX start-up flags of the older planes,
 // tested per wind at (KLO, jlo, ILO) as the reference does.
-__global__ void __launch_bounds__(256) k_ab(const MemberDesc *D, int mb) {
+// scratch: the result goes to copy 1 (u) and 2 (v) of sD, from where k_hv4
+// takes it, else to the field with its pads
+__global__ void __launch_bounds__(256) k_ab(const MemberDesc *D, int mb, int scratch) {
   MEMBER;
   FLAT2(0, d.nj + 1, 1, d.ni);
   const int K = 1 + blockIdx.y;
@@ -536,6 +538,10 @@ __global__ void __launch_bounds__(256) k_ab(const MemberDesc *D, int mb) {
     size_t q = ix3(d, K, J, I);
     const double y = val[q] + d.dt * (ab0 * tb[(size_t)dy.it0 * d.N3 + q] + ab1 * tb[(size_t)dy.itm1 * d.N3 + q] +
                                       ab2 * tb[(size_t)dy.itm2 * d.N3 + q]);
+    if (scratch) {
+      d.sD[(size_t)(1 + w) * d.N3 + q] = y;
+      continue;
+    }
     val[q] = y;
     // zonal pads (bc_lateral after the update)
     if (I == d.ni) val[ix3(d, K, J, 0)] = y;
@@ -544,7 +550,7 @@ __global__ void __launch_bounds__(256) k_ab(const MemberDesc *D, int mb) {
 }
 void L_ab(hipStream_t s, const Bucket &b) {
   if (b.mixed) { LM_ab(s, b); return; }
-  LAUNCH(k_ab, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
+  LAUNCH(k_ab, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb, hv_fused(b) ? 1 : 0);
 }
 
 // monotone filtered geopotential, K = nk-1 down to 0 (src/shared/epic_timestep.c:176-196)
@@ -974,140 +980,267 @@ __device__ __forceinline__ float mean_butterfly(float p, int ni) {
   return p / float(ni);
 }
 
-// del^4 after its meridional second differences, one row at a time (rows
-// of members whose highest order is del^4): the row of D (copy i of sB) is
-// zonally filtered and applied, A += DT*(-1)*D, then the zonal del^4 of the
-// updated row (two second differences, each less its zonal mean) is
-// applied, A += DT*(-1)*D_zonal; the zonal pads of every row 0..nj+1 hold
-// copies of points ni and 1.  The steps and expressions are those of
-// k_hv_apply (pass 1) followed by k_zonal_hv, with the row read and written
-// once instead of twice.  A row's ni/4 lanes (RowMap) each own the points
-// I = 1 + lane + (ni/4) q, q < 4; three row buffers in LDS (ni + 2 values,
-// pads included) carry the row, the first second difference and the input
-// of the second.  The zonal means: BFLY, the mixed mode's order for rows of
-// 256 points or more (mean_butterfly; a row's lanes are whole wavefronts);
-// otherwise sums left to right, as the reference and k_zonal_hv form them,
-// each lane of a row forming the same sum itself (which spares a barrier
-// to hand it round).
-template <bool WIDE, class T, bool BFLY>
-__global__ void __launch_bounds__(256) k_hv4_rows(const MemberDesc *D, int mb, int nm, FieldSet fs) {
+// del^4 of a field set in one launch, out of place (buckets whose members'
+// highest order is del^4).  A block takes 4 RW consecutive rows of one plane.
+// By columns first: thread c of G = 256/min(ni, 256) groups owns the columns
+// I = 1 + c + 256 q (q < CPT) of RB = 4 RW / G rows, loads them on rows
+// J0-2..J0+RB+1 and forms the two meridional second differences of del^4
+// (stencils shifted at rows 0 and jmax) into LDS rows.  By rows then:
+// wavefront w owns RW rows, a lane their points I = 1 + lane + 64 q (q < NQ);
+// it filters the rows of the filter band, applies A += DT*(-1)*D, forms the
+// zonal del^4 of the updated rows (two second differences, each less its
+// zonal mean) and applies that, with wavefront barriers only but around the
+// FP64 sums of long rows.  Every value is formed by the same expression as in
+// k_d2dy2_cols, k_hv_apply and k_zonal_hv, which members with higher orders
+// take; there the field and D cross memory three times, here the field is
+// read (twice by its block and on two halo rows either side, from L2) and
+// written.  Zonal means: the reference's sums left to right, a lane a row,
+// RW rows side by side; from 256 points on, where a wavefront has one row,
+// the block's four rows side by side in one wavefront instead (MEAN_BLOCK; a
+// lane a row in each wavefront took 45.7 us against 32 at 256x128x20);
+// the mixed mode's order for rows of 256 points or more (mean_butterfly;
+// MEAN_BFLY).
+// mode HV_TO_SCRATCH: field -> copy 1+i of sD (hdry and theta, which the
+// advection reads there); HV_FROM_SCRATCH: copy 1+i of sD, where the
+// Adams-Bashforth update left rows jbot..nj, -> field (u and v).  The zonal
+// pads of every row 0..nj+1 that the field keeps are written as copies of
+// points ni and 1.
+enum { HV_TO_SCRATCH = 0, HV_FROM_SCRATCH = 1 };
+enum { MEAN_WAVE, MEAN_BLOCK, MEAN_BFLY };
+template <class T, int NI, int RW, int MEAN>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_hv4(const MemberDesc *D, int mb, int nm, FieldSet fs, int mode) {
   SET_MEMBER;
+  constexpr int ni = NI, COLS = NI < 256 ? NI : 256, CPT = NI / COLS, G = 256 / COLS, ROWS = 4 * RW, RB = ROWS / G;
+  constexpr int NQ = NI < 64 ? 1 : NI / 64, WS = (NI + 2) | 1, NV = RW * NI < 64 ? 1 : RW * NI / 64;
+  static_assert(RB * G == ROWS, "rows split evenly over the column groups");
   extern __shared__ double lds_raw[];
-  const RowMap m = row_map(d.ni);
-  const int ni = d.ni, WS = ni + 2;
-  T *z0 = reinterpret_cast<T *>(lds_raw) + (size_t)m.g * 3 * WS, *z1 = z0 + WS, *z2 = z1 + WS;
-  HvRange r = hv_range(d, kind);
-  const int K = r.k0 + blockIdx.y, Jr = blockIdx.x * m.rpb + m.g;
-  if (K > r.k1 || hv_passes(d) != 2) return;  // uniform per block
-  const bool live = Jr <= d.nj + 1;
-  const int J = live ? Jr : 0, vg = (kind == 1);
-  const Plane<double> a{fld_ptr(d, f) + (size_t)K * d.N2};
-  const Plane<const T> dd{reinterpret_cast<const T *>(d.sB.get()) + (size_t)(fs.copy0 + fi) * d.N3 + (size_t)K * d.N2};
-  const bool upd = live && J >= r.jbot && J <= d.nj;
-  // the row of A and the row of D, both loads in flight together
-  double v[4];
-  T dq[4];
+  T *X = reinterpret_cast<T *>(lds_raw);
+  T *meanv = X + ROWS * WS;
+  int *on = reinterpret_cast<int *>(meanv + ROWS);
+  const int nj = d.nj, vg = (kind == 1);
+  const HvRange r = hv_range(d, kind);
+  const int K = r.k0 + blockIdx.y;
+  if (K > r.k1) return;  // uniform over the block
+  const int np = hv_passes(d);  // 0 or 2 (uniform)
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int Jb = blockIdx.x * ROWS;
+  const size_t o = (size_t)K * d.N2;
+  const Plane<double> a{fld_ptr(d, f) + o}, scr{d.sD + (size_t)(1 + fi) * d.N3 + o};
+  const int jmax = vg ? nj + 1 : nj;
+  // whether row j is updated, and the input on row j
+  auto upd = [&](int j) { return j >= r.jbot && j <= nj; };
+  auto in = [&](int j, int I) { return (mode == HV_FROM_SCRATCH && upd(j)) ? scr[ix2(d, j, I)] : a[ix2(d, j, I)]; };
+  const int *rflag = vg ? d.rflag_v : d.rflag_h;
+  if (np) {
+    int g = threadIdx.x / COLS;
+    if (COLS >= 64) g = __builtin_amdgcn_readfirstlane(g);  // the rows are the wavefront's: scalar
+    const int c = threadIdx.x % COLS, R0 = g * RB, J0 = Jb + R0;
+    if (threadIdx.x < ROWS) on[threadIdx.x] = upd(Jb + threadIdx.x) && rflag[Jb + threadIdx.x] != 0;
+    const Plane<const double> cx{vg ? d.vcx : d.hcx}, cy{vg ? d.vcy : d.hcy}, cz{vg ? d.vcz : d.hcz};
+    const T c2 = T(d.coef2), c4 = T(d.coef4);
+    // first pass at row j from rows (j0, j1, j2)
+    auto p1 = [&](int j, T h0, T h1, T h2) {
+      T a0 = c2 * T(cx[j]), a1 = c2 * T(cy[j]), a2 = c2 * T(cz[j]);
+      return a0 * h0 + a1 * h1 + a2 * h2;
+    };
+    // D of row J, column I (point e = I-1) to LDS, where the filter wants it
+    auto put = [&](int t, int e, T x) {
+      const bool band = upd(J0 + t) && rflag[J0 + t] != 0;
+      X[(R0 + t) * WS + (band ? rev_pos(e, d.nlogn - 1) : e)] = x;
+    };
+    if (J0 >= 2 && J0 + RB - 1 <= jmax - 2) {
+      // every stencil centred: the first pass of rows J0-1 .. J0+RB once each
+      T w[RB + 4][CPT];  // rows J0-2 .. J0+RB+1
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int I = 1 + m.lane + m.stride * q;
-    v[q] = live ? a[ix2(d, J, I)] : 0.;
-    dq[q] = upd ? dd[ix2(d, J, I)] : T(0.);
-  }
-  // the meridional part: D filtered (work = z1) where the row's wavefront or
-  // block holds a row of the filter band
-  const bool filt = upd && (vg ? d.rflag_v : d.rflag_h)[J] != 0;
-  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, dq, z1, J, vg, filt, m.lane);
-  const double sign = -1.;  // del^4
+      for (int t = 0; t < RB + 4; t++)
 #pragma unroll
-  for (int q = 0; q < 4; q++)
-    if (upd) v[q] += d.dt * sign * (double)dq[q];
-  // the updated row, pads included, as the zonal part reads it (each lane
-  // rewrites only the points it read)
+        for (int q = 0; q < CPT; q++) w[t][q] = T(in(J0 - 2 + t, 1 + c + 256 * q));
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int I = 1 + m.lane + m.stride * q;
-    const T t = T(v[q]);
-    z0[I] = t;
-    if (I == ni) z0[0] = t;
-    if (I == 1) z0[ni + 1] = t;
-  }
-  const int Jc = min(J, d.nj);
-  const double mm = fabs(d.lat[2 * Jc + r.jh]) > 45. ? d.m0z : d.m[2 * Jc + r.jh];
-  T y[4];
-  row_sync<WIDE>();
-  for (int pass = 0; pass < 2; pass++) {
-    // pass 0 reads z0 and leaves its raw result in z1; pass 1 reads z2 (pass
-    // 0 less its mean) and leaves its raw result in z0
-    const T *xin = pass ? z2 : z0;
-    T *raw = pass ? z0 : z1;
-    const T dcu = T(hv_coef(d, pass) * mm * mm);
+      for (int q = 0; q < CPT; q++) {
+        T P[RB + 2];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int I = 1 + m.lane + m.stride * q;
-      y[q] = dcu * (xin[I - 1] - T(2.) * xin[I] + xin[I + 1]);
-      raw[I] = y[q];
-    }
-    row_sync<WIDE>();
-    T fm;
-    if constexpr (BFLY) {
-      // each wavefront of the row's lanes forms the 64 partials itself
-      const int l = m.lane & 63;
-      T p = raw[1 + l];
-      for (int k = l + 64; k < ni; k += 64) p += raw[1 + k];
-      fm = mean_butterfly(p, ni);
-    } else {
-      fm = seq_acc(raw + 1, ni) / T(ni);
-    }
+        for (int t = 0; t < RB + 2; t++) P[t] = p1(J0 - 1 + t, w[t][q], w[t + 1][q], w[t + 2][q]);
 #pragma unroll
-    for (int q = 0; q < 4; q++) y[q] -= fm;
-    if (pass == 0) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int I = 1 + m.lane + m.stride * q;
-        z2[I] = y[q];
-        if (I == ni) z2[0] = y[q];
-        if (I == 1) z2[ni + 1] = y[q];
+        for (int t = 0; t < RB; t++) {
+          const int J = J0 + t;
+          const T a0 = c4 * T(cx[J]), a1 = c4 * T(cy[J]), a2 = c4 * T(cz[J]);
+          put(t, c + 256 * q, a0 * P[t] + a1 * P[t + 1] + a2 * P[t + 2]);
+        }
       }
-      row_sync<WIDE>();
+    } else {
+      // the stencil shifted at rows 0 and jmax (both passes)
+      auto p1_at = [&](int j, int I) {
+        const int m = min(max(j, 1), jmax - 1);
+        return p1(j, T(in(m - 1, I)), T(in(m, I)), T(in(m + 1, I)));
+      };
+#pragma unroll 1
+      for (int t = 0; t < RB; t++) {
+        const int J = J0 + t, m = min(max(J, 1), jmax - 1);
+        if (J > jmax) break;
+        const T a0 = c4 * T(cx[J]), a1 = c4 * T(cy[J]), a2 = c4 * T(cz[J]);
+#pragma unroll 1
+        for (int q = 0; q < CPT; q++) {
+          const int I = 1 + c + 256 * q;
+          put(t, I - 1, a0 * p1_at(m - 1, I) + a1 * p1_at(m, I) + a2 * p1_at(m + 1, I));
+        }
+      }
     }
   }
-  if (!live) return;
+  // by rows: row Jb + wv*RW + u in LDS at X + (wv*RW + u)*WS
+  const int R0 = wv * RW, Jw = Jb + R0;
+  T *Xw = X + R0 * WS;
+  const bool has = NI >= 64 || lane < NI;  // lane holds points of the row
+  double v[RW][NQ];
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int I = 1 + m.lane + m.stride * q;
-    if (upd) {
-      v[q] += d.dt * sign * (double)y[q];
-      a[ix2(d, J, I)] = v[q];
+  for (int u = 0; u < RW; u++)
+#pragma unroll
+    for (int q = 0; q < NQ; q++) v[u][q] = (has && upd(Jw + u)) ? in(Jw + u, 1 + lane + 64 * q) : 0.;
+  if (np) {
+    __syncthreads();
+    bool band = false;
+#pragma unroll
+    for (int u = 0; u < RW; u++) band |= on[R0 + u] != 0;
+    if (band) filter_wave<T, NV>(d, Xw, WS, RW, on + R0, Jw, vg, lane);
+    const double sign = -1.;  // del^4
+#pragma unroll
+    for (int u = 0; u < RW; u++) {
+      T *x = Xw + u * WS;
+      const T sc = on[R0 + u] ? T(2. / (ni)) : T(1.);
+      if (upd(Jw + u))
+#pragma unroll
+        for (int q = 0; q < NQ; q++)
+          if (has) v[u][q] += d.dt * sign * (double)(on[R0 + u] ? x[lane + 64 * q] * sc : x[lane + 64 * q]);
     }
-    if (I == ni) a[ix2(d, J, 0)] = v[q];
-    if (I == 1) a[ix2(d, J, ni + 1)] = v[q];
+    wave_sync();
+#pragma unroll
+    for (int u = 0; u < RW; u++)
+      if (has) {
+        T *x = Xw + u * WS;
+#pragma unroll
+        for (int q = 0; q < NQ; q++) x[1 + lane + 64 * q] = T(v[u][q]);
+        if (1 + lane + 64 * (NQ - 1) == ni) x[0] = T(v[u][NQ - 1]);
+        if (lane == 0) x[ni + 1] = T(v[u][0]);
+      }
+    wave_sync();
+#pragma unroll 1
+    for (int pass = 0; pass < 2; pass++) {
+      T part[RW];
+#pragma unroll
+      for (int u = 0; u < RW; u++) {
+        // m (or m0 poleward of LAT0) of the row; the pass's coefficient is
+        // (coef[2(p+1)] mm) mm, as the reference forms it
+        const int Jc = min(Jw + u, nj);
+        const double mm = fabs(d.lat[2 * Jc + r.jh]) > 45. ? d.m0z : d.m[2 * Jc + r.jh];
+        const T dcu = T(hv_coef(d, pass) * mm * mm);
+        T *x = Xw + u * WS + 1 + lane, y[NQ];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) y[q] = has ? dcu * (x[64 * q - 1] - T(2.) * x[64 * q] + x[64 * q + 1]) : T(0.);
+        wave_sync();
+        part[u] = y[0];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+          if (has) x[64 * q] = y[q];
+          if (q > 0) part[u] += y[q];
+        }
+      }
+      if constexpr (MEAN == MEAN_BLOCK) {
+        __syncthreads();
+        if (threadIdx.x < ROWS) meanv[threadIdx.x] = seq_acc(X + threadIdx.x * WS + 1, ni) / T(ni);
+        __syncthreads();
+      } else if constexpr (MEAN == MEAN_WAVE) {
+        wave_sync();
+        if (lane < RW) meanv[R0 + lane] = seq_acc(Xw + lane * WS + 1, ni) / T(ni);
+        wave_sync();
+      }
+#pragma unroll
+      for (int u = 0; u < RW; u++) {
+        T *x = Xw + u * WS + 1 + lane, y[NQ];
+        T fm;
+        if constexpr (MEAN == MEAN_BFLY) fm = mean_butterfly(part[u], ni);
+        else fm = meanv[R0 + u];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) y[q] = has ? x[64 * q] - fm : T(0.);
+        if (pass == 0) {
+          if (has) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) x[64 * q] = y[q];
+            if (1 + lane + 64 * (NQ - 1) == ni) Xw[u * WS] = y[NQ - 1];
+            if (lane == 0) Xw[u * WS + ni + 1] = y[0];
+          }
+        } else if (upd(Jw + u)) {
+#pragma unroll
+          for (int q = 0; q < NQ; q++) v[u][q] += d.dt * sign * (double)y[q];
+        }
+      }
+      wave_sync();
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < RW; u++) {
+    const int J = Jw + u;
+    if (upd(J)) {
+      const Plane<double> out{mode == HV_FROM_SCRATCH ? a.p : scr.p};
+      if (has) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) out[ix2(d, J, 1 + lane + 64 * q)] = v[u][q];
+        if (mode == HV_FROM_SCRATCH) {
+          if (1 + lane + 64 * (NQ - 1) == ni) a[ix2(d, J, 0)] = v[u][NQ - 1];
+          if (lane == 0) a[ix2(d, J, ni + 1)] = v[u][0];
+        }
+      }
+    } else if (np && J <= nj + 1 && lane == 0) {
+      // rows the update leaves alone: their pads
+      a[ix2(d, J, 0)] = a[ix2(d, J, ni)];
+      a[ix2(d, J, ni + 1)] = a[ix2(d, J, 1)];
+    }
   }
 }
 
-// del^4 (and higher orders) of a field set: the meridional part, then the
-// zonal part.  In the mixed mode with del^4 the highest order of the bucket
-// (the engine keeps such members apart from those with higher orders), the
-// filtered meridional update and the zonal part run as one row kernel
-// (k_hv4_rows); the FP64 path keeps the separate kernels (faster there: its
-// zonal means are the reference's serial sums, which k_zonal_hv spreads
-// over more rows at once).
-static void hv4_mixed(hipStream_t s, const Bucket &b, const FieldSet &fs) {
-  using T = float;
-  d2dy2_del4<T>(s, b, fs);
-  const int rpb = rows_per_block(b.ni);
-  const dim3 ga((b.nj + 2 + rpb - 1) / rpb, b.nk, fs.n * b.nm);
-  const size_t shm = sizeof(T) * rpb * 3 * (b.ni + 2);
-  if (b.ni > 256) LAUNCH_AS("k_hv4_rows", (k_hv4_rows<true, T, true>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
-  else if (b.ni == 256) LAUNCH_AS("k_hv4_rows", (k_hv4_rows<false, T, true>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
-  else LAUNCH_AS("k_hv4_rows", (k_hv4_rows<false, T, false>), ga, dim3(256), shm, s, b.D, b.mb, b.nm, fs);
+template <class T, int NI, int RW, int MEAN>
+static void hv4_ni(hipStream_t s, const Bucket &b, const FieldSet &fs, int mode) {
+  constexpr int rows = 4 * RW, WS = (NI + 2) | 1;
+  const size_t shm = sizeof(T) * (rows * WS + rows) + sizeof(int) * rows;
+  LAUNCH_AS("k_hv4", (k_hv4<T, NI, RW, MEAN>), dim3((b.nj + 2 + rows - 1) / rows, b.nk, fs.n * b.nm), dim3(256), shm, s,
+            b.D, b.mb, b.nm, fs, mode);
 }
-void L_hv(hipStream_t s, const Bucket &b, const FieldSet &fs) {
-  if (b.mixed && b.hv_passes == 2 && b.ni >= 16 && b.ni <= 1024) {
-    hv4_mixed(s, b, fs);
-    return;
+// whether a bucket's hyperviscosity runs as k_hv4
+bool hv_fused(const Bucket &b) { return b.hv_passes == 2; }
+// rows per wavefront: those that give a thread four rows of its columns
+template <class T, int MEAN>
+static void hv4_t(hipStream_t s, const Bucket &b, const FieldSet &fs, int mode) {
+  switch (b.ni) {
+    case 8: hv4_ni<T, 8, 8, MEAN_WAVE>(s, b, fs, mode); break;
+    case 16: hv4_ni<T, 16, 4, MEAN_WAVE>(s, b, fs, mode); break;
+    case 32: hv4_ni<T, 32, 4, MEAN_WAVE>(s, b, fs, mode); break;
+    case 64: hv4_ni<T, 64, 4, MEAN_WAVE>(s, b, fs, mode); break;
+    case 128: hv4_ni<T, 128, 2, MEAN_WAVE>(s, b, fs, mode); break;
+    case 256: hv4_ni<T, 256, 1, MEAN>(s, b, fs, mode); break;
+    case 512: hv4_ni<T, 512, 1, MEAN>(s, b, fs, mode); break;
+    default: hv4_ni<T, 1024, 1, MEAN>(s, b, fs, mode); break;
   }
+}
+static void hv4(hipStream_t s, const Bucket &b, const FieldSet &fs, int mode) {
+  if (b.mixed) hv4_t<float, MEAN_BFLY>(s, b, fs, mode);
+  else hv4_t<double, MEAN_BLOCK>(s, b, fs, mode);
+}
+
+// hyperviscosity of hdry and theta, which the advection then takes from sD's
+// copies 1 and 2 (hv_fused) or from the fields; and of u and v, which the
+// Adams-Bashforth update left in those copies or in the fields.  A bucket
+// with a member of higher order takes the separate kernels, in place.
+static void hv_inplace(hipStream_t s, const Bucket &b, const FieldSet &fs) {
   L_merid_hv(s, b, fs);
   L_zonal_hv(s, b, fs);
+}
+void L_hv_hth(hipStream_t s, const Bucket &b) {
+  const FieldSet hth = {2, {F_HDRY, F_THETA}, {2, 3}, 1};
+  if (hv_fused(b)) hv4(s, b, hth, HV_TO_SCRATCH);
+  else hv_inplace(s, b, hth);
+}
+void L_hv_uv(hipStream_t s, const Bucket &b) {
+  const FieldSet uv = {2, {F_U, F_V}, {0, 1}, 0};
+  if (hv_fused(b)) hv4(s, b, uv, HV_FROM_SCRATCH);
+  else hv_inplace(s, b, uv);
 }
 
 }  // namespace epic

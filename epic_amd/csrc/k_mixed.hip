@@ -276,7 +276,8 @@ __global__ void __launch_bounds__(256) km_divdamp(const MemberDesc *D, int mb) {
 // tendency is then stored, rounded to FP32, in the history slot IT_ZERO,
 // which the rotation at the end of the step makes IT_MINUS1.  Lanes cover
 // every cell of planes 1..nk-1 so the stored history is the whole plane.
-__global__ void __launch_bounds__(256) km_ab(const MemberDesc *D, int mb) {
+// scratch: as in k_ab.
+__global__ void __launch_bounds__(256) km_ab(const MemberDesc *D, int mb, int scratch) {
   MEMBER;
   FLAT2(0, d.nj + 1, 1, d.ni);
   const int K = 1 + blockIdx.y;
@@ -300,9 +301,13 @@ __global__ void __launch_bounds__(256) km_ab(const MemberDesc *D, int mb) {
       const double t1 = (ab1 != 0.) ? hist[(size_t)dy.itm1 * d.N3 + q] : 0.,
                    t2 = (ab2 != 0.) ? hist[(size_t)dy.itm2 * d.N3 + q] : 0.;
       const double y = val[q] + d.dt * (ab0 * t0 + ab1 * t1 + ab2 * t2);
-      val[q] = y;
-      if (I == d.ni) val[ix3(d, K, J, 0)] = y;
-      if (I == 1) val[ix3(d, K, J, d.ni + 1)] = y;
+      if (scratch) {
+        d.sD[(size_t)(1 + w) * d.N3 + q] = y;
+      } else {
+        val[q] = y;
+        if (I == d.ni) val[ix3(d, K, J, 0)] = y;
+        if (I == 1) val[ix3(d, K, J, d.ni + 1)] = y;
+      }
     }
     hist[(size_t)dy.it0 * d.N3 + q] = (float)t0;
   }
@@ -326,7 +331,7 @@ void LM_divdamp_apply(hipStream_t s, const Bucket &b) {
   LAUNCH(km_divdamp, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
 }
 void LM_ab(hipStream_t s, const Bucket &b) {
-  LAUNCH(km_ab, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
+  LAUNCH(km_ab, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb, hv_fused(b) ? 1 : 0);
 }
 
 }  // namespace epic

@@ -106,7 +106,11 @@ void L_gz_filtercopy(hipStream_t s, const Bucket &b);
 // part keeps its del^4 result in scratch copy i of sB)
 void L_merid_hv(hipStream_t s, const Bucket &b, const FieldSet &fs);
 void L_zonal_hv(hipStream_t s, const Bucket &b, const FieldSet &fs);
-void L_hv(hipStream_t s, const Bucket &b, const FieldSet &fs);
+// hyperviscosity of hdry and theta (before the advection) and of u and v;
+// hv_fused: as one launch each, through sD's copies 1 and 2
+bool hv_fused(const Bucket &b);
+void L_hv_hth(hipStream_t s, const Bucket &b);
+void L_hv_uv(hipStream_t s, const Bucket &b);
 
 // ---- mixed-precision momentum kernels (k_mixed.hip)
 void LM_uv_core(hipStream_t s, const Bucket &b);
