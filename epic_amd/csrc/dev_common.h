@@ -125,6 +125,11 @@ struct Plane {
     using C = typename std::conditional<std::is_const<T>::value, const char, char>::type;
     return *(T *)((C *)p + (uint32_t)(i * (uint32_t)sizeof(T)));
   }
+  // the point c cells to the east of i (c a constant: an immediate offset)
+  __device__ __forceinline__ T &at(uint32_t i, int c) const {
+    using C = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+    return *(T *)((C *)p + (uint32_t)(i * (uint32_t)sizeof(T)) + c * (int)sizeof(T));
+  }
 };
 
 __device__ __forceinline__ double dmax(double x, double y) { return x > y ? x : y; }

@@ -792,18 +792,29 @@ void L_heating(hipStream_t s, const Bucket &b, int adjust, bool in_thermo) {
 // reference's top/bottom statements write stale-index pad cells), so the
 // dF/dpbot term vanishes and is not formed.
 // With with_source (the step's call) the blocks past the ncb column tiles
-// first clear the step's tendency planes of u and v (the FP64 plane IT_ZERO,
-// or the mixed mode's one FP64 plane), which nothing in this launch reads.
+// first clear what the step does not write of its tendency planes of u and v
+// (the FP64 plane IT_ZERO, or the mixed mode's one FP64 plane; nothing in this
+// launch reads them): planes 0, nk and nk+1 and, of the planes between, rows
+// -1, 0 and nj+1.  k_uv_core forms the rest (row 0 of u again) and k_filter3
+// writes the pads of the rows it passes.
 template <bool F>
 __global__ void __launch_bounds__(1024) k_calc_w(const MemberDesc *D, int mb, int with_source, int C, int ncb) {
   MEMBER;
   if ((int)blockIdx.x >= ncb) {
     const size_t off = d.mixed ? 0 : (size_t)d.dyn->it0 * d.N3;
     double *du = d.DUDT + off, *dv = d.DVDT + off;
-    const size_t st = (size_t)(gridDim.x - ncb) * blockDim.x;
-    for (size_t i = (size_t)(blockIdx.x - ncb) * blockDim.x + threadIdx.x; i < (size_t)d.N3; i += st) {
-      du[i] = 0.;
-      dv[i] = 0.;
+    const int st = (gridDim.x - ncb) * blockDim.x, n = 3 * d.N2 + 3 * d.Ia * (d.nk - 1);
+    for (int i = (blockIdx.x - ncb) * blockDim.x + threadIdx.x; i < n; i += st) {
+      size_t q;
+      if (i < 3 * d.N2) {
+        const int p = i / d.N2;
+        q = (size_t)(p == 0 ? 0 : d.nk + p - 1) * d.N2 + (i - p * d.N2);
+      } else {
+        const int e = i - 3 * d.N2, row = e / d.Ia, k = row / 3, r = row - 3 * k;
+        q = ix3(d, 1 + k, r == 0 ? -1 : r == 1 ? 0 : d.nj + 1, e - row * d.Ia);
+      }
+      du[q] = 0.;
+      dv[q] = 0.;
     }
     return;  // a whole block: no barrier below waits for it
   }
@@ -902,9 +913,9 @@ void L_calc_w(hipStream_t s, const Bucket &b, int with_source) {
   dim3 g = tile_grid(b, C);
   const int ncb = (int)g.x;
   if (with_source) {
-    // blocks that clear the tendency planes: about 16 cells per lane
-    const size_t n3 = (size_t)(b.ni + 2) * (b.nj + 3) * (b.nk + 2);
-    g.x += (unsigned)std::max<size_t>(1, std::min<size_t>(1024, n3 / ((size_t)nt * 16)));
+    // blocks that clear the tendencies' edges: about 4 cells per lane
+    const size_t n = (size_t)(b.ni + 2) * (3 * (b.nj + 3) + 3 * (b.nk - 1));
+    g.x += (unsigned)std::max<size_t>(1, std::min<size_t>(1024, n / ((size_t)nt * 4)));
   }
   const size_t shm = sizeof(double) * (4 * C * (b.nk + 1) + C);
   if (b.mixed) LAUNCH_AS("k_calc_w", k_calc_w<true>, g, dim3(nt), shm, s, b.D, b.mb, with_source, C, ncb);

@@ -52,123 +52,172 @@ __device__ __forceinline__ double *cur_tend(const MemberDesc &d, double *base) {
 }
 
 // ------------------------------------------------------------- uv_core
-// UH (sA), VH (sB), KIN (sC) on planes K = 1..nk-1 with zonal pads; VH rows
-// 0 and nj+1 are zero as in the reference's cleared buffers
-__global__ void __launch_bounds__(256) k_uvh_kin(const MemberDesc *D, int mb) {
-  MEMBER_X;
-  FLAT2_X(0, d.nj + 2, 1, d.ni);
-  const int K = 1 + bx_.y;
-  const Plane<const double> u{d.U + (size_t)K * d.N2}, v{d.V + (size_t)K * d.N2}, h3{d.H3 + (size_t)K * d.N2};
-  const Plane<double> uh{d.sA + (size_t)K * d.N2}, vh{d.sB + (size_t)K * d.N2}, kin{d.sC + (size_t)K * d.N2};
-  const int ni = d.ni, nj = d.nj;
-  if (J <= nj) {
-    double havg = .5 * (h3[ix2(d, J, I)] + h3[ix2(d, J, I - 1)]);
-    double x = u[ix2(d, J, I)] * havg * d.ninv_h[J];
-    uh[ix2(d, J, I)] = x;
-    if (I == ni) uh[ix2(d, J, 0)] = x;
-    if (I == 1) uh[ix2(d, J, ni + 1)] = x;
-    // get_kin (src/shared/epic_funcs_diag.c:2694-2847)
-    const double *mn = d.mn, *mni = d.mn_inv;
-    int jj = 2 * J;
-    double u2 = u[ix2(d, J, I)], u4 = u[ix2(d, J, I + 1)], v2 = v[ix2(d, J, I)], v4 = v[ix2(d, J + 1, I)];
-    double kc = (u2 * u2 + u4 * u4 + mn[jj + 1] * (v2 * v2 * mni[jj] + v4 * v4 * mni[jj + 2])) * .25, k;
-    if (d.pv_al81 || J == 0 || J == nj) {
-      k = kc;
-    } else {
-      u2 = .5 * (u[ix2(d, J + 1, I)] + u[ix2(d, J - 1, I)]);
-      u4 = .5 * (u[ix2(d, J + 1, I + 1)] + u[ix2(d, J - 1, I + 1)]);
-      v2 = .5 * (v[ix2(d, J, I + 1)] + v[ix2(d, J, I - 1)]);
-      v4 = .5 * (v[ix2(d, J + 1, I + 1)] + v[ix2(d, J + 1, I - 1)]);
-      double ks = (u2 * u2 + u4 * u4 + mn[jj + 1] * (v2 * v2 * mni[jj] + v4 * v4 * mni[jj + 2])) * .25;
-      k = (5. / 6.) * kc + (1. / 6.) * ks;
-    }
-    kin[ix2(d, J, I)] = k;
-    if (I == ni) kin[ix2(d, J, 0)] = k;
-    if (I == 1) kin[ix2(d, J, ni + 1)] = k;
-  }
-  double y = 0.;
-  if (J >= 1 && J <= nj) {
-    double havg = .5 * (h3[ix2(d, J, I)] + h3[ix2(d, J - 1, I)]);
-    y = v[ix2(d, J, I)] * havg * d.minv_v[J];
-  }
-  vh[ix2(d, J, I)] = y;
-  if (I == ni) vh[ix2(d, J, 0)] = y;
-  if (I == 1) vh[ix2(d, J, ni + 1)] = y;
+// The step's first tendencies of u and v, formed (not accumulated: nothing
+// before uv_core adds to them) in one launch: Coriolis and kinetic-energy
+// terms with UH, VH and KIN, vertical advection, and the top sponge
+// (uv_drag).  A row team (RowMap) takes one row of one plane: it forms KIN at
+// its four points, filters it (the copy the u tendency takes) where the row
+// lies in the filter band, and hands its neighbours over through an LDS row;
+// UH, VH and the KIN of row J-1 are formed at each point that needs them, from
+// u, v and H3 in cache (4 products each), and never reach memory.  As arrays
+// (one launch to write them, one for each wind to read them) they and the
+// cleared, read and rewritten tendencies were 9.8 GB a step at 1024x512x64 of
+// which 2 GB are needed.  Marching several rows with what they share kept in
+// LDS and registers was slower at nearly every size (2 rows: +1 to +3 % of the
+// step, -1 % at 1024x512x64; 8 rows: +5 to +40 %): its waves wait at barriers.
+// Steps before and after: FP64 256x128x20 521 and 494 us, 1024x512x64 19.1 and
+// 18.7 ms; mixed, 64 members of 128x64x16, 3777 and 3630 us.
+// T = float: the mixed mode's arithmetic (k_mixed.hip); the tendencies are FP64
+// in both.  Plane K = 0 takes the sponge only, with its zonal pads: nothing
+// after uv_drag writes its interior, whose pads the reference fills in the
+// bc_lateral that ends the 3-D filter (the filter itself starts at K = 1 and
+// writes the other planes').
+template <class T>
+struct UvPlanes {
+  Plane<const double> u, v, h3;
+};
+// UH at point i of row j (0..nj)
+template <class T>
+__device__ __forceinline__ T uh_at(const MemberDesc &d, const UvPlanes<T> &p, int j, uint32_t i, int c) {
+  return T(p.u.at(i, c)) * (T(.5) * (T(p.h3.at(i, c)) + T(p.h3.at(i, c - 1)))) * T(d.ninv_h[j]);
 }
-
-// DVDT = (DVDT + PV*UH terms + dKIN/dy) - vertical advection
-__global__ void __launch_bounds__(256) k_dvdt_core(const MemberDesc *D, int mb) {
-  MEMBER_X;
-  FLAT2_X(1, d.nj, 1, d.ni);
-  const int K = 1 + bx_.y;
-  const size_t o = (size_t)K * d.N2;
-  const Plane<const double> uh{d.sA + o}, vh{d.sB + o}, kin{d.sC + o}, pv{d.PV3 + o};
-  const Plane<double> dv{cur_tend(d, d.DVDT) + o};
-  auto PV = [&](int j, int i) { return pv[ix2(d, j, i)]; };
-  const PvW<double> w = pv_weights_v<double>(d.pv_al81, PV, J, I);
-  double x = dv[ix2(d, J, I)];
-  x += ((-w.ga * uh[ix2(d, J, I + 1)] - w.de * uh[ix2(d, J, I)] - w.al * uh[ix2(d, J - 1, I)] -
-         w.be * uh[ix2(d, J - 1, I + 1)] + w.e2 * vh[ix2(d, J - 1, I)] - w.e1 * vh[ix2(d, J + 1, I)]) *
-            w.coef +
-        kin[ix2(d, J - 1, I)] - kin[ix2(d, J, I)]) *
-       d.n[2 * J];
-  int kk = 2 * K + 1;
-  double ds = d.sgth[kk - 2] - d.sgth[kk + 2];
-  x -= .5 * (d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K, J - 1, I)]) *
-       (d.V[ix3(d, K - 1, J, I)] - d.V[ix3(d, K + 1, J, I)]) / ds;
-  dv[ix2(d, J, I)] = x;
+// VH at point i of row j; rows 0 and nj+1 are zero as in the reference's
+// cleared buffers
+template <class T>
+__device__ __forceinline__ T vh_at(const MemberDesc &d, const UvPlanes<T> &p, int j, uint32_t i, int c) {
+  if (j < 1 || j > d.nj) return T(0.);
+  return T(p.v.at(i, c)) * (T(.5) * (T(p.h3.at(i, c)) + T(p.h3.at(i - d.Ia, c)))) * T(d.minv_v[j]);
 }
-
-// DUDT = (DUDT + PV*VH terms + dKIN/dx with filtered KIN) - vertical
-// advection.  One block per (K,J) u-row: the KIN row is zonally filtered in
-// LDS (rows of the filter band) and its pad refreshed, then one lane per I.
-template <bool WIDE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_dudt_core(const MemberDesc *D, int mb) {
+// KIN at point i of row j (get_kin, src/shared/epic_funcs_diag.c:2694-2847)
+template <class T>
+__device__ __forceinline__ T kin_at(const MemberDesc &d, const UvPlanes<T> &p, int j, uint32_t i) {
+  const int jj = 2 * j;
+  const uint32_t in = i + d.Ia, is = i - d.Ia;
+  const T mn1 = T(d.mn[jj + 1]), mi0 = T(d.mn_inv[jj]), mi2 = T(d.mn_inv[jj + 2]);
+  T u2 = T(p.u[i]), u4 = T(p.u.at(i, 1)), v2 = T(p.v[i]), v4 = T(p.v[in]);
+  const T kc = (u2 * u2 + u4 * u4 + mn1 * (v2 * v2 * mi0 + v4 * v4 * mi2)) * T(.25);
+  if (d.pv_al81 || j == 0 || j == d.nj) return kc;
+  u2 = T(.5) * (T(p.u[in]) + T(p.u[is]));
+  u4 = T(.5) * (T(p.u.at(in, 1)) + T(p.u.at(is, 1)));
+  v2 = T(.5) * (T(p.v.at(i, 1)) + T(p.v.at(i, -1)));
+  v4 = T(.5) * (T(p.v.at(in, 1)) + T(p.v.at(in, -1)));
+  const T ks = (u2 * u2 + u4 * u4 + mn1 * (v2 * v2 * mi0 + v4 * v4 * mi2)) * T(.25);
+  return (T(5.) / T(6.)) * kc + (T(1.) / T(6.)) * ks;
+}
+template <bool WIDE, class T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_uv_core(const MemberDesc *D, int mb) {
   MEMBER;
-  extern __shared__ double lds[];
+  constexpr bool F64 = std::is_same<T, double>::value;
+  extern __shared__ double lds_raw[];
   const RowMap m = row_map(d.ni);
-  const int Jr = blockIdx.x * m.rpb + m.g, K = 1 + blockIdx.y, ni = d.ni;
-  const bool live = Jr <= d.nj;
-  const int J = live ? Jr : 0;
+  const int ni = d.ni, nj = d.nj, K = blockIdx.y;
+  const int Jr = blockIdx.x * m.rpb + (WIDE ? __builtin_amdgcn_readfirstlane(m.g) : m.g);
+  const bool live = Jr <= nj;
+  const int J = live ? Jr : nj;
   const size_t o = (size_t)K * d.N2;
-  const Plane<const double> uh{d.sA + o}, vh{d.sB + o}, kin{d.sC + o}, pv{d.PV3 + o};
-  double *kr = lds + (size_t)m.g * ni;  // kr[I-1] = filtered KIN(J,I)
-  double kv[4];
+  const UvPlanes<T> p{{d.U + o}, {d.V + o}, {d.H3 + o}};
+  const Plane<const double> us{d.USPIN + o};
+  const Plane<double> du{cur_tend(d, d.DUDT) + o}, dv{cur_tend(d, d.DVDT) + o};
+  const bool sponge = K <= d.k_sponge;
+  const double ts = sponge ? d.t_sponge[K] : 0.;
+  auto drag = [&](double x, double w) { return F64 ? x - (ts) * w : x - (double)((float)ts * (float)w); };
+  if (K == 0) {  // uniform per block
+    if (!live) return;
 #pragma unroll
-  for (int q = 0; q < 4; q++) kv[q] = kin[ix2(d, J, 1 + m.lane + m.stride * q)];
+    for (int q = 0; q < 4; q++) {
+      const int I = 1 + m.lane + m.stride * q;
+      const uint32_t i = ix2(d, J, I);
+      const double x = drag(0., p.u[i] - us[i]);
+      du[i] = x;
+      if (I == ni) du[ix2(d, J, 0)] = x;
+      if (I == 1) du[ix2(d, J, ni + 1)] = x;
+      if (J < 1) continue;
+      const double y = drag(0., p.v[i] - 0.);
+      dv[i] = y;
+      if (I == ni) dv[ix2(d, J, 0)] = y;
+      if (I == 1) dv[ix2(d, J, ni + 1)] = y;
+    }
+    return;
+  }
+  const Plane<const double> pv{d.PV3 + o}, w3{d.W3 + o}, uu{d.U + o - d.N2}, ud{d.U + o + d.N2}, vu{d.V + o - d.N2},
+      vd{d.V + o + d.N2};
+  const bool al81 = d.pv_al81;
+  T *LK = reinterpret_cast<T *>(lds_raw) + (size_t)m.g * ni;  // [I-1]: filtered KIN
+  T kin[4], kf[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) kf[q] = kin[q] = kin_at<T>(d, p, J, ix2(d, J, 1 + m.lane + m.stride * q));
   const bool filt = live && d.rflag_h[J] != 0;
-  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, kv, kr, J, 0, filt, m.lane);
+  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, kf, LK, J, 0, filt, m.lane);
 #pragma unroll
-  for (int q = 0; q < 4; q++) kr[m.lane + m.stride * q] = kv[q];
+  for (int q = 0; q < 4; q++) LK[m.lane + m.stride * q] = kf[q];
   row_sync<WIDE>();
   if (!live) return;
-  const Plane<double> du{cur_tend(d, d.DUDT) + o};
-  for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-    auto PV = [&](int j, int i) { return pv[ix2(d, j, i)]; };
-    const PvW<double> w = pv_weights_u<double>(d.pv_al81, PV, J, I);
-    const double kin_w = kr[I == 1 ? ni - 1 : I - 2], kin_c = kr[I - 1];
-    double x = du[ix2(d, J, I)];
-    x += ((w.al * vh[ix2(d, J + 1, I)] + w.be * vh[ix2(d, J + 1, I - 1)] + w.ga * vh[ix2(d, J, I - 1)] +
-           w.de * vh[ix2(d, J, I)] + w.e2 * uh[ix2(d, J, I - 1)] - w.e1 * uh[ix2(d, J, I + 1)]) *
-              w.coef +
-          kin_w - kin_c) *
-         d.m[2 * J + 1];
-    int kk = 2 * K + 1;
-    double ds = d.sgth[kk - 2] - d.sgth[kk + 2];
-    x -= .5 * (d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K, J, I - 1)]) *
-         (d.U[ix3(d, K - 1, J, I)] - d.U[ix3(d, K + 1, J, I)]) / ds;
-    du[ix2(d, J, I)] = x;
+  const int kk = 2 * K + 1;
+  const double ds = d.sgth[kk - 2] - d.sgth[kk + 2];
+  const T ds_inv = T(1. / ds);  // the mixed mode's
+  // The stores wait for the last point: a store between two points keeps the
+  // second one's loads behind it.
+  double xu[4], xv[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const uint32_t i = ix2(d, J, 1 + m.lane + m.stride * q), in = i + d.Ia, is = i - d.Ia;
+    auto PV = [&](int j, int c) { return T(pv.at(j == J ? i : j > J ? in : is, c)); };
+    {
+      const PvW<T> w = pv_weights_u<T>(al81, PV, J, 0);
+      const T kw = LK[(m.lane + m.stride * q - 1) & (ni - 1)];
+      T a = w.al * vh_at<T>(d, p, J + 1, in, 0) + w.be * vh_at<T>(d, p, J + 1, in, -1) +
+            w.ga * vh_at<T>(d, p, J, i, -1) + w.de * vh_at<T>(d, p, J, i, 0);
+      if (al81) {
+        const uint32_t iw = (q == 0 && m.lane == 0) ? i + (ni - 1) : i - 1;  // UH's western pad is its point ni
+        a = a + w.e2 * uh_at<T>(d, p, J, iw, 0) - w.e1 * uh_at<T>(d, p, J, i, 1);
+      }
+      double x = 0.;
+      if constexpr (F64) {
+        x += (a * w.coef + kw - kf[q]) * d.m[2 * J + 1];
+        x -= .5 * (w3[i] + w3.at(i, -1)) * (uu[i] - ud[i]) / ds;
+      } else {
+        T y = (a * w.coef + (kw - kf[q])) * T(d.m[2 * J + 1]);
+        y -= T(.5) * T(w3[i] + w3.at(i, -1)) * T(uu[i] - ud[i]) * ds_inv;
+        x += (double)y;
+      }
+      if (sponge) x = drag(x, p.u[i] - us[i]);
+      xu[q] = x;
+    }
+    if (J >= 1) {
+      const PvW<T> w = pv_weights_v<T>(al81, PV, J, 0);
+      T a = -w.ga * uh_at<T>(d, p, J, i, 1) - w.de * uh_at<T>(d, p, J, i, 0) - w.al * uh_at<T>(d, p, J - 1, is, 0) -
+            w.be * uh_at<T>(d, p, J - 1, is, 1);
+      if (al81) a = a + w.e2 * vh_at<T>(d, p, J - 1, is, 0) - w.e1 * vh_at<T>(d, p, J + 1, in, 0);
+      const T ks = kin_at<T>(d, p, J - 1, is);
+      double x = 0.;
+      if constexpr (F64) {
+        x += (a * w.coef + ks - kin[q]) * d.n[2 * J];
+        x -= .5 * (w3[i] + w3[is]) * (vu[i] - vd[i]) / ds;
+      } else {
+        T y = (a * w.coef + (ks - kin[q])) * T(d.n[2 * J]);
+        y -= T(.5) * T(w3[i] + w3[is]) * T(vu[i] - vd[i]) * ds_inv;
+        x += (double)y;
+      }
+      if (sponge) x = drag(x, p.v[i] - 0.);
+      xv[q] = x;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const uint32_t i = ix2(d, J, 1 + m.lane + m.stride * q);
+    du[i] = xu[q];
+    if (J >= 1) dv[i] = xv[q];
   }
 }
-
-void L_uv_core(hipStream_t s, const Bucket &b) {
-  if (b.mixed) { LM_uv_core(s, b); return; }
-  const int nK = b.nk - 1;
-  LAUNCH(k_uvh_kin, grid2(b.nj + 2, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
-  LAUNCH(k_dvdt_core, grid2(b.nj, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
+template <class T>
+static void uv_core_t(hipStream_t s, const Bucket &b) {
   const int rpb = rows_per_block(b.ni);
-  ROWS_LAUNCH(b, "k_dudt_core", k_dudt_core<true>, k_dudt_core<false>, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(double) * rpb * b.ni, s,
-         b.D, b.mb);
+  ROWS_LAUNCH(b, "k_uv_core", (k_uv_core<true, T>), (k_uv_core<false, T>), dim3((b.nj + rpb) / rpb, b.nk, b.nm),
+              dim3(256), sizeof(T) * rpb * b.ni, s, b.D, b.mb);
+}
+void L_uv_core(hipStream_t s, const Bucket &b) {
+  if (b.mixed) uv_core_t<float>(s, b);
+  else uv_core_t<double>(s, b);
 }
 
 // ------------------------------------------------------------- uv_drag
@@ -183,31 +232,6 @@ __device__ __forceinline__ double t_rad(const MemberDesc &d, int K, int J, int I
   double amp = (p / pbot - 0.7) / (1. - 0.7);
   if (amp > 0.) kt += (ks - ka) * d.coslat4_h[J] * amp;  // host-libm table, as the oracle
   return 1. / kt;
-}
-
-// top sponge, K = 0..k_sponge (K = 0 runs even when k_sponge = 0)
-__global__ void __launch_bounds__(256) k_sponge(const MemberDesc *D, int mb) {
-  MEMBER;
-  FLAT2(0, d.nj + 1, 1, d.ni);
-  const int K = blockIdx.y;
-  if (K > d.k_sponge) return;
-  double *du = cur_tend(d, d.DUDT), *dv = cur_tend(d, d.DVDT);
-  size_t q = ix3(d, K, J, I);
-  double ts = d.t_sponge[K];
-  const double x = du[q] - (ts) * (d.U[q] - d.USPIN[q]);
-  du[q] = x;
-  // zonal pads: nothing after uv_drag writes the interior of plane K = 0,
-  // whose pads the reference fills in the bc_lateral that ends the 3-D
-  // filter of the tendency (the filter itself starts at K = 1); the pads
-  // of the other sponge planes are written again by the filter
-  if (I == d.ni) du[ix3(d, K, J, 0)] = x;
-  if (I == 1) du[ix3(d, K, J, d.ni + 1)] = x;
-  if (J >= 1) {
-    const double y = dv[q] - (ts) * (d.V[q] - 0.);
-    dv[q] = y;
-    if (I == d.ni) dv[ix3(d, K, J, 0)] = y;
-    if (I == 1) dv[ix3(d, K, J, d.ni + 1)] = y;
-  }
 }
 
 // Rayleigh drag (tau_drag, or prandtl / t_rad): one block per (K,J) row, the
@@ -277,7 +301,7 @@ __global__ void __launch_bounds__(256) k_hs_pbl(const MemberDesc *D, int mb) {
 
 void L_uv_drag(hipStream_t s, const Bucket &b) {
   if (b.mixed) { LM_uv_drag(s, b); return; }
-  LAUNCH(k_sponge, grid2(b.nj + 1, b.ni, b.nk, b.nm), dim3(TPB), 0, s, b.D, b.mb);
+  // (the top sponge is in k_uv_core)
   if (b.any_ray)
     LAUNCH(k_rayleigh, dim3(b.nj + 1, b.nk, b.nm), dim3(b.ni < 64 ? 64 : b.ni > 256 ? 256 : b.ni),
            sizeof(double) * (2 * b.ni + 2), s, b.D, b.mb);

@@ -47,141 +47,8 @@ static inline dim3 grid2(int nJ, int nI, int nK, int nm) {
 // the current step's tendency plane (FP64) and the FP32 history ring
 __device__ __forceinline__ double *curU(const MemberDesc &d) { return d.DUDT; }
 __device__ __forceinline__ double *curV(const MemberDesc &d) { return d.DVDT; }
-__device__ __forceinline__ float *sAf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sA.get()); }
-__device__ __forceinline__ float *sBf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sB.get()); }
-__device__ __forceinline__ float *sCf(const MemberDesc &d) { return reinterpret_cast<float *>(d.sC.get()); }
-
-// ------------------------------------------------------------ tendencies
-// UH, VH, KIN (FP32 views of sA, sB, sC) on planes 1..nk-1 with zonal pads
-__global__ void __launch_bounds__(256) km_uvh_kin(const MemberDesc *D, int mb) {
-  MEMBER_X;
-  FLAT2_X(0, d.nj + 2, 1, d.ni);
-  const int K = 1 + bx_.y;
-  const size_t o = (size_t)K * d.N2;
-  const Plane<const double> u{d.U + o}, v{d.V + o}, h3{d.H3 + o};
-  const Plane<float> uh{sAf(d) + o}, vh{sBf(d) + o}, kin{sCf(d) + o};
-  const int ni = d.ni, nj = d.nj;
-  if (J <= nj) {
-    float havg = .5f * ((float)h3[ix2(d, J, I)] + (float)h3[ix2(d, J, I - 1)]);
-    float x = (float)u[ix2(d, J, I)] * havg * (float)d.ninv_h[J];
-    uh[ix2(d, J, I)] = x;
-    if (I == ni) uh[ix2(d, J, 0)] = x;
-    if (I == 1) uh[ix2(d, J, ni + 1)] = x;
-    const int jj = 2 * J;
-    const float mn1 = (float)d.mn[jj + 1], mi0 = (float)d.mn_inv[jj], mi2 = (float)d.mn_inv[jj + 2];
-    float u2 = (float)u[ix2(d, J, I)], u4 = (float)u[ix2(d, J, I + 1)];
-    float v2 = (float)v[ix2(d, J, I)], v4 = (float)v[ix2(d, J + 1, I)];
-    float kc = (u2 * u2 + u4 * u4 + mn1 * (v2 * v2 * mi0 + v4 * v4 * mi2)) * .25f, k;
-    if (d.pv_al81 || J == 0 || J == nj) {
-      k = kc;
-    } else {
-      u2 = .5f * ((float)u[ix2(d, J + 1, I)] + (float)u[ix2(d, J - 1, I)]);
-      u4 = .5f * ((float)u[ix2(d, J + 1, I + 1)] + (float)u[ix2(d, J - 1, I + 1)]);
-      v2 = .5f * ((float)v[ix2(d, J, I + 1)] + (float)v[ix2(d, J, I - 1)]);
-      v4 = .5f * ((float)v[ix2(d, J + 1, I + 1)] + (float)v[ix2(d, J + 1, I - 1)]);
-      float ks = (u2 * u2 + u4 * u4 + mn1 * (v2 * v2 * mi0 + v4 * v4 * mi2)) * .25f;
-      k = (5.f / 6.f) * kc + (1.f / 6.f) * ks;
-    }
-    kin[ix2(d, J, I)] = k;
-    if (I == ni) kin[ix2(d, J, 0)] = k;
-    if (I == 1) kin[ix2(d, J, ni + 1)] = k;
-  }
-  float y = 0.f;
-  if (J >= 1 && J <= nj) {
-    float havg = .5f * ((float)h3[ix2(d, J, I)] + (float)h3[ix2(d, J - 1, I)]);
-    y = (float)v[ix2(d, J, I)] * havg * (float)d.minv_v[J];
-  }
-  vh[ix2(d, J, I)] = y;
-  if (I == ni) vh[ix2(d, J, 0)] = y;
-  if (I == 1) vh[ix2(d, J, ni + 1)] = y;
-}
-
-__global__ void __launch_bounds__(256) km_dvdt_core(const MemberDesc *D, int mb) {
-  MEMBER_X;
-  FLAT2_X(1, d.nj, 1, d.ni);
-  const int K = 1 + bx_.y;
-  const size_t o = (size_t)K * d.N2;
-  const Plane<const float> uh{sAf(d) + o}, vh{sBf(d) + o}, kin{sCf(d) + o};
-  const Plane<const double> pv{d.PV3 + o};
-  const Plane<double> dv{curV(d) + o};
-  auto PV = [&](int j, int i) { return (float)pv[ix2(d, j, i)]; };
-  const PvW<float> w = pv_weights_v<float>(d.pv_al81, PV, J, I);
-  float t = -w.ga * uh[ix2(d, J, I + 1)] - w.de * uh[ix2(d, J, I)] - w.al * uh[ix2(d, J - 1, I)] -
-            w.be * uh[ix2(d, J - 1, I + 1)];
-  if (d.pv_al81) t = t + w.e2 * vh[ix2(d, J - 1, I)] - w.e1 * vh[ix2(d, J + 1, I)];
-  float x = (t * w.coef + (kin[ix2(d, J - 1, I)] - kin[ix2(d, J, I)])) * (float)d.n[2 * J];
-  const int kk = 2 * K + 1;
-  const float ds_inv = (float)(1. / (d.sgth[kk - 2] - d.sgth[kk + 2]));
-  const float dvz = (float)(d.V[ix3(d, K - 1, J, I)] - d.V[ix3(d, K + 1, J, I)]);
-  x -= .5f * (float)(d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K, J - 1, I)]) * dvz * ds_inv;
-  dv[ix2(d, J, I)] += (double)x;
-}
-
-// One block per (K,J) u-row group: the row of KIN is zonally filtered in
-// LDS (rows of the filter band, the FP32 filter of the 2-D zonal filter),
-// then one lane per I forms the u tendency, as k_dudt_core does in FP64.
-template <bool WIDE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) km_dudt_core(const MemberDesc *D, int mb) {
-  MEMBER;
-  extern __shared__ double lds_raw[];
-  float *lds = reinterpret_cast<float *>(lds_raw);
-  const RowMap m = row_map(d.ni);
-  const int Jr = blockIdx.x * m.rpb + m.g, K = 1 + blockIdx.y, ni = d.ni;
-  const bool live = Jr <= d.nj;
-  const int J = live ? Jr : 0;
-  const size_t o = (size_t)K * d.N2;
-  const Plane<const float> uh{sAf(d) + o}, vh{sBf(d) + o}, kin{sCf(d) + o};
-  float *kr = lds + (size_t)m.g * ni;  // kr[I-1] = filtered KIN(J,I)
-  float kv[4];
-#pragma unroll
-  for (int q = 0; q < 4; q++) kv[q] = kin[ix2(d, J, 1 + m.lane + m.stride * q)];
-  const bool filt = live && d.rflag_h[J] != 0;
-  if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, kv, kr, J, 0, filt, m.lane);
-#pragma unroll
-  for (int q = 0; q < 4; q++) kr[m.lane + m.stride * q] = kv[q];
-  row_sync<WIDE>();
-  if (!live) return;
-  const Plane<const double> pv{d.PV3 + o};
-  const Plane<double> du{curU(d) + o};
-  const int kk = 2 * K + 1;
-  const float ds_inv = (float)(1. / (d.sgth[kk - 2] - d.sgth[kk + 2])), mj = (float)d.m[2 * J + 1];
-  for (int I = 1 + m.lane; I <= ni; I += m.stride) {
-    auto PV = [&](int j, int i) { return (float)pv[ix2(d, j, i)]; };
-    const PvW<float> w = pv_weights_u<float>(d.pv_al81, PV, J, I);
-    float t = w.al * vh[ix2(d, J + 1, I)] + w.be * vh[ix2(d, J + 1, I - 1)] + w.ga * vh[ix2(d, J, I - 1)] +
-              w.de * vh[ix2(d, J, I)];
-    if (d.pv_al81) t = t + w.e2 * uh[ix2(d, J, I - 1)] - w.e1 * uh[ix2(d, J, I + 1)];
-    const float kin_w = kr[I == 1 ? ni - 1 : I - 2], kin_c = kr[I - 1];
-    float x = (t * w.coef + (kin_w - kin_c)) * mj;
-    const float duz = (float)(d.U[ix3(d, K - 1, J, I)] - d.U[ix3(d, K + 1, J, I)]);
-    x -= .5f * (float)(d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K, J, I - 1)]) * duz * ds_inv;
-    du[ix2(d, J, I)] += (double)x;
-  }
-}
 
 // ------------------------------------------------------------- uv_drag
-__global__ void __launch_bounds__(256) km_sponge(const MemberDesc *D, int mb) {
-  MEMBER;
-  FLAT2(0, d.nj + 1, 1, d.ni);
-  const int K = blockIdx.y;
-  if (K > d.k_sponge) return;
-  double *du = curU(d), *dv = curV(d);
-  const size_t q = ix3(d, K, J, I);
-  const float ts = (float)d.t_sponge[K];
-  const double x = du[q] - (double)(ts * (float)(d.U[q] - d.USPIN[q]));
-  du[q] = x;
-  // zonal pads of plane K = 0, which no later kernel writes (the 3-D
-  // filter's bc_lateral does in the reference)
-  if (I == d.ni) du[ix3(d, K, J, 0)] = x;
-  if (I == 1) du[ix3(d, K, J, d.ni + 1)] = x;
-  if (J >= 1) {
-    const double y = dv[q] - (double)(ts * (float)d.V[q]);
-    dv[q] = y;
-    if (I == d.ni) dv[ix3(d, K, J, 0)] = y;
-    if (I == 1) dv[ix3(d, K, J, d.ni + 1)] = y;
-  }
-}
-
 __device__ __forceinline__ float t_rad_f(const MemberDesc &d, int K, int J, int I) {
   if (d.is_hj) return (float)d.tau_rad;
   if (d.is_tab) return (float)tab_cool_time(d, -crm_log(d.P3[ix3(d, K, J, I)]));
@@ -314,16 +181,7 @@ __global__ void __launch_bounds__(256) km_ab(const MemberDesc *D, int mb, int sc
 }
 
 // ------------------------------------------------------------- launchers
-void LM_uv_core(hipStream_t s, const Bucket &b) {
-  const int nK = b.nk - 1;
-  LAUNCH(km_uvh_kin, grid2(b.nj + 2, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
-  LAUNCH(km_dvdt_core, grid2(b.nj, b.ni, nK, b.nm), dim3(TPB), 0, s, b.D, b.mb);
-  const int rpb = rows_per_block(b.ni);
-  ROWS_LAUNCH(b, "km_dudt_core", km_dudt_core<true>, km_dudt_core<false>, dim3((b.nj + 1 + rpb - 1) / rpb, nK, b.nm), dim3(256), sizeof(float) * rpb * b.ni, s,
-         b.D, b.mb);
-}
 void LM_uv_drag(hipStream_t s, const Bucket &b) {
-  LAUNCH(km_sponge, grid2(b.nj + 1, b.ni, b.nk, b.nm), dim3(TPB), 0, s, b.D, b.mb);
   if (b.any_ray) LAUNCH(km_rayleigh, dim3(b.nj + 1, b.nk, b.nm), dim3(64), 0, s, b.D, b.mb);
   if (b.any_hs) LAUNCH(km_hs_pbl, grid2(b.nj + 1, b.ni, 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
 }

@@ -113,7 +113,6 @@ void L_hv_hth(hipStream_t s, const Bucket &b);
 void L_hv_uv(hipStream_t s, const Bucket &b);
 
 // ---- mixed-precision momentum kernels (k_mixed.hip)
-void LM_uv_core(hipStream_t s, const Bucket &b);
 void LM_uv_drag(hipStream_t s, const Bucket &b);
 void LM_divdamp_apply(hipStream_t s, const Bucket &b);
 void LM_ab(hipStream_t s, const Bucket &b);
