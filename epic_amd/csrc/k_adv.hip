@@ -6,11 +6,10 @@
 //
 // Directions are split as in the reference: vertical column pass, then a
 // meridional pass on every level, then a zonal pass on a zonally filtered
-// copy.  The column pass works on LDS column tiles, the meridional pass on
-// LDS tiles of a few rows by up to 64 columns (each intermediate of the
-// tile formed once), the zonal pass on LDS rows; every intermediate value
-// is formed by the same expression as in the reference, so nothing changes
-// but where it is computed.
+// copy.  The column and meridional passes hold a few cells of a line with
+// their reach in a lane's registers (Akima's: LDS tiles), the zonal pass works
+// on LDS rows; every intermediate value is formed by the same expression as
+// in the reference, so nothing changes but where it is computed.
 //
 // The three advected fields (unity on the pressure grid, theta, hdry) are
 // independent of one another until the theta correction that follows them,
@@ -68,12 +67,6 @@ __device__ __forceinline__ double adv_value(const MemberDesc &d, int which, int 
 // first level of a field that is advected
 __device__ __forceinline__ int adv_kfirst(const MemberDesc &d, int which) { return which == AV_HDRY ? 1 : d.ks - 1; }
 
-// ------------------------------------------------------------ vertical
-// Column tiles of C columns (J = 0..nj, I = 1..ni) with every level in LDS.
-// The pass is a chain of K-stencils (first-guess flux, predictor, centred
-// flux, limiter correction, update) with no recurrence, so each stage runs
-// on all lanes over (column, level) pairs, separated by barriers.
-//
 // The advection passes are templated on the arithmetic type T of the fluxes:
 // double reproduces the reference operation for operation; float is the
 // mixed mode's (the fields stay FP64: each update adds the FP32 flux
@@ -81,21 +74,38 @@ __device__ __forceinline__ int adv_kfirst(const MemberDesc &d, int which) { retu
 template <class T> __device__ __forceinline__ T tmin(T x, T y) { return x < y ? x : y; }
 template <class T> __device__ __forceinline__ T tmax(T x, T y) { return x > y ? x : y; }
 
-template <class T>
-__device__ __forceinline__ T tt_layer(const T *wa, int K, int nk, T ep) {
-  T tt;
-  if (K == 1) tt = fabs(wa[K + 1] - wa[K]) + ep;
-  else if (K == nk) tt = fabs(-wa[K] + wa[K - 1]) + ep;
-  else tt = fabs(wa[K + 1] - T(2.) * wa[K] + wa[K - 1]) + ep;
-  return tt * tt;
+// x / 6, correctly rounded, for finite x of ordinary size: the product with
+// the rounded reciprocal is within an ulp, and one fused correction of its
+// exact remainder rounds it right (Markstein, IBM J. Res. Dev. 34, 1990)
+__device__ __forceinline__ double div6(double x) {
+  const double q = x * (1. / 6.);
+  return fma(fma(-6., q, x), 1. / 6., q);
 }
+__device__ __forceinline__ float div6(float x) {
+  const float q = x * (1.f / 6.f);
+  return fmaf(fmaf(-6.f, q, x), 1.f / 6.f, q);
+}
+
+// The corrected flux through the face between cells m and j; v > 0 carries m
+// into j.  The reference forms it from v split by sign, as the sum of a
+// positive and a negative part of which one is zero; here the part that is
+// not is formed alone, with the donor's (D) and the receiver's (R) values
+// picked by v's sign: the same operations in the same order, half the
+// divisions and square roots.  (Only a zero's sign, and how many cells a NaN
+// spreads in one pass, can differ.)  dh: the predicted change from the cell
+// behind the donor to the donor; nb: the velocity of the face behind it; qD:
+// its smoothness term; prod: (a_D - min)(a_R - min); c: the metric factor of
+// the Courant number.
 template <class T>
-__device__ __forceinline__ T tt_iface(const T *wa, int K, int nk, T ep) {
-  T tt;
-  if (K == 0) tt = fabs(wa[K + 1] - wa[K]) + ep;
-  else if (K == nk) tt = fabs(-wa[K] + wa[K - 1]) + ep;
-  else tt = fabs(wa[K + 1] - T(2.) * wa[K] + wa[K - 1]) + ep;
-  return tt * tt;
+__device__ __forceinline__ T hsu_flux(T v, T aD, T pR, T dh, T qD, T nb, T prod, T c, T DT) {
+  const T fc = T(.5) * (v * (pR + aD));
+  const T x = v * nb;
+  const T vh = copysign(sqrt(x < T(0.) ? T(0.) : x), v);
+  const T al = div6(T(1.) + fabs(v) * c * DT);
+  T g = qD / (qD + prod);
+  g = g * g;
+  const T b = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * g;
+  return fc + -al * (v * b * (pR - aD) - vh * (T(1.) - g) * dh);
 }
 
 // The FP64 value a pass updates: the staged copy itself when the pass
@@ -107,226 +117,207 @@ __device__ __forceinline__ double col_value(float, const MemberDesc &d, int whic
   return adv_value(d, which, K, q, hv);
 }
 
-template <class T>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_hsu_vert(const MemberDesc *D, int mb, int nm, int C, int hv) {
-  ADV_MEMBER;
-  if (d.adv_akima[which]) return;  // the field takes the Akima scheme (uniform per block)
-  extern __shared__ double lds_raw[];
-  T *lds = reinterpret_cast<T *>(lds_raw);
-  const int c = threadIdx.x % C, kk = threadIdx.x / C, KS = blockDim.x / C;
-  const int col = blockIdx.x * C + c;
-  const bool live = col < (d.nj + 1) * d.ni;
-  const int J = live ? col >> d.nlogn : 0, I = live ? 1 + (col & (d.ni - 1)) : 1;
-  const int nk = d.nk, L = nk + 2;
-  const int layer = (which == AV_HDRY);
-  const int kf = (which == AV_THETA) ? d.ks - 1 : 1;
+// ------------------------------------------------------------ vertical
+// A lane takes one column (J = 0..nj, I = 1..ni) and KC of its levels in
+// registers, with the two levels above and below them that the K-stencils
+// (first-guess flux, predictor, centred flux, limiter correction, update)
+// reach: cells K0-2..K0+KC+1 and the velocities of the faces K0-2..K0+KC,
+// face k lying between cells k and k+1 (for unity and theta, whose cells are
+// the interfaces, the mean of W3 above and below).  Every load is issued
+// before the first flux; nothing passes through LDS and the level's metric
+// terms are scalar.  Cells and faces outside the column are formed from
+// whatever the clamped loads gave and replaced.
+// (As stages over an LDS column tile with barriers between, the addresses
+// and waits were most of it: 1730 us against 681 at 1024x512x64, 23.2 against
+// 14.7 at 256x128x20, both FP64.)
+// LAYER: hdry.  EDGE: the reach K0-2..K0+KC+1 touches the top or the bottom
+// (interior chunks carry none of the tests).
+template <class T, int KC, bool LAYER, bool EDGE>
+__device__ __forceinline__ void hsu_vert_cells(const MemberDesc &d, int which, int hv, int K0, int kf, int kout, uint32_t i) {
+  const int nk = d.nk;
   const T ep = T(1.e-10), DT = T(d.dt);
-  const double *dsi = d.dsgth_inv;
-  double *out = adv_out(d, which);
-  T *wa = lds + c * L, *wv = lds + (C + c) * L, *pr = lds + (2 * C + c) * L, *ff = lds + (3 * C + c) * L;
-  // stage 1: field and vertical velocity (wv holds w on the points the
-  // field lives on: W3 itself for layers, the interface average otherwise)
-  if (live) {
-    for (int K = kk; K <= nk + 1; K += KS) {
-      double x = 0., w = 0.;
-      if (layer) {
-        if (K >= kf && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I), hv);
-        if (K >= kf - 1 && K <= nk) w = d.W3[ix3(d, K, J, I)];
-      } else {
-        if (K >= kf - 1 && K <= nk) x = adv_value(d, which, K, ix3(d, K, J, I), hv);
-        if (K >= kf && K <= nk) w = (K == 1 || K == nk) ? 0. : .5 * (d.W3[ix3(d, K, J, I)] + d.W3[ix3(d, K - 1, J, I)]);
-        // statics left by the unity pass (wm[kf-1], wa[kf-2] of its last column)
-        if (which == AV_THETA && K == kf - 1 && K >= 1) {
-          const int Jl = d.nj, Il = d.ni + 1;
-          w = dmin(0., (K == 1 || K == nk) ? 0. : .5 * (d.W3[ix3(d, K, Jl, Il)] + d.W3[ix3(d, K - 1, Jl, Il)]));
-        }
-        if (which == AV_THETA && K == kf - 2) x = 1.;
-      }
-      wa[K] = T(x);
-      wv[K] = T(w);
+  const double *dsi = d.dsgth_inv + (LAYER ? 0 : 1);  // [2k]: of cell k; [2k+1]: of face k
+  const double *in = adv_in(d, which, hv);
+  auto lev = [&](int k, int k0) { return EDGE ? min(max(k, k0), nk) : k; };
+  double f[KC + 4], w[KC + 4];  // the field on cells K0-2 .., W3
+#pragma unroll
+  for (int r = 0; r < KC + 4; r++) f[r] = 1.;  // unity
+  if (LAYER || which == AV_THETA) {
+#pragma unroll
+    for (int r = 0; r < KC + 4; r++) {
+      const int k = lev(K0 - 2 + r, LAYER ? 1 : kf - 1);
+      // theta above its first advected level is the field's own
+      const double *x = (EDGE && !LAYER && k < d.ks - 1) ? d.THETA : in;
+      f[r] = Plane<const double>{x + (size_t)k * d.N2}[i];
     }
   }
-  __syncthreads();
-#define WM(k) tmin(T(0.), wv[k])
-#define WP(k) tmax(T(0.), wv[k])
-  if (layer) {
-    // first-guess flux on interfaces kf..nk-1 (zero at kf-1 and nk)
-    if (live)
-      for (int K = kf - 1 + kk; K <= nk; K += KS)
-        ff[K] = (K == kf - 1 || K == nk) ? T(0.) : WP(K) * wa[K + 1] + WM(K) * wa[K];
-    __syncthreads();
-    if (live)
-      for (int K = kf + kk; K <= nk; K += KS) pr[K] = wa[K] + (ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT;
-    __syncthreads();
-    if (live)
-      for (int K = kf + kk; K < nk; K += KS)
-        ff[K] = T(.5) * (WP(K) * (pr[K] + wa[K + 1]) + WM(K) * (pr[K + 1] + wa[K]));
-    __syncthreads();
-    if (live)
-      for (int K = kf + kk; K < nk; K += KS) {
-        const T d1K = pr[K] - wa[K + 1];
-        const T d1P = (K + 1 == nk) ? T(0.) : pr[K + 1] - wa[K + 2];
-        const T d2K = (K == 1) ? T(0.) : pr[K] - wa[K - 1];
-        const T d2P = pr[K + 1] - wa[K];
-        const T aaK = tt_layer(wa, K, nk, ep), aaP = tt_layer(wa, K + 1, nk, ep);
-        const T aminK = (K >= kf) ? T(d.h_min[K]) : T(0.), aminP = T(d.h_min[K + 1]);
-        const T wpK = WP(K), wmK = WM(K);
-        T whp = sqrt(wpK * WP(K + 1)), whm = -sqrt(wmK * WM(K - 1));
-        T mu = (wpK - wmK) * T(dsi[2 * K + 1]) * DT, al = (T(1.) + mu) / T(6.);
-        T gp = aaP / (aaP + (wa[K + 1] - aminP) * (wa[K] - aminK));
-        gp = gp * gp;
-        T gm = aaK / (aaK + (wa[K + 1] - aminP) * (wa[K] - aminK));
-        gm = gm * gm;
-        T bp = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gp, bm = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gm;
-        T bhp = T(1.) - gp, bhm = T(1.) - gm;
-        ff[K] += -al * (wpK * bp * d1K - whp * bhp * d1P + wmK * bm * d2P - whm * bhm * d2K);
-      }
-    __syncthreads();
-    if (live)
-      for (int K = kf + kk; K <= nk; K += KS)
-        out[ix3(d, K, J, I)] =
-            col_value(wa[K], d, which, K, ix3(d, K, J, I), hv) + (double)((ff[K] - ff[K - 1]) * T(dsi[2 * K]) * DT);
-  } else {
-    // unity's levels above k_sigma-1 serve their neighbours only: flux and
-    // predictor from k_sigma-2, the corrected flux from k_sigma-1
-    const int k1 = max(kf, d.ks - 2), k2 = max(kf, d.ks - 1);
-    // first-guess flux on layers kf..nk (zero below the bottom)
-    if (live)
-      for (int K = k1 + kk; K <= nk + 1; K += KS) ff[K] = (K == nk + 1) ? T(0.) : WP(K) * wa[K] + WM(K) * wa[K - 1];
-    __syncthreads();
-    if (live)
-      for (int K = max(kf - 1, d.ks - 2) + kk; K <= nk; K += KS)
-        pr[K] = (K == kf - 1) ? wa[K] : wa[K] + (ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT;
-    __syncthreads();
-    if (live)
-      for (int K = k2 + kk; K <= nk; K += KS)
-        ff[K] = T(.5) * (WP(K) * (pr[K - 1] + wa[K]) + WM(K) * (pr[K] + wa[K - 1]));
-    __syncthreads();
-    if (live)
-      for (int K = k2 + kk; K <= nk; K += KS) {
-        const T d1K = pr[K - 1] - wa[K];
-        const T d2K = pr[K] - wa[K - 1];
-        const T d2M = (K == kf) ? T(0.) : pr[K - 1] - wa[K - 2];
-        const T aaK = tt_iface(wa, K, nk, ep), aaM = tt_iface(wa, K - 1, nk, ep);
-        const T wpK = WP(K), wmK = WM(K);
-        T whm = (K == 1) ? T(0.) : -sqrt(wmK * WM(K - 1));
-        T whp = (K == nk) ? T(0.) : sqrt(wpK * WP(K + 1));
-        T mu = (wpK - wmK) * T(dsi[2 * K]) * DT, al = (T(1.) + mu) / T(6.);
-        T gp = aaK / (aaK + (wa[K] - T(0.)) * (wa[K - 1] - T(0.)));
-        gp = gp * gp;
-        T gm = aaM / (aaM + (wa[K] - T(0.)) * (wa[K - 1] - T(0.)));
-        gm = gm * gm;
-        T bp = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gp, bm = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gm;
-        T bhp = T(1.) - gp, bhm = T(1.) - gm, g;
-        if (K < nk) {
-          const T d1P = pr[K] - wa[K + 1];
-          g = -al * (wpK * bp * d1K - whp * bhp * d1P + wmK * bm * d2K - whm * bhm * d2M);
-        } else {
-          g = -al * (wpK * bp * d1K + wmK * bm * d2K - whm * bhm * d2M);
-        }
-        ff[K] += g;
-      }
-    __syncthreads();
-    if (live)
-      for (int K = k2 + kk; K <= nk; K += KS)
-        out[ix3(d, K, J, I)] =
-            col_value(wa[K], d, which, K, ix3(d, K, J, I), hv) + (double)((ff[K + 1] - ff[K]) * T(dsi[2 * K + 1]) * DT);
+#pragma unroll
+  for (int r = 0; r < KC + (LAYER ? 3 : 4); r++) w[r] = Plane<const double>{d.W3 + (size_t)lev(K0 - 2 + r, 0) * d.N2}[i];
+  if (LAYER) {
+#pragma unroll
+    for (int r = 0; r < KC + 4; r++) f[r] = dmax(d.h_min[lev(K0 - 2 + r, 1)], f[r]);
+  } else if (EDGE && which == AV_THETA) {  // the reference's static work column holds unity there
+#pragma unroll
+    for (int r = 0; r < KC + 4; r++)
+      if (K0 - 2 + r < kf - 1) f[r] = 1.;
   }
-#undef WM
-#undef WP
+  __builtin_amdgcn_sched_barrier(0);  // every load before the first flux
+  // from here on one face after another, each with the cell it enters
+  T a[KC + 4], v[KC + 3], g0[KC + 3], p[KC + 2], q[KC + 2], F[KC + 1];
+#pragma unroll
+  for (int r = 0; r < KC + 4; r++) a[r] = T(f[r]);
+  // the velocity of face k = K0-2+r and its first-guess flux (none through the
+  // bottom, nor through a layer's top)
+  auto guess = [&](int r) {
+    const int k = K0 - 2 + r;
+    v[r] = T(LAYER ? w[r] : .5 * (w[r + 1] + w[r]));
+    if (EDGE && !LAYER && (k < max(kf - 1, 1) || k >= nk - 1)) v[r] = T(0.);
+    g0[r] = v[r] * (v[r] > T(0.) ? a[r + 1] : a[r]);
+    if (EDGE && (k >= nk || (LAYER && k <= 0))) g0[r] = T(0.);
+  };
+  // predictor and smoothness term of cell k = K0-1+r
+  auto cell = [&](int r) {
+    const int k = K0 - 1 + r;
+    p[r] = a[r + 1] + (g0[r + 1] - g0[r]) * T(dsi[2 * lev(k, 0)]) * DT;
+    if (EDGE && !LAYER && k == kf - 1) p[r] = a[r + 1];
+    T t = a[r + 2] - T(2.) * a[r + 1] + a[r];
+    if (EDGE && k == (LAYER ? 1 : 0)) t = a[r + 2] - a[r + 1];
+    else if (EDGE && k == nk) t = -a[r + 1] + a[r];
+    t = fabs(t) + ep;
+    q[r] = t * t;
+  };
+  double *out = adv_out(d, which);
+  guess(0);
+  guess(1);
+  cell(0);
+#pragma unroll
+  for (int r = 0; r < KC + 1; r++) {
+    // corrected flux through face k: cell j = k above, m = k+1 below
+    const int k = K0 - 1 + r, kk = EDGE ? min(k, nk - 1) : k;
+    guess(r + 2);
+    cell(r + 1);
+    const bool up = v[r + 1] > T(0.);
+    const T aj = a[r + 1], am = a[r + 2];
+    const T prod = LAYER ? (am - T(d.h_min[kk + 1])) * (aj - T(d.h_min[EDGE ? max(kk, 1) : kk])) : am * aj;
+    // the predicted change behind the donor; none at the column's ends
+    T dm = p[r + 1] - a[r + 3], dj = p[r] - a[r];
+    if (EDGE && k + 1 == nk) dm = T(0.);
+    if (EDGE && k == (LAYER ? 1 : kf - 1)) dj = T(0.);
+    F[r] = hsu_flux<T>(v[r + 1], up ? am : aj, up ? p[r] : p[r + 1], up ? dm : dj, up ? q[r + 1] : q[r],
+                       up ? v[r + 2] : v[r], prod, T(dsi[2 * kk + 1]), DT);
+    if (EDGE && (k >= nk || (LAYER && k <= 0))) F[r] = T(0.);
+    if (r > 0 && !(EDGE && (k < kout || k > nk)))
+      Plane<double>{out + (size_t)k * d.N2}[i] = f[r + 1] + (double)((F[r] - F[r - 1]) * T(dsi[2 * k]) * DT);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+template <class T, int KC>
+__global__ void __launch_bounds__(256) k_hsu_vert(const MemberDesc *D, int mb, int nm, int hv) {
+  ADV_MEMBER;
+  const int nk = d.nk, K0 = 1 + (int)blockIdx.y * KC;
+  const bool layer = (which == AV_HDRY);
+  const int kf = (which == AV_THETA) ? d.ks - 1 : 1;
+  // unity's levels above k_sigma-1 serve their neighbours only
+  const int kout = layer ? 1 : max(kf, d.ks - 1);
+  if (d.adv_akima[which] || K0 + KC <= kout) return;  // uniform per block
+  const int col = blockIdx.x * TPB + threadIdx.x;
+  if (col >= (d.nj + 1) * d.ni) return;
+  const uint32_t i = ix2(d, col >> d.nlogn, 1 + (col & (d.ni - 1)));
+  const bool edge = K0 - 2 < max(kout, 2) || K0 + KC + 1 >= nk;  // uniform per block
+  if (layer) {
+    if (edge) hsu_vert_cells<T, KC, true, true>(d, which, hv, K0, kf, kout, i);
+    else hsu_vert_cells<T, KC, true, false>(d, which, hv, K0, kf, kout, i);
+  } else {
+    if (edge) hsu_vert_cells<T, KC, false, true>(d, which, hv, K0, kf, kout, i);
+    else hsu_vert_cells<T, KC, false, false>(d, which, hv, K0, kf, kout, i);
+  }
 }
 
 // ---------------------------------------------------------- meridional
-// One launch: a block holds a tile of TJ rows x CW columns of one plane of
-// one field in LDS, with halos: the field on rows J0-2..J0+TJ+1, the
-// meridional velocities vp, vm (v times 1/m, split by sign) on v-rows
-// J0-1..J0+TJ+1, the smoothness terms aq and the predictor ap on rows
-// J0-1..J0+TJ and the corrected flux on v-rows J0..J0+TJ, each formed once per
-// cell by the reference's expression (the halo rows are formed again by the
-// neighbouring tile: the same values).  The update goes to sA.
-template <class T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_hsu_mer(const MemberDesc *D, int mb, int nm, int CW, int MER_TJ) {
-  ADV_MEMBER;
+// A lane takes one longitude of a plane and TJ rows in registers, with the
+// rows around them as the column pass does: the field on rows J0-2..J0+TJ+1,
+// the velocity v/m on v-rows J0-1..J0+TJ+1 (v-row J lies between rows J-1 and
+// J), predictor and smoothness terms on rows J0-1..J0+TJ and the corrected
+// flux on v-rows J0..J0+TJ; the halo rows are formed again by the
+// neighbouring lane (the same values).  SROW: a wavefront lies in one row
+// tile, whose metric terms are scalar.  The update goes to sA.
+// (From an LDS tile of 64 columns: 1700 us against 680 at 1024x512x64, 26.6
+// against 14.6 at 256x128x20, both FP64; 423 vector instructions a cell.)
+// EDGE: the reach touches a pole (the tiles between carry none of the tests).
+template <class T, int TJ, bool EDGE>
+__device__ __forceinline__ void hsu_mer_cells(const MemberDesc &d, int which, int K, int J0, int I) {
+  const int nj = d.nj;
+  const bool layer = (which == AV_HDRY);
+  const size_t o = (size_t)K * d.N2;
+  const Plane<const double> A{adv_out(d, which) + o}, V{d.V + o}, VU{d.V + o - d.N2};
+  const T amin = layer ? T(d.h_min[K]) : T(0.), DT = T(d.dt), ep = T(1.e-10);
+  auto row = [&](int J, int lo, int hi) { return EDGE ? min(max(J, lo), hi) : J; };
+  double f[TJ + 4], v64[TJ + 3];
+#pragma unroll
+  for (int r = 0; r < TJ + 4; r++) f[r] = A[ix2(d, row(J0 - 2 + r, -1, nj + 1), I)];
+#pragma unroll
+  for (int r = 0; r < TJ + 3; r++) v64[r] = V[ix2(d, row(J0 - 1 + r, 0, nj + 1), I)];
+  if (layer) {
+#pragma unroll
+    for (int r = 0; r < TJ + 3; r++) {
+      const int J = J0 - 1 + r;
+      v64[r] = .5 * (v64[r] + VU[ix2(d, row(J, 0, nj + 1), I)]);
+      if (EDGE && (J < 1 || J > nj)) v64[r] = 0.;
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load before the first flux
+  T a[TJ + 4], v[TJ + 3], g0[TJ + 3], p[TJ + 2], q[TJ + 2], F[TJ + 1];
+#pragma unroll
+  for (int r = 0; r < TJ + 4; r++) a[r] = T(f[r]);
+  auto guess = [&](int r) {
+    const int J = J0 - 1 + r;
+    v[r] = T(v64[r] * d.minv_v[row(J, 0, nj + 1)]);
+    g0[r] = v[r] * (v[r] > T(0.) ? a[r] : a[r + 1]);
+    if (EDGE && (J < 1 || J > nj)) g0[r] = T(0.);
+  };
+  auto cell = [&](int r) {
+    const int J = J0 - 1 + r;
+    p[r] = a[r + 1] + (g0[r] - g0[r + 1]) * T(d.mn[2 * row(J, 0, nj) + 1]) * DT;
+    T t = a[r] - T(2.) * a[r + 1] + a[r + 2];
+    if (EDGE && J == 0) t = -a[r + 1] + a[r + 2];
+    else if (EDGE && J == nj) t = a[r] - a[r + 1];
+    t = fabs(t) + ep;
+    q[r] = t * t;
+  };
+  const Plane<double> sA{d.sA + (size_t)which * d.N3 + o};
+  guess(0);
+  guess(1);
+  cell(0);
+#pragma unroll
+  for (int r = 0; r < TJ + 1; r++) {
+    const int J = J0 + r;
+    guess(r + 2);
+    cell(r + 1);
+    const bool up = v[r + 1] > T(0.);
+    const T am = a[r + 1], aj = a[r + 2];
+    // the predicted change behind the donor; none at the poles
+    T dm = p[r] - a[r], dj = p[r + 1] - a[r + 3];
+    if (EDGE && J == 1) dm = T(0.);
+    if (EDGE && J == nj) dj = T(0.);
+    F[r] = hsu_flux<T>(v[r + 1], up ? am : aj, up ? p[r + 1] : p[r], up ? dm : dj, up ? q[r] : q[r + 1],
+                       up ? v[r] : v[r + 2], (am - amin) * (aj - amin), T(d.mn[2 * row(J, 0, nj)]), DT);
+    if (EDGE && (J < 1 || J > nj)) F[r] = T(0.);
+    if (r > 0 && !(EDGE && J - 1 > nj))
+      sA[ix2(d, J - 1, I)] = f[r + 1] + (double)((F[r - 1] - F[r]) * T(d.mn[2 * J - 1]) * DT);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+template <class T, int TJ, bool SROW>
+__global__ void __launch_bounds__(256) k_hsu_mer(const MemberDesc *D, int mb, int nm) {
+  const int which = (int)blockIdx.z / nm;
+  const MemberDesc &d = D[mb + (int)blockIdx.z - which * nm];
   const int K = 1 + blockIdx.y;
   if (d.adv_akima[which] || K < adv_kfirst(d, which)) return;  // uniform per block
-  extern __shared__ double sh_raw[];
-  T *sh = reinterpret_cast<T *>(sh_raw);
-  const int nj = d.nj, nchunk = d.ni / CW;
-  const int tile = blockIdx.x / nchunk, chunk = blockIdx.x - tile * nchunk;
-  const int J0 = tile * MER_TJ, c = threadIdx.x % CW, r0 = threadIdx.x / CW, RS = blockDim.x / CW;
-  const int I = 1 + chunk * CW + c;
-  const int RA = MER_TJ + 4, RV = MER_TJ + 3, RP = MER_TJ + 2;
-  T *ta = sh, *tvp = ta + RA * CW, *tvm = tvp + RV * CW, *taq = tvm + RV * CW, *tap = taq + RP * CW;
-  T *tff = tap + RP * CW;
-  const size_t o = (size_t)K * d.N2;
-  const Plane<const double> A{adv_out(d, which) + o};
-  const T amin = (which == AV_HDRY) ? T(d.h_min[K]) : T(0.), DT = T(d.dt), ep = T(1.e-10);
-  // row index helpers: field rows from J0-2, v-rows and predictor rows from J0-1
-  auto a = [&](int J) { return ta[(J - J0 + 2) * CW + c]; };
-  auto vp = [&](int J) { return tvp[(J - J0 + 1) * CW + c]; };
-  auto vm = [&](int J) { return tvm[(J - J0 + 1) * CW + c]; };
-  auto aq = [&](int J) { return taq[(J - J0 + 1) * CW + c]; };
-  auto ap = [&](int J) { return tap[(J - J0 + 1) * CW + c]; };
-  // the field (rows outside -1..nj+1 are never read) and the velocities
-  for (int r = r0; r < RA; r += RS) {
-    const int J = J0 - 2 + r;
-    ta[r * CW + c] = (J >= -1 && J <= nj + 1) ? T(A[ix2(d, J, I)]) : T(0.);
-  }
-  for (int r = r0; r < RV; r += RS) {
-    const int J = J0 - 1 + r;
-    if (J < 0 || J > nj + 1) continue;
-    double v2;
-    if (which == AV_HDRY) v2 = (J < 1 || J > nj) ? 0. : .5 * (d.V[ix3(d, K, J, I)] + d.V[ix3(d, K - 1, J, I)]);
-    else v2 = d.V[ix3(d, K, J, I)];
-    const double mi = d.minv_v[J];
-    tvm[r * CW + c] = T(dmin(0., v2 * mi));
-    tvp[r * CW + c] = T(dmax(0., v2 * mi));
-  }
-  __syncthreads();
-  // smoothness terms and predictor on rows J0-1 .. J0+MER_TJ within 0..nj
-  for (int r = r0; r < RP; r += RS) {
-    const int J = J0 - 1 + r;
-    if (J < 0 || J > nj) continue;
-    T t;
-    if (J == 0) t = fabs(-a(0) + a(1)) + ep;
-    else if (J == nj) t = fabs(a(J - 1) - a(J)) + ep;
-    else t = fabs(a(J - 1) - T(2.) * a(J) + a(J + 1)) + ep;
-    taq[r * CW + c] = t * t;
-    const T f0 = (J < 1) ? T(0.) : vp(J) * a(J - 1) + vm(J) * a(J);
-    const T f1 = (J + 1 > nj) ? T(0.) : vp(J + 1) * a(J) + vm(J + 1) * a(J + 1);
-    tap[r * CW + c] = a(J) + (f0 - f1) * T(d.mn[2 * J + 1]) * DT;
-  }
-  __syncthreads();
-  // corrected flux on v-rows J0 .. J0+MER_TJ within 1..nj
-  for (int r = r0; r <= MER_TJ; r += RS) {
-    const int J = J0 + r;
-    if (J < 1 || J > nj) continue;
-    T VP = vp(J), VM = vm(J), APj = ap(J), APm = ap(J - 1), Am = a(J - 1), Aj = a(J);
-    T fc = T(.5) * (VP * (APj + Am) + VM * (APm + Aj));
-    T vhp = sqrt(VP * vp(J - 1)), vhm = -sqrt(VM * vm(J + 1));
-    T mu = (VP - VM) * T(d.mn[2 * J]) * DT, al = (T(1.) + mu) / T(6.);
-    T q0 = aq(J - 1), q1 = aq(J);
-    T gp = q0 / (q0 + (Am - amin) * (Aj - amin));
-    gp = gp * gp;
-    T gm = q1 / (q1 + (Am - amin) * (Aj - amin));
-    gm = gm * gm;
-    T bp = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gp, bm = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gm;
-    T bhp = T(1.) - gp, bhm = T(1.) - gm;
-    T d1J = (APj - Am);
-    T d1m = (J - 1 == 0) ? T(0.) : APm - a(J - 2);
-    T d2m = APm - a(J);
-    T d2J = (J == nj) ? T(0.) : APj - a(J + 1);
-    tff[r * CW + c] = fc + -al * (VP * bp * d1J - vhp * bhp * d1m + VM * bm * d2m - vhm * bhm * d2J);
-  }
-  __syncthreads();
-  // update on the tile's rows: the FP64 field plus the flux divergence
-  const Plane<double> sA{d.sA + so + o};
-  for (int r = r0; r < MER_TJ; r += RS) {
-    const int J = J0 + r;
-    if (J > nj) break;
-    const T f0 = (J >= 1) ? tff[r * CW + c] : T(0.), f1 = (J + 1 <= nj) ? tff[(r + 1) * CW + c] : T(0.);
-    sA[ix2(d, J, I)] = old_value(a(J), &A[ix2(d, J, I)]) + (double)((f0 - f1) * T(d.mn[2 * J + 1]) * DT);
-  }
+  const int t0 = blockIdx.x * TPB + threadIdx.x, tile = t0 >> d.nlogn;
+  const int J0 = TJ * (SROW ? __builtin_amdgcn_readfirstlane(tile) : tile), I = 1 + (t0 & (d.ni - 1));
+  if (J0 > d.nj) return;
+  if (SROW && J0 >= 2 && J0 + TJ < d.nj) hsu_mer_cells<T, TJ, false>(d, which, K, J0, I);
+  else hsu_mer_cells<T, TJ, true>(d, which, K, J0, I);
 }
 
 // --------------------------------------------------------------- zonal
@@ -381,37 +372,26 @@ __device__ __forceinline__ void hsu_zonal_row(const MemberDesc &d, const RowMap 
     UV[0] = T(adv_u(d, layer, K, J, 0) * ninv);
   }
   row_sync<WIDE>();
-  // T(min(0, x)) = min(0, T(x)): rounding is monotone and keeps zero
-  auto UP = [UV](int I) { return tmax(T(0.), UV[I]); };
-  auto UM = [UV](int I) { return tmin(T(0.), UV[I]); };
-  auto FP = [&](int c) { return UP(c) * A[c - 1] + UM(c) * A[c]; };
+  auto FP = [&](int c) { return UV[c] * (UV[c] > T(0.) ? A[c - 1] : A[c]); };
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     const int c = 1 + m.lane + m.stride * q;
     AP[c] = A[c] + (FP(c) - FP(wr(c + 1))) * mn * DT;
   }
   row_sync<WIDE>();
-  // a lane's four corrected fluxes (c = 1 + lane + q*stride) in registers
+  // a lane's four corrected fluxes (c = 1 + lane + q*stride) in registers:
+  // the face between cells cm = c-1 and c
   T ffr[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    const int c = 1 + m.lane + q * m.stride;
-    const int cm = wr(c - 1);
-    T UPc = UP(c), UMc = UM(c), APc = AP[c], APm = AP[cm], Am = A[c - 1], Ac = A[c];
-    T fc = T(.5) * (UPc * (APc + Am) + UMc * (APm + Ac));
-    T d1c = APc - Am, d2c = APc - A[c + 1];
-    T d1m = APm - A[cm - 1], d2m = APm - A[cm + 1];
-    T uhp = sqrt(UPc * UP(c - 1)), uhm = -sqrt(UMc * UM(c + 1));
-    T mu = (UPc - UMc) * mn * DT, al = (T(1.) + mu) / T(6.);
-    T t0 = fabs(A[cm - 1] - T(2.) * A[cm] + A[cm + 1]) + T(1.e-10), q0 = t0 * t0;
-    T t1 = fabs(A[c - 1] - T(2.) * A[c] + A[c + 1]) + T(1.e-10), q1 = t1 * t1;
-    T gp = q0 / (q0 + (Am - amin) * (Ac - amin));
-    gp = gp * gp;
-    T gm = q1 / (q1 + (Am - amin) * (Ac - amin));
-    gm = gm * gm;
-    T bp = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gp, bm = T(1.) + (T(1.) / (T(2.) * al) - T(1.)) * gm;
-    T bhp = T(1.) - gp, bhm = T(1.) - gm;
-    ffr[q] = fc + -al * (UPc * bp * d1c - uhp * bhp * d1m + UMc * bm * d2m - uhm * bhm * d2c);
+    const int c = 1 + m.lane + q * m.stride, cm = wr(c - 1);
+    const T u = UV[c];
+    const bool up = u > T(0.);
+    const int e = up ? cm : c;  // the donor
+    const T aD = A[e], aR = A[up ? c : cm], aW = A[e - 1], aE = A[e + 1];
+    const T t = fabs(aW - T(2.) * aD + aE) + T(1.e-10);
+    ffr[q] = hsu_flux<T>(u, aD, AP[up ? c : cm], AP[e] - (up ? aW : aE), t * t, UV[up ? c - 1 : c + 1],
+                         (aD - amin) * (aR - amin), mn, DT);
     // one point at a time: interleaved, the four need 192 VGPRs
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -689,6 +669,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 // mode forms the fluxes in FP32.  Each scheme's launches run where some field
 // of the bucket takes it.  set_p2etc(DONT_UPDATE_THETA) follows, with
 // store_pgrad_vars.
+template <class T, int KC>
+static void hsu_vert(hipStream_t s, const Bucket &b, int hv) {
+  LAUNCH_AS("k_hsu_vert<T>", (k_hsu_vert<T, KC>), dim3(((b.nj + 1) * b.ni + TPB - 1) / TPB, (b.nk + KC - 1) / KC, ADV_FIELDS * b.nm),
+            dim3(TPB), 0, s, b.D, b.mb, b.nm, hv);
+}
+template <class T, int TJ>
+static void hsu_mer(hipStream_t s, const Bucket &b) {
+  const int tiles = (b.nj + TJ) / TJ;
+  const dim3 g((tiles * b.ni + TPB - 1) / TPB, b.nk, ADV_FIELDS * b.nm);
+  if (b.ni >= 64) LAUNCH_AS("k_hsu_mer<T>", (k_hsu_mer<T, TJ, true>), g, dim3(TPB), 0, s, b.D, b.mb, b.nm);
+  else LAUNCH_AS("k_hsu_mer<T>", (k_hsu_mer<T, TJ, false>), g, dim3(TPB), 0, s, b.D, b.mb, b.nm);
+}
 template <class T>
 static void advection_t(hipStream_t s, const Bucket &b) {
   const int hv = hv_fused(b) ? 1 : 0;
@@ -700,15 +692,24 @@ static void advection_t(hipStream_t s, const Bucket &b) {
   if (v) C = knob_cols(v);
   const bool hsu = b.adv_schemes & 1, akima = b.adv_schemes & 2;
   const dim3 gv((ncol + C - 1) / C, 1, nz);
-  if (hsu)
-    LAUNCH(k_hsu_vert<T>, gv, dim3(knob_threads(v, b.nk + 2)), sizeof(T) * 4 * C * (b.nk + 2), s, b.D, b.mb, b.nm, C, hv);
+  // More cells per lane form fewer halo cells again and leave fewer lanes: 8
+  // of each from 2^22 points up (16.51 against 16.66 ms a step with 4 at
+  // 1024x512x64, no difference at 2^22), 4 below (473 against 476 us with 8 at
+  // 256x128x20, 156 against 159 us at 32x19x7)
+  const bool big = (size_t)b.ni * (b.nj + 1) * b.nk * b.nm >= ((size_t)1 << 22);
+  if (hsu) {
+    if (big) hsu_vert<T, 8>(s, b, hv);
+    else hsu_vert<T, 4>(s, b, hv);
+  }
   if (akima) LAUNCH(k_ak_vert<T>, gv, dim3(knob_threads(v, b.nk + 2)), sizeof(T) * 4 * C * (b.nk + 2), s, b.D, b.mb, b.nm, C, hv);
-  const int TJ = b.knob[KN_ROWS_MER] ? b.knob[KN_ROWS_MER] : 4;
+  const int kn = b.knob[KN_ROWS_MER], TJ = kn ? kn : 4, TJH = kn ? kn : big ? 8 : 4;
   const int CW = b.ni < 64 ? b.ni : 64, tiles = (b.nj + 1 + TJ - 1) / TJ;
   const dim3 gm(tiles * (b.ni / CW), b.nk, nz);
-  if (hsu)
-    LAUNCH(k_hsu_mer<T>, gm, dim3(256), sizeof(T) * CW * ((TJ + 4) + 2 * (TJ + 3) + 2 * (TJ + 2) + (TJ + 1)), s, b.D,
-           b.mb, b.nm, CW, TJ);
+  if (hsu) {
+    if (TJH == 2) hsu_mer<T, 2>(s, b);
+    else if (TJH == 4) hsu_mer<T, 4>(s, b);
+    else hsu_mer<T, 8>(s, b);
+  }
   if (akima)
     LAUNCH(k_ak_mer<T>, gm, dim3(256), sizeof(T) * CW * ((TJ + 4) + 2 * (TJ + 1) + (TJ + 2)), s, b.D, b.mb, b.nm, CW,
            TJ);
