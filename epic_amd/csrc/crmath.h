@@ -52,11 +52,17 @@ CRM_FN void crm_two_sum(double a, double b, double *s, double *e) {
   *s = t;
   *e = (a - (t - bb)) + (b - bb);
 }
-// s + e = a + b exactly, |a| >= |b| (Dekker)
+// s + e = a + b exactly, |a| >= |b| or a = 0 (Dekker)
 CRM_FN void crm_fast_two_sum(double a, double b, double *s, double *e) {
   const double t = a + b;
   *s = t;
   *e = b - (t - a);
+}
+// s + e = a + c b exactly, c b exact, |a| >= |c b| or a = 0
+CRM_FN void crm_fast_two_sum_mul(double a, double c, double b, double *s, double *e) {
+  const double t = __builtin_fma(c, b, a);
+  *s = t;
+  *e = __builtin_fma(c, b, a - t);
 }
 // p + e = a b exactly
 CRM_FN void crm_two_prod(double a, double b, double *p, double *e) {
@@ -65,31 +71,23 @@ CRM_FN void crm_two_prod(double a, double b, double *p, double *e) {
   *e = __builtin_fma(a, b, -t);
 }
 
-// log(x) as a double-double hi + lo, x positive and finite
-CRM_FN void crm_log_dd(double x, double *hi, double *lo) {
-  uint64_t ix = crm_bits(x);
-  int k = (int)(ix >> 52) - 1023;
-  if ((ix >> 52) == 0) {  // subnormal
-    ix = crm_bits(x * 0x1p54);
-    k = (int)(ix >> 52) - 1023 - 54;
-  }
-  double m = crm_double((ix & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);  // [1, 2)
-  // nearest table point 1 + i/256: the top nine mantissa bits, rounded
-  int i = (int)(((ix >> 43) & 0x1ff) + 1) >> 1;
-  double rh, rl;
-  if (i == CRM_N) {  // m near 2: log(x) = (k+1) ln2 + log1p(m/2 - 1)
-    k += 1;
-    m *= 0.5;
-    i = 0;
-  }
-  if (i == 0) {
-    rh = m - 1.0;  // exact (Sterbenz)
-    rl = 0.0;
-  } else {
-    double p, e;
-    crm_two_prod(m, CRM_LOG_INVC[i], &p, &e);
-    crm_two_sum(p - 1.0, e, &rh, &rl);  // p - 1 is exact (Sterbenz)
-  }
+// The main paths below are free of branches (whatever the argument, the table
+// index is in range), so that several calls of one cell can be computed side
+// by side: the waits of a call's two dependent table reads were the time of the
+// kernels that make them.  An argument outside a main path's range takes the
+// result of the *_rare function at the end.
+
+// log(x 2^k0) as a double-double hi + lo, x positive and normal
+CRM_FN void crm_log_dd(double x, int k0, double *hi, double *lo) {
+  const uint64_t ix = crm_bits(x);
+  // nearest table point 1 + i/256: the top nine mantissa bits, rounded; from
+  // 1 + 511/512 up (i = 256) log(x) = (k+1) ln2 + log(m/2), m/2 near 1
+  const int i = (int)(((ix >> 43) & 0x1ff) + 1) >> 1, wrap = i >> 8, j = i & (CRM_N - 1);
+  const int k = (int)(ix >> 52) - 1023 + k0 + wrap;
+  const double m = crm_double((ix & 0x000fffffffffffffULL) | ((uint64_t)(0x3ff - wrap) << 52));  // [1/2, 2)
+  double p, e, rh, rl;
+  crm_two_prod(m, CRM_LOG_INVC[j], &p, &e);
+  crm_fast_two_sum(p - 1.0, e, &rh, &rl);  // p - 1 is exact (Sterbenz), a multiple of 2^-53, |e| <= 2^-54 below 1
   // log1p(rh + rl) = rh - rh^2/2 + rh^3/3 - ... + rl (1 - rh + rh^2) + ...
   double sh, sl;
   crm_two_prod(rh, rh, &sh, &sl);
@@ -97,31 +95,42 @@ CRM_FN void crm_log_dd(double x, double *hi, double *lo) {
       rh * sh *
       (1. / 3. + rh * (-1. / 4. + rh * (1. / 5. + rh * (-1. / 6. + rh * (1. / 7. + rh * (-1. / 8. + rh * (1. / 9.)))))));
   double a, ea;
-  crm_two_sum(rh, -0.5 * sh, &a, &ea);
-  const double l1 = ea + (rl + ((-0.5 * sl) + (-(rh * rl) + (sh * rl + poly))));
-  // k ln2 + T_i + a + l1
-  const double kd = (double)k;
-  double b, eb, c, ec;
-  crm_two_sum(kd * CRM_LN2_HI, CRM_LOG_T[2 * i], &b, &eb);
-  crm_two_sum(b, a, &c, &ec);
-  const double low = eb + ec + (kd * CRM_LN2_LO + CRM_LOG_T[2 * i + 1] + l1);
+  crm_fast_two_sum_mul(rh, -0.5, sh, &a, &ea);
+  const double l1 = ea + (rl + __builtin_fma(-0.5, sl, -(rh * rl) + (sh * rl + poly)));
+  // k ln2 + T_j + a + l1: k LN2_HI is exact and 0 or above T_j, their sum 0 or above a
+  const double kd = (double)k, T = CRM_LOG_T[2 * j];
+  const double b = __builtin_fma(kd, CRM_LN2_HI, T), eb = T - __builtin_fma(-kd, CRM_LN2_HI, b);
+  double c, ec;
+  crm_fast_two_sum(b, a, &c, &ec);
+  const double low = eb + ec + (kd * CRM_LN2_LO + CRM_LOG_T[2 * j + 1] + l1);
   crm_fast_two_sum(c, low, hi, lo);
 }
+CRM_FN int crm_log_main(double x) { return x >= 0x1p-1022 && x < __builtin_inf(); }
+// log of a subnormal as a double-double
+CRM_FN void crm_log_sub(double x, double *hi, double *lo) { crm_log_dd(x * 0x1p54, -54, hi, lo); }
 
-CRM_FN double crm_log(double x) {
+CRM_FN double crm_log_rare(double x) {
   if (!(x > 0.) || x == __builtin_inf()) return log(x);
   double hi, lo;
-  crm_log_dd(x, &hi, &lo);
+  crm_log_sub(x, &hi, &lo);
   return hi + lo;
+}
+CRM_FN double crm_log(double x) {
+  double hi, lo;
+  crm_log_dd(x, 0, &hi, &lo);
+  double r = hi + lo;
+  if (__builtin_expect(!crm_log_main(x), 0)) r = crm_log_rare(x);
+  return r;
 }
 
 // exp(xh + xl), |xl| <= ulp(xh), |xh| < 700
 CRM_FN double crm_exp_dd(double xh, double xl) {
-  const double kd = __builtin_rint(xh * CRM_INV_LN2N);
-  const int k = (int)kd;
+  // the nearest whole number, by adding it to the last place of 1.5 2^52
+  const double kt = xh * CRM_INV_LN2N + 0x1.8p52, kd = kt - 0x1.8p52;
+  const int k = (int)(uint32_t)crm_bits(kt);
   // r = xh + xl - k ln2/256, ln2/256 = C1 + C2 + C3
   double rh, rl;
-  crm_two_sum(xh - kd * CRM_LN2N_C1, -(kd * CRM_LN2N_C2), &rh, &rl);  // both products exact
+  crm_two_sum(__builtin_fma(-kd, CRM_LN2N_C1, xh), -(kd * CRM_LN2N_C2), &rh, &rl);  // both products exact
   rl += xl - kd * CRM_LN2N_C3;
   crm_fast_two_sum(rh, rl, &rh, &rl);
   // expm1(rh + rl) = rh + rh^2/2 + rh^3/6 + ... + rl (1 + rh)
@@ -129,11 +138,11 @@ CRM_FN double crm_exp_dd(double xh, double xl) {
   crm_two_prod(rh, rh, &sh, &sl);
   const double poly = rh * sh * (1. / 6. + rh * (1. / 24. + rh * (1. / 120. + rh * (1. / 720. + rh * (1. / 5040.)))));
   double a, ea;
-  crm_two_sum(rh, 0.5 * sh, &a, &ea);
+  crm_fast_two_sum_mul(rh, 0.5, sh, &a, &ea);
   double ph, pl;
-  crm_fast_two_sum(a, ea + (rl + (0.5 * sl + (rh * rl + poly))), &ph, &pl);
+  crm_fast_two_sum(a, ea + (rl + __builtin_fma(0.5, sl, rh * rl + poly)), &ph, &pl);
   // 2^(j/256) (1 + p)
-  const int j = k & (CRM_N - 1), e = (k - j) / CRM_N;
+  const int j = k & (CRM_N - 1), e = k >> 8;
   const double th = CRM_EXP_T[2 * j], tl = CRM_EXP_T[2 * j + 1];
   double q1, q2, s, es;
   crm_two_prod(th, ph, &q1, &q2);
@@ -144,19 +153,34 @@ CRM_FN double crm_exp_dd(double xh, double xl) {
 }
 
 CRM_FN double crm_exp(double x) {
-  if (!(__builtin_fabs(x) < 700.)) return exp(x);
-  return crm_exp_dd(x, 0.);
+  double r = crm_exp_dd(x, 0.);
+  if (__builtin_expect(!(__builtin_fabs(x) < 700.), 0)) r = exp(x);
+  return r;
 }
 
-CRM_FN double crm_pow(double x, double y) {
+// y (lh + ll) as a double-double
+CRM_FN void crm_pow_arg(double lh, double ll, double y, double *zh, double *zl) {
+  double h, l;
+  crm_two_prod(y, lh, &h, &l);
+  l += y * ll;
+  crm_fast_two_sum(h, l, zh, zl);
+}
+CRM_FN double crm_pow_rare(double x, double y) {
   if (x == 1. || y == 0.) return 1.;
   if (!(x > 0.) || x == __builtin_inf() || !(__builtin_fabs(y) < __builtin_inf())) return pow(x, y);
-  double lh, ll;
-  crm_log_dd(x, &lh, &ll);
-  double zh, zl;
-  crm_two_prod(y, lh, &zh, &zl);
-  zl += y * ll;
-  crm_fast_two_sum(zh, zl, &zh, &zl);
+  double lh, ll, zh, zl;
+  if (x >= 0x1p-1022) crm_log_dd(x, 0, &lh, &ll);
+  else crm_log_sub(x, &lh, &ll);
+  crm_pow_arg(lh, ll, y, &zh, &zl);
   if (!(__builtin_fabs(zh) < 700.)) return pow(x, y);
   return crm_exp_dd(zh, zl);
+}
+CRM_FN double crm_pow(double x, double y) {
+  double lh, ll, zh, zl;
+  crm_log_dd(x, 0, &lh, &ll);
+  crm_pow_arg(lh, ll, y, &zh, &zl);
+  double r = crm_exp_dd(zh, zl);
+  // (y infinite or NaN: zh is too)
+  if (__builtin_expect(!(crm_log_main(x) && __builtin_fabs(zh) < 700.), 0)) r = crm_pow_rare(x, y);
+  return r;
 }
