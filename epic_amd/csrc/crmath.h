@@ -184,3 +184,43 @@ CRM_FN double crm_pow(double x, double y) {
   if (__builtin_expect(!(crm_log_main(x) && __builtin_fabs(zh) < 700.), 0)) r = crm_pow_rare(x, y);
   return r;
 }
+
+// two calls side by side
+CRM_FN void crm_log2(double x0, double x1, double *r0, double *r1) {
+  double h0, l0, h1, l1;
+  crm_log_dd(x0, 0, &h0, &l0);
+  crm_log_dd(x1, 0, &h1, &l1);
+  double a = h0 + l0, b = h1 + l1;
+  const int ok0 = crm_log_main(x0), ok1 = crm_log_main(x1);
+  if (__builtin_expect(!(ok0 & ok1), 0)) {
+    if (!ok0) a = crm_log_rare(x0);
+    if (!ok1) b = crm_log_rare(x1);
+  }
+  *r0 = a;
+  *r1 = b;
+}
+CRM_FN void crm_exp2(double x0, double x1, double *r0, double *r1) {
+  double a = crm_exp_dd(x0, 0.), b = crm_exp_dd(x1, 0.);
+  const int ok0 = __builtin_fabs(x0) < 700., ok1 = __builtin_fabs(x1) < 700.;
+  if (__builtin_expect(!(ok0 & ok1), 0)) {
+    if (!ok0) a = exp(x0);
+    if (!ok1) b = exp(x1);
+  }
+  *r0 = a;
+  *r1 = b;
+}
+CRM_FN void crm_pow2(double x0, double y0, double x1, double y1, double *r0, double *r1) {
+  double lh, ll, z0, w0, z1, w1;
+  crm_log_dd(x0, 0, &lh, &ll);
+  crm_pow_arg(lh, ll, y0, &z0, &w0);
+  crm_log_dd(x1, 0, &lh, &ll);
+  crm_pow_arg(lh, ll, y1, &z1, &w1);
+  double a = crm_exp_dd(z0, w0), b = crm_exp_dd(z1, w1);
+  const int ok0 = crm_log_main(x0) & (__builtin_fabs(z0) < 700.), ok1 = crm_log_main(x1) & (__builtin_fabs(z1) < 700.);
+  if (__builtin_expect(!(ok0 & ok1), 0)) {
+    if (!ok0) a = crm_pow_rare(x0, y0);
+    if (!ok1) b = crm_pow_rare(x1, y1);
+  }
+  *r0 = a;
+  *r1 = b;
+}

@@ -230,6 +230,21 @@ template <bool F> __device__ __forceinline__ double m_pow(double x, double y) {
   else return crm_pow(x, y);
 }
 
+// two at a time
+template <bool F> __device__ __forceinline__ void m_exp2(double x0, double x1, double *r0, double *r1) {
+  if constexpr (F) *r0 = exp(x0), *r1 = exp(x1);
+  else crm_exp2(x0, x1, r0, r1);
+}
+template <bool F> __device__ __forceinline__ void m_log2(double x0, double x1, double *r0, double *r1) {
+  if constexpr (F) *r0 = log(x0), *r1 = log(x1);
+  else crm_log2(x0, x1, r0, r1);
+}
+template <bool F>
+__device__ __forceinline__ void m_pow2(double x0, double y0, double x1, double y1, double *r0, double *r1) {
+  if constexpr (F) *r0 = pow(x0, y0), *r1 = pow(x1, y1);
+  else crm_pow2(x0, y0, x1, y1, r0, r1);
+}
+
 // hybrid sigma-theta coordinate (src/shared/epic_funcs_diag.c:1238-1314,1751-1770)
 template <bool F = false>
 __device__ __forceinline__ double get_sigma(double pbot, double p, double ptop) {
@@ -276,30 +291,36 @@ __device__ __forceinline__ double sgth_of(const MemberDesc &d, double theta, dou
   return 0.;
 }
 
-// The same three functions with the column's log(ptop/pbot) formed once by
+// The same with the column's log(ptop/pbot) formed once by
 // the caller: identical operations on identical operands, so identical
 // results, with one logarithm fewer per call.
 template <bool F = false>
 __device__ __forceinline__ double get_sigma_l(double pbot, double p, double lr) { return m_log<F>(p / pbot) / lr; }
 template <bool F = false>
 __device__ __forceinline__ double get_p_sigma_l(double pbot, double s, double lr) { return pbot * m_exp<F>(s * lr); }
-template <bool F = false>
-__device__ __forceinline__ double sgth_of_l(const MemberDesc &d, double theta, double p, double pbot, double ptop,
-                                            double lr, int *bad) {
-  if (p <= ptop) return theta;
-  if (p <= pbot) {
-    const double s = get_sigma_l<F>(pbot, p, lr);
-    // f_sig(s) + g_sig(s) * theta with g_sigma's exponential formed once (the
-    // same operations as the two calls, so the same result)
-    const bool mid = (s > d.sigma_sigma && s < 1.);
-    const double gm = mid ? d.g_coeff * (1. - m_exp<F>(-d.alpha * (s - d.sigma_sigma))) : 0.;
+// sgth_of at p2 less sgth_of at p4, ptop <= p2 < p4 <= pbot (p4 > ptop), the
+// transcendentals of the two side by side: f_sig(s) + g_sig(s) theta with
+// g_sigma's exponential formed once (the same operations as the two calls, so
+// the same result); *bad as sgth_of sets it
+template <bool F>
+__device__ __forceinline__ double sgth_diff_l(const MemberDesc &d, double theta, double p2, double p4, double pbot,
+                                              double ptop, double lr, int *bad) {
+  double s2, s4, e2 = 0., e4 = 0.;
+  m_log2<F>(p2 / pbot, p4 / pbot, &s2, &s4);
+  s2 = s2 / lr;
+  s4 = s4 / lr;
+  const bool mid2 = s2 > d.sigma_sigma && s2 < 1., mid4 = s4 > d.sigma_sigma && s4 < 1.;
+  if (mid2 || mid4) m_exp2<F>(-d.alpha * (s2 - d.sigma_sigma), -d.alpha * (s4 - d.sigma_sigma), &e2, &e4);
+  auto value = [&](double s, bool mid, double e, double p) {
+    const double gm = mid ? d.g_coeff * (1. - e) : 0., lin = d.zeta0 + s * (d.zeta1 - d.zeta0);
     const double g = (s <= d.sigma_sigma) ? 0. : (s >= 1. ? 1. : gm);
-    const double f = (s < 0.) ? d.zeta0 : (s <= d.sigma_sigma ? d.zeta0 + s * (d.zeta1 - d.zeta0)
-                                                              : (s < 1. ? (1. - gm) * (d.zeta0 + s * (d.zeta1 - d.zeta0)) : 0.));
-    return f + g * theta;
-  }
-  *bad = 1;
-  return 0.;
+    const double f = (s < 0.) ? d.zeta0 : (s <= d.sigma_sigma ? lin : (s < 1. ? (1. - gm) * lin : 0.));
+    double x = f + g * theta;
+    if (p <= ptop) x = theta;
+    else if (!(p <= pbot)) *bad = 1, x = 0.;
+    return x;
+  };
+  return value(s2, mid2, e2, p2) - value(s4, mid4, e4, p4);
 }
 
 // The block's tile as a logical (x, y, z), renumbered for the XCDs: a

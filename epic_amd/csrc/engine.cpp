@@ -317,7 +317,7 @@ static void rec_step(hipStream_t s, const Bucket &b, bool hv, bool divd, bool ad
   // store_diag, then the time planes rotated (in the same launch: nothing
   // after the Adams-Bashforth update reads them)
   rec_store_diag(s, b, 1);
-  L_heating(s, b, adjust, true);  // the relaxation itself was formed with T3 (thermo_cell)
+  L_heating(s, b, adjust, true);  // the relaxation itself was formed with T3 (k_thermo)
 }
 
 void member_record(hipStream_t s, const Bucket &b, bool sync_only, bool hv, bool divd, bool adjust) {

@@ -6,13 +6,13 @@
 //   calc_heating      src/shared/epic_funcs_diag.c:4793-4869 +
 //                     src/shared/epic_sensible_heating.c:51-463 (Held-Suarez,
 //                     and the hot Jupiter's day-night relaxation; inside the
-//                     step it is formed with T3 by thermo_cell)
+//                     step it is formed with T3 by k_thermo)
 //   calc_w            src/shared/epic_flux.c:123-335           (column scan)
 //   vorticity         src/shared/epic_funcs_diag.c:4131-4445
 //   divergence        src/shared/epic_funcs_diag.c:4064-4117
 //
-// Column work runs in LDS column tiles (per-level arithmetic on every lane,
-// the K recurrences in one lane per column); zonal means stage the row in
+// Column work runs in column tiles (a few levels in a lane's registers, the K
+// recurrences in one lane per column over LDS); zonal means stage the row in
 // LDS and sum it in one lane in the reference's order.  The arithmetic of
 // each expression follows the reference's operation order.
 #include <algorithm>
@@ -58,183 +58,251 @@ void L_fill(hipStream_t s, const Bucket &b, int f, double v) {
 }
 
 // ------------------------------------------------------------ column tiles
-// A block holds C consecutive (J,I) columns (J = 0..nj, I = 0..ni+1) and
-// all their levels.  The per-level work (transcendentals, Leslie-Purser
-// weights) runs on all lanes, (column, level) pairs strided over the block;
-// the recurrences in K (pressure from the top, geopotential from the
-// bottom, the running SUM_DIV) run in one lane per column over values staged
-// in LDS, in the reference's order.  C is 64 where the block's LDS stays
-// small; deep grids take 32 or 16 columns so that several blocks still fit
-// in a CU's LDS.
+// A block holds C consecutive (J,I) columns (J = 0..nj, I = 0..ni+1) and all
+// their levels.  A lane takes one column and KC of its levels 1..nk,
+// K0..K0+KC-1, in registers, with the levels around them that it needs read
+// (and their logarithms formed) again; the first lane has level 0 too; the recurrences in K (pressure from the top,
+// geopotential from the bottom, the running SUM_DIV) run in one lane per
+// column over one array in LDS, in the reference's order, between two
+// barriers.  With C = 64 a wavefront's lanes share their levels (U): what
+// depends on the level alone is scalar and the tests on it are scalar
+// branches.  (With the levels strided over the lanes of 32 columns, and every
+// per-level value of the others read from LDS, those tables were three of
+// every five vector loads and the logarithms' and quotients' operands came
+// from memory up to four times.)
+template <bool U>
 struct Tile {
-  int C, c, kk, KS, J, I;
-  bool live;
+  int C, c, K0, J, I;
+  bool live, scan;  // a column of the grid; runs the column's recurrence
+  uint32_t i;       // the column in a plane
+  __device__ __forceinline__ Tile(const MemberDesc &d, int C_, int KC) : C(C_) {
+    const int g = U ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : (int)threadIdx.x / C;
+    c = U ? (int)threadIdx.x & 63 : (int)threadIdx.x - g * C;
+    K0 = 1 + g * KC;
+    const int nI = d.ni + 2, n = (d.nj + 1) * nI, col = blockIdx.x * C + c;
+    live = col < n;
+    scan = g == 0;
+    const int q = live ? col : n - 1;  // lanes past the last column repeat it and store nothing
+    J = q / nI;
+    I = q - J * nI;
+    i = ix2(d, J, I);
+  }
+  __device__ __forceinline__ Plane<const double> at(const MemberDesc &d, const double *f, int K) const {
+    return {f + (size_t)K * d.N2};
+  }
 };
-__device__ __forceinline__ Tile tile_of(const MemberDesc &d, int C) {
-  Tile t;
-  t.C = C;
-  t.c = threadIdx.x % C;
-  t.kk = threadIdx.x / C;
-  t.KS = blockDim.x / C;
-  const int nI = d.ni + 2, col = blockIdx.x * C + t.c;
-  t.live = col < (d.nj + 1) * nI;
-  t.J = t.live ? col / nI : 0;
-  t.I = t.live ? col % nI : 0;
-  return t;
-}
-// columns per block for a kernel keeping `arrays` (nk+1)-long columns in LDS
-static inline int tile_cols(const Bucket &b, int arrays) {
-  int C = 64;
-  while (C > 16 && (size_t)arrays * C * (b.nk + 1) * sizeof(double) > 40 * 1024) C /= 2;
-  return C;
+// a tile kernel's shape: columns, levels per lane, threads
+struct ColShape {
+  int C, KC, nt;
+};
+static inline ColShape col_shape(const Bucket &b, int knob) {
+  const int lev = b.nk;
+  ColShape s{64, 2, 0};
+  if (knob) {
+    s.C = knob_cols(knob);
+    const int groups = std::max(1, knob_threads(knob, lev + 1) / s.C);
+    while (s.KC < 8 && groups * s.KC < lev) s.KC *= 2;
+  } else {
+    // More levels a lane read and form fewer around them again, but leave
+    // fewer wavefronts: the most that leave 8192 (8 levels) or 2048 (4) of
+    // them.  Steps with 2, 4 and 8 levels: 64x32x10 170, 181, 208 us;
+    // 256x128x20 441, 442, 469; 23 members of 128x51x13 955, 952, 981; 64 mixed
+    // ones of 128x64x16 3510, 3414, 3310; mixed 512x256x32 1786, 1786, 1759.
+    const size_t tiles = ((size_t)(b.nj + 1) * (b.ni + 2) + 63) / 64 * b.nm;
+    s.KC = tiles * ((lev + 7) / 8) >= 8192 ? 8 : tiles * ((lev + 3) / 4) >= 2048 ? 4 : 2;
+  }
+  // (any depth: 8 columns take up to 1024 levels)
+  while (s.KC < 8 && (lev + s.KC - 1) / s.KC * s.C > 1024) s.KC *= 2;
+  while (s.C > 1 && (lev + s.KC - 1) / s.KC * s.C > 1024) s.C /= 2;
+  s.nt = s.C * ((lev + s.KC - 1) / s.KC);
+  return s;
 }
 static inline dim3 tile_grid(const Bucket &b, int C) {
   return dim3((unsigned)(((b.nj + 1) * (b.ni + 2) + C - 1) / C), 1, (unsigned)b.nm);
 }
+#define COLS_LAUNCH_U(name, kern, U, sh, ...)                     \
+  do {                                                            \
+    if ((sh).KC == 2) LAUNCH_AS(name, (kern(2, U)), __VA_ARGS__);      \
+    else if ((sh).KC == 4) LAUNCH_AS(name, (kern(4, U)), __VA_ARGS__); \
+    else LAUNCH_AS(name, (kern(8, U)), __VA_ARGS__);                   \
+  } while (0)
+#define COLS_LAUNCH(name, kern, sh, ...)                        \
+  do {                                                          \
+    if ((sh).C == 64) COLS_LAUNCH_U(name, kern, true, sh, __VA_ARGS__); \
+    else COLS_LAUNCH_U(name, kern, false, sh, __VA_ARGS__);             \
+  } while (0)
 
 // ------------------------------------------------------------ set_p2etc
 // P3 from the top down (prefix of dsgth*g*h), the sigma-region pressures,
 // h = max(h_min, dp/(g dsgth)), and the layer diagnostics P2, H3, THETA2
 // (and the theta of the sigma region when update_theta)
 // The FULL = 0 launch then forms store_pgrad_vars' T3 and RHO3 of its
-// columns (thermo_cell).
+// columns.
 // FULL = 1: set_p2etc(UPDATE_THETA) with P2, H3, THETA2.  FULL = 0: the
 // call that follows the advection inside the step forms P3 and h (and the
 // pressure-range check) only: the P2 and H3 it would form are written again
 // by the step's second set_p2etc before anything reads them, so the values
 // the step leaves are the same.
-template <bool F>
-__device__ __forceinline__ void thermo_cell(const MemberDesc &d, int K, int J, int I, bool full, double th, double p);
+// T3 and RHO3 of an interface cell (return_temp and return_density with
+// x_h2 = 0); pk = (p/press0)^kappa
+__device__ __forceinline__ double t3_of(double th, double pk) { return th * pk; }
+__device__ __forceinline__ double rho3_of(const MemberDesc &d, double p, double t) {
+  const double R_GAS = 8.314472e+3;
+  return p * d.mu3 / (R_GAS * t);
+}
 // F: the mixed mode's exp/log/pow (m_exp)
-template <int FULL, bool F>
+// FP64, 1024x512x64: FULL = 0 912 us before (the levels strided over a tile's
+// lanes), 533 now; FULL = 1 1346 and 1114; 256x128x20: 22 and 19, 39 and 36.
+template <int FULL, bool F, int KC, bool U>
 __global__ void __launch_bounds__(1024) k_set_p2etc(const MemberDesc *D, int mb, int C) {
-  constexpr bool update_theta = FULL;
   MEMBER;
   extern __shared__ double lds[];
-  const Tile T = tile_of(d, C);
-  const int nk = d.nk, ks = d.ks, W = nk + 1, J = T.J, I = T.I;
-  double *a = lds + T.c * W, *pw = lds + C * W + T.c * W;
-  // theta(ks-2), H3(1), P2(1), log(ptop/pbot) of the column
-  double *aux = lds + 2 * C * W + 4 * T.c;
-  double *P3 = d.P3, *H = d.HDRY;
-  const double g = d.g[2 * J + 1];
-  if (T.live)
-    for (int K = T.kk; K <= nk; K += T.KS)
-      a[K] = (K == 0) ? P3[ix3(d, 0, J, I)] : d.dsgth[2 * K] * g * H[ix3(d, K, J, I)];
+  const Tile<U> T(d, C, KC);
+  const int nk = d.nk, ks = d.ks, K0 = T.K0;
+  double *L = lds + T.c;  // [K C]: the pressure's terms, then P3
+  const double g = d.g[2 * T.J + 1], zr = d.zeta1 - d.zeta0;
+  double h[KC];
+#pragma unroll
+  for (int r = 0; r < KC; r++) h[r] = T.at(d, d.HDRY, min(K0 + r, nk))[T.i];
+  if (T.scan) L[0] = T.at(d, d.P3, 0)[T.i];
+#pragma unroll
+  for (int r = 0; r < KC; r++) {
+    const int K = K0 + r;
+    if (K <= nk) L[K * C] = d.dsgth[2 * K] * g * h[r];
+  }
   __syncthreads();
-  // running sum in a register (a[K-1] + a[K], in order), not through LDS,
-  // its terms read eight at a time ahead of the chain
-  if (T.live && T.kk == 0) {
-    double acc = a[0];
+  // the running sum in a register, its terms read eight at a time ahead of
+  // the chain
+  if (T.scan) {
+    double acc = L[0];
     int K = 1;
     for (; K + 7 <= nk; K += 8) {
       double t8[8];
 #pragma unroll
-      for (int u = 0; u < 8; u++) t8[u] = a[K + u];
+      for (int u = 0; u < 8; u++) t8[u] = L[(K + u) * C];
 #pragma unroll
       for (int u = 0; u < 8; u++) {
         acc = acc + t8[u];
-        a[K + u] = acc;
+        L[(K + u) * C] = acc;
       }
     }
     for (; K <= nk; K++) {
-      acc = acc + a[K];
-      a[K] = acc;
-    }
-    // log(ptop/pbot) once per column (the sigma-region formulas read it)
-    aux[3] = m_log<F>(a[0] / a[nk]);
-  }
-  __syncthreads();
-  if (T.live) {
-    const double pbot = a[nk], lr = aux[3];
-    for (int K = ks - 1 + T.kk; K < nk; K += T.KS) {
-      double sigma = (d.sgth[2 * K + 1] - d.zeta0) / (d.zeta1 - d.zeta0);
-      a[K] = get_p_sigma_l<F>(pbot, sigma, lr);
+      acc = acc + L[K * C];
+      L[K * C] = acc;
     }
   }
   __syncthreads();
-  // p^(kappa+1) once per interface (each is the top of one layer and the
-  // bottom of the next)
-  if (FULL && T.live)
-    for (int K = T.kk; K <= nk; K += T.KS) pw[K] = m_pow<F>(a[K], d.kappa + 1.);
-  __syncthreads();
-  if (T.live) {
-    const double pbot = a[nk], kp1 = d.kappa + 1., lr = aux[3];
-    const double *tx = d.sgth + 2 * nk + 1;  // tx[kay*(-2)] = sgth[2*(nk-kay)+1]
-    for (int K = T.kk; K <= nk; K += T.KS) {
-      const size_t q = ix3(d, K, J, I);
-      P3[q] = a[K];
-      if (update_theta && K < ks - 1) {
-        double sigma = get_sigma_l<F>(pbot, a[K], lr);
-        double th = theta_of_sigma<F>(d, d.sgth[2 * K + 1], sigma);
-        d.THETA[q] = th;
-        if (K == ks - 2) aux[0] = th;
-      }
-      if (K == 0) continue;
-      double hl = (a[K] - a[K - 1]) / (g * d.dsgth[2 * K]);
-      H[q] = dmax(d.h_min[K], hl);
-      if (!FULL) {
-        if (fcmp_d(a[K], a[K - 1]) != 0 && (a[K - 1] < 0. || a[K] < 0.)) atomicOr(&d.dyn->err, 2);
-        continue;
-      }
-      double top = a[K - 1], bot = a[K], pp;
+  const double ptop = L[0], pbot = L[nk * C], lr = m_log<F>(ptop / pbot);
+  // P3 on K0-1 .. K0+KC
+  double p[KC + 2];
+#pragma unroll
+  for (int r = 0; r < KC + 2; r++) {
+    const int K = min(K0 - 1 + r, nk);
+    p[r] = L[K * C];
+    if (K >= ks - 1 && K < nk) p[r] = get_p_sigma_l<F>(pbot, (d.sgth[2 * K + 1] - d.zeta0) / zr, lr);
+  }
+  if (!T.live) return;
+  auto in = [&](double *f, int K) { return T.at(d, f, K)[T.i]; };
+  auto out = [&](double *f, int K, double x) { Plane<double>{f + (size_t)K * d.N2}[T.i] = x; };
+  if constexpr (!FULL) {
+    // P3, h and store_pgrad_vars' per-cell part (T3, RHO3)
+    double th[KC], pk[KC];
+#pragma unroll
+    for (int r = 0; r < KC; r++) th[r] = in(d.THETA, min(K0 + r, nk));
+#pragma unroll
+    for (int r = 0; r < KC; r += 2)
+      m_pow2<F>(p[r + 1] / d.press0, d.kappa, p[r + 2] / d.press0, d.kappa, &pk[r], &pk[r + 1]);
+    if (T.scan) {
+      const double t0 = t3_of(in(d.THETA, 0), m_pow<F>(ptop / d.press0, d.kappa));
+      out(d.T3, 0, t0);
+      out(d.RHO3, 0, rho3_of(d, ptop, t0));
+    }
+#pragma unroll
+    for (int r = 0; r < KC; r++) {
+      const int K = K0 + r;
+      if (K > nk) break;
+      const double a = p[r + 1], am = p[r];
+      const double hl = (a - am) / (g * d.dsgth[2 * K]), t = t3_of(th[r], pk[r]);
+      out(d.P3, K, a);
+      out(d.HDRY, K, dmax(d.h_min[K], hl));
+      if (fcmp_d(a, am) != 0 && (am < 0. || a < 0.)) atomicOr(&d.dyn->err, 2);
+      out(d.T3, K, t);
+      out(d.RHO3, K, rho3_of(d, a, t));
+    }
+  } else {
+    // p^(kappa+1) of a level's interface, formed beside P2 of the level above
+    const double kp1 = d.kappa + 1., ki = 1. / d.kappa;
+    double pwm, pw;
+    m_pow2<F>(p[0], kp1, p[1], kp1, &pwm, &pw);
+    double th = 0., thm = 0.;  // theta around a level above k_sigma-1
+    if (K0 <= ks - 1) thm = theta_of_sigma<F>(d, d.sgth[2 * K0 - 1], get_sigma_l<F>(pbot, p[0], lr));
+    if (T.scan && ks > 1) out(d.THETA, 0, thm);
+#pragma unroll
+    for (int r = 0; r < KC; r++) {
+      const int K = K0 + r;
+      if (K > nk) break;
+      const double bot = p[r + 1], top = p[r];
+      // from k_sigma down, theta2 is a linear interpolation of theta against
+      // sigmatheta, table ordered from the bottom interface up
+      // (src/shared/epic_funcs_diag.c:3522-3562); the interval is the same in
+      // every column, found once on the host by the same search
+      const int kay = K >= ks ? d.t2_kay[K] : 0;
+      double y0 = 0., y1 = 0.;
+      if (K >= ks) y0 = in(d.THETA, nk - kay), y1 = in(d.THETA, nk - kay - 1);
+      else if (K == ks - 1) y0 = in(d.THETA, K);
+      double pp, pwn = 0.;
+      const double x = (pw - pwm) / (kp1 * (bot - top));
+      if (r + 1 < KC) m_pow2<F>(x, ki, p[r + 2], kp1, &pp, &pwn);
+      else pp = m_pow<F>(x, ki);
       if (fcmp_d(bot, top) == 0) pp = .5 * (bot + top);
       else if (top < 0. || bot < 0.) { atomicOr(&d.dyn->err, 2); pp = 0.; }
-      else pp = m_pow<F>((pw[K] - pw[K - 1]) / (kp1 * (bot - top)), 1. / d.kappa);
-      if (K == 1) aux[2] = pp;
-      d.P2[q] = pp;
-      double h3;
+      const double hl = (bot - top) / (g * d.dsgth[2 * K]);
+      double h3 = hl;
       if (K < nk) {
-        int kk = 2 * K + 1;
-        double topwt = d.dsgth[kk - 1], botwt = d.dsgth[kk + 1];
-        double hl1 = (a[K + 1] - a[K]) / (g * d.dsgth[2 * (K + 1)]);
+        const int kk = 2 * K + 1;
+        const double topwt = d.dsgth[kk - 1], botwt = d.dsgth[kk + 1];
+        const double hl1 = (p[r + 2] - bot) / (g * d.dsgth[2 * (K + 1)]);
         h3 = (topwt * hl + botwt * hl1) / (topwt + botwt);
+      }
+      double th2;
+      if (K < ks - 1) {
+        double s3, s2;
+        m_log2<F>(bot / pbot, pp / pbot, &s3, &s2);
+        th = theta_of_sigma<F>(d, d.sgth[2 * K + 1], s3 / lr);
+        th2 = theta_of_sigma<F>(d, d.sgth[2 * K], s2 / lr);
+        out(d.THETA, K, th);
+      } else if (K >= ks) {
+        const double sg = d.sgth[2 * K], hh = d.t2_h[K];
+        th2 = y0 + (y1 - y0) * (sg - d.sgth[2 * (nk - kay) + 1]) / hh;
       } else {
-        h3 = hl;
+        th2 = .5 * (y0 + thm);
       }
-      d.H3[q] = h3;
-      if (K == 1) aux[1] = h3;
-      if (update_theta) {
-        if (K < ks - 1) {
-          double sigma = get_sigma_l<F>(pbot, pp, lr);
-          d.THETA2[q] = theta_of_sigma<F>(d, d.sgth[2 * K], sigma);
-        } else if (K >= ks) {
-          // linear interpolation of theta against sigmatheta, table ordered
-          // from the bottom interface up (src/shared/epic_funcs_diag.c:3522-3562);
-          // the interval is the same in every column, found once on the host
-          // by the same search
-          const double sg = d.sgth[2 * K], h = d.t2_h[K];
-          const int kay = d.t2_kay[K];
-          double y0 = d.THETA[ix3(d, nk - kay, J, I)], y1 = d.THETA[ix3(d, nk - kay - 1, J, I)];
-          d.THETA2[q] = y0 + (y1 - y0) * (sg - tx[-2 * kay]) / h;
-        }
+      out(d.P3, K, bot);
+      out(d.HDRY, K, dmax(d.h_min[K], hl));
+      out(d.P2, K, pp);
+      out(d.H3, K, h3);
+      out(d.THETA2, K, th2);
+      if (T.scan && r == 0) {
+        out(d.P2, 0, ptop * ptop / pp);
+        out(d.H3, 0, h3);
       }
+      pwm = pw;
+      pw = pwn;
+      thm = th;
     }
   }
-  __syncthreads();
-  if (FULL && T.live && T.kk == 0) {
-    const size_t q0 = ix3(d, 0, J, I);
-    d.P2[q0] = a[0] * a[0] / aux[2];
-    d.H3[q0] = aux[1];
-    if (update_theta) d.THETA2[ix3(d, ks - 1, J, I)] = .5 * (d.THETA[ix3(d, ks - 1, J, I)] + aux[0]);
-  }
-  // FULL = 0: store_pgrad_vars' per-cell part (T3, RHO3) on the column's
-  // levels from the P3 in LDS.  FULL = 1 leaves its larger per-cell part to
-  // k_thermo, whose one lane per cell hides the latency of its pow chains
-  // better than the tile's few lanes per column.
-  if (!FULL && T.live)
-    for (int K = T.kk; K <= nk; K += T.KS) thermo_cell<F>(d, K, J, I, false, d.THETA[ix3(d, K, J, I)], a[K]);
+}
+template <int FULL, bool F>
+static void set_p2etc_t(hipStream_t s, const Bucket &b) {
+  const ColShape sh = col_shape(b, b.knob[KN_COLS_P2ETC]);
+#define K_(KC, U) k_set_p2etc<FULL, F, KC, U>
+  COLS_LAUNCH(FULL ? "k_set_p2etc<1>" : "k_set_p2etc<0>", K_, sh, tile_grid(b, sh.C), dim3(sh.nt),
+              sizeof(double) * sh.C * (b.nk + 1), s, b.D, b.mb, sh.C);
+#undef K_
 }
 void L_set_p2etc(hipStream_t s, const Bucket &b, int update_theta) {
-  const int v = b.knob[KN_COLS_P2ETC], C = v ? knob_cols(v) : tile_cols(b, 2), nt = knob_threads(v, b.nk + 1);
-  size_t shm = sizeof(double) * (2 * C * (b.nk + 1) + 4 * C);
-  if (b.mixed) {
-    if (update_theta) LAUNCH_AS("k_set_p2etc<1>", (k_set_p2etc<1, true>), tile_grid(b, C), dim3(nt), shm, s, b.D, b.mb, C);
-    else LAUNCH_AS("k_set_p2etc<0>", (k_set_p2etc<0, true>), tile_grid(b, C), dim3(nt), shm, s, b.D, b.mb, C);
-  } else {
-    if (update_theta) LAUNCH_AS("k_set_p2etc<1>", (k_set_p2etc<1, false>), tile_grid(b, C), dim3(nt), shm, s, b.D, b.mb, C);
-    else LAUNCH_AS("k_set_p2etc<0>", (k_set_p2etc<0, false>), tile_grid(b, C), dim3(nt), shm, s, b.D, b.mb, C);
-  }
+  if (b.mixed) update_theta ? set_p2etc_t<1, true>(s, b) : set_p2etc_t<0, true>(s, b);
+  else update_theta ? set_p2etc_t<1, false>(s, b) : set_p2etc_t<0, false>(s, b);
 }
 
 // ------------------------------------------------- store_pgrad_vars parts
@@ -253,63 +321,17 @@ __device__ __forceinline__ double hj_relax(const MemberDesc &d, int J, int I, do
 // nothing changes between here and the end of the step, where the reference
 // forms it, and it takes the p^kappa formed here for T3 (a pad takes the
 // value of the column it copies)
-// T3 and RHO3 of an interface cell from its theta and p (return_temp and
-// return_density with x_h2 = 0); pk = (p/press0)^kappa
-template <bool F = false>
-__device__ __forceinline__ double t3_of(const MemberDesc &d, double th, double p, double *pk) {
-  *pk = m_pow<F>(p / d.press0, d.kappa);
-  return th * *pk;
-}
-__device__ __forceinline__ double rho3_of(const MemberDesc &d, double p, double t) {
-  const double R_GAS = 8.314472e+3;
-  return p * d.mu3 / (R_GAS * t);
-}
+// store_pgrad_vars' per-cell part with full = 1 (after the FULL set_p2etc), one
+// lane per (K,J,I), K = 1..nk, J = 0..nj, I = 0..ni+1: the operands loaded
+// together (a load behind a store waits for it: the fields may overlap for all
+// the compiler knows) and the cell's two powers formed side by side.  The lane
+// of level 1 has level 0 too, whose RHO2 it needs.  966 us at 1024x512x64 FP64
+// before, 816 now; two or four levels a lane are no faster.
 template <bool F>
-__device__ __forceinline__ void thermo_cell(const MemberDesc &d, int K, int J, int I, bool full, double th, double p) {
-  const size_t q = ix3(d, K, J, I);
-  if (full && K >= 1 && d.dyn->itime > 1 && I >= 1 && I <= d.ni) d.DZDT3[q] = d.GZ3[q];
-  const double R_GAS = 8.314472e+3;
-  double pk;
-  double t = t3_of<F>(d, th, p, &pk);
-  double rho3 = rho3_of(d, p, t);
-  d.T3[q] = t;
-  d.RHO3[q] = rho3;
-  if (!full) return;
-  if (K >= 1 && newt_relax_on(d)) {
-    double h;
-    if (d.is_tab) {
-      h = 0. + tab_relax(d, p, t);
-    } else if (d.is_hj) {
-      h = hj_relax<F>(d, J, (I == 0) ? d.ni : (I == d.ni + 1 ? 1 : I), p, t, pk);
-    } else {
-      const double pk0 = (d.press0 == 1000. * 100.) ? pk : m_pow<F>(p / (1000. * 100.), d.kappa);
-      h = 0. + hs_relax<F>(d, J, p, t, d.P3[ix3(d, d.nk, J, I)], pk0);
-    }
-    d.HEAT3[q] = h;
-  }
-  d.EXNER3[q] = d.cp * t / th;
-  if (K >= 1) {
-    double p2 = d.P2[q], th2 = d.THETA2[q];
-    double t2 = th2 * m_pow<F>(p2 / d.press0, d.kappa);
-    d.T2[q] = t2;
-    d.RHO2[q] = p2 * d.mu2 / (R_GAS * t2);
-  } else {
-    const size_t q1 = ix3(d, 1, J, I);
-    double p21 = d.P2[q1], th21 = d.THETA2[q1];
-    double t21 = th21 * m_pow<F>(p21 / d.press0, d.kappa);
-    double rho21 = p21 * d.mu2 / (R_GAS * t21);
-    d.RHO2[q] = rho3 * rho3 / rho21;
-    d.THETA2[q] = d.sgth[0];
-    d.T2[q] = t;
-  }
-}
-
-// store_pgrad_vars' per-cell part with full = 1, one lane per (K,J,I),
-// K = 0..nk, J = 0..nj, I = 0..ni+1 (after the FULL set_p2etc)
-template <bool F>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_thermo(const MemberDesc *D, int mb) {
+__global__ void __launch_bounds__(256) k_thermo(const MemberDesc *D, int mb) {
   MEMBER;
-  if (d.dyn->itime <= 1) {
+  const long itime = d.dyn->itime;
+  if (itime <= 1) {
     // no lane of this kernel writes DZDT3 while itime <= 1
     const size_t nthr = (size_t)gridDim.x * gridDim.y * blockDim.x;
     for (size_t i = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x; i < (size_t)d.N3;
@@ -317,13 +339,50 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
       d.DZDT3[i] = 0.;
   }
   FLAT2(0, d.nj + 1, 0, d.ni + 2);
-  const int K = blockIdx.y;
-  const size_t q = ix3(d, K, J, I);
-  thermo_cell<F>(d, K, J, I, true, d.THETA[q], d.P3[q]);
+  const int K = 1 + (int)blockIdx.y;
+  const uint32_t i = ix2(d, J, I);
+  auto in = [&](const double *f, int K) { return Plane<const double>{f + (size_t)K * d.N2}[i]; };
+  auto out = [&](double *f, int K, double x) { Plane<double>{f + (size_t)K * d.N2}[i] = x; };
+  const double R_GAS = 8.314472e+3;
+  const bool rate = itime > 1 && I >= 1 && I <= d.ni;  // DZDT3 <- GZ3
+  const double p = in(d.P3, K), th = in(d.THETA, K), p2 = in(d.P2, K), th2 = in(d.THETA2, K), gz = in(d.GZ3, K);
+  double pk, pk2;
+  m_pow2<F>(p / d.press0, d.kappa, p2 / d.press0, d.kappa, &pk, &pk2);
+  const double t = t3_of(th, pk), t2 = t3_of(th2, pk2), rho2 = p2 * d.mu2 / (R_GAS * t2);
+  const double ex = d.cp * t / th, rho3 = rho3_of(d, p, t);
+  if (newt_relax_on(d)) {
+    double h;
+    if (d.is_tab) {
+      h = 0. + tab_relax(d, p, t);
+    } else if (d.is_hj) {
+      h = hj_relax<F>(d, J, (I == 0) ? d.ni : (I == d.ni + 1 ? 1 : I), p, t, pk);
+    } else {
+      const double pk0 = (d.press0 == 1000. * 100.) ? pk : m_pow<F>(p / (1000. * 100.), d.kappa);
+      h = 0. + hs_relax<F>(d, J, p, t, in(d.P3, d.nk), pk0);
+    }
+    out(d.HEAT3, K, h);
+  }
+  if (rate) out(d.DZDT3, K, gz);
+  out(d.T3, K, t);
+  out(d.RHO3, K, rho3);
+  out(d.EXNER3, K, ex);
+  out(d.T2, K, t2);
+  out(d.RHO2, K, rho2);
+  if (K == 1) {
+    const double p0 = in(d.P3, 0), th0 = in(d.THETA, 0), t0 = t3_of(th0, m_pow<F>(p0 / d.press0, d.kappa));
+    const double rho0 = rho3_of(d, p0, t0);
+    out(d.T3, 0, t0);
+    out(d.RHO3, 0, rho0);
+    out(d.EXNER3, 0, d.cp * t0 / th0);
+    out(d.RHO2, 0, rho0 * rho0 / rho2);
+    out(d.THETA2, 0, d.sgth[0]);
+    out(d.T2, 0, t0);
+  }
 }
 void L_thermo(hipStream_t s, const Bucket &b) {
-  if (b.mixed) LAUNCH_AS("k_thermo", k_thermo<true>, grid2(b.nj + 1, b.ni + 2, b.nk + 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
-  else LAUNCH_AS("k_thermo", k_thermo<false>, grid2(b.nj + 1, b.ni + 2, b.nk + 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
+  const dim3 g = grid2(b.nj + 1, b.ni + 2, b.nk, b.nm);
+  if (b.mixed) LAUNCH_AS("k_thermo", k_thermo<true>, g, dim3(TPB), 0, s, b.D, b.mb);
+  else LAUNCH_AS("k_thermo", k_thermo<false>, g, dim3(TPB), 0, s, b.D, b.mb);
 }
 
 // ------------------------------------------------------------ RI2
@@ -414,10 +473,9 @@ __global__ void __launch_bounds__(256) k_gzu_means(const MemberDesc *D, int mb) 
   for (int i = threadIdx.x; i < ni; i += blockDim.x) {
     const size_t q = ix3(d, nk, J, i + 1);
     const double p = d.P3[q];
-    double pk;
     row[i] = d.U[q];
     row[ni + i] = p;
-    row[2 * ni + i] = rho3_of(d, p, t3_of<F>(d, d.THETA[q], p, &pk));
+    row[2 * ni + i] = rho3_of(d, p, t3_of(d.THETA[q], m_pow<F>(p / d.press0, d.kappa)));
   }
   __syncthreads();
   if (threadIdx.x < 3) d.rowbuf[threadIdx.x * R + J] = seq_acc(row + threadIdx.x * ni, ni) / ni;
@@ -534,103 +592,121 @@ void L_gz_from_u(hipStream_t s, const Bucket &b) {
 
 // hydrostatic GZ3 and MONT3 from the bottom up (Leslie-Purser 4-point
 // integral in ln p) and the monotonicity screen
-template <bool F>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) k_gz3(const MemberDesc *D, int mb, int C) {
+// FP64, 1024x512x64: 650 us before, 415 now; 256x128x20: 20 and 15.
+template <bool F, int KC, bool U>
+__global__ void __launch_bounds__(1024) k_gz3(const MemberDesc *D, int mb, int C) {
   MEMBER;
   extern __shared__ double lds[];
-  const Tile T = tile_of(d, C);
-  const int nk = d.nk, W = nk + 1, J = T.J, I = T.I;
-  double *inc = lds + T.c * W, *tt = lds + C * W + T.c * W, *lg = lds + 2 * C * W + T.c * W;
-  const double *P = d.P3, *RH = d.RHO3;
-#define PP(k) P[ix3(d, k, J, I)]
-#define RR(k) RH[ix3(d, k, J, I)]
+  const Tile<U> T(d, C, KC);
+  const int nk = d.nk, J = T.J, I = T.I, K0 = T.K0;
+  double *L = lds + T.c;  // [K C]: the increment of layer K, then GZ3
   // the column's surface geopotential, read ahead by the lane that runs the
   // chain; on a gas giant gz_from_u's results for this column: GZ_SURFACE,
   // and plane nk+1 of PV3 (the absolute vorticity of the uniform rows; row
   // nj+1 by the columns of row nj)
   double gs = 0.;
-  if (T.live && T.kk == 0) {
+  if (T.live && T.scan) {
     if (d.is_gas) {
       const int R = d.nj + 3;
       gs = d.rowbuf[4 * R + J];
-      d.GZS[ix2(d, J, I)] = gs;
+      d.GZS[T.i] = gs;
       double *pv = d.PV3 + (size_t)(d.nk + 1) * d.N2;
-      pv[ix2(d, J, I)] = d.rowbuf[3 * R + J];
+      pv[T.i] = d.rowbuf[3 * R + J];
       if (J == d.nj) pv[ix2(d, J + 1, I)] = d.rowbuf[3 * R + J + 1];
     } else {
-      gs = d.GZS[ix2(d, J, I)];
+      gs = d.GZS[T.i];
     }
   }
-  // lg[k] = log(P3(k)/P3(k-1)): every ln-p interval the integral uses, once
-  if (T.live)
-    for (int K = T.kk; K <= nk; K += T.KS) {
-      tt[K] = d.T3[ix3(d, K, J, I)];
-      if (K >= 1) lg[K] = m_log<F>(PP(K) / PP(K - 1));
+  // P3 and RHO3 on K0-2 .. K0+KC
+  double p[KC + 3], rho[KC + 3];
+#pragma unroll
+  for (int r = 0; r < KC + 3; r++) {
+    const int K = min(max(K0 - 2 + r, 0), nk);
+    p[r] = T.at(d, d.P3, K)[T.i];
+    rho[r] = T.at(d, d.RHO3, K)[T.i];
+  }
+  // log(P3(K)/P3(K-1)) and P3/RHO3, each once per level of the chunk
+  double lg[KC + 2], df[KC + 3];
+  m_log2<F>(p[1] / p[0], p[2] / p[1], &lg[0], &lg[1]);
+#pragma unroll
+  for (int r = 0; r < 3; r++) df[r] = p[r] / rho[r];
+#pragma unroll
+  for (int r = 0; r < KC; r++) {
+    const int K = K0 + r;
+    if (r % 2 == 0) m_log2<F>(p[r + 3] / p[r + 2], p[min(r + 4, KC + 2)] / p[r + 3], &lg[r + 2], &lg[min(r + 3, KC + 1)]);
+    df[r + 3] = p[r + 3] / rho[r + 3];
+    double v;
+    if (K >= nk || K == 1) {
+      v = ((p[r + 2] + p[r + 1]) / (rho[r + 2] + rho[r + 1])) * lg[r + 1];
+    } else {
+      const double dz10 = lg[r + 2], dz21 = lg[r + 1], dz32 = lg[r];
+      const double dz20 = dz21 + dz10, dz30 = dz32 + dz20, dz31 = dz32 + dz21;
+      const double df0 = df[r + 3], df1 = df[r + 2], df2 = df[r + 1], df3 = df[r];
+      v = -(df0 * (dz21 * dz21 * dz21 * (dz31 + dz32)) / (dz10 * dz20 * dz30) +
+            df1 * (dz21 * (dz21 * (dz21 + 2. * (dz10 - dz31)) - 6. * dz10 * dz31)) / (dz10 * dz31) +
+            df2 * (dz21 * (dz21 * (dz21 + 2. * (dz32 - dz20)) - 6. * dz20 * dz32)) / (dz20 * dz32) +
+            df3 * (dz21 * dz21 * dz21 * (dz10 + dz20)) / (dz30 * dz31 * dz32)) /
+          12.;
     }
+    if (K <= nk) L[K * C] = v;
+  }
+  double t[KC];
+#pragma unroll
+  for (int r = 0; r < KC; r++) t[r] = T.at(d, d.T3, min(K0 + r, nk))[T.i];
   __syncthreads();
-  if (T.live)
-    for (int K = 1 + T.kk; K <= nk; K += T.KS) {
-      double v;
-      if (K == nk || K == 1) {
-        v = ((PP(K) + PP(K - 1)) / (RR(K) + RR(K - 1))) * lg[K];
-      } else {
-        double dz10 = lg[K + 1], dz21 = lg[K], dz32 = lg[K - 1];
-        double dz20 = dz21 + dz10, dz30 = dz32 + dz20, dz31 = dz32 + dz21;
-        double df0 = PP(K + 1) / RR(K + 1), df1 = PP(K) / RR(K), df2 = PP(K - 1) / RR(K - 1),
-               df3 = PP(K - 2) / RR(K - 2);
-        v = -(df0 * (dz21 * dz21 * dz21 * (dz31 + dz32)) / (dz10 * dz20 * dz30) +
-              df1 * (dz21 * (dz21 * (dz21 + 2. * (dz10 - dz31)) - 6. * dz10 * dz31)) / (dz10 * dz31) +
-              df2 * (dz21 * (dz21 * (dz21 + 2. * (dz32 - dz20)) - 6. * dz20 * dz32)) / (dz20 * dz32) +
-              df3 * (dz21 * dz21 * dz21 * (dz10 + dz20)) / (dz30 * dz31 * dz32)) /
-            12.;
-      }
-      inc[K] = v;
-    }
-#undef PP
-#undef RR
-  __syncthreads();
-  if (T.live && T.kk == 0) {
-    const double cpr = d.cpr, rgas = d.rgas;
-    double *G = d.GZ3, *M = d.MONT3;
-    double gprev = d.topo_scale * gs;
-    G[ix3(d, nk, J, I)] = gprev;
-    M[ix3(d, nk, J, I)] = gprev + cpr * tt[nk] * rgas;
-    const bool inner = (I >= 1 && I <= d.ni);
+  if (T.scan) {
+    double gp = d.topo_scale * gs;
+    const bool inner = T.live && (I >= 1 && I <= d.ni);
     int bad = 0;
-    // the increments and temperatures are read eight levels at a time ahead
-    // of the chain
+    // the increments are read eight levels at a time ahead of the chain
     int K = nk;
     for (; K - 7 >= 1; K -= 8) {
-      double i8[8], t8[8];
+      double i8[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) i8[u] = L[(K - u) * C];
 #pragma unroll
       for (int u = 0; u < 8; u++) {
-        i8[u] = inc[K - u];
-        t8[u] = tt[K - u - 1];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        double gn = gprev + i8[u];
-        G[ix3(d, K - u - 1, J, I)] = gn;
-        M[ix3(d, K - u - 1, J, I)] = gn + cpr * t8[u] * rgas;
-        if (inner && gprev >= gn) bad = 1;
-        gprev = gn;
+        const double gn = gp + i8[u];
+        L[(K - u) * C] = gp;
+        if (inner && gp >= gn) bad = 1;
+        gp = gn;
       }
     }
     for (; K >= 1; K--) {
-      double gn = gprev + inc[K];
-      G[ix3(d, K - 1, J, I)] = gn;
-      M[ix3(d, K - 1, J, I)] = gn + cpr * tt[K - 1] * rgas;
-      if (inner && gprev >= gn) bad = 1;
-      gprev = gn;
+      const double gn = gp + L[K * C];
+      L[K * C] = gp;
+      if (inner && gp >= gn) bad = 1;
+      gp = gn;
     }
+    L[0] = gp;
     if (bad) atomicOr(&d.dyn->err, 1);
   }
+  __syncthreads();
+  if (!T.live) return;
+  const double cpr = d.cpr, rgas = d.rgas;
+  auto out = [&](int K, double tk) {
+    const double gz = L[K * C];
+    Plane<double>{d.GZ3 + (size_t)K * d.N2}[T.i] = gz;
+    Plane<double>{d.MONT3 + (size_t)K * d.N2}[T.i] = gz + cpr * tk * rgas;
+  };
+  if (T.scan) out(0, T.at(d, d.T3, 0)[T.i]);
+#pragma unroll
+  for (int r = 0; r < KC; r++) {
+    const int K = K0 + r;
+    if (K > nk) break;
+    out(K, t[r]);
+  }
+}
+template <bool F>
+static void gz3_t(hipStream_t s, const Bucket &b) {
+  const ColShape sh = col_shape(b, b.knob[KN_COLS_GZ3]);
+#define K_(KC, U) k_gz3<F, KC, U>
+  COLS_LAUNCH("k_gz3", K_, sh, tile_grid(b, sh.C), dim3(sh.nt), sizeof(double) * sh.C * (b.nk + 1), s, b.D, b.mb, sh.C);
+#undef K_
 }
 void L_gz3(hipStream_t s, const Bucket &b) {
-  const int v = b.knob[KN_COLS_GZ3], C = v ? knob_cols(v) : tile_cols(b, 3);
-  const size_t shm = sizeof(double) * 3 * C * (b.nk + 1);
-  if (b.mixed) LAUNCH_AS("k_gz3", k_gz3<true>, tile_grid(b, C), dim3(knob_threads(v, b.nk + 1)), shm, s, b.D, b.mb, C);
-  else LAUNCH_AS("k_gz3", k_gz3<false>, tile_grid(b, C), dim3(knob_threads(v, b.nk + 1)), shm, s, b.D, b.mb, C);
+  if (b.mixed) gz3_t<true>(s, b);
+  else gz3_t<false>(s, b);
 }
 
 // finish DZDT3 (diagnostic vertical velocity)
@@ -768,7 +844,7 @@ __global__ void __launch_bounds__(256) k_heat_adjust_apply(const MemberDesc *D, 
   const size_t q = ix3(d, K, J, I);
   d.HEAT3[q] = 0. + (d.HEAT3[q] - d.sD[K]);
 }
-// in_thermo: the relaxation was formed by this step's thermo_cell (full = 1),
+// in_thermo: the relaxation was formed by this step's k_thermo,
 // and every other cell of HEAT3 is zero (a member's blob is cleared when it
 // is created, a drop-in upload brings the caller's array, which the
 // reference zeroes there, and no kernel writes outside K = 1..nk, J = 0..nj),
@@ -797,7 +873,8 @@ void L_heating(hipStream_t s, const Bucket &b, int adjust, bool in_thermo) {
 // launch reads them): planes 0, nk and nk+1 and, of the planes between, rows
 // -1, 0 and nj+1.  k_uv_core forms the rest (row 0 of u again) and k_filter3
 // writes the pads of the rows it passes.
-template <bool F>
+// FP64, 1024x512x64: 1065 us before, 774 now; 256x128x20: 35 both.
+template <bool F, int KC, bool U>
 __global__ void __launch_bounds__(1024) k_calc_w(const MemberDesc *D, int mb, int with_source, int C, int ncb) {
   MEMBER;
   if ((int)blockIdx.x >= ncb) {
@@ -819,107 +896,127 @@ __global__ void __launch_bounds__(1024) k_calc_w(const MemberDesc *D, int mb, in
     return;  // a whole block: no barrier below waits for it
   }
   extern __shared__ double lds[];
-  const Tile T = tile_of(d, C);
-  const int nk = d.nk, ks = d.ks, W = nk + 1, J = T.J, I = T.I;
-  double *dsv = lds + T.c * W, *dfv = lds + C * W + T.c * W, *wbv = lds + 2 * C * W + T.c * W;
-  double *lg = lds + 3 * C * W + T.c * W, *lrv = lds + 4 * C * W + T.c;
-  const double *P = d.P3;
-  double *TH = d.THETA;
+  const Tile<U> T(d, C, KC);
+  const int nk = d.nk, ks = d.ks, K0 = T.K0;
+  double *L = lds + T.c;  // [K C]: the increment of SUM_DIV, then SUM_DIV
   int bad = 0;
-#define PP(k) P[ix3(d, k, J, I)]
-#define DV(k) d.DIV[ix3(d, k, J, I)]
-  // lg[k] = log(P3(k)/P3(k-1)), the ln-p intervals of the Leslie-Purser weights
-  // and log(ptop/pbot) once per column
-  if (T.live) {
-    for (int K = 1 + T.kk; K <= nk; K += T.KS) lg[K] = m_log<F>(PP(K) / PP(K - 1));
-    if (T.kk == 0) lrv[0] = m_log<F>(PP(0) / PP(nk));
-  }
-  __syncthreads();
-  if (T.live) {
-    const double ptop = P[ix3(d, 0, J, I)], pbot = P[ix3(d, nk, J, I)], psig = P[ix3(d, ks - 1, J, I)];
-    const double eps = d.eps13, lr = lrv[0];
-    for (int K = 1 + T.kk; K <= nk; K += T.KS) {
-      const size_t q = ix3(d, K, J, I);
-      double th = TH[q];
-      if (with_source && K >= ks - 1) {
-        th += d.dt * d.HEAT3[q] / d.EXNER3[q];
-        TH[q] = th;
-      }
-      if (K == nk) continue;
-      double wb = 0.;
-      if (K < ks - 1) {
-        double sigma = get_sigma_l<F>(pbot, P[q], lr);
-        wb = g_sig<F>(d, sigma) * d.HEAT3[q] / d.EXNER3[q];
-      }
+  const double ptop = T.at(d, d.P3, 0)[T.i], pbot = T.at(d, d.P3, nk)[T.i], psig = T.at(d, d.P3, ks - 1)[T.i];
+  // SUM_DIV's increments: P3 and the divergence on K0-2 .. K0+KC, their
+  // product and log(P3(K)/P3(K-1)), the ln-p interval of the Leslie-Purser
+  // weights, once per level of the chunk
+  double p3[KC];
+  {
+    double p[KC + 3], f[KC + 3], lg[KC + 2];
+#pragma unroll
+    for (int r = 0; r < KC + 3; r++) {
+      const int K = min(max(K0 - 2 + r, 0), nk);
+      p[r] = T.at(d, d.P3, K)[T.i];
+      f[r] = T.at(d, d.DIV, K)[T.i];
+    }
+#pragma unroll
+    for (int r = 0; r < KC; r++) p3[r] = p[r + 2];
+#pragma unroll
+    for (int r = 0; r < KC + 3; r++) f[r] = p[r] * f[r];
+    m_log2<F>(p[1] / p[0], p[2] / p[1], &lg[0], &lg[1]);
+#pragma unroll
+    for (int r = 0; r < KC; r++) {
+      const int K = K0 + r;
+      if (r % 2 == 0) m_log2<F>(p[r + 3] / p[r + 2], p[min(r + 4, KC + 2)] / p[r + 3], &lg[r + 2], &lg[min(r + 3, KC + 1)]);
       double ds = 0.;
       if (K >= 2) {
-        double dz10 = lg[K - 1], dz21 = lg[K], dz32 = lg[K + 1];
-        double dz20 = dz21 + dz10, dz30 = dz32 + dz20, dz31 = dz32 + dz21;
-        double df0 = PP(K - 2) * DV(K - 2), df1 = PP(K - 1) * DV(K - 1), df2 = PP(K) * DV(K),
-               df3 = PP(K + 1) * DV(K + 1);
+        const double dz10 = lg[r], dz21 = lg[r + 1], dz32 = lg[r + 2];
+        const double dz20 = dz21 + dz10, dz30 = dz32 + dz20, dz31 = dz32 + dz21;
+        const double df0 = f[r], df1 = f[r + 1], df2 = f[r + 2], df3 = f[r + 3];
         ds = -(df0 * (dz21 * dz21 * dz21 * (dz31 + dz32)) / (dz10 * dz20 * dz30) +
                df1 * (dz21 * (dz21 * (dz21 + 2. * (dz10 - dz31)) - 6. * dz10 * dz31)) / (dz10 * dz31) +
                df2 * (dz21 * (dz21 * (dz21 + 2. * (dz32 - dz20)) - 6. * dz20 * dz32)) / (dz20 * dz32) +
                df3 * (dz21 * dz21 * dz21 * (dz10 + dz20)) / (dz30 * dz31 * dz32)) /
              12.;
       }
-      double p3 = P[q], pb3 = pbot;
-      double dp = p3 * eps;
-      double p2 = dmax(p3 - dp * .5, ptop), p4 = dmin(p3 + dp * .5, pbot);
-      if (p2 < psig && p4 >= psig) p2 = p3;
-      double dFdp = 0.;
-      if (p2 < p4)
-        dFdp = (sgth_of_l<F>(d, th, p2, pb3, ptop, lr, &bad) - sgth_of_l<F>(d, th, p4, pb3, ptop, lr, &bad)) / (p2 - p4);
-      else
-        bad = 1;
-      dsv[K] = ds;
-      dfv[K] = dFdp;
-      wbv[K] = wb;
+      if (K < nk) L[K * C] = ds;
     }
   }
-#undef PP
-#undef DV
   __syncthreads();
-  if (T.live && T.kk == 0) {
-    double *Wf = d.W3;
-    Wf[ix3(d, 0, J, I)] = 0.;
-    Wf[ix3(d, nk, J, I)] = 0.;
-    // (the three columns read eight levels at a time ahead of the chain)
+  if (T.scan) {
+    // (read eight levels at a time ahead of the chain)
     double S = 0.;
-    int K = 1;
+    int K = 2;
     for (; K + 7 < nk; K += 8) {
-      double s8[8], w8[8], f8[8];
+      double s8[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) s8[u] = L[(K + u) * C];
 #pragma unroll
       for (int u = 0; u < 8; u++) {
-        s8[u] = dsv[K + u];
-        w8[u] = wbv[K + u];
-        f8[u] = dfv[K + u];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        if (K + u >= 2) S = S + s8[u];
-        Wf[ix3(d, K + u, J, I)] = w8[u] - S * f8[u];
+        S = S + s8[u];
+        L[(K + u) * C] = S;
       }
     }
     for (; K < nk; K++) {
-      if (K >= 2) S = S + dsv[K];
-      Wf[ix3(d, K, J, I)] = wbv[K] - S * dfv[K];
+      S = S + L[K * C];
+      L[K * C] = S;
+    }
+  }
+  __syncthreads();
+  // theta with its heating, the heating's part of W3 and dF/dp
+  const double eps = d.eps13, lr = m_log<F>(ptop / pbot);
+  auto out = [&](double *f, int K, double x) {
+    if (T.live) Plane<double>{f + (size_t)K * d.N2}[T.i] = x;
+  };
+  if (T.scan) out(d.W3, 0, 0.);
+  constexpr int KB = 2;  // levels loaded together
+#pragma unroll
+  for (int rb = 0; rb < KC; rb += KB) {
+    double th[KB], heat[KB], ex[KB];
+#pragma unroll
+    for (int r = 0; r < KB; r++) {
+      const int K = min(K0 + rb + r, nk);
+      th[r] = T.at(d, d.THETA, K)[T.i];
+      heat[r] = T.at(d, d.HEAT3, K)[T.i];
+      ex[r] = T.at(d, d.EXNER3, K)[T.i];
+    }
+#pragma unroll
+    for (int r = 0; r < KB; r++) {
+      const int K = K0 + rb + r;
+      if (K > nk) break;
+      const double pc = p3[rb + r];
+      if (with_source && K >= ks - 1) {
+        th[r] += d.dt * heat[r] / ex[r];
+        out(d.THETA, K, th[r]);
+      }
+      if (K == nk) {
+        out(d.W3, nk, 0.);
+        break;
+      }
+      double wb = 0.;
+      if (K < ks - 1) wb = g_sig<F>(d, get_sigma_l<F>(pbot, pc, lr)) * heat[r] / ex[r];
+      const double dp = pc * eps;
+      double p2 = dmax(pc - dp * .5, ptop), dF = 0.;
+      const double p4 = dmin(pc + dp * .5, pbot);
+      if (p2 < psig && p4 >= psig) p2 = pc;
+      if (p2 < p4) dF = sgth_diff_l<F>(d, th[r], p2, p4, pbot, ptop, lr, &bad) / (p2 - p4);
+      else bad = 1;
+      out(d.W3, K, wb - L[K * C] * dF);  // (SUM_DIV(1) is 0, as its L was left)
     }
   }
   if (bad) atomicOr(&d.dyn->err, 2);
 }
-void L_calc_w(hipStream_t s, const Bucket &b, int with_source) {
-  const int v = b.knob[KN_COLS_CALCW], C = v ? knob_cols(v) : tile_cols(b, 4), nt = knob_threads(v, b.nk + 1);
-  dim3 g = tile_grid(b, C);
+template <bool F>
+static void calc_w_t(hipStream_t s, const Bucket &b, int with_source) {
+  const ColShape sh = col_shape(b, b.knob[KN_COLS_CALCW]);
+  dim3 g = tile_grid(b, sh.C);
   const int ncb = (int)g.x;
   if (with_source) {
     // blocks that clear the tendencies' edges: about 4 cells per lane
     const size_t n = (size_t)(b.ni + 2) * (3 * (b.nj + 3) + 3 * (b.nk - 1));
-    g.x += (unsigned)std::max<size_t>(1, std::min<size_t>(1024, n / ((size_t)nt * 4)));
+    g.x += (unsigned)std::max<size_t>(1, std::min<size_t>(1024, n / ((size_t)sh.nt * 4)));
   }
-  const size_t shm = sizeof(double) * (4 * C * (b.nk + 1) + C);
-  if (b.mixed) LAUNCH_AS("k_calc_w", k_calc_w<true>, g, dim3(nt), shm, s, b.D, b.mb, with_source, C, ncb);
-  else LAUNCH_AS("k_calc_w", k_calc_w<false>, g, dim3(nt), shm, s, b.D, b.mb, with_source, C, ncb);
+#define K_(KC, U) k_calc_w<F, KC, U>
+  COLS_LAUNCH("k_calc_w", K_, sh, g, dim3(sh.nt), sizeof(double) * sh.C * (b.nk + 1), s, b.D, b.mb, with_source, sh.C, ncb);
+#undef K_
+}
+void L_calc_w(hipStream_t s, const Bucket &b, int with_source) {
+  if (b.mixed) calc_w_t<true>(s, b, with_source);
+  else calc_w_t<false>(s, b, with_source);
 }
 
 // ------------------------------------------------ vorticity / divergence
