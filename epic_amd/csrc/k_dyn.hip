@@ -329,45 +329,28 @@ __global__ void __launch_bounds__(256) k_gz_polefill(const MemberDesc *D, int mb
   for (int I = threadIdx.x; I <= ni + 1; I += blockDim.x) d.GZ3[ix3(d, K, Jd, I)] = v;
 }
 
-// finite-volume pressure-gradient force.  Longitudinal: the east face of
-// cell I-1 is this cell's west face.  Latitudinal: the north face of row
-// J-1 is this row's south face.
-__device__ __forceinline__ double face_lon(const MemberDesc &d, int K, int J, int I, double &zbse, double &zbne,
-                                           double &ztse, double &ztne, double &zbe, double &zte, double &pbe,
-                                           double &pte) {
-  const double *G = d.GZ3, *P2 = d.P2;
-#define Z(k, j, i) G[ix3(d, k, j, i)]
-  zbse = .25 * (Z(K, J, I) + Z(K, J - 1, I) + Z(K + 1, J, I) + Z(K + 1, J - 1, I));
-  zbne = .25 * (Z(K, J, I) + Z(K, J + 1, I) + Z(K + 1, J, I) + Z(K + 1, J + 1, I));
-  ztse = .25 * (Z(K, J, I) + Z(K, J - 1, I) + Z(K - 1, J, I) + Z(K - 1, J - 1, I));
-  ztne = .25 * (Z(K, J, I) + Z(K, J + 1, I) + Z(K - 1, J, I) + Z(K - 1, J + 1, I));
-  zbe = .5 * (Z(K, J, I) + Z(K + 1, J, I));
-  zte = .5 * (Z(K, J, I) + Z(K - 1, J, I));
-#undef Z
-  pbe = P2[ix3(d, K + 1, J, I)];
-  pte = P2[ix3(d, K, J, I)];
-  double a1 = ztne + ztse, b1 = ztne * ztse, a2 = zbne + zbse, b2 = zbne * zbse;
-  double t1 = a1 * a1 - b1 - (a2 * a2 - b2), t2 = 3. * (a1 - a2);
-  return (-t1 * (pbe - pte) + t2 * (zte * pbe - zbe * pte)) / (zte - zbe);
-}
-
-__device__ __forceinline__ double face_lat(const MemberDesc &d, int K, int J, int I, double rlnn, double &zbnw,
-                                           double &zbne, double &ztnw, double &ztne, double &zbn, double &ztn,
-                                           double &pbn, double &ptn) {
-  const double *G = d.GZ3, *P2 = d.P2;
-#define Z(k, j, i) G[ix3(d, k, j, i)]
-  zbnw = .25 * (Z(K, J, I) + Z(K, J, I - 1) + Z(K + 1, J, I) + Z(K + 1, J, I - 1));
-  zbne = .25 * (Z(K, J, I) + Z(K, J, I + 1) + Z(K + 1, J, I) + Z(K + 1, J, I + 1));
-  ztnw = .25 * (Z(K, J, I) + Z(K, J, I - 1) + Z(K - 1, J, I) + Z(K - 1, J, I - 1));
-  ztne = .25 * (Z(K, J, I) + Z(K, J, I + 1) + Z(K - 1, J, I) + Z(K - 1, J, I + 1));
-  zbn = .5 * (Z(K, J, I) + Z(K + 1, J, I));
-  ztn = .5 * (Z(K, J, I) + Z(K - 1, J, I));
-#undef Z
-  pbn = P2[ix3(d, K + 1, J, I)];
-  ptn = P2[ix3(d, K, J, I)];
-  double a1 = ztne + ztnw, b1 = ztne * ztnw, a2 = zbne + zbnw, b2 = zbne * zbnw;
-  double t1 = a1 * a1 - b1 - (a2 * a2 - b2), t2 = 3. * (a1 - a2);
-  return rlnn * (-t1 * (pbn - ptn) + t2 * (ztn * pbn - zbn * ptn)) / (ztn - zbn);
+// finite-volume pressure-gradient force.  A face of cell (K,J,I) from GZ3 on
+// the levels K-1, K, K+1 of its column (C) and of the columns beside it, and P2
+// above (pt) and below (pb): the corner geopotentials bottom/top, first and
+// second side, the edge means b, t, and the force f.
+struct PgFace {
+  double b1, b2, t1, t2, b, t, pb, pt, f;
+};
+__device__ __forceinline__ PgFace pg_face(const double (&A)[3], const double (&C)[3], const double (&B)[3], double pt,
+                                          double pb) {
+  PgFace r;
+  r.b1 = .25 * (C[1] + A[1] + C[2] + A[2]);
+  r.b2 = .25 * (C[1] + B[1] + C[2] + B[2]);
+  r.t1 = .25 * (C[1] + A[1] + C[0] + A[0]);
+  r.t2 = .25 * (C[1] + B[1] + C[0] + B[0]);
+  r.b = .5 * (C[1] + C[2]);
+  r.t = .5 * (C[1] + C[0]);
+  r.pb = pb;
+  r.pt = pt;
+  const double a1 = r.t2 + r.t1, b1 = r.t2 * r.t1, a2 = r.b2 + r.b1, b2 = r.b2 * r.b1;
+  const double x1 = a1 * a1 - b1 - (a2 * a2 - b2), x2 = 3. * (a1 - a2);
+  r.f = (-x1 * (pb - pt) + x2 * (r.t * pb - r.b * pt));
+  return r;
 }
 
 // uv_pgrad_traditional (src/shared/epic_timestep.c:806-884, the reference's
@@ -400,119 +383,133 @@ __device__ __forceinline__ void pgrad_traditional(const MemberDesc &d, int K, in
   }
 }
 
+// One lane per (K,J,I); with SROW (rows of whole wavefronts) a wavefront lies in
+// one row, whose metric terms are then scalar.  GZ3 and P2 are held as columns
+// of three levels, each value loaded once.
+// FP64: 1198 us at 1024x512x64 with the metric terms per lane and the flat
+// indices, 916 now; 256x128x20 27.5 and 20.6.  Marching 2-8 rows a lane with
+// the shared face kept needs 190 VGPRs and is no faster (2 rows slower), nor
+// are 128 VGPRs with spills (1390 us).
+template <bool SROW>
 __global__ void __launch_bounds__(256) k_pgrad(const MemberDesc *D, int mb) {
   MEMBER_X;
-  FLAT2_X(0, d.nj + 1, 1, d.ni);
-  const int K = 1 + bx_.y;
+  const int t0 = bx_.x * TPB + threadIdx.x, Jl = t0 >> d.nlogn, K = 1 + bx_.y;
+  const int J = SROW ? __builtin_amdgcn_readfirstlane(Jl) : Jl, I = 1 + (t0 & (d.ni - 1));
+  if (J > d.nj) return;
   const double TOL = 1.e-2, DG = M_PI / 180.;
-  const double *G = d.GZ3, *P2 = d.P2;
-  double *du = cur_tend(d, d.DUDT), *dv = cur_tend(d, d.DVDT);
   if (d.pgrad_trad) {
-    pgrad_traditional(d, K, J, I, du, dv);
+    pgrad_traditional(d, K, J, I, cur_tend(d, d.DUDT), cur_tend(d, d.DVDT));
     return;
   }
-#define Z(k, j, i) G[ix3(d, k, j, i)]
-#define PZ(k, j, i) P2[ix3(d, k, j, i)]
+  const size_t o = (size_t)K * d.N2;
+  const uint32_t i = ix2(d, J, I), is = i - d.Ia, in = i + d.Ia;
+  const Plane<const double> G[3] = {{d.GZ3 + o - d.N2}, {d.GZ3 + o}, {d.GZ3 + o + d.N2}};
+  const Plane<const double> P[2] = {{d.P2 + o}, {d.P2 + o + d.N2}}, rho3{d.RHO3 + o};
+  const Plane<double> du{cur_tend(d, d.DUDT) + o}, dv{cur_tend(d, d.DVDT) + o};
+  // rows S (J-1), C (J), N (J+1): [column I-1, I, I+1][level K-1, K, K+1]
+  double S[3][3], C[3][3], N[2][3], pc[3][2];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      S[c][k] = G[k].at(is, c - 1);
+      C[c][k] = G[k].at(i, c - 1);
+      if (c < 2) N[c][k] = G[k].at(in, c - 1);
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) pc[c][k] = P[k].at(i, c - 1);
+  }
+  const double rho = rho3.at(i, 0), dln = d.lon[2 * I + 1] * DG - d.lon[2 * (I - 1) + 1] * DG;
   {
     // ---- longitudinal component at u-point (J,I)
-    double rlns = d.rln[2 * J], rlnn = d.rln[2 * J + 2];
-    double zbsw, zbnw, ztsw, ztnw, zbw, ztw, pbw, ptw;
-    double west = face_lon(d, K, J, I - 1, zbsw, zbnw, ztsw, ztnw, zbw, ztw, pbw, ptw);
-    double lnw = d.lon[2 * (I - 1) + 1] * DG;
-    double zbse, zbne, ztse, ztne, zbe, zte, pbe, pte;
-    double east = face_lon(d, K, J, I, zbse, zbne, ztse, ztne, zbe, zte, pbe, pte);
-    double lne = d.lon[2 * I + 1] * DG;
-    double rho = .5 * (d.RHO3[ix3(d, K, J, I)] + d.RHO3[ix3(d, K, J, I - 1)]);
+    const double rlns = d.rln[2 * J], rlnn = d.rln[2 * J + 2];
+    PgFace w = pg_face(S[0], C[0], N[0], pc[0][0], pc[0][1]), e = pg_face(S[1], C[1], N[1], pc[1][0], pc[1][1]);
+    const double west = w.f / (w.t - w.b), east = e.f / (e.t - e.b);
+    const double rm = .5 * (rho + rho3.at(i, -1));
     double top, bottom, a1, a2, b1, b2, t1, t2;
-    a1 = ztne + ztse; a2 = ztnw + ztsw;
+    a1 = e.t2 + e.t1; a2 = w.t2 + w.t1;
     t2 = 3. * (a1 - a2);
-    if (fabs(2. * (zte - ztw) / (zte + ztw - zbe - zbw)) > TOL) {
-      b1 = ztne * ztse; b2 = ztnw * ztsw;
+    if (fabs(2. * (e.t - w.t) / (e.t + w.t - e.b - w.b)) > TOL) {
+      b1 = e.t2 * e.t1; b2 = w.t2 * w.t1;
       t1 = a1 * a1 - b1 - (a2 * a2 - b2);
-      top = (-t1 * (ptw - pte) + t2 * (zte * ptw - ztw * pte)) / (zte - ztw);
+      top = (-t1 * (w.pt - e.pt) + t2 * (e.t * w.pt - w.t * e.pt)) / (e.t - w.t);
     } else {
-      top = .5 * (ptw + pte) * t2;
+      top = .5 * (w.pt + e.pt) * t2;
     }
-    a1 = zbne + zbse; a2 = zbnw + zbsw;
+    a1 = e.b2 + e.b1; a2 = w.b2 + w.b1;
     t2 = 3. * (a1 - a2);
-    if (fabs(2. * (zbe - zbw) / (zte + ztw - zbe - zbw)) > TOL) {
-      b1 = zbne * zbse; b2 = zbnw * zbsw;
+    if (fabs(2. * (e.b - w.b) / (e.t + w.t - e.b - w.b)) > TOL) {
+      b1 = e.b2 * e.b1; b2 = w.b2 * w.b1;
       t1 = a1 * a1 - b1 - (a2 * a2 - b2);
-      bottom = (-t1 * (pbw - pbe) + t2 * (zbe * pbw - zbw * pbe)) / (zbe - zbw);
+      bottom = (-t1 * (w.pb - e.pb) + t2 * (e.b * w.pb - w.b * e.pb)) / (e.b - w.b);
     } else {
-      bottom = .5 * (pbw + pbe) * t2;
+      bottom = .5 * (w.pb + e.pb) * t2;
     }
     double north = 0., south = 0.;
     double pgf = top - bottom + south - north + west - east;
-    double dzn = ztne - zbne + ztnw - zbnw, dzs = ztse - zbse + ztsw - zbsw;
-    pgf /= (lne - lnw) * rho * (rlns * (dzs + .5 * dzn) + rlnn * (dzn + .5 * dzs));
-    du[ix3(d, K, J, I)] += pgf;
+    const double dzn = e.t2 - e.b2 + w.t2 - w.b2, dzs = e.t1 - e.b1 + w.t1 - w.b1;
+    pgf /= dln * rm * (rlns * (dzs + .5 * dzn) + rlnn * (dzn + .5 * dzs));
+    du[i] += pgf;
   }
-  if (J >= 1) {
-    // ---- latitudinal component at v-point (J,I)
-    double rlns = d.rln[2 * J - 1], lts = d.lat[2 * J - 1] * DG;
-    double zbsw, zbse, ztsw, ztse, zbs, zts, pbs, pts;
-    double south = face_lat(d, K, J - 1, I, rlns, zbsw, zbse, ztsw, ztse, zbs, zts, pbs, pts);
-    double rlnn = d.rln[2 * J + 1], ltn = d.lat[2 * J + 1] * DG;
-    double zbnw, zbne, ztnw, ztne, zbn, ztn, pbn, ptn;
-    double north = face_lat(d, K, J, I, rlnn, zbnw, zbne, ztnw, ztne, zbn, ztn, pbn, ptn);
-    double rho = .5 * (d.RHO3[ix3(d, K, J, I)] + d.RHO3[ix3(d, K, J - 1, I)]);
-    double rlt = d.rlt[2 * J];
-    double a1, a2, b1, b2, b3, t1, t2;
-    double zbe = .125 * (Z(K, J, I) + Z(K, J, I + 1) + Z(K, J - 1, I) + Z(K, J - 1, I + 1) + Z(K + 1, J, I) +
-                         Z(K + 1, J, I + 1) + Z(K + 1, J - 1, I) + Z(K + 1, J - 1, I + 1));
-    double zte = .125 * (Z(K - 1, J, I) + Z(K - 1, J, I + 1) + Z(K - 1, J - 1, I) + Z(K - 1, J - 1, I + 1) +
-                         Z(K, J, I) + Z(K, J, I + 1) + Z(K, J - 1, I) + Z(K, J - 1, I + 1));
-    double pbe = .25 * (PZ(K + 1, J, I) + PZ(K + 1, J, I + 1) + PZ(K + 1, J - 1, I) + PZ(K + 1, J - 1, I + 1));
-    double pte = .25 * (PZ(K, J, I) + PZ(K, J, I + 1) + PZ(K, J - 1, I) + PZ(K, J - 1, I + 1));
-    a1 = ztne + ztse; b1 = ztne * ztse; a2 = zbne + zbse; b2 = zbne * zbse;
+  if (J < 1) return;
+  __builtin_amdgcn_sched_barrier(0);  // (the parts one after the other)
+  // ---- latitudinal component at v-point (J,I)
+  double ps[3][2];
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+#pragma unroll
+    for (int k = 0; k < 2; k++) ps[c][k] = P[k].at(is, c - 1);
+  const double rlnn = d.rln[2 * J + 1];
+  PgFace n = pg_face(C[0], C[1], C[2], pc[1][0], pc[1][1]), fs = pg_face(S[0], S[1], S[2], ps[1][0], ps[1][1]);
+  const double rlns = d.rln[2 * J - 1], lts = d.lat[2 * J - 1] * DG, ltn = d.lat[2 * J + 1] * DG;
+  const double rm = .5 * (rho + rho3.at(is, 0)), rlt = d.rlt[2 * J];
+  n.f = rlnn * n.f / (n.t - n.b);
+  fs.f = rlns * fs.f / (fs.t - fs.b);
+  double a1, a2, b1, b2, b3, t1, t2;
+  // east (c = 2) and west (c = 0) edges
+  auto side = [&](int c, double ta, double tb, double ba, double bb) {
+    const double zb = .125 * (C[1][1] + C[c][1] + S[1][1] + S[c][1] + C[1][2] + C[c][2] + S[1][2] + S[c][2]);
+    const double zt = .125 * (C[1][0] + C[c][0] + S[1][0] + S[c][0] + C[1][1] + C[c][1] + S[1][1] + S[c][1]);
+    const double pb = .25 * (pc[1][1] + pc[c][1] + ps[1][1] + ps[c][1]);
+    const double pt = .25 * (pc[1][0] + pc[c][0] + ps[1][0] + ps[c][0]);
+    const double x1 = ta + tb, y1 = ta * tb, x2 = ba + bb, y2 = ba * bb;
+    const double u1 = x1 * x1 - y1 - (x2 * x2 - y2), u2 = 3. * (x1 - x2);
+    return .5 * (rlns - rlnn) * (-u1 * (pb - pt) + u2 * (zt * pb - zb * pt)) / (zt - zb);
+  };
+  const double east = side(2, n.t2, fs.t2, n.b2, fs.b2), west = side(0, n.t1, fs.t1, n.b1, fs.b1);
+  double top, bottom;
+  a1 = n.t2 + n.t1; a2 = fs.t2 + fs.t1;
+  t2 = 3. * (a1 - a2);
+  if (fabs(2. * (n.t - fs.t) / (n.t + fs.t - n.b - fs.b)) > TOL) {
+    b1 = n.t2 * n.t1; b2 = fs.t2 * fs.t1; b3 = n.t2 * fs.t2 + n.t1 * fs.t1;
     t1 = a1 * a1 - b1 - (a2 * a2 - b2);
-    t2 = 3. * (a1 - a2);
-    double east = .5 * (rlns - rlnn) * (-t1 * (pbe - pte) + t2 * (zte * pbe - zbe * pte)) / (zte - zbe);
-    double zbw = .125 * (Z(K, J, I) + Z(K, J, I - 1) + Z(K, J - 1, I) + Z(K, J - 1, I - 1) + Z(K + 1, J, I) +
-                         Z(K + 1, J, I - 1) + Z(K + 1, J - 1, I) + Z(K + 1, J - 1, I - 1));
-    double ztw = .125 * (Z(K - 1, J, I) + Z(K - 1, J, I - 1) + Z(K - 1, J - 1, I) + Z(K - 1, J - 1, I - 1) +
-                         Z(K, J, I) + Z(K, J, I - 1) + Z(K, J - 1, I) + Z(K, J - 1, I - 1));
-    double pbw = .25 * (PZ(K + 1, J, I) + PZ(K + 1, J, I - 1) + PZ(K + 1, J - 1, I) + PZ(K + 1, J - 1, I - 1));
-    double ptw = .25 * (PZ(K, J, I) + PZ(K, J, I - 1) + PZ(K, J - 1, I) + PZ(K, J - 1, I - 1));
-    a1 = ztnw + ztsw; b1 = ztnw * ztsw; a2 = zbnw + zbsw; b2 = zbnw * zbsw;
-    t1 = a1 * a1 - b1 - (a2 * a2 - b2);
-    t2 = 3. * (a1 - a2);
-    double west = .5 * (rlns - rlnn) * (-t1 * (pbw - ptw) + t2 * (ztw * pbw - zbw * ptw)) / (ztw - zbw);
-    double top, bottom;
-    a1 = ztne + ztnw; a2 = ztse + ztsw;
-    t2 = 3. * (a1 - a2);
-    if (fabs(2. * (ztn - zts) / (ztn + zts - zbn - zbs)) > TOL) {
-      b1 = ztne * ztnw; b2 = ztse * ztsw; b3 = ztne * ztse + ztnw * ztsw;
-      t1 = a1 * a1 - b1 - (a2 * a2 - b2);
-      top = .5 * ((ptn - pts) * ((rlnn + rlns) * t1 + (rlnn - rlns) * (b1 + b2 - b3)) +
-                  (rlnn + rlns) * t2 * (ztn * pts - zts * ptn)) / (ztn - zts);
-    } else {
-      top = .25 * (rlnn + rlns) * (pts + ptn) * t2;
-    }
-    a1 = zbne + zbnw; a2 = zbse + zbsw;
-    t2 = 3. * (a1 - a2);
-    if (fabs(2. * (zbn - zbs) / (ztn + zts - zbn - zbs)) > TOL) {
-      b1 = zbne * zbnw; b2 = zbse * zbsw; b3 = zbne * zbse + zbnw * zbsw;
-      t1 = a1 * a1 - b1 - (a2 * a2 - b2);
-      bottom = .5 * ((pbn - pbs) * ((rlnn + rlns) * t1 + (rlnn - rlns) * (b1 + b2 - b3)) +
-                     (rlnn + rlns) * t2 * (zbn * pbs - zbs * pbn)) / (zbn - zbs);
-    } else {
-      bottom = .25 * (rlnn + rlns) * (pbs + pbn) * t2;
-    }
-    double pgf = top - bottom + south - (north + west + east);
-    double dzn = ztne - zbne + ztnw - zbnw, dzs = ztse - zbse + ztsw - zbsw;
-    pgf /= (ltn - lts) * rho * rlt * (rlns * (dzs + .5 * dzn) + rlnn * (dzn + .5 * dzs));
-    dv[ix3(d, K, J, I)] += pgf;
+    top = .5 * ((n.pt - fs.pt) * ((rlnn + rlns) * t1 + (rlnn - rlns) * (b1 + b2 - b3)) +
+                (rlnn + rlns) * t2 * (n.t * fs.pt - fs.t * n.pt)) / (n.t - fs.t);
+  } else {
+    top = .25 * (rlnn + rlns) * (fs.pt + n.pt) * t2;
   }
-#undef Z
-#undef PZ
+  a1 = n.b2 + n.b1; a2 = fs.b2 + fs.b1;
+  t2 = 3. * (a1 - a2);
+  if (fabs(2. * (n.b - fs.b) / (n.t + fs.t - n.b - fs.b)) > TOL) {
+    b1 = n.b2 * n.b1; b2 = fs.b2 * fs.b1; b3 = n.b2 * fs.b2 + n.b1 * fs.b1;
+    t1 = a1 * a1 - b1 - (a2 * a2 - b2);
+    bottom = .5 * ((n.pb - fs.pb) * ((rlnn + rlns) * t1 + (rlnn - rlns) * (b1 + b2 - b3)) +
+                   (rlnn + rlns) * t2 * (n.b * fs.pb - fs.b * n.pb)) / (n.b - fs.b);
+  } else {
+    bottom = .25 * (rlnn + rlns) * (fs.pb + n.pb) * t2;
+  }
+  double pgf = top - bottom + fs.f - (n.f + west + east);
+  const double dzn = n.t2 - n.b2 + n.t1 - n.b1, dzs = fs.t2 - fs.b2 + fs.t1 - fs.b1;
+  pgf /= (ltn - lts) * rm * rlt * (rlns * (dzs + .5 * dzn) + rlnn * (dzn + .5 * dzs));
+  dv[i] += pgf;
 }
 
 void L_pgrad(hipStream_t s, const Bucket &b) {
   LAUNCH(k_gz_polefill, dim3(2 * (b.nk + 1), 1, b.nm), dim3(64), sizeof(double) * (b.ni + 1), s, b.D, b.mb);
   // FP64 in both precision modes (k_mixed.hip says why)
-  LAUNCH(k_pgrad, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
+  const dim3 g = grid2(b.nj + 1, b.ni, b.nk - 1, b.nm);
+  if (b.ni >= 64) LAUNCH_AS("k_pgrad", k_pgrad<true>, g, dim3(TPB), 0, s, b.D, b.mb);
+  else LAUNCH_AS("k_pgrad", k_pgrad<false>, g, dim3(TPB), 0, s, b.D, b.mb);
 }
 
 // ------------------------------------------------------ divergence damping
