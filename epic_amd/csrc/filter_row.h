@@ -50,14 +50,39 @@ template <> __device__ __forceinline__ const float *tw_inv<float>(const MemberDe
 template <> __device__ __forceinline__ const float *tr_fwd<float>(const MemberDesc &d) { return d.tr_f32; }
 template <> __device__ __forceinline__ const float *tr_inv<float>(const MemberDesc &d) { return d.tr_i32; }
 
-// unit `lane` (of n/8) of the stages s and s+1, h = 2^s, on a row in LDS: the
+// Where complex element p of a row lies in the transform's scratch: the low
+// four bits of its place mixed with the next four.  In natural order the
+// bit-reversed stores of 64 lanes fall 16 elements (256 bytes, all 64 banks)
+// apart at ni = 1024 and the points of the first stage pairs 4 or 16: waiting
+// for the same banks was over a third of the row kernels' time.  A permutation
+// of each 16 elements, linear over exclusive or: swz(p ^ q) = swz(p) ^ swz(q).
+// FP64 steps before and after: 256x128x20 429 and 413 us, 23 members of
+// 128x51x13 945 and 920, 1024x512x64 14.39 and 14.26 ms.  (k_hv4's rows are
+// summed in place in natural order and keep it.)
+__device__ __forceinline__ int swz(int p) { return p ^ ((p >> 4) & 15); }
+// the same for value e of the row (element e/2, real or imaginary)
+__device__ __forceinline__ int swz_val(int e) { return 2 * swz(e >> 1) + (e & 1); }
+
+// unit `lane` (of n/8) of the stages s and s+1, h = 2^s, on a row in LDS (SW:
+// its elements at swz): the
 // four points p, p+h, p+2h, p+3h go through stage s as (p, p+h) and
 // (p+2h, p+3h) and through stage s+1 as (p, p+2h) and (p+h, p+3h), in
 // registers
-template <class T>
+template <bool SW = false, class T>
 __device__ __forceinline__ void four1_pair(T *buf, int s, int lane, const T *tw) {
-  const int half = 1 << s, mm = lane & (half - 1), g = lane >> s;
-  const int i0 = 2 * (mm + g * 4 * half), i1 = i0 + 2 * half, i2 = i1 + 2 * half, i3 = i2 + 2 * half;
+  const int half = 1 << s, mm = lane & (half - 1), g = lane >> s, p = mm + g * 4 * half;
+  int i0, i1, i2, i3;
+  if constexpr (SW) {  // p has zeros where half and 2 half have their bit
+    i0 = 2 * swz(p);
+    i1 = i0 ^ (2 * swz(half));
+    i2 = i0 ^ (2 * swz(2 * half));
+    i3 = i0 ^ (2 * swz(3 * half));
+  } else {
+    i0 = 2 * p;
+    i1 = i0 + 2 * half;
+    i2 = i1 + 2 * half;
+    i3 = i2 + 2 * half;
+  }
   T x0r = buf[i0], x0i = buf[i0 + 1], x1r = buf[i1], x1i = buf[i1 + 1];
   T x2r = buf[i2], x2i = buf[i2 + 1], x3r = buf[i3], x3i = buf[i3 + 1];
   const int ka = half - 1 + mm, kb = 2 * half - 1 + mm;
@@ -77,10 +102,10 @@ __device__ __forceinline__ void four1_pair(T *buf, int s, int lane, const T *tw)
   buf[i3 + 1] = x3i;
 }
 // unit `lane` (of n/4) of one stage s: the odd last one
-template <class T>
+template <bool SW = false, class T>
 __device__ __forceinline__ void four1_last(T *buf, int s, int lane, const T *tw) {
-  const int mmax = 2 << s, half = 1 << s, g = lane >> s, mm = lane & (half - 1);
-  const int i0 = 2 * mm + g * 2 * mmax, j0 = i0 + mmax, k = half - 1 + mm;
+  const int half = 1 << s, g = lane >> s, mm = lane & (half - 1), p = mm + g * 2 * half, k = half - 1 + mm;
+  const int i0 = 2 * (SW ? swz(p) : p), j0 = SW ? i0 ^ (2 * swz(half)) : i0 + 2 * half;
   T xr = buf[i0], xi = buf[i0 + 1], yr = buf[j0], yi = buf[j0 + 1];
   bfly(xr, xi, yr, yi, tw[2 * k], tw[2 * k + 1]);
   buf[i0] = xr;
@@ -89,7 +114,7 @@ __device__ __forceinline__ void four1_last(T *buf, int s, int lane, const T *tw)
   buf[j0 + 1] = yi;
 }
 
-// complex radix-2 stages on buf[0..n) (n doubles = n/2 complex), in the
+// complex radix-2 stages on buf[0..n) (n doubles = n/2 complex, at swz), in the
 // reference's stage order.  Stages go two at a time: a lane loads the four
 // points p, p+h, p+2h, p+3h (h = 2^s) into registers, applies stage s to
 // (p, p+h) and (p+2h, p+3h) and stage s+1 to (p, p+2h) and (p+h, p+3h), and
@@ -103,11 +128,11 @@ __device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const T *t
   while ((2 << S) < n) S++;  // stages s with 2 << s < n
   int s = 0;
   for (; s + 1 < S; s += 2) {
-    if (active && lane < (n >> 3)) four1_pair(buf, s, lane, tw);
+    if (active && lane < (n >> 3)) four1_pair<true>(buf, s, lane, tw);
     row_sync<WIDE>();
   }
   if (s < S) {
-    if (active) four1_last(buf, s, lane, tw);
+    if (active) four1_last<true>(buf, s, lane, tw);
     row_sync<WIDE>();
   }
 }
@@ -212,22 +237,23 @@ __device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], 
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int e = lane + q * nq;
-      work[(brev(e >> 1, bits) << 1) | (e & 1)] = v[q];
+      work[2 * swz(brev(e >> 1, bits)) + (e & 1)] = v[q];
     }
   row_sync<WIDE>();
   four1_stages<WIDE>(work, n, lane, tw_fwd<T>(d), active);
   const int ka = unit_k(n, lane), kb = unit_kb(n, lane);
   T ar, ai, br, bi;
   if (active) {
-    ar = work[2 * ka];
-    ai = work[2 * ka + 1];
-    br = work[2 * kb];
-    bi = work[2 * kb + 1];
+    const int pa = 2 * swz(ka), pb = 2 * swz(kb);
+    ar = work[pa];
+    ai = work[pa + 1];
+    br = work[pb];
+    bi = work[pb + 1];
     split_gain(ar, ai, br, bi, n, lane, tr_fwd<T>(d), tr_inv<T>(d), hl);
   }
   row_sync<WIDE>();
   if (active) {
-    const int pa = brev(ka, bits) << 1, pb = brev(kb, bits) << 1;
+    const int pa = 2 * swz(brev(ka, bits)), pb = 2 * swz(brev(kb, bits));
     work[pa] = ar;
     work[pa + 1] = ai;
     work[pb] = br;
@@ -237,7 +263,7 @@ __device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], 
   four1_stages<WIDE>(work, n, lane, tw_inv<T>(d), active);
   if (active)
 #pragma unroll
-    for (int q = 0; q < 4; q++) v[q] = work[lane + q * nq] * T(2. / (n));
+    for (int q = 0; q < 4; q++) v[q] = work[swz_val(lane + q * nq)] * T(2. / (n));
   row_sync<WIDE>();
 }
 
