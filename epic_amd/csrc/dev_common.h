@@ -573,6 +573,33 @@ template <> __device__ __forceinline__ float *fld_ptr_t<float>(const MemberDesc 
   return nullptr;
 }
 
+// DZDT3 of a cell on K = 1..nk, J = 0..nj, with its zonal pads
+// (store_pgrad_vars, src/shared/epic_funcs_diag.c:3595-3950): what k_thermo
+// left there (the geopotential before this call, or 0 while itime <= 1) made a
+// rate, the vertical velocity's part, and the advection of geopotential
+__device__ __forceinline__ void dzdt3_at(const MemberDesc &d, int K, int J, int I) {
+  const size_t o = (size_t)K * d.N2;
+  const uint32_t i = ix2(d, J, I), is = i - d.Ia, in = i + d.Ia;
+  const Plane<const double> G{d.GZ3 + o}, u{d.U + o}, v{d.V + o}, w{d.W3 + o}, h3{d.H3 + o}, rho3{d.RHO3 + o};
+  const Plane<double> Dz{d.DZDT3 + o};
+  double z = Dz[i];
+  if (d.dyn->itime > 1) {
+    double dtg_inv = -1. / (d.dt * d.g[2 * J + 1]);
+    z -= G[i];
+    z *= dtg_inv;
+  }
+  z += w[i] * h3[i] / rho3[i];
+  int jj = 2 * J;
+  double gx3 = .5 * d.m[jj + 1] / d.g[jj + 1];
+  double gy2 = .5 * d.n[jj] / d.g[jj];
+  double gy4 = .5 * d.n[jj + 2] / d.g[jj + 2];
+  z += v[i] * (G[i] - G[is]) * gy2 + v[in] * (G[in] - G[i]) * gy4 + u[i] * (G[i] - G.at(i, -1)) * gx3 +
+       u.at(i, 1) * (G.at(i, 1) - G[i]) * gx3;
+  Dz[i] = z;
+  if (I == d.ni) Dz[ix2(d, J, 0)] = z;
+  if (I == 1) Dz[ix2(d, J, d.ni + 1)] = z;
+}
+
 // launch geometry shared by host and device
 constexpr int TPB = 256;
 

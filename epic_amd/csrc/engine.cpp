@@ -240,9 +240,10 @@ static int rebuild_buckets(epic_engine *E) {
 // With `side` (full = 1, gas giants), gz_from_u runs on the second stream
 // beside k_thermo: it reads U, P3 and theta of the bottom interface (forming
 // RHO3 there itself) and writes its own row buffer, k_thermo writes the
-// per-cell diagnostics; k_gz3 waits for both.
+// per-cell diagnostics; k_gz3 waits for both.  dzdt3 = false: k_ab finishes
+// DZDT3 behind it.
 static bool fork_worth(const Bucket &b) { return (size_t)b.ni * (b.nj + 1) * b.nk * b.nm >= ((size_t)1 << 18); }
-static void rec_p2etc_pgrad_vars(hipStream_t s, const Bucket &b, int full, const SideStream *side) {
+static void rec_p2etc_pgrad_vars(hipStream_t s, const Bucket &b, int full, const SideStream *side, bool dzdt3 = true) {
   L_set_p2etc(s, b, full);  // full = 0: with store_pgrad_vars' T3, RHO3
   const bool fork = full && side && b.any_gas && fork_worth(b);
   if (fork) {
@@ -255,7 +256,7 @@ static void rec_p2etc_pgrad_vars(hipStream_t s, const Bucket &b, int full, const
   if (fork) (void)hipStreamWaitEvent(s, side->join, 0);
   else L_gz_from_u(s, b);
   L_gz3(s, b);
-  if (full) L_dzdt3(s, b);
+  if (full && dzdt3) L_dzdt3(s, b);
 }
 
 // store_diag (src/shared/epic_funcs_diag.c:3963-4053); the filtered copies
@@ -309,7 +310,7 @@ static void rec_step(hipStream_t s, const Bucket &b, bool hv, bool divd, bool ad
   // them, is applied to the filtered hdry as it is stored
   const FieldSet f4 = {4, {F_DUDT_T, F_DVDT_T, F_HDRY, F_THETA}, {0, 1, 2, 3}};
   L_filter3(s, b, f4);
-  rec_p2etc_pgrad_vars(s, b, 1, side);
+  rec_p2etc_pgrad_vars(s, b, 1, side, !ab_dzdt3_fused(b));
   L_pgrad(s, b);
   if (divd) L_divdamp(s, b);
   L_ab(s, b);

@@ -709,31 +709,12 @@ void L_gz3(hipStream_t s, const Bucket &b) {
   else gz3_t<false>(s, b);
 }
 
-// finish DZDT3 (diagnostic vertical velocity)
+// finish DZDT3 (diagnostic vertical velocity); in the step k_ab does it where
+// it can
 __global__ void __launch_bounds__(256) k_dzdt3(const MemberDesc *D, int mb) {
   MEMBER_X;
   FLAT2_X(0, d.nj + 1, 1, d.ni);
-  const int K = 1 + bx_.y;
-  size_t q = ix3(d, K, J, I);
-  const double *G = d.GZ3;
-  double z = d.DZDT3[q];
-  if (d.dyn->itime > 1) {
-    double dtg_inv = -1. / (d.dt * d.g[2 * J + 1]);
-    z -= G[q];
-    z *= dtg_inv;
-  }
-  z += d.W3[q] * d.H3[q] / d.RHO3[q];
-  int jj = 2 * J;
-  double gx3 = .5 * d.m[jj + 1] / d.g[jj + 1];
-  double gy2 = .5 * d.n[jj] / d.g[jj];
-  double gy4 = .5 * d.n[jj + 2] / d.g[jj + 2];
-  z += d.V[q] * (G[q] - G[ix3(d, K, J - 1, I)]) * gy2 +
-       d.V[ix3(d, K, J + 1, I)] * (G[ix3(d, K, J + 1, I)] - G[q]) * gy4 +
-       d.U[q] * (G[q] - G[ix3(d, K, J, I - 1)]) * gx3 +
-       d.U[ix3(d, K, J, I + 1)] * (G[ix3(d, K, J, I + 1)] - G[q]) * gx3;
-  d.DZDT3[q] = z;
-  if (I == d.ni) d.DZDT3[ix3(d, K, J, 0)] = z;
-  if (I == 1) d.DZDT3[ix3(d, K, J, d.ni + 1)] = z;
+  dzdt3_at(d, 1 + bx_.y, J, I);
 }
 void L_dzdt3(hipStream_t s, const Bucket &b) {
   LAUNCH(k_dzdt3, grid2(b.nj + 1, b.ni, b.nk, b.nm), dim3(TPB), 0, s, b.D, b.mb);

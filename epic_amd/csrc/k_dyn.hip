@@ -534,44 +534,88 @@ void L_divdamp(hipStream_t s, const Bucket &b) {
 }
 
 // ------------------------------------------------------ Adams-Bashforth
-// Coefficients from the FLAT_MAX start-up flags of the older planes,
-// tested per wind at (KLO, jlo, ILO) as the reference does.
-// scratch: the result goes to copy 1 (u) and 2 (v) of sD, from where k_hv4
-// takes it, else to the field with its pads
-__global__ void __launch_bounds__(256) k_ab(const MemberDesc *D, int mb, int scratch) {
-  MEMBER;
-  FLAT2(0, d.nj + 1, 1, d.ni);
-  const int K = 1 + blockIdx.y;
-  const MemberDyn dy = *d.dyn;
-  const double FMAX = 1.7976931348623157e308;
-  for (int w = 0; w < 2; w++) {
-    const int jlo = w;  // u: JLO = 0, v: JFIRST = 1
-    if (J < jlo) continue;
-    double *val = w ? d.V : d.U;
-    double *tb = w ? d.DVDT : d.DUDT;
-    double ab0, ab1, ab2;
-    if (tb[(size_t)dy.itm2 * d.N3 + ix3(d, 1, jlo, 1)] == FMAX) {
-      if (tb[(size_t)dy.itm1 * d.N3 + ix3(d, 1, jlo, 1)] == FMAX) { ab0 = 1.; ab1 = 0.; ab2 = 0.; }
-      else { ab0 = 3. / 2.; ab1 = -1. / 2.; ab2 = 0.; }
-    } else {
-      ab0 = 23. / 12.; ab1 = -16. / 12.; ab2 = 5. / 12.;
-    }
-    size_t q = ix3(d, K, J, I);
-    const double y = val[q] + d.dt * (ab0 * tb[(size_t)dy.it0 * d.N3 + q] + ab1 * tb[(size_t)dy.itm1 * d.N3 + q] +
-                                      ab2 * tb[(size_t)dy.itm2 * d.N3 + q]);
-    if (scratch) {
-      d.sD[(size_t)(1 + w) * d.N3 + q] = y;
-      continue;
-    }
-    val[q] = y;
-    // zonal pads (bc_lateral after the update)
-    if (I == d.ni) val[ix3(d, K, J, 0)] = y;
-    if (I == 1) val[ix3(d, K, J, d.ni + 1)] = y;
-  }
+// Coefficients from the start-up flags of the older planes (FLOAT_MAX; the
+// mixed mode's FP32 planes hold FP32's largest value), tested per wind at
+// (KLO, jlo, ILO) as the reference does (jlo: u 0, v 1).
+struct AbCoef {
+  double c0, c1, c2;
+};
+template <class H>
+__device__ __forceinline__ AbCoef ab_coef(const MemberDesc &d, const MemberDyn &dy, const H *hist, int jlo, H flag) {
+  const size_t q = ix3(d, 1, jlo, 1);
+  if (hist[(size_t)dy.itm2 * d.N3 + q] != flag) return {23. / 12., -16. / 12., 5. / 12.};
+  if (hist[(size_t)dy.itm1 * d.N3 + q] != flag) return {3. / 2., -1. / 2., 0.};
+  return {1., 0., 0.};
 }
+// the wind w (0 u, 1 v) of cell i of plane K after the step, from its value x;
+// o: the plane's offset.  MIXED: FP64 accumulation of the current tendency and
+// the FP32 history planes; the current tendency is then stored, rounded, in
+// the history slot IT_ZERO, which the rotation at the end of the step makes
+// IT_MINUS1.
+template <bool MIXED>
+__device__ __forceinline__ double ab_wind(const MemberDesc &d, const MemberDyn &dy, int w, size_t o, uint32_t i, double x,
+                                          bool upd) {
+  if constexpr (MIXED) {
+    float *hist = w ? d.DVDTf : d.DUDTf;
+    const AbCoef ab = ab_coef<float>(d, dy, hist, w, 3.40282347e+38f);
+    const double t0 = Plane<const double>{(w ? d.DVDT : d.DUDT) + o}[i];
+    if (upd) {
+      const Plane<const float> h1{hist + (size_t)dy.itm1 * d.N3 + o}, h2{hist + (size_t)dy.itm2 * d.N3 + o};
+      const double t1 = (ab.c1 != 0.) ? h1[i] : 0., t2 = (ab.c2 != 0.) ? h2[i] : 0.;
+      x += d.dt * (ab.c0 * t0 + ab.c1 * t1 + ab.c2 * t2);
+    }
+    Plane<float>{hist + (size_t)dy.it0 * d.N3 + o}[i] = (float)t0;
+  } else if (upd) {
+    const double *tb = w ? d.DVDT : d.DUDT;
+    const AbCoef ab = ab_coef<double>(d, dy, tb, w, 1.7976931348623157e308);
+    const Plane<const double> h0{tb + (size_t)dy.it0 * d.N3 + o}, h1{tb + (size_t)dy.itm1 * d.N3 + o},
+        h2{tb + (size_t)dy.itm2 * d.N3 + o};
+    x += d.dt * (ab.c0 * h0[i] + ab.c1 * h1[i] + ab.c2 * h2[i]);
+  }
+  return x;
+}
+// TO_FIELD: the update alone, to the field with its pads.  Else to copy 1 (u)
+// and 2 (v) of sD, from where k_hv4 takes it; the fields still hold the winds
+// of before, and the same launch (planes 1..nk, the wind on 1..nk-1) finishes
+// DZDT3, which reads them at the cell's neighbours.  (The two as launches of
+// their own were 490 + 485 us at 1024x512x64 FP64, 10.5 + 11 at 256x128x20;
+// together
+// 867 and 16.9.)
+template <bool MIXED, bool TO_FIELD>
+__global__ void __launch_bounds__(256) k_ab(const MemberDesc *D, int mb) {
+  MEMBER_X;
+  FLAT2_X(0, d.nj + 1, 1, d.ni);
+  const int K = 1 + bx_.y;
+  const size_t o = (size_t)K * d.N2;
+  const uint32_t i = ix2(d, J, I);
+  const MemberDyn dy = *d.dyn;
+  if (TO_FIELD || K < d.nk) {
+#pragma unroll
+    for (int w = 0; w < 2; w++) {
+      double *val = w ? d.V : d.U;
+      const double x = ab_wind<MIXED>(d, dy, w, o, i, Plane<const double>{val + o}[i], J >= w);
+      if (J < w) continue;
+      if constexpr (!TO_FIELD) {
+        Plane<double>{d.sD + (size_t)(1 + w) * d.N3 + o}[i] = x;
+      } else {
+        const Plane<double> out{val + o};
+        out[i] = x;
+        // zonal pads (bc_lateral after the update)
+        if (I == d.ni) out[ix2(d, J, 0)] = x;
+        if (I == 1) out[ix2(d, J, d.ni + 1)] = x;
+      }
+    }
+  }
+  if constexpr (!TO_FIELD) dzdt3_at(d, K, J, I);
+}
+bool ab_dzdt3_fused(const Bucket &b) { return hv_fused(b); }
 void L_ab(hipStream_t s, const Bucket &b) {
-  if (b.mixed) { LM_ab(s, b); return; }
-  LAUNCH(k_ab, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb, hv_fused(b) ? 1 : 0);
+  const bool all = ab_dzdt3_fused(b);
+  const dim3 g = grid2(b.nj + 1, b.ni, all ? b.nk : b.nk - 1, b.nm);
+  if (all && b.mixed) LAUNCH_AS("k_ab", (k_ab<true, false>), g, dim3(TPB), 0, s, b.D, b.mb);
+  else if (all) LAUNCH_AS("k_ab", (k_ab<false, false>), g, dim3(TPB), 0, s, b.D, b.mb);
+  else if (b.mixed) LAUNCH_AS("k_ab", (k_ab<true, true>), g, dim3(TPB), 0, s, b.D, b.mb);
+  else LAUNCH_AS("k_ab", (k_ab<false, true>), g, dim3(TPB), 0, s, b.D, b.mb);
 }
 
 // monotone filtered geopotential, K = nk-1 down to 0 (src/shared/epic_timestep.c:176-196)

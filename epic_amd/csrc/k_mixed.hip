@@ -137,49 +137,6 @@ __global__ void __launch_bounds__(256) km_divdamp(const MemberDesc *D, int mb) {
   }
 }
 
-// ------------------------------------------------------- Adams-Bashforth
-// FP64 accumulation: the current (FP64) tendency and the FP32 history
-// planes IT_MINUS1, IT_MINUS2 (FLT_MAX flags start AB1/AB2); the current
-// tendency is then stored, rounded to FP32, in the history slot IT_ZERO,
-// which the rotation at the end of the step makes IT_MINUS1.  Lanes cover
-// every cell of planes 1..nk-1 so the stored history is the whole plane.
-// scratch: as in k_ab.
-__global__ void __launch_bounds__(256) km_ab(const MemberDesc *D, int mb, int scratch) {
-  MEMBER;
-  FLAT2(0, d.nj + 1, 1, d.ni);
-  const int K = 1 + blockIdx.y;
-  const MemberDyn dy = *d.dyn;
-  const float FMAX = 3.40282347e+38f;
-  for (int w = 0; w < 2; w++) {
-    const int jlo = w;
-    double *val = w ? d.V : d.U;
-    const double *cur = w ? d.DVDT : d.DUDT;
-    float *hist = w ? d.DVDTf : d.DUDTf;
-    const size_t q = ix3(d, K, J, I);
-    const double t0 = cur[q];
-    if (J >= jlo) {
-      double ab0, ab1, ab2;
-      if (hist[(size_t)dy.itm2 * d.N3 + ix3(d, 1, jlo, 1)] == FMAX) {
-        if (hist[(size_t)dy.itm1 * d.N3 + ix3(d, 1, jlo, 1)] == FMAX) { ab0 = 1.; ab1 = 0.; ab2 = 0.; }
-        else { ab0 = 3. / 2.; ab1 = -1. / 2.; ab2 = 0.; }
-      } else {
-        ab0 = 23. / 12.; ab1 = -16. / 12.; ab2 = 5. / 12.;
-      }
-      const double t1 = (ab1 != 0.) ? hist[(size_t)dy.itm1 * d.N3 + q] : 0.,
-                   t2 = (ab2 != 0.) ? hist[(size_t)dy.itm2 * d.N3 + q] : 0.;
-      const double y = val[q] + d.dt * (ab0 * t0 + ab1 * t1 + ab2 * t2);
-      if (scratch) {
-        d.sD[(size_t)(1 + w) * d.N3 + q] = y;
-      } else {
-        val[q] = y;
-        if (I == d.ni) val[ix3(d, K, J, 0)] = y;
-        if (I == 1) val[ix3(d, K, J, d.ni + 1)] = y;
-      }
-    }
-    hist[(size_t)dy.it0 * d.N3 + q] = (float)t0;
-  }
-}
-
 // ------------------------------------------------------------- launchers
 void LM_uv_drag(hipStream_t s, const Bucket &b) {
   if (b.any_ray) LAUNCH(km_rayleigh, dim3(b.nj + 1, b.nk, b.nm), dim3(64), 0, s, b.D, b.mb);
@@ -187,9 +144,6 @@ void LM_uv_drag(hipStream_t s, const Bucket &b) {
 }
 void LM_divdamp_apply(hipStream_t s, const Bucket &b) {
   LAUNCH(km_divdamp, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb);
-}
-void LM_ab(hipStream_t s, const Bucket &b) {
-  LAUNCH(km_ab, grid2(b.nj + 1, b.ni, b.nk - 1, b.nm), dim3(TPB), 0, s, b.D, b.mb, hv_fused(b) ? 1 : 0);
 }
 
 }  // namespace epic

@@ -99,6 +99,8 @@ void L_uv_core(hipStream_t s, const Bucket &b);
 void L_uv_drag(hipStream_t s, const Bucket &b);
 void L_pgrad(hipStream_t s, const Bucket &b);
 void L_divdamp(hipStream_t s, const Bucket &b);
+// the Adams-Bashforth update; where ab_dzdt3_fused, DZDT3 too
+bool ab_dzdt3_fused(const Bucket &b);
 void L_ab(hipStream_t s, const Bucket &b);
 void L_gz_mono(hipStream_t s, const Bucket &b);
 void L_gz_filtercopy(hipStream_t s, const Bucket &b);
@@ -115,7 +117,6 @@ void L_hv_uv(hipStream_t s, const Bucket &b);
 // ---- mixed-precision momentum kernels (k_mixed.hip)
 void LM_uv_drag(hipStream_t s, const Bucket &b);
 void LM_divdamp_apply(hipStream_t s, const Bucket &b);
-void LM_ab(hipStream_t s, const Bucket &b);
 
 // ---- advection (k_adv.hip)
 void L_advection(hipStream_t s, const Bucket &b);
