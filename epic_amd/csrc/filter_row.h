@@ -57,32 +57,23 @@ template <> __device__ __forceinline__ const float *tr_inv<float>(const MemberDe
 // for the same banks was over a third of the row kernels' time.  A permutation
 // of each 16 elements, linear over exclusive or: swz(p ^ q) = swz(p) ^ swz(q).
 // FP64 steps before and after: 256x128x20 429 and 413 us, 23 members of
-// 128x51x13 945 and 920, 1024x512x64 14.39 and 14.26 ms.  (k_hv4's rows are
-// summed in place in natural order and keep it.)
+// 128x51x13 945 and 920, 1024x512x64 14.39 and 14.26 ms; k_hv4, 1024x512x64:
+// 853 and 750 us.
 __device__ __forceinline__ int swz(int p) { return p ^ ((p >> 4) & 15); }
 // the same for value e of the row (element e/2, real or imaginary)
 __device__ __forceinline__ int swz_val(int e) { return 2 * swz(e >> 1) + (e & 1); }
 
-// unit `lane` (of n/8) of the stages s and s+1, h = 2^s, on a row in LDS (SW:
-// its elements at swz): the
+// unit `lane` (of n/8) of the stages s and s+1, h = 2^s, on a row in LDS, its elements
+// at swz: the
 // four points p, p+h, p+2h, p+3h go through stage s as (p, p+h) and
 // (p+2h, p+3h) and through stage s+1 as (p, p+2h) and (p+h, p+3h), in
 // registers
-template <bool SW = false, class T>
+template <class T>
 __device__ __forceinline__ void four1_pair(T *buf, int s, int lane, const T *tw) {
-  const int half = 1 << s, mm = lane & (half - 1), g = lane >> s, p = mm + g * 4 * half;
-  int i0, i1, i2, i3;
-  if constexpr (SW) {  // p has zeros where half and 2 half have their bit
-    i0 = 2 * swz(p);
-    i1 = i0 ^ (2 * swz(half));
-    i2 = i0 ^ (2 * swz(2 * half));
-    i3 = i0 ^ (2 * swz(3 * half));
-  } else {
-    i0 = 2 * p;
-    i1 = i0 + 2 * half;
-    i2 = i1 + 2 * half;
-    i3 = i2 + 2 * half;
-  }
+  const int half = 1 << s, mm = lane & (half - 1), g = lane >> s;
+  // (mm + 4 half g has zeros where half and 2 half have their bit)
+  const int i0 = 2 * swz(mm + g * 4 * half), i1 = i0 ^ (2 * swz(half)), i2 = i0 ^ (2 * swz(2 * half)),
+            i3 = i0 ^ (2 * swz(3 * half));
   T x0r = buf[i0], x0i = buf[i0 + 1], x1r = buf[i1], x1i = buf[i1 + 1];
   T x2r = buf[i2], x2i = buf[i2 + 1], x3r = buf[i3], x3i = buf[i3 + 1];
   const int ka = half - 1 + mm, kb = 2 * half - 1 + mm;
@@ -102,10 +93,10 @@ __device__ __forceinline__ void four1_pair(T *buf, int s, int lane, const T *tw)
   buf[i3 + 1] = x3i;
 }
 // unit `lane` (of n/4) of one stage s: the odd last one
-template <bool SW = false, class T>
+template <class T>
 __device__ __forceinline__ void four1_last(T *buf, int s, int lane, const T *tw) {
-  const int half = 1 << s, g = lane >> s, mm = lane & (half - 1), p = mm + g * 2 * half, k = half - 1 + mm;
-  const int i0 = 2 * (SW ? swz(p) : p), j0 = SW ? i0 ^ (2 * swz(half)) : i0 + 2 * half;
+  const int half = 1 << s, g = lane >> s, mm = lane & (half - 1), k = half - 1 + mm;
+  const int i0 = 2 * swz(mm + g * 2 * half), j0 = i0 ^ (2 * swz(half));
   T xr = buf[i0], xi = buf[i0 + 1], yr = buf[j0], yi = buf[j0 + 1];
   bfly(xr, xi, yr, yi, tw[2 * k], tw[2 * k + 1]);
   buf[i0] = xr;
@@ -128,11 +119,11 @@ __device__ __forceinline__ void four1_stages(T *buf, int n, int lane, const T *t
   while ((2 << S) < n) S++;  // stages s with 2 << s < n
   int s = 0;
   for (; s + 1 < S; s += 2) {
-    if (active && lane < (n >> 3)) four1_pair<true>(buf, s, lane, tw);
+    if (active && lane < (n >> 3)) four1_pair(buf, s, lane, tw);
     row_sync<WIDE>();
   }
   if (s < S) {
-    if (active) four1_last<true>(buf, s, lane, tw);
+    if (active) four1_last(buf, s, lane, tw);
     row_sync<WIDE>();
   }
 }
@@ -274,8 +265,8 @@ __device__ __forceinline__ void filter_row_regs(const MemberDesc &d, T (&v)[4], 
 // all rows, so that short rows fill the wavefront too, and only wavefront
 // barriers separate the stages.  On entry (behind a barrier) a row that is on
 // holds its points in bit-reversed order (rev_pos); on exit (behind one) the
-// unscaled result in natural order, to be multiplied by 2/ni.
-__device__ __forceinline__ int rev_pos(int e, int bits) { return (brev(e >> 1, bits) << 1) | (e & 1); }
+// unscaled result, value e at swz_val(e), to be multiplied by 2/ni.
+__device__ __forceinline__ int rev_pos(int e, int bits) { return 2 * swz(brev(e >> 1, bits)) + (e & 1); }
 template <class T, int NV>
 __device__ __forceinline__ void filter_wave(const MemberDesc &d, T *X, int WS, int rows, const int *on, int J,
                                             int vgrid, int lane) {
@@ -307,10 +298,11 @@ __device__ __forceinline__ void filter_wave(const MemberDesc &d, T *X, int WS, i
     if (r < rows && on[r]) {
       const T *x = X + r * WS;
       const int ka = unit_k(n, l), kb = unit_kb(n, l);
-      ar[i] = x[2 * ka];
-      ai[i] = x[2 * ka + 1];
-      br[i] = x[2 * kb];
-      bi[i] = x[2 * kb + 1];
+      const int pa = 2 * swz(ka), pb = 2 * swz(kb);
+      ar[i] = x[pa];
+      ai[i] = x[pa + 1];
+      br[i] = x[pb];
+      bi[i] = x[pb + 1];
       const double *hl = (vgrid ? d.hl_pv : d.hl_h) + (size_t)(J + r) * (n / 2 + 2);
       split_gain(ar[i], ai[i], br[i], bi[i], n, l, tr_fwd<T>(d), tr_inv<T>(d), hl);
     }
@@ -321,7 +313,7 @@ __device__ __forceinline__ void filter_wave(const MemberDesc &d, T *X, int WS, i
     const int u = lane + 64 * i, r = u >> (lg - 2), l = u & ((n >> 2) - 1);
     if (r < rows && on[r]) {
       T *x = X + r * WS;
-      const int pa = brev(unit_k(n, l), bits) << 1, pb = brev(unit_kb(n, l), bits) << 1;
+      const int pa = 2 * swz(brev(unit_k(n, l), bits)), pb = 2 * swz(brev(unit_kb(n, l), bits));
       x[pa] = ar[i];
       x[pa + 1] = ai[i];
       x[pb] = br[i];

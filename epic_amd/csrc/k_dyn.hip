@@ -1174,7 +1174,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
       if (upd(Jw + u))
 #pragma unroll
         for (int q = 0; q < NQ; q++)
-          if (has) v[u][q] += d.dt * sign * (double)(on[R0 + u] ? x[lane + 64 * q] * sc : x[lane + 64 * q]);
+          if (has) v[u][q] += d.dt * sign * (double)(on[R0 + u] ? x[swz_val(lane + 64 * q)] * sc : x[lane + 64 * q]);
     }
     wave_sync();
 #pragma unroll
