@@ -65,16 +65,21 @@ KERNEL_BYTES = {
     # rho2, heat3, dzdt3
     "k_set_p2etc<1>": (56, 1), "k_set_p2etc<0>": (48, 1), "k_thermo": (88, 1),
     "k_gz3": (40, 1), "k_calc_w": (56, 1), "k_dzdt3": (72, 1),
-    "k_hsu_vert": (24, 3), "k_hsu_mer": (40, 3),
-    "k_hsu_zonal": (32, 3), "k_fft_filter": (16, 3),
-    "k_filter3": (24, 4), "k_zonal_hv": (16, 2), "k_d2dy2_cols": (16, 2), "k_hv_apply": (24, 2),
-    # the mixed mode's fused del^4 rows: D (FP32) read, the field read and written
-    "k_hv4_rows": (20, 2),
-    "k_pgrad": (48, 1), "k_uvh_kin": (48, 1), "k_dvdt_core": (40, 1), "k_dudt_core": (40, 1), "k_ab": (80, 1),
-    "k_divdamp": (40, 1), "km_uvh_kin": (36, 1), "km_dvdt_core": (32, 1), "km_dudt_core": (32, 1), "km_ab": (64, 1),
-    "km_divdamp": (40, 1), "k_gz_mono": (16, 1),
-    "k_zero_tend": (16, 1), "k_adv_elem": (16, 1), "k_heating": (24, 1), "k_sponge": (24, 1), "k_hs_pbl": (32, 1),
-    "k_divergence": (24, 1), "k_store_diag": (40, 1),
+    # the advection's column pass reads w3, theta, h (unity is 1) and writes
+    # three fields; the meridional pass reads v and the three, writes them; the
+    # zonal pass reads u, the three and the old theta, writes theta and h
+    "k_hsu_vert": (16, 3), "k_hsu_mer": (56 / 3, 3), "k_hsu_zonal": (56 / 3, 3),
+    # the 3-D filter reads and writes four fields and reads the filtered gz
+    "k_filter3": (18, 4), "k_zonal_hv": (16, 2), "k_d2dy2_cols": (16, 2), "k_hv_apply": (24, 2),
+    # del^4 in one launch: a field read once and written once
+    "k_hv4": (16, 2),
+    # uv_core reads u, v, h3, pv, w3 and writes du, dv; the pressure gradient
+    # reads gz3, p2, rho3 and adds to du, dv; the Adams-Bashforth update reads
+    # six tendency planes, u, v and writes u, v, and finishes dzdt3 from gz3,
+    # w3, h3, rho3
+    "k_uv_core": (56, 1), "k_pgrad": (56, 1), "k_ab": (128, 1),
+    "k_divdamp": (40, 1), "km_divdamp": (40, 1), "k_gz_mono": (16, 1),
+    "k_heating": (24, 1), "k_hs_pbl": (32, 1), "k_divergence": (24, 1), "k_store_diag": (40, 1),
 }
 
 
@@ -118,11 +123,7 @@ def kernel_bytes(name, ni, nj, nk, members):
         per_cell, fields = KERNEL_BYTES[base]
     else:
         return None
-    if base == "k_fft_filter":
-        cells = ni * filtered_rows(nj) * nk
-    else:
-        cells = ni * (nj + 1) * nk
-    return per_cell * cells * fields * members
+    return per_cell * ni * (nj + 1) * nk * fields * members
 
 
 REF_EXE = os.path.join(HERE, "oracle", "_ref", "epic_ref")

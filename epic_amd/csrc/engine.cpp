@@ -275,7 +275,7 @@ static void rec_sync(hipStream_t s, const Bucket &b, bool adjust, const SideStre
 // src/shared/epic_timestep.c:104-327.  With `side`, the hyperviscosity of
 // hdry and theta runs on the second stream beside uv_core and uv_drag: the
 // two branches read what calc_w leaves and write disjoint arrays (the
-// tendencies and scratch copy 0; hdry, theta and scratch copies 1, 2), so
+// tendencies; hdry, theta and scratch copies 1, 2), so
 // the results are those of the reference's order.
 static void rec_step(hipStream_t s, const Bucket &b, bool hv, bool divd, bool adjust, const SideStream *side) {
   L_calc_w(s, b, 1);  // source_sink + calc_w, and the step's tendency planes cleared

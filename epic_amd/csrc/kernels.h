@@ -25,9 +25,7 @@ extern bool g_prof_on;
 
 // Up to four fields processed by one launch of a batched kernel, each with
 // its kind (0 U, 1 V, 2 HDRY, 3 THETA); blockIdx.z = field index * members
-// + member, and field i uses scratch copy copy0 + i (the hyperviscosity
-// launches of hdry and theta take copies 1 and 2, so that they can run beside
-// uv_core, which uses copy 0).
+// + member, and field i uses scratch copy copy0 + i.
 struct FieldSet {
   int n;
   int f[4], kind[4];
