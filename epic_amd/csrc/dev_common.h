@@ -247,29 +247,14 @@ __device__ __forceinline__ void m_pow2(double x0, double y0, double x1, double y
 
 // hybrid sigma-theta coordinate (src/shared/epic_funcs_diag.c:1238-1314,1751-1770)
 template <bool F = false>
-__device__ __forceinline__ double get_sigma(double pbot, double p, double ptop) {
-  return m_log<F>(p / pbot) / m_log<F>(ptop / pbot);
-}
-template <bool F = false>
-__device__ __forceinline__ double get_p_sigma(double pbot, double s, double ptop) {
-  return pbot * m_exp<F>(s * m_log<F>(ptop / pbot));
-}
-template <bool F = false>
 __device__ __forceinline__ double g_sig(const MemberDesc &d, double s) {
   if (s <= d.sigma_sigma) return 0.;
   if (s >= 1.) return 1.;
   return d.g_coeff * (1. - m_exp<F>(-d.alpha * (s - d.sigma_sigma)));
 }
-template <bool F = false>
-__device__ __forceinline__ double f_sig(const MemberDesc &d, double s) {
-  if (s < 0.) return d.zeta0;
-  if (s <= d.sigma_sigma) return d.zeta0 + s * (d.zeta1 - d.zeta0);
-  if (s < 1.) return (1. - g_sig<F>(d, s)) * (d.zeta0 + s * (d.zeta1 - d.zeta0));
-  return 0.;
-}
 // (sigmatheta - f_sigma(s)) / g_sigma(s), the theta of a hybrid level at
 // sigma s, with g_sigma formed once for both terms (the same operations as
-// calling f_sig and g_sig, so the same result)
+// forming each by itself, so the same result)
 template <bool F = false>
 __device__ __forceinline__ double theta_of_sigma(const MemberDesc &d, double sgth, double s) {
   const bool mid = (s > d.sigma_sigma && s < 1.);
@@ -279,29 +264,16 @@ __device__ __forceinline__ double theta_of_sigma(const MemberDesc &d, double sgt
   const double f = (s < 0.) ? d.zeta0 : (s <= d.sigma_sigma ? lin : (s < 1. ? (1. - gm) * lin : 0.));
   return (sgth - f) / g;
 }
-// return_sigmatheta; sets *bad when p is outside [ptop, pbot]
-__device__ __forceinline__ double sgth_of(const MemberDesc &d, double theta, double p, double pbot, double ptop,
-                                          int *bad) {
-  if (p <= ptop) return theta;
-  if (p <= pbot) {
-    double s = get_sigma(pbot, p, ptop);
-    return f_sig(d, s) + g_sig(d, s) * theta;
-  }
-  *bad = 1;
-  return 0.;
-}
-
-// The same with the column's log(ptop/pbot) formed once by
-// the caller: identical operations on identical operands, so identical
-// results, with one logarithm fewer per call.
+// sigma of a pressure and the pressure of a sigma, lr the column's
+// log(ptop/pbot)
 template <bool F = false>
 __device__ __forceinline__ double get_sigma_l(double pbot, double p, double lr) { return m_log<F>(p / pbot) / lr; }
 template <bool F = false>
 __device__ __forceinline__ double get_p_sigma_l(double pbot, double s, double lr) { return pbot * m_exp<F>(s * lr); }
-// sgth_of at p2 less sgth_of at p4, ptop <= p2 < p4 <= pbot (p4 > ptop), the
-// transcendentals of the two side by side: f_sig(s) + g_sig(s) theta with
-// g_sigma's exponential formed once (the same operations as the two calls, so
-// the same result); *bad as sgth_of sets it
+// return_sigmatheta at p2 less that at p4, the transcendentals of the two side
+// by side: theta at or above ptop, below it f_sigma(s) + g_sigma(s) theta (g_sig)
+// with g_sigma's exponential formed once for both; sets *bad when a pressure
+// lies outside [ptop, pbot]
 template <bool F>
 __device__ __forceinline__ double sgth_diff_l(const MemberDesc &d, double theta, double p2, double p4, double pbot,
                                               double ptop, double lr, int *bad) {

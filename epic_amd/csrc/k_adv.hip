@@ -71,8 +71,6 @@ __device__ __forceinline__ int adv_kfirst(const MemberDesc &d, int which) { retu
 // double reproduces the reference operation for operation; float is the
 // mixed mode's (the fields stay FP64: each update adds the FP32 flux
 // divergence to the FP64 value).
-template <class T> __device__ __forceinline__ T tmin(T x, T y) { return x < y ? x : y; }
-template <class T> __device__ __forceinline__ T tmax(T x, T y) { return x > y ? x : y; }
 
 // x / 6, correctly rounded, for finite x of ordinary size: the product with
 // the rounded reciprocal is within an ulp, and one fused correction of its

@@ -42,9 +42,6 @@ static inline dim3 grid2(int nJ, int nI, int nK, int nm) {
   return dim3((unsigned)((nJ * nI + TPB - 1) / TPB), (unsigned)nK, (unsigned)nm);
 }
 
-__device__ __forceinline__ double *tend(const MemberDesc &d, double *base, int plane) {
-  return base + (size_t)plane * d.N3;
-}
 // the plane the current step's tendency accumulates in: the time plane
 // IT_ZERO, or the mixed mode's single FP64 plane
 __device__ __forceinline__ double *cur_tend(const MemberDesc &d, double *base) {

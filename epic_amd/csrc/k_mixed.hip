@@ -29,16 +29,6 @@ namespace epic {
   if (t_ >= (nJ) * (nI)) return;                       \
   const int J = (j0) + t_ / (nI);                      \
   const int I = (i0) + t_ % (nI);
-// the same with the block renumbered for the XCDs (xcd_block): bx_.y and
-// bx_.z stand for blockIdx.y and blockIdx.z
-#define MEMBER_X                                       \
-  const uint3 bx_ = xcd_block();                       \
-  const MemberDesc &d = D[mb + bx_.z]
-#define FLAT2_X(j0, nJ, i0, nI)                        \
-  int t_ = bx_.x * TPB + threadIdx.x;                  \
-  if (t_ >= (nJ) * (nI)) return;                       \
-  const int J = (j0) + t_ / (nI);                      \
-  const int I = (i0) + t_ % (nI);
 
 static inline dim3 grid2(int nJ, int nI, int nK, int nm) {
   return dim3((unsigned)((nJ * nI + TPB - 1) / TPB), (unsigned)nK, (unsigned)nm);
