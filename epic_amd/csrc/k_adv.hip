@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(256) k_hsu_mer(const MemberDesc *D, int mb, in
 // follow on all lanes, periodic in I.  The filter runs here, on the row in registers, rather than
 // in a launch of its own over a copy: the copy was a write and two reads of
 // every field, and a wavefront without a row in the band skips the transform.
-// Three row arrays: field, velocity (split by sign where it is used; the
+// Three row arrays: field, velocity (the
 // corrected flux overwrites it once every lane has read it) and predictor
 // (before that, the filter's scratch); the first-guess flux is formed where
 // the predictor needs it (twice per cell, by the same expression).

@@ -9,7 +9,7 @@
 //   zonal/meridional hyperviscosity, d2dy2  src/shared/epic_subgrid.c:590-1232
 //
 // (restore_mass, src/shared/epic_adjust.c:45-96, runs inside the launches
-// next to each of its calls: k_adv_elem in k_adv.hip, k_filter3 in
+// next to each of its calls: the advection in k_adv.hip, k_filter3 in
 // k_filter.hip.)
 //
 // The reference carries the finite-volume faces west->east and
