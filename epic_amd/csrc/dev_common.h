@@ -407,19 +407,22 @@ __device__ __forceinline__ int table_place_near(int n, const double *x, double x
   *dx = x[g + 1] - x[g];
   return g;
 }
-// whether x[0..n) is such a table (then table_place_near may replace table_place)
-__device__ __forceinline__ bool table_well_separated(int n, const double *x) {
+// whether x[0..n) is such a table (then table_place_near may replace
+// table_place), by the lanes of one wavefront; every lane gets the answer
+__device__ __forceinline__ bool table_well_separated(int n, const double *x, int lane) {
   double mx = 0.;
-  for (int e = 0; e < n; e++) mx = dmax(mx, fabs(x[e]));
+  for (int e = lane; e < n; e += 64) mx = dmax(mx, fabs(x[e]));
+  for (int off = 32; off > 0; off >>= 1) mx = dmax(mx, __shfl_xor(mx, off, 64));
   int ex;
   frexp(mx, &ex);
   const double gap = 2. * ldexp(2.220446049250313e-16, ex + 1);
   const bool ascend = (x[n - 1] >= x[0]);
-  for (int e = 0; e + 1 < n; e++) {
+  bool close = n < 2;
+  for (int e = lane; e + 1 < n; e += 64) {
     const double dd = ascend ? x[e + 1] - x[e] : x[e] - x[e + 1];
-    if (!(dd > gap)) return false;
+    if (!(dd > gap)) close = true;
   }
-  return n >= 2;
+  return !__any(close);
 }
 
 // strided variant: table entries at x[k*stride]
