@@ -1243,10 +1243,16 @@ static std::vector<int> knob_candidates(int k) {
   return k == KN_ROWS_ZHV ? std::vector<int>(zhv, zhv + 3) : std::vector<int>(mer, mer + 3);
 }
 
+// whether a launch takes its shape from knob k (cols_hsuv: the Akima column
+// pass alone, the other scheme's holds its cells in registers; rows_zhv and
+// rows_d2: buckets with an order past del^4, k_hv4 has neither)
 static bool knob_times(const char *kernel, int k) {
-  static const char *const pfx[KN_COUNT] = {"k_set_p2etc", "k_gz3", "k_calc_w", "k_hsu_vert", "k_zonal_hv",
-                                            "k_hsu_mer", "k_d2dy2_cols"};
-  return strncmp(kernel, pfx[k], strlen(pfx[k])) == 0;
+  static const char *const pfx[KN_COUNT][2] = {{"k_set_p2etc", ""}, {"k_gz3", ""},         {"k_calc_w", ""},
+                                               {"k_ak_vert", ""},   {"k_zonal_hv", ""},    {"k_hsu_mer", "k_ak_mer"},
+                                               {"k_d2dy2_cols", ""}};
+  for (const char *p : pfx[k])
+    if (*p && strncmp(kernel, p, strlen(p)) == 0) return true;
+  return false;
 }
 
 extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int cap) {
@@ -1286,6 +1292,7 @@ extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int
     for (int k = 0; k < KN_COUNT; k++) {
       double best = 1e300;
       int bestv = b.knob[k];
+      bool launched = true;
       for (int v : knob_candidates(k)) {
         if (!v || !knob_fits(b, k, v)) continue;
         b.knob[k] = v;
@@ -1299,12 +1306,16 @@ extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int
         g_prof_on = false;
         HIPCHK(hipStreamSynchronize(E->stream));
         double t = 0.;
+        launched = false;
         for (auto &r : g_prof) {
           if (!knob_times(r.name, k)) continue;
+          launched = true;
           float ms = 0.f;
           (void)hipEventElapsedTime(&ms, r.a, r.b);
           t += ms;
         }
+        // nothing of this bucket reads the knob: it stays as it was
+        if (!launched) break;
         if (t < best) {
           best = t;
           bestv = v;
@@ -1314,11 +1325,16 @@ extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int
       if (report && used < (size_t)cap) {
         char shape[32];
         const int lev = (k == KN_COLS_HSUV) ? b.nk + 2 : b.nk + 1;
-        if (k <= KN_COLS_HSUV && knob_threads(bestv, lev) != 256)
+        if (!bestv)
+          snprintf(shape, sizeof(shape), "built-in");
+        else if (k <= KN_COLS_HSUV && knob_threads(bestv, lev) != 256)
           snprintf(shape, sizeof(shape), "%d/%dthr", knob_cols(bestv), knob_threads(bestv, lev));
         else
           snprintf(shape, sizeof(shape), "%d", bestv);
-        if (best < 1e300)
+        if (!launched)
+          used += snprintf(report + used, cap - used, "%dx%dx%d x%d %s=%s (not launched)\n", b.ni, b.nj, b.nk, b.nm,
+                           knob_name[k], shape);
+        else if (best < 1e300)
           used += snprintf(report + used, cap - used, "%dx%dx%d x%d %s=%s (%.1f us/step)\n", b.ni, b.nj, b.nk,
                            b.nm, knob_name[k], shape, best / steps * 1e3);
         else

@@ -1,0 +1,50 @@
+"""The launch shapes of the tunable kernels: what the autotuner times and
+picks, and that no shape changes a result."""
+import pytest
+
+import epic_amd as ea
+from tests.gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+# the default operators, and the ones with kernels of their own: del^8 after
+# del^4's pieces, monotonized fourth-order advection of every field
+PLAIN = ea.spec(ea.JUPITER_LIKE, 64, 32, 20, 60, 5, 0.5, 0.0, 0.0, 0.5)
+OTHER = ea.spec(ea.JUPITER_LIKE, 64, 32, 20, 60, 6, 0.0, 0.0, 0.0, 0.5, nu8=0.5, adv_mass=1, adv_nonmass=1)
+
+
+def engine(*specs, precision=ea.FP64):
+    e = ea.Engine(precision, len(specs))
+    for sp in specs:
+        e.add(sp)
+    return e
+
+
+def report(e):
+    """{knob: what the autotuner says of it} of a one-bucket engine."""
+    rep = e.autotune(1)
+    say(rep)
+    return dict(line.split(" ", 2)[2].split("=", 1) for line in rep.strip().splitlines())
+
+
+def test_a_knob_no_launch_reads_stays_as_it_was():
+    """del^4 alone runs in k_hv4 and the predictor-corrector's column pass in
+    registers: neither reads rows_zhv, rows_d2 or cols_hsuv.  Set by hand or
+    not, these stay, and the report says why."""
+    say("knobs not launched")
+    e = engine(PLAIN)
+    e.set_shape("rows_zhv", 8)
+    got = report(e)
+    assert got["rows_zhv"] == "8 (not launched)"
+    assert got["rows_d2"] == got["cols_hsuv"] == "built-in (not launched)"
+    e.close()
+
+
+def test_every_knob_is_timed_on_the_kernels_that_read_it():
+    say("knobs launched")
+    e = engine(OTHER)
+    got = report(e)
+    assert sorted(got) == sorted(ea.SHAPE_KNOBS)
+    for k, v in got.items():
+        assert v.endswith(" us/step)") and "(0.0 " not in v, (k, v)
+    e.close()
