@@ -1199,8 +1199,8 @@ extern "C" int epic_engine_restore(epic_engine *E, const epic_case *c, const cha
 // --------------------------------------------------------------- autotune
 // Picks, per bucket, the launch shape of each tunable kernel (columns per
 // column tile, rows per zonal-hyperviscosity block or meridional-advection
-// tile) by timing every
-// candidate over a few steps of the bucket's own members.  The members'
+// tile) by timing the built-in shape and every candidate that fits
+// over a few steps of the bucket's own members.  The members'
 // blobs are copied aside first and put back after every candidate and at
 // the end, so tuning leaves the state (and the step counts) as it found
 // them; the shapes never change a result.  The graph is re-captured with
@@ -1209,25 +1209,18 @@ static const char *const knob_name[KN_COUNT] = {"cols_p2etc", "cols_gz3", "cols_
                                                 "cols_hsuv",  "rows_zhv", "rows_mer", "rows_d2"};
 
 static bool knob_fits(const Bucket &b, int k, int v) {
-  const size_t W = (size_t)b.nk + 1, L = (size_t)b.nk + 2, lim = 128 * 1024;
-  if (k <= KN_COLS_HSUV) {
-    // lanes per column beyond twice the column's length would idle
-    // the kernel's levels per column: nk+2 for the vertical advection pass,
-    // nk+1 for the others
-    const int C = knob_cols(v), lev = (k == KN_COLS_HSUV) ? (int)L : (int)W, nt = knob_threads(v, lev);
-    if (nt > 1024 || (size_t)(nt / C) > 2 * L) return false;
-    v = C;
-  }
+  const size_t lim = 128 * 1024;
   switch (k) {
-    case KN_COLS_P2ETC: return sizeof(double) * (2 * v * W + 4 * v) <= lim;
-    case KN_COLS_GZ3: return sizeof(double) * 3 * v * W <= lim;
-    case KN_COLS_CALCW: return sizeof(double) * (4 * v * W + v) <= lim;
-    case KN_COLS_HSUV: return sizeof(double) * 4 * v * L <= lim;
-    case KN_ROWS_MER: return sizeof(double) * (size_t)(b.ni < 64 ? b.ni : 64) * (6 * v + 15) <= lim;
-    case KN_ROWS_D2: return true;  // registers only
-    default:  // KN_ROWS_ZHV: one row array per row, and at most 16 points per lane
+    case KN_ROWS_MER: return true;  // registers; the Akima tile's 8 rows of 64 columns are 20 KB of LDS
+    case KN_ROWS_D2: return true;   // registers only
+    case KN_ROWS_ZHV:  // one row array per row, and at most 16 points per lane
       return sizeof(double) * ((size_t)v * ((b.ni + 2) | 1) + v) <= lim && v / 4 * (b.ni >= 64 ? b.ni / 64 : 1) <= 16;
   }
+  // no more threads than twice the column's length for each column (nk+2
+  // levels in the Akima column pass, nk+1 in the others)
+  const bool ak = (k == KN_COLS_HSUV);
+  const int C = knob_cols(v), nt = knob_threads(v, ak ? b.nk + 2 : b.nk + 1);
+  return nt <= 1024 && nt / C <= 2 * (b.nk + 2) && (ak ? ak_col_lds(b, C) : col_lds(b, C)) <= lim;
 }
 
 // the candidates: column tiles of 8-64 columns per block of 256, 512 or
@@ -1293,8 +1286,10 @@ extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int
       double best = 1e300;
       int bestv = b.knob[k];
       bool launched = true;
-      for (int v : knob_candidates(k)) {
-        if (!v || !knob_fits(b, k, v)) continue;
+      std::vector<int> cand{0};  // the built-in shape first
+      for (int v : knob_candidates(k))
+        if (knob_fits(b, k, v)) cand.push_back(v);
+      for (int v : cand) {
         b.knob[k] = v;
         restore();
         rec_step(E->stream, b, hv, divd, adj, &E->side);  // warm-up, not timed
@@ -1334,12 +1329,9 @@ extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int
         if (!launched)
           used += snprintf(report + used, cap - used, "%dx%dx%d x%d %s=%s (not launched)\n", b.ni, b.nj, b.nk, b.nm,
                            knob_name[k], shape);
-        else if (best < 1e300)
+        else
           used += snprintf(report + used, cap - used, "%dx%dx%d x%d %s=%s (%.1f us/step)\n", b.ni, b.nj, b.nk,
                            b.nm, knob_name[k], shape, best / steps * 1e3);
-        else
-          used += snprintf(report + used, cap - used, "%dx%dx%d x%d %s=built-in (no candidate fits)\n", b.ni,
-                           b.nj, b.nk, b.nm, knob_name[k]);
       }
     }
     std::array<int, KN_COUNT> kv;

@@ -685,7 +685,7 @@ static void advection_t(hipStream_t s, const Bucket &b) {
   const int ncol = (b.nj + 1) * b.ni, nz = ADV_FIELDS * b.nm;
   // columns per block: as many as keep the four LDS columns within 40 KB
   int C = 64;
-  while (C > 16 && (size_t)4 * C * (b.nk + 2) * sizeof(double) > 40 * 1024) C /= 2;
+  while (C > 16 && ak_col_lds(b, C) > 40 * 1024) C /= 2;
   const int v = b.knob[KN_COLS_HSUV];
   if (v) C = knob_cols(v);
   const bool hsu = b.adv_schemes & 1, akima = b.adv_schemes & 2;

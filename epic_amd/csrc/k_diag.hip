@@ -91,32 +91,6 @@ struct Tile {
     return {f + (size_t)K * d.N2};
   }
 };
-// a tile kernel's shape: columns, levels per lane, threads
-struct ColShape {
-  int C, KC, nt;
-};
-static inline ColShape col_shape(const Bucket &b, int knob) {
-  const int lev = b.nk;
-  ColShape s{64, 2, 0};
-  if (knob) {
-    s.C = knob_cols(knob);
-    const int groups = std::max(1, knob_threads(knob, lev + 1) / s.C);
-    while (s.KC < 8 && groups * s.KC < lev) s.KC *= 2;
-  } else {
-    // More levels a lane read and form fewer around them again, but leave
-    // fewer wavefronts: the most that leave 8192 (8 levels) or 2048 (4) of
-    // them.  Steps with 2, 4 and 8 levels: 64x32x10 170, 181, 208 us;
-    // 256x128x20 441, 442, 469; 23 members of 128x51x13 955, 952, 981; 64 mixed
-    // ones of 128x64x16 3510, 3414, 3310; mixed 512x256x32 1786, 1786, 1759.
-    const size_t tiles = ((size_t)(b.nj + 1) * (b.ni + 2) + 63) / 64 * b.nm;
-    s.KC = tiles * ((lev + 7) / 8) >= 8192 ? 8 : tiles * ((lev + 3) / 4) >= 2048 ? 4 : 2;
-  }
-  // (any depth: 8 columns take up to 1024 levels)
-  while (s.KC < 8 && (lev + s.KC - 1) / s.KC * s.C > 1024) s.KC *= 2;
-  while (s.C > 1 && (lev + s.KC - 1) / s.KC * s.C > 1024) s.C /= 2;
-  s.nt = s.C * ((lev + s.KC - 1) / s.KC);
-  return s;
-}
 static inline dim3 tile_grid(const Bucket &b, int C) {
   return dim3((unsigned)(((b.nj + 1) * (b.ni + 2) + C - 1) / C), 1, (unsigned)b.nm);
 }
@@ -297,7 +271,7 @@ static void set_p2etc_t(hipStream_t s, const Bucket &b) {
   const ColShape sh = col_shape(b, b.knob[KN_COLS_P2ETC]);
 #define K_(KC, U) k_set_p2etc<FULL, F, KC, U>
   COLS_LAUNCH(FULL ? "k_set_p2etc<1>" : "k_set_p2etc<0>", K_, sh, tile_grid(b, sh.C), dim3(sh.nt),
-              sizeof(double) * sh.C * (b.nk + 1), s, b.D, b.mb, sh.C);
+              col_lds(b, sh.C), s, b.D, b.mb, sh.C);
 #undef K_
 }
 void L_set_p2etc(hipStream_t s, const Bucket &b, int update_theta) {
@@ -701,7 +675,7 @@ template <bool F>
 static void gz3_t(hipStream_t s, const Bucket &b) {
   const ColShape sh = col_shape(b, b.knob[KN_COLS_GZ3]);
 #define K_(KC, U) k_gz3<F, KC, U>
-  COLS_LAUNCH("k_gz3", K_, sh, tile_grid(b, sh.C), dim3(sh.nt), sizeof(double) * sh.C * (b.nk + 1), s, b.D, b.mb, sh.C);
+  COLS_LAUNCH("k_gz3", K_, sh, tile_grid(b, sh.C), dim3(sh.nt), col_lds(b, sh.C), s, b.D, b.mb, sh.C);
 #undef K_
 }
 void L_gz3(hipStream_t s, const Bucket &b) {
@@ -992,7 +966,7 @@ static void calc_w_t(hipStream_t s, const Bucket &b, int with_source) {
     g.x += (unsigned)std::max<size_t>(1, std::min<size_t>(1024, n / ((size_t)sh.nt * 4)));
   }
 #define K_(KC, U) k_calc_w<F, KC, U>
-  COLS_LAUNCH("k_calc_w", K_, sh, g, dim3(sh.nt), sizeof(double) * sh.C * (b.nk + 1), s, b.D, b.mb, with_source, sh.C, ncb);
+  COLS_LAUNCH("k_calc_w", K_, sh, g, dim3(sh.nt), col_lds(b, sh.C), s, b.D, b.mb, with_source, sh.C, ncb);
 #undef K_
 }
 void L_calc_w(hipStream_t s, const Bucket &b, int with_source) {

@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "dev_common.h"
 
 namespace epic {
@@ -63,7 +65,37 @@ struct Bucket {
   int adv_schemes;
 };
 
-
+// The shape of a column-tile kernel (set_p2etc, gz3, calc_w): columns, levels
+// per lane, threads
+struct ColShape {
+  int C, KC, nt;
+};
+inline ColShape col_shape(const Bucket &b, int knob) {
+  const int lev = b.nk;
+  ColShape s{64, 2, 0};
+  if (knob) {
+    s.C = knob_cols(knob);
+    const int groups = std::max(1, knob_threads(knob, lev + 1) / s.C);
+    while (s.KC < 8 && groups * s.KC < lev) s.KC *= 2;
+  } else {
+    // More levels a lane read and form fewer around them again, but leave
+    // fewer wavefronts: the most that leave 8192 (8 levels) or 2048 (4) of
+    // them.  Steps with 2, 4 and 8 levels: 64x32x10 170, 181, 208 us;
+    // 256x128x20 441, 442, 469; 23 members of 128x51x13 955, 952, 981; 64 mixed
+    // ones of 128x64x16 3510, 3414, 3310; mixed 512x256x32 1786, 1786, 1759.
+    const size_t tiles = ((size_t)(b.nj + 1) * (b.ni + 2) + 63) / 64 * b.nm;
+    s.KC = tiles * ((lev + 7) / 8) >= 8192 ? 8 : tiles * ((lev + 3) / 4) >= 2048 ? 4 : 2;
+  }
+  // (any depth: 8 columns take up to 1024 levels)
+  while (s.KC < 8 && (lev + s.KC - 1) / s.KC * s.C > 1024) s.KC *= 2;
+  while (s.C > 1 && (lev + s.KC - 1) / s.KC * s.C > 1024) s.C /= 2;
+  s.nt = s.C * ((lev + s.KC - 1) / s.KC);
+  return s;
+}
+// its LDS: one column of nk+1 values for each of its columns
+inline size_t col_lds(const Bucket &b, int C) { return sizeof(double) * C * (b.nk + 1); }
+// the Akima column pass's LDS (of FP64 values): four columns of nk+2 values each
+inline size_t ak_col_lds(const Bucket &b, int C) { return sizeof(double) * 4 * C * (b.nk + 2); }
 
 // the Bucket::adv_schemes bits of one member
 inline int adv_schemes(const MemberDesc &d) {

@@ -48,3 +48,21 @@ def test_every_knob_is_timed_on_the_kernels_that_read_it():
     for k, v in got.items():
         assert v.endswith(" us/step)") and "(0.0 " not in v, (k, v)
     e.close()
+
+
+@pytest.mark.parametrize("precision", [ea.FP64, ea.MIXED])
+@pytest.mark.parametrize("knob", ["cols_p2etc", "cols_gz3", "cols_calcw"])
+def test_the_widest_column_tile_fits_the_deepest_grid(knob, precision):
+    """64 columns of 64 levels are one LDS array of 33 KB, and the built-in
+    tile of a deep grid: the same shape by hand gives the same bits."""
+    sp = ea.spec(ea.HELD_SUAREZ, 16, 8, 64, 300, 3, 0.5, 0.0, 0.1, 0.3)
+    say("64 columns of 64 levels", knob, precision)
+    out = []
+    for v in (0, 64, 2064, 4064):
+        e = engine(sp, precision=precision)
+        e.set_shape(knob, v)
+        e.step(3)
+        out.append({f: e.read(0, f).tobytes() for f in ea.FIELDS if f[:4] not in ("DUDT", "DVDT")})
+        e.close()
+    for got in out[1:]:
+        assert got == out[0]
