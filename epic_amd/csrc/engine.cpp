@@ -90,8 +90,9 @@ struct epic_engine {
   MemberDesc *dD;       // device descriptor array (bucket order)
   std::vector<int> order;  // bucket order -> slot
   std::vector<Bucket> buckets;
-  // launch shapes chosen by epic_engine_autotune, by (ni, nj, nk, members)
-  std::map<std::array<int, 4>, std::array<int, KN_COUNT>> tuned;
+  // launch shapes chosen by epic_engine_autotune, by what decides which kernels
+  // a bucket launches and over how many cells (tuned_key)
+  std::map<std::array<int, 6>, std::array<int, KN_COUNT>> tuned;
   bool dirty;
   hipStream_t stream;
   // a second stream (default priority) for the step's one independent
@@ -105,6 +106,10 @@ struct epic_engine {
   std::vector<hipGraphExec_t> bgexec;
   char err[512];
 };
+
+static std::array<int, 6> tuned_key(const Bucket &b) {
+  return {b.ni, b.nj, b.nk, b.nm, b.hv_passes, b.adv_schemes};
+}
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -220,7 +225,7 @@ static int rebuild_buckets(epic_engine *E) {
       b.any_ray |= ((h.newt_cool_on && h.prandtl > 0.) || (h.tau_drag > 0. && h.tau_drag < 1.e+20));
       b.adv_schemes |= adv_schemes(h);
     }
-    auto t = E->tuned.find({b.ni, b.nj, b.nk, b.nm});
+    auto t = E->tuned.find(tuned_key(b));
     for (int k = 0; k < KN_COUNT; k++) b.knob[k] = (t == E->tuned.end()) ? 0 : t->second[k];
     E->buckets.push_back(b);
     i = j;
@@ -1336,7 +1341,7 @@ extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int
     }
     std::array<int, KN_COUNT> kv;
     for (int k = 0; k < KN_COUNT; k++) kv[k] = b.knob[k];
-    E->tuned[{b.ni, b.nj, b.nk, b.nm}] = kv;
+    E->tuned[tuned_key(b)] = kv;
   }
   restore();
   HIPCHK(hipStreamSynchronize(E->stream));
@@ -1365,11 +1370,11 @@ extern "C" int epic_engine_set_shape(epic_engine *E, int knob, int value) {
   HIPCHK(hipStreamSynchronize(E->stream));
   for (Bucket &b : E->buckets) {
     b.knob[knob] = value;
-    auto t = E->tuned.find({b.ni, b.nj, b.nk, b.nm});
+    auto t = E->tuned.find(tuned_key(b));
     if (t == E->tuned.end()) {
       std::array<int, KN_COUNT> kv{};
       kv[knob] = value;
-      E->tuned[{b.ni, b.nj, b.nk, b.nm}] = kv;
+      E->tuned[tuned_key(b)] = kv;
     } else {
       t->second[knob] = value;
     }

@@ -66,3 +66,25 @@ def test_the_widest_column_tile_fits_the_deepest_grid(knob, precision):
         e.close()
     for got in out[1:]:
         assert got == out[0]
+
+
+def test_shapes_belong_to_buckets_of_the_same_kernels():
+    """A shape chosen for a bucket serves later buckets of the grid, member
+    count, hyperviscosity order and advection schemes it was chosen for, and
+    no other: here the report of knobs that no launch of the new bucket reads
+    shows what they hold."""
+    say("shapes of other kernels")
+    e = engine(OTHER)
+    e.set_shape("cols_hsuv", 2016)
+    e.set_shape("rows_zhv", 8)
+    e.remove(0)
+    e.add(PLAIN)
+    got = report(e)
+    assert got["cols_hsuv"] == got["rows_zhv"] == "built-in (not launched)"
+    e.close()
+    e = engine(PLAIN)
+    e.set_shape("rows_zhv", 8)
+    e.remove(0)
+    e.add(PLAIN)
+    assert report(e)["rows_zhv"] == "8 (not launched)"
+    e.close()
