@@ -1228,8 +1228,9 @@ static bool knob_fits(const Bucket &b, int k, int v) {
   return nt <= 1024 && nt / C <= 2 * (b.nk + 2) && (ak ? ak_col_lds(b, C) : col_lds(b, C)) <= lim;
 }
 
-// the candidates: column tiles of 8-64 columns per block of 256, 512 or
-// 1024 threads, or of 4-16 columns with one lane per level; 4-16 rows per zonal-hyperviscosity block; 2-8 rows per
+// the candidates: column tiles of 8-64 columns with threads for 256, 512 or
+// 1024 (column, level) pairs, or of 4-16 columns with threads for every level;
+// 4-16 rows per zonal-hyperviscosity block; 2-8 rows per
 // meridional-advection tile; 8-32 rows per column tile of the del^4
 // meridional second differences
 static std::vector<int> knob_candidates(int k) {
@@ -1324,11 +1325,13 @@ extern "C" int epic_engine_autotune(epic_engine *E, int steps, char *report, int
       b.knob[k] = bestv;
       if (report && used < (size_t)cap) {
         char shape[32];
-        const int lev = (k == KN_COLS_HSUV) ? b.nk + 2 : b.nk + 1;
+        // column tiles with the threads their blocks have
         if (!bestv)
           snprintf(shape, sizeof(shape), "built-in");
-        else if (k <= KN_COLS_HSUV && knob_threads(bestv, lev) != 256)
-          snprintf(shape, sizeof(shape), "%d/%dthr", knob_cols(bestv), knob_threads(bestv, lev));
+        else if (k < KN_COLS_HSUV)
+          snprintf(shape, sizeof(shape), "%d/%dthr", col_shape(b, bestv).C, col_shape(b, bestv).nt);
+        else if (k == KN_COLS_HSUV)
+          snprintf(shape, sizeof(shape), "%d/%dthr", knob_cols(bestv), knob_threads(bestv, b.nk + 2));
         else
           snprintf(shape, sizeof(shape), "%d", bestv);
         if (!launched)

@@ -427,25 +427,29 @@ int  epic_engine_write_nc(epic_engine *e, int slot, const epic_case *c, const ch
 const char *epic_nc_error(void);
 void epic_nc_header_free(void *header);
 /* Autotuner (no counterpart in the reference, whose loops have no launch
- * shapes): for each bucket, time every candidate launch shape of the tunable
- * kernels (columns per column tile of set_p2etc, gz3, calc_w and the
- * vertical advection pass, and the tile's threads; rows per
- * zonal-hyperviscosity block, per meridional-advection tile and per column
- * tile of the del^4 meridional second differences) over
- * `steps` steps of the bucket's own members and keep the fastest.  The
- * members' state is copied aside and put back, so the call changes no
- * result and no state; it needs room for one copy of every member.  Writes
- * one line per choice into report (up to cap bytes).  0 or a negative code. */
+ * shapes): for each bucket, time the built-in and every candidate launch
+ * shape of the tunable kernels (columns per column tile of set_p2etc, gz3,
+ * calc_w and the Akima scheme's column pass, and the tile's threads; rows per
+ * meridional-advection tile and, where an order past del^4 is on, per
+ * zonal-hyperviscosity block and per column tile of the del^4 meridional
+ * second differences) over `steps` steps of the bucket's own members and keep
+ * the fastest.  A shape that no launch of the bucket reads stays as it was.
+ * The members' state is copied aside and put back, so the call changes no
+ * result and no state; it needs room for one copy of every member.  Writes one line per
+ * choice into report (up to cap bytes).  0 or a negative code. */
 int  epic_engine_autotune(epic_engine *e, int steps, char *report, int cap);
 /* One launch shape set by hand for every bucket (knob: 0 columns per
- * set_p2etc tile, 1 gz3, 2 calc_w, 3 vertical advection, 4 rows per
- * zonal-hyperviscosity block, 5 rows per meridional-advection tile, 6 rows
- * per column tile of the del^4 meridional second differences (8, 16, 32); a
- * column-tile value is C, 1000 n + C for blocks of 256 n threads, n = 2
- * or 4, or 10000 + C for one thread per level of each of the C columns; 0
- * restores the built-in choice).  Values outside the candidates the
- * autotuner tries, or whose LDS would not fit, are refused (-1).  For tests
- * that every shape gives the same bits. */
+ * set_p2etc tile, 1 gz3, 2 calc_w, 3 the Akima scheme's column pass, 4 rows
+ * per zonal-hyperviscosity block, 5 rows per meridional-advection tile, 6 rows
+ * per column tile of the del^4 meridional second differences (8, 16, 32); 0
+ * restores the built-in choice).  A column-tile value names C columns and N
+ * threads: C for 256 threads, 1000 n + C for 256 n (n = 2 or 4), 10000 + C for
+ * one thread per level of each of the C columns.  The Akima pass's block has N
+ * threads; in the other three a thread takes 2, 4 or 8 levels, the fewest with
+ * which N threads cover the columns (8 where they cannot), and the block has
+ * the threads that this needs.  Values outside the candidates the autotuner
+ * tries, or whose LDS would not fit, are refused (-1).  For tests that every
+ * shape gives the same bits. */
 int  epic_engine_set_shape(epic_engine *e, int knob, int value);
 const char *epic_engine_last_error(epic_engine *e);
 

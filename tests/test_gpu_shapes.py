@@ -88,3 +88,21 @@ def test_shapes_belong_to_buckets_of_the_same_kernels():
     e.add(PLAIN)
     assert report(e)["rows_zhv"] == "8 (not launched)"
     e.close()
+
+
+def test_the_report_names_the_threads_that_are_launched():
+    """set_p2etc, gz3 and calc_w give a thread 2, 4 or 8 of a column's 20
+    levels (10, 5 or 3 threads a column); the Akima column pass has 256, 512 or
+    1024 threads, or one for each of 22 levels."""
+    say("threads in the report")
+    e = engine(OTHER)
+    for knob, text in report(e).items():
+        if not knob.startswith("cols_") or text.startswith("built-in"):
+            continue
+        c, threads = text.split()[0].removesuffix("thr").split("/")
+        c, threads = int(c), int(threads)
+        if knob == "cols_hsuv":
+            assert threads in (256, 512, 1024, 22 * c), (knob, text)
+        else:
+            assert threads in (10 * c, 5 * c, 3 * c), (knob, text)
+    e.close()
