@@ -432,6 +432,14 @@ int member_check(const epic_case *c, int precision, char *err, size_t cap) {
     snprintf(err, cap, "k_sponge=%d outside 0..nk-1", c->k_sponge);
     return -1;
   }
+  // theta is prognostic from interface k_sigma-1 down: at least the bottom two
+  // interfaces (the 3-D filter's profile of theta has an entry for each, and
+  // the reference's spline refuses fewer than two), and not the top one,
+  // above which there is no level for the advection's stencils to read
+  if (c->k_sigma < 2 || c->k_sigma > c->nk) {
+    snprintf(err, cap, "k_sigma=%d outside 2..nk", c->k_sigma);
+    return -1;
+  }
   if (precision != EPIC_FP64 && precision != EPIC_MIXED) {
     snprintf(err, cap, "unknown precision mode %d", precision);
     return -1;

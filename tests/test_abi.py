@@ -135,3 +135,26 @@ def test_case_builder_through_the_binding():
         assert ts[0] == 1.0 / (30.0 * 60) and ts[2] == 0.0 and 0 < ts[1] < ts[0]
     finally:
         ea.free_case(c)
+
+
+@pytest.mark.parametrize("k_sigma,ok", [(-1, False), (0, False), (1, False), (2, True), (6, True), (10, True),
+                                        (11, False), (12, False)])
+def test_k_sigma_outside_the_column_is_refused(k_sigma, ok):
+    """k_sigma is 2..nk (here nk = 10): the kernels would read levels outside
+    the column for others.  The configuration is checked before any device
+    memory is looked at, so the null field table below is what stops a call
+    with a good one."""
+    fn = ea.lib().epic_step_noalloc
+    fn.restype = ctypes.c_int
+    c = ea.build_case(ea.spec(ea.HELD_SUAREZ, 16, 8, 10))
+    try:
+        c.k_sigma = k_sigma
+        fields = (ctypes.c_void_p * len(ea.FIELDS))()
+        it = (ctypes.c_int * 4)(0, 1, 2, 0)
+        err = ctypes.create_string_buffer(256)
+        rc = fn(ctypes.byref(c), fields, it, ctypes.c_int(ea.SYNC_DIAGS_ONLY), ctypes.c_int(0), None, err,
+                ctypes.c_size_t(256))
+    finally:
+        ea.free_case(c)
+    assert rc == -1
+    assert err.value.decode() == ("field 0 has no device array" if ok else f"k_sigma={k_sigma} outside 2..nk")
