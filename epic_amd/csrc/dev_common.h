@@ -54,8 +54,8 @@ struct MemberDesc {
   int ni, nj, nk, Ia, N2, N3;
   int ks, k_sponge;  // k_sigma, k_sponge
   int is_hs, is_gas, newt_cool_on, newt_cool_adjust, drag_v, drag_zonal_avg, jtp;
-  int nrow_h, nrow_v, nlogn;  // filtered rows (h- and v-grid), log2(ni)
-  int mixed;                  // precision mode
+  int nlogn;  // log2(ni)
+  int mixed;  // precision mode
   double dt, kappa, cp, cpr, rgas, press0, zeta0, zeta1, alpha, sigma_sigma;
   double topo_scale, prandtl, tau_drag;
   double coef2, coef4, nu4, m0z, nudiv, eps13, mu3, mu2, g_coeff;
@@ -93,7 +93,6 @@ struct MemberDesc {
   gptr<const double> mn_inv, hl_h, hl_pv, hcx, hcy, hcz, vcx, vcy, vcz;
   gptr<const double> tw_f, tw_i, tr_f, tr_i;  // four1 / realft twiddles, forward and inverse
   gptr<const float> tw_f32, tw_i32, tr_f32, tr_i32;
-  gptr<const int> rows_h, rows_v;
   gptr<const int> rflag_h, rflag_v;  // 1 where row J is in the filter band
   // state and diagnostics
   gptr<double> U, V, DUDT, DVDT, HDRY, THETA, P3, P2, THETA2, H3, T2, T3, RHO2, RHO3;
@@ -425,26 +424,6 @@ __device__ __forceinline__ bool table_well_separated(int n, const double *x, int
   return !__any(close);
 }
 
-// strided variant: table entries at x[k*stride]
-__device__ __forceinline__ int table_place_s(int n, const double *x, int st, double xx, double *dx) {
-  int il = -1, iu = n;
-  int ascend = (x[(n - 1) * st] >= x[0]);
-  int lo = fcmp_d(xx, x[0]), hi = fcmp_d(xx, x[(n - 1) * st]);
-  if (ascend) {
-    if (lo <= 0) { *dx = x[st] - x[0]; return 0; }
-    if (hi >= 0) { *dx = x[(n - 1) * st] - x[(n - 2) * st]; return n - 2; }
-  } else {
-    if (lo >= 0) { *dx = x[st] - x[0]; return 0; }
-    if (hi <= 0) { *dx = x[(n - 1) * st] - x[(n - 2) * st]; return n - 2; }
-  }
-  while (iu - il > 1) {
-    int im = (iu + il) >> 1;
-    if ((fcmp_d(xx, x[im * st]) >= 0) == ascend) il = im; else iu = im;
-  }
-  *dx = x[(il + 1) * st] - x[il * st];
-  return il;
-}
-
 // Barrier among the lanes of one wavefront (LDS traffic of a single wave is
 // ordered; the fences keep the compiler from moving accesses across it).
 __device__ __forceinline__ void wave_sync() {
@@ -528,22 +507,6 @@ __device__ __forceinline__ double *fld_ptr(const MemberDesc &d, int f) {
     // the mixed mode keeps one FP64 plane for the current step's tendency
     case F_DUDT_T: return d.mixed ? d.DUDT : d.DUDT + (size_t)d.dyn->it0 * d.N3;
     case F_DVDT_T: return d.mixed ? d.DVDT : d.DVDT + (size_t)d.dyn->it0 * d.N3;
-  }
-  return nullptr;
-}
-
-// FP32 views used by the mixed mode: the tendency planes and the scratch
-// arrays (an FP32 view of a scratch array uses the first half of its bytes)
-template <class T> __device__ __forceinline__ T *fld_ptr_t(const MemberDesc &d, int f);
-template <> __device__ __forceinline__ double *fld_ptr_t<double>(const MemberDesc &d, int f) { return fld_ptr(d, f); }
-template <> __device__ __forceinline__ float *fld_ptr_t<float>(const MemberDesc &d, int f) {
-  switch (f) {
-    case F_DUDT_T: return d.DUDTf + (size_t)d.dyn->it0 * d.N3;
-    case F_DVDT_T: return d.DVDTf + (size_t)d.dyn->it0 * d.N3;
-    case F_SA: return reinterpret_cast<float *>(d.sA.get());
-    case F_SB: return reinterpret_cast<float *>(d.sB.get());
-    case F_SC: return reinterpret_cast<float *>(d.sC.get());
-    case F_SD: return reinterpret_cast<float *>(d.sD.get());
   }
   return nullptr;
 }

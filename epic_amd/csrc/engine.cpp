@@ -368,9 +368,10 @@ extern "C" size_t epic_engine_bytes_in_use(epic_engine *E) { return E ? E->in_us
 // Upload a case into a free slot.  hdry_src: the prognostic h of the caller
 // (nullptr: reconstitute it from p3 as epic_main does).  prime: run the
 // SYNC_DIAGS_ONLY sequence for the new member.
-// Host copies of the device's fcmp_d / table_place_s (dev_common.h), for
-// searches whose table and argument are the same in every column: the
-// index (and interval width) is formed once here, by the same operations.
+// Host copies of the device's fcmp_d and table_place (dev_common.h), the
+// table's entries st apart, for searches whose table and argument are the same
+// in every column: the index (and interval width) is formed once here, by the
+// same operations.
 static int fcmp_host(double x1, double x2) {
   int e;
   frexp(fabs(x1) > fabs(x2) ? x1 : x2, &e);
@@ -542,8 +543,6 @@ void member_plan(const epic_case *c, bool mixed, const epic_tables &T, MemberDes
   add(&d.tw_i32, sizeof(float) * T.n_tw, hold.twi32.data());
   add(&d.tr_f32, sizeof(float) * T.n_tr, hold.trf32.data());
   add(&d.tr_i32, sizeof(float) * T.n_tr, hold.tri32.data());
-  add(&d.rows_h, sizeof(int) * (c->nj + 2), T.rows_h);
-  add(&d.rows_v, sizeof(int) * (c->nj + 2), T.rows_v);
   hold.flag_h.assign(c->nj + 2, 0);
   hold.flag_v.assign(c->nj + 2, 0);
   for (int r = 0; r < T.nrow_h; r++) hold.flag_h[T.rows_h[r]] = 1;
@@ -608,7 +607,6 @@ void member_plan(const epic_case *c, bool mixed, const epic_tables &T, MemberDes
   }
   d.newt_cool_on = c->newt_cool_on; d.newt_cool_adjust = c->newt_cool_adjust;
   d.drag_v = c->drag_v; d.drag_zonal_avg = c->drag_zonal_avg; d.jtp = c->jtp;
-  d.nrow_h = T.nrow_h; d.nrow_v = T.nrow_v;
   int lg = 0;
   while ((1 << lg) < c->ni) lg++;
   d.nlogn = lg;

@@ -120,7 +120,7 @@ __device__ int pchip_wave(int n, const double *x, const double *y, double *dd, i
   const int f = fs.f[fi], kind = fs.kind[fi]
 
 // F: the mixed mode's exp/log (m_exp)
-template <class T, bool F>
+template <bool F>
 __global__ void __launch_bounds__(256) k_spline_prep(const MemberDesc *D, int mb, int nm, FieldSet fs) {
   SET_MEMBER;
   F3 r = f3_range(d, kind);
@@ -148,11 +148,11 @@ __global__ void __launch_bounds__(256) k_spline_prep(const MemberDesc *D, int mb
     }
   }
   const int Imin = (bi == 0x7fffffff) ? 1 : bi;
-  const T *b = fld_ptr_t<T>(d, f);
+  const double *b = fld_ptr(d, f);
   for (int e = lane; e < n; e += 64) {
     const int K = r.kend - e;
     sx[e] = geez(d, kind, K, J, Imin);
-    double v = (double)b[ix3(d, K, J, Imin)];
+    double v = b[ix3(d, K, J, Imin)];
     sy[e] = (kind == 2) ? m_log<F>(v) : v;
   }
   wave_sync();
@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(256) k_spline_prep(const MemberDesc *D, int mb
 // band come out as (a - v) + v, as in the reference, which subtracts and adds
 // the profile on every row.  HDRY is stored with the restore_mass that
 // follows the filters in the step.  RB rows per block, ni/4 lanes per row.
-template <bool WIDE, class T, bool F>
+template <bool WIDE, bool F>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k_filter3(const MemberDesc *D, int mb, int nm, FieldSet fs) {
   SET_MEMBER;
   extern __shared__ double lds_raw[];
@@ -194,12 +194,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
   const bool filt = live && (vg ? d.rflag_v[J] : d.rflag_h[J]);
   const int KT = d.nk + 2, nt = r.kend - r.kstart + 1;
   double *tab = tabs + (size_t)rs * 5 * KT;
-  T *buf = reinterpret_cast<T *>(tabs + (size_t)RB * 5 * KT) + (size_t)rs * n;
+  double *buf = tabs + (size_t)RB * 5 * KT + (size_t)rs * n;
   // the lane's four points and their filtered geopotential, on their way
   // while the row's table is set up
-  const Plane<T> a{fld_ptr_t<T>(d, f) + (size_t)K * d.N2};
-  double xx[4];
-  T x[4];
+  const Plane<double> a{fld_ptr(d, f) + (size_t)K * d.N2};
+  double xx[4], x[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     const int I = lane + q * nq + 1;
@@ -234,7 +233,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
       double val = ty[k] + xr * (tz[k] + xr * (tc2[k] + xr * tc3[k]));
       if (kind == 2) val = m_exp<F>(val);
       v[q] = val;
-      x[q] = T((double)x[q] - val);
+      x[q] -= val;
     }
   if (filter_any<WIDE>(filt)) filter_row_regs<WIDE>(d, x, buf, J, vg, filt, lane);
   // hdry leaves with restore_mass applied (max(h_min, h), every cell of
@@ -244,8 +243,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int e = lane + q * nq;
-      T out = T((double)x[q] + v[q]);
-      if (kind == 2) out = T(dmax(hmin, (double)out));
+      double out = x[q] + v[q];
+      if (kind == 2) out = dmax(hmin, out);
       a[ix2(d, J, e + 1)] = out;
       if (e == n - 1) a[ix2(d, J, 0)] = out;
       if (e == 0) a[ix2(d, J, n + 1)] = out;
@@ -256,13 +255,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 // cover 0..nj and the kernels drop the rows outside the kind's range)
 void L_filter3(hipStream_t s, const Bucket &b, const FieldSet &fs) {
   const int nrow = b.nj + 1, nz = fs.n * b.nm;
-  if (b.mixed) LAUNCH_AS("k_spline_prep<double>", (k_spline_prep<double, true>), dim3(nrow, 1, nz), dim3(64), 0, s, b.D, b.mb, b.nm, fs);
-  else LAUNCH_AS("k_spline_prep<double>", (k_spline_prep<double, false>), dim3(nrow, 1, nz), dim3(64), 0, s, b.D, b.mb, b.nm, fs);
+  if (b.mixed) LAUNCH_AS("k_spline_prep", k_spline_prep<true>, dim3(nrow, 1, nz), dim3(64), 0, s, b.D, b.mb, b.nm, fs);
+  else LAUNCH_AS("k_spline_prep", k_spline_prep<false>, dim3(nrow, 1, nz), dim3(64), 0, s, b.D, b.mb, b.nm, fs);
   const int nq = b.ni / 4, RB = (256 / nq) < 16 ? (256 / nq) : 16;
   dim3 g((nrow + RB - 1) / RB, b.nk, nz);
   size_t shm = sizeof(double) * (size_t)RB * 5 * (b.nk + 2) + sizeof(double) * (size_t)RB * b.ni;
-  if (b.mixed) ROWS_LAUNCH(b, "k_filter3<double>", (k_filter3<true, double, true>), (k_filter3<false, double, true>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
-  else ROWS_LAUNCH(b, "k_filter3<double>", (k_filter3<true, double, false>), (k_filter3<false, double, false>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
+  if (b.mixed) ROWS_LAUNCH(b, "k_filter3", (k_filter3<true, true>), (k_filter3<false, true>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
+  else ROWS_LAUNCH(b, "k_filter3", (k_filter3<true, false>), (k_filter3<false, false>), g, dim3(RB * nq), shm, s, b.D, b.mb, b.nm, fs);
 }
 
 }  // namespace epic
