@@ -106,3 +106,42 @@ def test_the_report_names_the_threads_that_are_launched():
         else:
             assert threads in (10 * c, 5 * c, 3 * c), (knob, text)
     e.close()
+
+
+# 35 rows (36 on the v grid) and 13 levels: a remainder over every tile
+ODD = dict(ni=64, nj=34, nk=13, dt=60)
+BY_KERNEL = {
+    # the Akima scheme's column pass and its meridional tile
+    "akima_cols": ("cols_hsuv", (16, 32, 64, 2032, 4064, 10004, 10012), dict(adv_mass=1, adv_nonmass=1)),
+    "akima_rows": ("rows_mer", (2, 4, 8), dict(adv_mass=1, adv_nonmass=1)),
+    # the predictor-corrector's meridional pass, a template instance each
+    "hsu_rows": ("rows_mer", (2, 4, 8), {}),
+    # the separate hyperviscosity kernels, which orders past del^4 take
+    "del8_zonal": ("rows_zhv", (4, 8, 16), dict(nu4=0.0, nu8=0.5)),
+    "del8_meridional": ("rows_d2", (8, 16, 32), dict(nu4=0.0, nu8=0.5)),
+    "del6_zonal": ("rows_zhv", (4, 8, 16), dict(nu4=0.25, nu6=0.2)),
+}
+
+
+@pytest.mark.parametrize("precision", [ea.FP64, ea.MIXED])
+@pytest.mark.parametrize("name", sorted(BY_KERNEL))
+def test_every_shape_of_a_kernel_gives_the_same_bits(name, precision):
+    """Each candidate on a member whose step launches the kernel that reads
+    it (the report's time shows that it does)."""
+    knob, values, opt = BY_KERNEL[name]
+    sp = ea.spec(ea.JUPITER_LIKE, ODD["ni"], ODD["nj"], ODD["nk"], ODD["dt"], seed=9,
+                 **dict(dict(nu4=0.5, noise_theta=0.0, noise_uv=0.5), **opt))
+    e = engine(sp, precision=precision)
+    assert report(e)[knob].endswith(" us/step)")
+    e.close()
+    out = {}
+    for v in (0,) + values:
+        say(name, precision, v)
+        e = engine(sp, precision=precision)
+        e.set_shape(knob, v)
+        e.step(3)
+        out[v] = {f: e.read(0, f).tobytes() for f in ea.FIELDS if f[:4] not in ("DUDT", "DVDT")}
+        e.sync()
+        e.close()
+    bad = [(v, f) for v in values for f in out[0] if out[v][f] != out[0][f]]
+    assert not bad
