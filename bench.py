@@ -74,10 +74,13 @@ KERNEL_BYTES = {
     # del^4 in one launch: a field read once and written once
     "k_hv4": (16, 2),
     # uv_core reads u, v, h3, pv, w3 and writes du, dv; the pressure gradient
-    # reads gz3, p2, rho3 and adds to du, dv; the Adams-Bashforth update reads
-    # six tendency planes, u, v and writes u, v, and finishes dzdt3 from gz3,
-    # w3, h3, rho3
-    "k_uv_core": (56, 1), "k_pgrad": (56, 1), "k_ab": (128, 1),
+    # reads gz3, p2, rho3 and adds to du, dv; the Adams-Bashforth update
+    # <mixed, in place> reads six tendency planes, u, v and writes u, v (mixed:
+    # two planes in FP64 and four in FP32, and writes two in FP32), and, where
+    # it is out of place, finishes dzdt3 from gz3, w3, h3, rho3 (48 bytes)
+    "k_uv_core": (56, 1), "k_pgrad": (56, 1),
+    "k_ab<false, true>": (80, 1), "k_ab<true, true>": (72, 1),
+    "k_ab<false, false>": (128, 1), "k_ab<true, false>": (120, 1),
     "k_divdamp": (40, 1), "km_divdamp": (40, 1), "k_gz_mono": (16, 1),
     "k_heating": (24, 1), "k_hs_pbl": (32, 1), "k_divergence": (24, 1), "k_store_diag": (40, 1),
 }

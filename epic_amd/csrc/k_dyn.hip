@@ -609,10 +609,10 @@ bool ab_dzdt3_fused(const Bucket &b) { return hv_fused(b); }
 void L_ab(hipStream_t s, const Bucket &b) {
   const bool all = ab_dzdt3_fused(b);
   const dim3 g = grid2(b.nj + 1, b.ni, all ? b.nk : b.nk - 1, b.nm);
-  if (all && b.mixed) LAUNCH_AS("k_ab", (k_ab<true, false>), g, dim3(TPB), 0, s, b.D, b.mb);
-  else if (all) LAUNCH_AS("k_ab", (k_ab<false, false>), g, dim3(TPB), 0, s, b.D, b.mb);
-  else if (b.mixed) LAUNCH_AS("k_ab", (k_ab<true, true>), g, dim3(TPB), 0, s, b.D, b.mb);
-  else LAUNCH_AS("k_ab", (k_ab<false, true>), g, dim3(TPB), 0, s, b.D, b.mb);
+  if (all && b.mixed) LAUNCH_AS("k_ab<true, false>", (k_ab<true, false>), g, dim3(TPB), 0, s, b.D, b.mb);
+  else if (all) LAUNCH_AS("k_ab<false, false>", (k_ab<false, false>), g, dim3(TPB), 0, s, b.D, b.mb);
+  else if (b.mixed) LAUNCH_AS("k_ab<true, true>", (k_ab<true, true>), g, dim3(TPB), 0, s, b.D, b.mb);
+  else LAUNCH_AS("k_ab<false, true>", (k_ab<false, true>), g, dim3(TPB), 0, s, b.D, b.mb);
 }
 
 // monotone filtered geopotential, K = nk-1 down to 0 (src/shared/epic_timestep.c:176-196)

@@ -65,3 +65,12 @@ def test_reference_cpu_leg_times_the_reference_build():
     v, n, el = bench.cpu_baseline_reference(ea.HELD_SUAREZ, 32, 16, 8, 600, 0.5)
     assert n >= 2 and el > 0
     assert abs(v - 32 * 17 * 8 * n / el) < 1e-6 * v
+
+
+def test_kernel_bytes_of_the_adams_bashforth_forms():
+    """u and v read and written and six tendency planes read are 80 bytes a
+    cell; the mixed mode's FP32 history takes 8 off (four planes read at half
+    the size, two written); DZDT3 in the same launch adds six arrays."""
+    cells = 256 * 129 * 20
+    got = [bench.kernel_bytes(f"k_ab<{m}, {f}>", 256, 128, 20, 1) for m in ("false", "true") for f in ("true", "false")]
+    assert got == [80 * cells, 128 * cells, 72 * cells, 120 * cells]
