@@ -2,7 +2,9 @@
 algorithmic bytes of a launch, the lookup of the committed counter
 summaries (including kernels whose launch name hides template arguments)
 and the CPU baseline's run of the reference build."""
+import json
 import os
+import re
 import subprocess
 import sys
 
@@ -74,3 +76,34 @@ def test_kernel_bytes_of_the_adams_bashforth_forms():
     cells = 256 * 129 * 20
     got = [bench.kernel_bytes(f"k_ab<{m}, {f}>", 256, 128, 20, 1) for m in ("false", "true") for f in ("true", "false")]
     assert got == [80 * cells, 128 * cells, 72 * cells, 120 * cells]
+
+
+STEP_KERNELS = ["k_set_p2etc<0>", "k_set_p2etc<1>", "k_thermo", "k_gz3", "k_calc_w", "k_hsu_vert<T>", "k_hsu_mer<T>",
+                "k_hsu_zonal<T>", "k_filter3", "k_hv4", "k_uv_core", "k_pgrad", "k_store_diag", "k_gz_mono"]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("workload", ["jupiter_256x128x20", "jupiter_ensemble_64x128x64x16", "hot_jupiter_1024x512x64"])
+def test_traffic_summaries_hold_the_kernels_of_the_step(workload, precision):
+    """Every kernel that a step of the workload launches is found under its
+    launch name, with the dispatches of one run; a row of another run or of an
+    earlier build says so."""
+    for name in STEP_KERNELS + [f"k_ab<{'true' if precision == 'mixed' else 'false'}, false>"]:
+        t, _ = bench.measured_traffic(workload, precision, name)
+        assert t and t > 0, name
+    with open(os.path.join(ROOT, "profiles", f"traffic_{workload}_{precision}.json")) as f:
+        summary = json.load(f)
+    assert summary["build"]
+    src = "".join(open(os.path.join(ROOT, "epic_amd", "csrc", n)).read()
+                  for n in os.listdir(os.path.join(ROOT, "epic_amd", "csrc")) if n.endswith(".hip"))
+    rows = summary["kernels"]
+    once = next(v["dispatches"] for n, v in rows.items() if n.startswith("k_uv_core"))
+    for name, row in rows.items():
+        base = name.split("<")[0]
+        if "build" in row:
+            continue
+        assert re.search(rf"\b{base}\(const MemberDesc", src), name
+        # the workloads run del^4, whose one kernel is k_hv4
+        assert ("run" in row) == (base in ("k_hv_apply", "k_zonal_hv", "k_d2dy2_cols", "k_d2dy2_pass")), name
+        if base == "k_hv4":
+            assert row["dispatches"] == 2 * once
