@@ -30,8 +30,8 @@
 // The reference keeps its column work arrays in statics across calls: the
 // theta call starts at K = k_sigma-1 and reads wm[k_sigma-2] and
 // w_a[k_sigma-3] as left by the last column (J = nj, I = ni+1) of the
-// preceding unity call.  Both are functions of W3 and of unity before its
-// advection (1 everywhere), so the theta blocks form them themselves.
+// preceding unity call.  w_a is unity before its advection, 1 everywhere; wm
+// meets the predicted change behind that face, which is 0 there.
 #include "kernels.h"
 #include "filter_row.h"
 
